@@ -10,9 +10,9 @@
 // This file keeps those phases but maps them to the GPU as follows.
 //
 // Column tiers (by flop_j, after sorting columns by flop descending):
-//   hash tier  flop_j <= small_flop_max: one workgroup per column with an LDS
-//              linear-probing hash table of 2^ceil(log2(2*size)) slots, then
-//              in-LDS compaction and a bitonic sort of the surviving rows.
+//   hash tier  flop_j <= small_flop_max: one workgroup per column; the rows
+//              are counted in an LDS linear-probing hash table, and the
+//              products sorted by row in LDS (k_num_sort).
 //   dense tier the rest: one workgroup per column walks the rows in tiles of
 //              TR rows; each tile accumulates into a dense LDS array with a
 //              presence bitmap and is emitted in row order by a block scan
@@ -911,12 +911,27 @@ __global__ __launch_bounds__(NT) void k_sym_dense(const int32_t* __restrict__ or
   if (threadIdx.x == 0) nnzcol[col] = tot;
 }
 
-// ---------------------------------------------------------- numeric: hash
-// Hash accumulation (mtSpGEMM.h:362-423 / :595-622), compaction (:425-432)
-// and sort by row (:434); SORT=false keeps hash order like LocalSpGEMMHash
-// with sort=false (:624-634).
-template <int K, class T, int HMAX, int NT, bool SORT>
-__global__ __launch_bounds__(NT) void k_num_hash(const int32_t* __restrict__ order, int64_t first,
+// ---------------------------------------------------------- numeric: sort
+// Columns with tiny_flop < flop_j <= 4 * NT products, one workgroup each:
+// the heap / hash accumulation and sort of mtSpGEMM.h:311-440 as a radix sort
+// of the products.  Every thread gathers four products into registers; their
+// rows are sorted in LDS with the product's number as payload (least
+// significant digit first, at most 7 bits a pass, over the bits in which the
+// column's rows differ); the heads of equal rows, numbered by a block scan,
+// give every product its rank, and the products then accumulate from the
+// registers at vals[rank].  Rows and values leave in rank order, coalesced.
+//
+// A digit pass ranks 64 keys at a time by wave ballots: every wave counts its
+// own 256 keys, so the pass needs one block scan over (digit, wave) and no
+// atomics.  At R-MAT s19 ef16 (int64) the columns of 1025 to 4096 products
+// take 3.2 ms and the smaller ones 0.35 ms; a hash table with LDS compaction
+// and a bitonic sort took 17.3 ms (one 119 KB workgroup per CU, 78 barriers a
+// sort) and 1.2 ms.  Bound by VALU (the ballots) and LDS; 60 KB at 1024
+// threads: two workgroups per CU, all 32 waves.  The workgroup has a quarter
+// of the tier's product bound in threads, so that none idles: bounds of 1024,
+// 2048 and 4096 products.
+template <int K, class T, int NT>
+__global__ __launch_bounds__(NT) void k_num_sort(const int32_t* __restrict__ order, int64_t first,
                                                  const int64_t* __restrict__ nnzcol, const int64_t* __restrict__ cpB,
                                                  const int32_t* __restrict__ bpos, const T* __restrict__ valB,
                                                  const int64_t* __restrict__ cpA, const int32_t* __restrict__ rowsA,
@@ -925,119 +940,209 @@ __global__ __launch_bounds__(NT) void k_num_hash(const int32_t* __restrict__ ord
                                                  int* __restrict__ err, Filter<T> flt = {}) {
   using SR = Sem<K, T>;
   using Acc = typename SR::Acc;
-  __shared__ int32_t keys[HMAX];
-  __shared__ Acc acc[HMAX];
-  __shared__ long long wsum[NT / kWave];
-  __shared__ SegStage<T, NT> st;
+  constexpr int U = 4, CAP = U * NT, NW = NT / kWave;
+  constexpr int kDigit = 7;  // bits per pass at most: 128 * NW 16-bit counters, two per thread
+  static_assert((1 << kDigit) * NW == 2 * NT, "one pair of counters per thread");
+  union Window {
+    SegStage<T, NT> st;  // while the products are gathered
+    Acc vals[CAP];       // once their ranks are known
+  };
+  __shared__ __align__(16) uint32_t keys[CAP];
+  __shared__ __align__(8) uint16_t pay[CAP];  // product numbers, then the products' ranks
+  __shared__ uint32_t hist32[NT];
+  __shared__ __align__(16) unsigned char window_mem[sizeof(Window)];
+  __shared__ long long wsum[NW];
+  __shared__ int isum[NW];
+  Window& win = *reinterpret_cast<Window*>(window_mem);
+  uint16_t* hist = reinterpret_cast<uint16_t*>(hist32);
+  const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
   const int col = order[first + blockIdx.x];
-  const int64_t nz = nnzcol[col];
-  const int lg = min(ceil_log2_dev(max(2 * nz, 64ll)), ceil_log2_dev(HMAX));
-  const int H = 1 << lg;
-  for (int i = threadIdx.x; i < H; i += NT) {
-    keys[i] = -1;
-    acc[i] = SR::ident();
-  }
-  __syncthreads();
   const int64_t b0 = cpB[col], b1 = cpB[col + 1];
+  // products tid * U .. tid * U + U - 1 of the column
+  uint32_t key[U], num[U];
+  Acc prod[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    key[u] = 0;
+    num[u] = (uint32_t)(tid * U + u);
+    prod[u] = SR::ident();
+  }
+  int total = 0;
   for (int64_t eb = b0; eb < b1; eb += NT) {
     int64_t base;
     int len, nseg;
     T bv;
-    load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, nullptr, 0, 0, 0, true, valB, base, len, bv);
-    const int tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
-    visit_staged<T, NT, 4>(st, nseg, tot, [&](const int64_t(&idx)[4], const T(&bvs)[4]) {
-      int32_t rr[4];
-      T aa[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        rr[u] = -1;
-        if (idx[u] >= 0) {
-          rr[u] = rowsA[idx[u]];
-          aa[u] = valA[idx[u]];
-        }
+    load_seg<T, true>(eb + tid, b1, bpos, cpA, nullptr, 0, 0, 0, true, valB, base, len, bv);
+    const int tot = stage_chunk<T, NT>(win.st, wsum, base, len, bv, nseg);
+    const int x0 = tid * U - total;  // this chunk's number of the thread's first product
+    if (x0 + U > 0 && x0 < tot) {
+      const int xf = max(x0, 0);
+      int lo = 0, hi = nseg;  // largest k with off[k] <= xf
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (win.st.off[mid] <= xf) lo = mid;
+        else hi = mid;
       }
+      int k = lo, cur = win.st.off[k], nxt = win.st.off[k + 1];
+      int64_t idx[U];
+      T bvs[U];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int32_t r = rr[u];
-        if (r < 0) continue;
-        const Acc v = SR::mul(aa[u], bvs[u]);
-        uint32_t h = hash_slot(r, lg);
-        int probe = 0;
-        for (; probe < H; ++probe) {  // the table is at least twice the column's nnz
-          const int32_t old = atomicCAS(&keys[h], -1, r);
-          if (old == -1 || old == r) break;
-          h = (h + 1) & (H - 1);
-        }
-        if (probe < H) SR::acc(&acc[h], v);
-        else atomicOr(err, 2);
-      }
-    });
-  }
-  __syncthreads();
-  // in-place compaction, NT slots at a time
-  int base = 0;
-  for (int c0 = 0; c0 < H; c0 += NT) {
-    const int i = c0 + threadIdx.x;
-    const int32_t k = i < H ? keys[i] : -1;
-    const Acc a = i < H ? acc[i] : SR::ident();
-    long long tot;
-    const int ex = (int)block_excl_scan_ll<NT>(k != -1 ? 1 : 0, wsum, tot);
-    if (k != -1) {
-      keys[base + ex] = k;
-      acc[base + ex] = a;
-    }
-    base += tot;
-    __syncthreads();
-  }
-  if (base != nz && threadIdx.x == 0) atomicOr(err, 8);
-  const int cnt = min(base, (int)nz);
-  if constexpr (SORT) {
-    int N = 1;
-    while (N < cnt) N <<= 1;
-    for (int i = cnt + threadIdx.x; i < N; i += NT) keys[i] = 0x7fffffff;
-    __syncthreads();
-    for (int k = 2; k <= N; k <<= 1) {
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        for (int i = threadIdx.x; i < N; i += NT) {
-          const int ixj = i ^ j;
-          if (ixj > i) {
-            const int32_t ki = keys[i], kx = keys[ixj];
-            const bool up = (i & k) == 0;
-            if ((ki > kx) == up) {
-              keys[i] = kx;
-              keys[ixj] = ki;
-              const Acc t = acc[i];
-              acc[i] = acc[ixj];
-              acc[ixj] = t;
-            }
+      for (int u = 0; u < U; ++u) {
+        const int x = x0 + u;
+        idx[u] = -1;
+        if (x >= 0 && x < tot) {
+          if (x >= nxt) {
+            ++k;
+            cur = nxt;
+            nxt = win.st.off[k + 1];
           }
+          idx[u] = win.st.base[k] + (x - cur);
+          bvs[u] = win.st.bval[k];
         }
-        __syncthreads();
       }
+      T a[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (idx[u] >= 0) {
+          key[u] = (uint32_t)rowsA[idx[u]];
+          a[u] = valA[idx[u]];
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (idx[u] >= 0) prod[u] = SR::mul(a[u], bvs[u]);
+    }
+    total += tot;
+  }
+  if (total > CAP) {  // the tier's bound keeps it below; guard anyway (uniform)
+    if (tid == 0) atomicOr(err, 2);
+    total = CAP;
+  }
+  // the bits in which the rows differ from the column's first
+  if (tid == 0) isum[0] = (int)key[0];
+  __syncthreads();
+  const uint32_t key0 = (uint32_t)isum[0];
+  uint32_t diff = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (tid * U + u < total) diff |= key[u] ^ key0;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) diff |= (uint32_t)__shfl_xor((int)diff, d, kWave);
+  __syncthreads();
+  if (lane == 0) isum[w] = (int)diff;
+  hist32[tid] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NW; ++i) diff |= (uint32_t)isum[i];
+  const int nbits = 32 - __clz((int)diff);  // 0 when every row is the same
+  const int npass = max(1, (nbits + kDigit - 1) / kDigit);
+  const int width = (nbits + npass - 1) / npass;
+  const uint32_t dmask = (1u << width) - 1u;
+  for (int p = 0, shift = 0; p < npass; ++p, shift += width) {
+    // in the first pass a wave's keys are those it gathered, later the sorted positions [256 w, 256 w + 256)
+    int rank[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool valid = p == 0 ? tid * U + u < total : (w * U + u) * kWave + lane < total;
+      const uint32_t d = (key[u] >> shift) & dmask;
+      unsigned long long same = __ballot(valid);
+      for (int b = 0; b < width; ++b) {
+        const bool bit = (d >> b) & 1u;
+        const unsigned long long m = __ballot(bit);
+        same &= bit ? m : ~m;
+      }
+      const int before = __popcll(same & ((1ull << lane) - 1ull));
+      uint16_t* h = &hist[d * NW + w];
+      int seen = 0;
+      if (valid) seen = *h;
+      wave_lds_sync();
+      if (valid && before == 0) *h = (uint16_t)(seen + __popcll(same));
+      wave_lds_sync();
+      rank[u] = valid ? seen + before : -1;
+    }
+    __syncthreads();
+    {
+      const uint32_t pair = hist32[tid];
+      const int c0 = (int)(pair & 0xffffu), c1 = (int)(pair >> 16);
+      int all;
+      const int ex = block_excl_scan<NT>(c0 + c1, isum, all);
+      hist32[tid] = (uint32_t)ex | ((uint32_t)(ex + c0) << 16);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (rank[u] >= 0) {
+        const int at = (int)hist[((key[u] >> shift) & dmask) * NW + w] + rank[u];
+        keys[at] = key[u];
+        pay[at] = (uint16_t)num[u];
+      }
+    __syncthreads();
+    if (p + 1 < npass) {
+      hist32[tid] = 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = (w * U + u) * kWave + lane;
+        key[u] = e < total ? keys[e] : 0u;
+        num[u] = pay[e];
+      }
+      __syncthreads();
     }
   }
+  // heads of equal rows among the thread's four sorted positions, and their numbers
+  uint32_t prev = tid > 0 && tid * U - 1 < total ? keys[tid * U - 1] : 0u;
+  bool head[U];
+  int heads = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int e = tid * U + u;
+    key[u] = e < total ? keys[e] : 0u;
+    num[u] = pay[e];
+    head[u] = e < total && (e == 0 || key[u] != prev);
+    prev = key[u];
+    heads += head[u];
+  }
+  int cnt;
+  int rk = block_excl_scan<NT>(heads, isum, cnt) - 1;  // its barriers: every position has been read
+  const int64_t nz = nnzcol[col];
+  if (cnt != nz && tid == 0) atomicOr(err, 8);
+  cnt = (int)min((int64_t)cnt, nz);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (tid * U + u >= total) continue;
+    rk += head[u];
+    if (head[u]) keys[rk] = key[u];  // the output rows
+    pay[num[u]] = (uint16_t)rk;
+  }
+  for (int i = tid; i < cnt; i += NT) win.vals[i] = SR::ident();
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (tid * U + u < total) {
+      const int q = pay[tid * U + u];
+      if (q < cnt) SR::acc(&win.vals[q], prod[u]);
+    }
+  __syncthreads();
   const int64_t out = cpC[col];
   if (!flt.on) {
-    for (int i = threadIdx.x; i < cnt; i += NT) {
-      irC[out + i] = keys[i];
-      valC[out + i] = SR::out(acc[i]);
+    for (int i = tid; i < cnt; i += NT) {
+      irC[out + i] = (int64_t)keys[i];
+      valC[out + i] = SR::out(win.vals[i]);
     }
     return;
   }
   int kept = 0;  // the fused threshold: the kept entries, in order, at out
   for (int c0 = 0; c0 < cnt; c0 += NT) {
-    const int i = c0 + threadIdx.x;
-    const T v = i < cnt ? SR::out(acc[i]) : T{};
+    const int i = c0 + tid;
+    const T v = i < cnt ? SR::out(win.vals[i]) : T{};
     const bool keep = i < cnt && !(v < flt.thr);
     long long tot;
     const int ex = (int)block_excl_scan_ll<NT>(keep ? 1 : 0, wsum, tot);
     if (keep) {
-      irC[out + kept + ex] = keys[i];
+      irC[out + kept + ex] = (int64_t)keys[i];
       valC[out + kept + ex] = v;
     }
     kept += (int)tot;
   }
-  if (threadIdx.x == 0) filter_add_run(flt, out, kept, col, err);
+  if (tid == 0) filter_add_run(flt, out, kept, col, err);
 }
 
 // --------------------------------------------------------- numeric: dense
@@ -3274,26 +3379,27 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   tmp_bytes = std::max(tmp_bytes, tmp2);
   CBX_HIP(hipcub::DeviceSelect::Flagged(nullptr, tmp2, B->jc, flags, (int64_t*)nullptr, nsel, (int)nzcB, s));
   tmp_bytes = std::max(tmp_bytes, tmp2);
-  CBX_HIP(hipcub::DeviceReduce::Sum(nullptr, tmp2, flop, bounds + 5, (int)nzcB, s));
+  CBX_HIP(hipcub::DeviceReduce::Sum(nullptr, tmp2, flop, bounds + 6, (int)nzcB, s));
   tmp_bytes = std::max(tmp_bytes, tmp2);
   void* tmp;
   CBX_TRY(dalloc(b_tmp, tmp_bytes, s, (uint8_t**)&tmp));
   CBX_HIP(hipcub::DeviceRadixSort::SortPairsDescending(tmp, tmp_bytes, flop, flop_s, order, order_s, (int)nzcB, 0, 64,
                                                        s));
-  CBX_HIP(hipcub::DeviceReduce::Sum(tmp, tmp_bytes, flop, bounds + 5, (int)nzcB, s));
+  CBX_HIP(hipcub::DeviceReduce::Sum(tmp, tmp_bytes, flop, bounds + 6, (int)nzcB, s));
 
   // class thresholds: units > small_max ; hash8k > mid ; hash2k > tiny ; tiny (one wave) > 0 ;
-  // large units possible > unit_split_nnz
-  int64_t hthr[5] = {cfg.small_flop_max, cfg.hash_mid_flop, cfg.tiny_flop, 0, cfg.unit_split_nnz};
+  // large units possible > unit_split_nnz ; 1024-thread sort > 2048
+  int64_t hthr[6] = {cfg.small_flop_max, cfg.hash_mid_flop, cfg.tiny_flop, 0, cfg.unit_split_nnz, 2048};
   CBX_HIP(hipMemcpyAsync(thr, hthr, sizeof(hthr), hipMemcpyHostToDevice, s));
-  k_class_bounds<<<1, 64, 0, s>>>(flop_s, nzcB, thr, 5, bounds);
-  int64_t hb[6];
+  k_class_bounds<<<1, 64, 0, s>>>(flop_s, nzcB, thr, 6, bounds);
+  int64_t hb[7];
   CBX_HIP(hipMemcpyAsync(hb, bounds, sizeof(hb), hipMemcpyDeviceToHost, s));
   CBX_HIP(hipMemsetAsync(nnzcol, 0, sizeof(int64_t) * (nzcB + 1), s));
   CBX_HIP(hipStreamSynchronize(s));
   const int64_t n_dense = hb[0], n_h8 = hb[1] - hb[0], n_h2 = hb[2] - hb[1], n_h256 = hb[3] - hb[2];
   const int64_t n_heavy_max = hb[4];  // columns whose flops (an upper bound of nnz) exceed unit_split_nnz
-  const int64_t total_flop = hb[5];
+  const int64_t total_flop = hb[6];
+  const int64_t n_s4k = std::min(n_h8, std::max<int64_t>(hb[5] - hb[0], 0));  // of n_h8, those above 2048 products
   // one workgroup per column (hash tiers, symbolic units): a dispatch holds
   // fewer than 2^32 work-items
   CBX_RETURN_IF(n_dense * 1024 >= (1ll << 32) || n_h8 * 1024 >= (1ll << 32) || n_h2 * kHashNT >= (1ll << 32),
@@ -3419,9 +3525,9 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   CBX_HIP(hipGetLastError());
   CBX_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, nnzcol, cpC, (int)(nzcB + 1), s));
   if (n_dense) {
-    CBX_HIP(hipMemsetAsync(bounds + 6, 0, sizeof(int64_t), s));
-    k_sum_ordered<<<nblk(n_dense, 256), 256, 0, s>>>(order_s, n_dense, nnzcol, (unsigned long long*)(bounds + 6));
-    CBX_HIP(hipMemcpyAsync(&nnz_main, bounds + 6, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    CBX_HIP(hipMemsetAsync(bounds + 7, 0, sizeof(int64_t), s));
+    k_sum_ordered<<<nblk(n_dense, 256), 256, 0, s>>>(order_s, n_dense, nnzcol, (unsigned long long*)(bounds + 7));
+    CBX_HIP(hipMemcpyAsync(&nnz_main, bounds + 7, sizeof(int64_t), hipMemcpyDeviceToHost, s));
   }
   CBX_HIP(hipMemcpyAsync(&nnzC, cpC + nzcB, sizeof(int64_t), hipMemcpyDeviceToHost, s));
   CBX_HIP(hipMemcpyAsync(hu, ucnt, sizeof(hu), hipMemcpyDeviceToHost, s));
@@ -3502,26 +3608,23 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   }
   tm.mark(4, s);
   }  // !learned_done
-  const bool sort = mode != CBX_SPGEMM_UNSORTED;
-#define CBX_LAUNCH_HASH(HM, HNT, NCOL, FIRST)                                                                     \
-  if (NCOL) {                                                                                                     \
-    if (sort)                                                                                                     \
-      k_num_hash<K, T, HM, HNT, true><<<(unsigned)(NCOL), HNT, 0, s>>>(                                           \
-          order_s, FIRST, nnzcol, B->cp, bpos, valB, A->cp, rowsA, valA, cpC, C->ir, (T*)C->val, err, flt);      \
-    else                                                                                                          \
-      k_num_hash<K, T, HM, HNT, false><<<(unsigned)(NCOL), HNT, 0, s>>>(                                          \
-          order_s, FIRST, nnzcol, B->cp, bpos, valB, A->cp, rowsA, valA, cpC, C->ir, (T*)C->val, err, flt);      \
-  }
-  // the 8192-slot table takes ~100 KB of LDS, so one workgroup per CU: give it 16 waves
-  CBX_LAUNCH_HASH(8192, 1024, n_h8, hb[0]);
-  CBX_LAUNCH_HASH(2048, kHashNT, n_h2, hb[1]);
+  // hash-tier columns by the products that a workgroup holds (four per thread)
+  if (n_s4k)
+    k_num_sort<K, T, 1024><<<(unsigned)n_s4k, 1024, 0, s>>>(order_s, hb[0], nnzcol, B->cp, bpos, valB, A->cp, rowsA,
+                                                            valA, cpC, C->ir, (T*)C->val, err, flt);
+  if (n_h8 - n_s4k)
+    k_num_sort<K, T, 512><<<(unsigned)(n_h8 - n_s4k), 512, 0, s>>>(order_s, hb[0] + n_s4k, nnzcol, B->cp, bpos, valB,
+                                                                  A->cp, rowsA, valA, cpC, C->ir, (T*)C->val, err,
+                                                                  flt);
+  if (n_h2)
+    k_num_sort<K, T, 256><<<(unsigned)n_h2, 256, 0, s>>>(order_s, hb[1], nnzcol, B->cp, bpos, valB, A->cp, rowsA, valA,
+                                                        cpC, C->ir, (T*)C->val, err, flt);
   if (n_h256 && tiny_staged)
     k_tiny_place<T><<<wave_grid(n_h256), 256, 0, s>>>(order_s, hb[2], n_h256, stage_off, nnzcol, cpC, stage_ir,
                                                        stage_val, C->ir, (T*)C->val, flt, err);
   else if (n_h256)
     launch_tiny<K, T, false>(cfg, order_s, hb[2], n_h256, B->cp, bpos, valB, A->cp, rowsA, valA, nnzcol, cpC, C->ir,
                              (T*)C->val, err, nullptr, s, flt);
-#undef CBX_LAUNCH_HASH
   CBX_HIP(hipGetLastError());
 
   if (flt.on) {  // the fused threshold's runs into the final arrays
