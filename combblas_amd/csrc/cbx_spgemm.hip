@@ -168,13 +168,24 @@ __device__ __forceinline__ void filter_add_run(const Filter<T>& f, int64_t src, 
   }
 }
 
-// Segment of B entry e restricted to P tiles [t_lo, t_hi) (or the whole A
+// Tile pointers of the unit tier: at[t * ncols + p] is the index of the first
+// entry of A's p-th stored column with row >= t * kBR (t = 0 .. S; the index
+// runs over all of A's entries).  Tile-major: the units in flight share a few
+// tiles (they are sorted by first block), so a look-up's lines stay in the
+// L2 caches (4 B per stored column and tile, 1.4 MB at R-MAT s19).  Stored
+// column by column, every look-up fetched a line of its own for two of its
+// words, and the column's start another.
+struct Tiles {
+  const int32_t* at = nullptr;
+  int64_t ncols = 0;
+};
+
+// Segment of B entry e restricted to tiles [t_lo, t_hi) (or the whole A
 // column when `full`).
 template <class T, bool VAL>
 __device__ __forceinline__ void load_seg(int64_t e, int64_t b1, const int32_t* __restrict__ bpos,
-                                         const int64_t* __restrict__ cpA, const int32_t* __restrict__ P, int S,
-                                         int t_lo, int t_hi, bool full, const T* __restrict__ valB, int64_t& base,
-                                         int& len, T& bv) {
+                                         const int64_t* __restrict__ cpA, const Tiles& P, int t_lo, int t_hi,
+                                         bool full, const T* __restrict__ valB, int64_t& base, int& len, T& bv) {
   base = 0;
   len = 0;
   bv = T{};
@@ -185,10 +196,9 @@ __device__ __forceinline__ void load_seg(int64_t e, int64_t b1, const int32_t* _
         base = cpA[p];
         len = (int)(cpA[p + 1] - base);
       } else {
-        const int32_t* pp = P + (int64_t)p * (S + 1);
-        const int a0 = pp[t_lo];
-        base = cpA[p] + a0;
-        len = pp[t_hi] - a0;
+        const int32_t a0 = P.at[t_lo * P.ncols + p];
+        base = a0;
+        len = P.at[t_hi * P.ncols + p] - a0;
       }
       if constexpr (VAL) bv = valB[e];
     }
@@ -376,7 +386,7 @@ __global__ __launch_bounds__(NT) void k_sym_hash(const int32_t* __restrict__ ord
     int64_t base;
     int len, nseg;
     uint8_t dummy;
-    load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, nullptr, 0, 0, 0, true, nullptr, base, len, dummy);
+    load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, Tiles{}, 0, 0, true, nullptr, base, len, dummy);
     const int tot = stage_chunk<uint8_t, NT>(st, wsum, base, len, 0, nseg);
     visit_staged<uint8_t, NT, 4>(st, nseg, tot, [&](const int64_t(&idx)[4], const uint8_t(&)[4]) {
       int32_t rr[4];
@@ -590,7 +600,7 @@ __device__ __forceinline__ int tiny_gather(int64_t b0, int64_t b1, const int32_t
     int64_t base;
     int len;
     T bv;
-    load_seg<T, !SYM>(eb + lane, b1, bpos, cpA, nullptr, 0, 0, 0, true, valB, base, len, bv);
+    load_seg<T, !SYM>(eb + lane, b1, bpos, cpA, Tiles{}, 0, 0, true, valB, base, len, bv);
     const int inc = wave_incl_scan(len);
     const int off = filled + inc - len;  // first element of this lane's segment
     const int total = __shfl(inc, kWave - 1, kWave);
@@ -972,7 +982,7 @@ __global__ __launch_bounds__(NT) void k_num_sort(const int32_t* __restrict__ ord
     int64_t base;
     int len, nseg;
     T bv;
-    load_seg<T, true>(eb + tid, b1, bpos, cpA, nullptr, 0, 0, 0, true, valB, base, len, bv);
+    load_seg<T, true>(eb + tid, b1, bpos, cpA, Tiles{}, 0, 0, true, valB, base, len, bv);
     const int tot = stage_chunk<T, NT>(win.st, wsum, base, len, bv, nseg);
     const int x0 = tid * U - total;  // this chunk's number of the thread's first product
     if (x0 + U > 0 && x0 < tot) {
@@ -1241,7 +1251,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
     const int32_t* __restrict__ order, int64_t first,
                                                   const int64_t* __restrict__ cpB, const int32_t* __restrict__ bpos,
                                                   const int64_t* __restrict__ cpA, const int32_t* __restrict__ rowsA,
-                                                  const int32_t* __restrict__ P, int S, int kmax_l, int rblk_l,
+                                                  const Tiles P, int S, int kmax_l, int rblk_l,
                                                   int kmax_h, int rblk_h, int64_t heavy_thr,
                                                   int64_t* __restrict__ nnzcol, Unit* __restrict__ units_l,
                                                   int* __restrict__ n_l, int cap_l, Unit* __restrict__ units_h,
@@ -1293,7 +1303,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         int64_t base;
         int len;
         uint8_t dummy;
-        load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, P, S, i_lo, i_hi, whole, nullptr, base, len,
+        load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, P, i_lo, i_hi, whole, nullptr, base, len,
                                  dummy);
         int nseg;
         const int tot = stage_chunk<uint8_t, NT>(st, wsum, base, len, 0, nseg);
@@ -1453,7 +1463,7 @@ template <int NT, int U, int IBLK>
 __global__ __launch_bounds__(NT) void k_sym_band(const int32_t* __restrict__ order, int64_t first,
                                                  const int64_t* __restrict__ cpB, const int32_t* __restrict__ bpos,
                                                  const int64_t* __restrict__ cpA, const int32_t* __restrict__ rowsA,
-                                                 const int32_t* __restrict__ P, int S, int32_t* __restrict__ bcnt,
+                                                 const Tiles P, int S, int32_t* __restrict__ bcnt,
                                                  uint32_t* __restrict__ rmap, int64_t rm_cols) {
   constexpr int BMW = IBLK * kBRW;  // bitmap words of one band
   __shared__ uint32_t bits[BMW];
@@ -1471,7 +1481,7 @@ __global__ __launch_bounds__(NT) void k_sym_band(const int32_t* __restrict__ ord
     int64_t base;
     int len;
     uint8_t dummy;
-    load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, P, S, i_lo, i_hi, whole, nullptr, base, len, dummy);
+    load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, P, i_lo, i_hi, whole, nullptr, base, len, dummy);
     int nseg;
     const int tot = stage_chunk<uint8_t, NT>(st, wsum, base, len, 0, nseg);
     visit_staged<uint8_t, NT, U>(st, nseg, tot, [&](const int64_t(&idx)[U], const uint8_t(&)[U]) {
@@ -1692,7 +1702,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
                                                                             const int64_t* __restrict__ cpB,
                                                   const int32_t* __restrict__ bpos, const T* __restrict__ valB,
                                                   const int64_t* __restrict__ cpA, const int32_t* __restrict__ rowsA,
-                                                  const T* __restrict__ valA, const int32_t* __restrict__ P, int S,
+                                                  const T* __restrict__ valA, const Tiles P, int S,
                                                   const int64_t* __restrict__ cpC, int64_t* __restrict__ irC,
                                                   T* __restrict__ valC, int* __restrict__ err, Filter<T> flt = {}, int xg = 0) {
   using SR = Sem<K, T>;
@@ -1765,7 +1775,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
     int64_t base;
     int len;
     T bv;
-    load_seg<T, true>(b0 + threadIdx.x, b1, bpos, cpA, P, S, t_lo, t_hi, false, valB, base, len, bv);
+    load_seg<T, true>(b0 + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
     tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
     // sweep 1, cached rounds
 #pragma unroll
@@ -1814,7 +1824,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
       int64_t base;
       int len;
       T bv;
-      load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, S, t_lo, t_hi, false, valB, base, len, bv);
+      load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
       tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
       if (direct) visit_staged<T, NT, U>(st, nseg, tot, acc_direct);
       else visit_staged<T, NT, U>(st, nseg, tot, set_bits);
@@ -1864,7 +1874,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
       int64_t base;
       int len;
       T bv;
-      load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, S, t_lo, t_hi, false, valB, base, len, bv);
+      load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
       int ns2;
       const int t2 = stage_chunk<T, NT>(st, wsum, base, len, bv, ns2);
       visit_staged<T, NT, U>(st, ns2, t2, accumulate);
@@ -1885,7 +1895,7 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
                                                      const int64_t* __restrict__ cpB, const int32_t* __restrict__ bpos,
                                                      const T* __restrict__ valB, const int64_t* __restrict__ cpA,
                                                      const int32_t* __restrict__ rowsA, const T* __restrict__ valA,
-                                                     const int32_t* __restrict__ P, int S, int64_t rm_cols,
+                                                     const Tiles P, int S, int64_t rm_cols,
                                                      const int64_t* __restrict__ cpC, int64_t* __restrict__ irC,
                                                      T* __restrict__ valC, int* __restrict__ err,
                                                      Filter<T> flt = {}, int xg = 0) {
@@ -1965,7 +1975,7 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
     int64_t base;
     int len;
     T bv;
-    load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, S, t_lo, t_hi, false, valB, base, len, bv);
+    load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
     int nseg;
     const int tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
     visit_staged<T, NT, U>(st, nseg, tot, accumulate);
@@ -1989,7 +1999,7 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
                                                  const uint16_t* __restrict__ bcnt16, const int64_t* __restrict__ cpB,
                                                  const int32_t* __restrict__ bpos, const T* __restrict__ valB,
                                                  const int64_t* __restrict__ cpA, const int32_t* __restrict__ rowsA,
-                                                 const T* __restrict__ valA, const int32_t* __restrict__ P, int S,
+                                                 const T* __restrict__ valA, const Tiles P, int S,
                                                  const int64_t* __restrict__ cpC, int64_t* __restrict__ irC,
                                                  T* __restrict__ valC, int* __restrict__ err, Filter<T> flt = {}, int xg = 0) {
   using SR = Sem<K, T>;
@@ -2059,7 +2069,7 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
     int64_t base;
     int len;
     T bv;
-    load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, S, t_lo, t_hi, false, valB, base, len, bv);
+    load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
     int nseg;
     const int tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
     visit_staged<T, NT, U>(st, nseg, tot, accumulate);
@@ -2297,7 +2307,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
     const UnitL* __restrict__ units, int* __restrict__ ticket, unsigned long long* __restrict__ status,
     const int64_t* __restrict__ hcs, const int64_t* __restrict__ cpB, const int32_t* __restrict__ bpos,
     const T* __restrict__ valB, const int64_t* __restrict__ cpA, const int32_t* __restrict__ rowsA,
-    const T* __restrict__ valA, const int32_t* __restrict__ P, int S, int64_t cap, int64_t* __restrict__ irC,
+    const T* __restrict__ valA, const Tiles P, int S, int64_t cap, int64_t* __restrict__ irC,
     T* __restrict__ valC, unsigned long long* __restrict__ col_total, int* __restrict__ ovf_units,
     int* __restrict__ err) {
   using SR = Sem<K, T>;
@@ -2392,7 +2402,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
       int64_t base;
       int len;
       T bv;
-      load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, S, t_lo, t_hi, false, valB, base, len, bv);
+      load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
       tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
       visit_staged<T, NT, U>(st, nseg, tot, acc_direct);
     }
@@ -2400,7 +2410,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
     int64_t base;
     int len;
     T bv;
-    load_seg<T, true>(b0 + threadIdx.x, b1, bpos, cpA, P, S, t_lo, t_hi, false, valB, base, len, bv);
+    load_seg<T, true>(b0 + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
     if (!valid) len = 0;
     tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
 #pragma unroll
@@ -2430,7 +2440,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
       int64_t base;
       int len;
       T bv;
-      load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, S, t_lo, t_hi, false, valB, base, len, bv);
+      load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
       if (!valid) len = 0;
       tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
       visit_staged<T, NT, U>(st, nseg, tot, set_bits);
@@ -2532,7 +2542,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
         int64_t base;
         int len;
         T bv;
-        load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, S, t_lo, t_hi, false, valB, base, len, bv);
+        load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
         if (!valid) len = 0;
         int ns2;
         const int t2 = stage_chunk<T, NT>(st, wsum, base, len, bv, ns2);
@@ -2567,25 +2577,32 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   }
 }
 
-// Tile pointers at kBR granularity, one wave per stored A column:
-// P[p*(S+1)+t] = #entries of column p with row < t*kBR (binary search).
-__global__ void k_ptable_wave(const int64_t* __restrict__ cpA, int64_t nzcA, const int32_t* __restrict__ rowsA,
-                              int S, int32_t* __restrict__ P) {
-  const int64_t p = global_wave();
+// Tile pointers (Tiles): thread per stored A column and run of kTileRun tiles,
+// so a wave's stores cover 64 consecutive columns of one tile.  Each pointer
+// is searched for from the previous one, doubling the step: one or two probes
+// for the short segments of sparse columns, a logarithm for the long ones.
+constexpr int kTileRun = 32;
+__global__ __launch_bounds__(256) void k_tiles(const int64_t* __restrict__ cpA, int64_t nzcA,
+                                               const int32_t* __restrict__ rowsA, int S, int32_t* __restrict__ at) {
+  const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (p >= nzcA) return;
-  const int64_t b = cpA[p];
-  const int len = (int)(cpA[p + 1] - b);
-  const int32_t* rows = rowsA + b;
-  int32_t* out = P + p * (int64_t)(S + 1);
-  for (int t = lane_id(); t <= S; t += kWave) {
+  const int32_t end = (int32_t)cpA[p + 1];
+  int32_t lo = (int32_t)cpA[p];
+  const int t0 = (int)blockIdx.y * kTileRun, t1 = min(S + 1, t0 + kTileRun);
+  for (int t = t0; t < t1; ++t) {
     const int64_t key = (int64_t)t * kBR;
-    int lo = 0, hi = len;  // first i with rows[i] >= key
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (rows[mid] < key) lo = mid + 1;
+    int32_t step = 1, hi = lo;  // rows before lo are below key
+    while (hi < end && rowsA[hi] < key) {
+      lo = hi + 1;
+      hi = min(end, lo + step);
+      step = min(step * 2, 1 << 29);
+    }
+    while (lo < hi) {  // first entry in [lo, hi] with row >= key
+      const int32_t mid = lo + (hi - lo) / 2;
+      if (rowsA[mid] < key) lo = mid + 1;
       else hi = mid;
     }
-    out[t] = lo;
+    at[t * nzcA + p] = lo;
   }
 }
 
@@ -2889,7 +2906,7 @@ static cbx_status alloc_unit_lists(const int32_t* order, const int64_t* flop, in
 // small units' row lists) or banded (the band height in row blocks, 16 or 64;
 // bcnt_buf receives the block counts).
 cbx_status launch_sym_units(const SpgemmConfig& cfg, const int32_t* order, int64_t ncols, const cbx_dcsc* A,
-                            const cbx_dcsc* B, const int32_t* bpos, const int32_t* rowsA, const int32_t* P, int S,
+                            const cbx_dcsc* B, const int32_t* bpos, const int32_t* rowsA, const Tiles& P, int S,
                             int64_t* nnzcol, Unit* units_l, int* n_l, int cap_l, Unit* units_h, int* n_h, int cap_h,
                             uint32_t* rmap, int64_t rm_cols, int* err, DevBuf& bcnt_buf, int kmax_h, hipStream_t s,
                             const UnitLists& ul = {}) {
@@ -2931,7 +2948,7 @@ struct LearnedInfo {
 // written, nnzcol holds every column's size and cpC its exclusive scan.
 template <int K, class T>
 static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const SpgemmConfig& cfg, hipStream_t s,
-                                  const int32_t* rowsA, const int32_t* bpos, const int64_t* flop, const int32_t* P,
+                                  const int32_t* rowsA, const int32_t* bpos, const int64_t* flop, const Tiles& P,
                                   int S, int64_t* nnzcol, int64_t* cpC, void* tmp, size_t tmp_bytes, cbx_dcsc* C,
                                   int* err, LearnedInfo& info) {
   const int64_t nzcB = B->nzc, m = A->m;
@@ -3410,10 +3427,11 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   if (n_dense) {
     CBX_TRY(dalloc(b_P, (size_t)nzcA * (S + 1), s, &P));
     if (use_units)
-      k_ptable_wave<<<wave_grid(nzcA), 256, 0, s>>>(A->cp, nzcA, rowsA, S, P);
+      k_tiles<<<dim3(nblk(nzcA, 256), nblk(S + 1, kTileRun)), 256, 0, s>>>(A->cp, nzcA, rowsA, S, P);
     else
       k_ptable<<<nblk(nzcA, 256), 256, 0, s>>>(A->cp, nzcA, rowsA, S, TR, P);
   }
+  const Tiles tiles{P, nzcA};
   tm.mark(1, s);
 
   // --- learned single pass (unit-tier columns), with the exact hash-tier
@@ -3432,7 +3450,7 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
                               nullptr, nullptr, err, nullptr, s);
     tm.mark(2, s);
     tm.mark(3, s);
-    CBX_TRY((learned_numeric<K, T>(A, B, cfg, s, rowsA, bpos, flop, P, S, nnzcol, cpC, tmp, tmp_bytes, C, err, linfo)));
+    CBX_TRY((learned_numeric<K, T>(A, B, cfg, s, rowsA, bpos, flop, tiles, S, nnzcol, cpC, tmp, tmp_bytes, C, err, linfo)));
     if (linfo.over_capacity) {  // predictions too small overall: redo exactly
       dev_free(C->ir);
       dev_free(C->val);
@@ -3487,7 +3505,7 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
                                tmp, tmp_bytes, b_lsz, b_loff, b_lists, b_lbc, b_us, s, ul));
       if (ul.lists && lists_used) *lists_used = true;
     }
-    CBX_TRY(launch_sym_units(cfg, order_s, n_dense, A, B, bpos, rowsA, P, S, nnzcol, units_l, ucnt, (int)cap_l, units_h,
+    CBX_TRY(launch_sym_units(cfg, order_s, n_dense, A, B, bpos, rowsA, tiles, S, nnzcol, units_l, ucnt, (int)cap_l, units_h,
                              ucnt + 1, (int)cap_h, rmap, rm_cols, err, b_bcnt, heavy_k<K, T>(), s, ul));
   } else if (n_dense) {
     k_sym_dense<kSymNT, kSymRBW><<<(unsigned)n_dense, kSymNT, 0, s>>>(order_s, 0, B->cp, bpos, A->cp, rowsA, P, S, G,
@@ -3590,17 +3608,17 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
     // registers
     if (hu[1] && rmap)
       k_num_units_rm<K, T, kHeavyNT, 4, heavy_k<K, T>(), kHeavyRB><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
-          units_h, rmap, B->cp, bpos, valB, A->cp, rowsA, valA, P, S, rm_cols, cpC, C->ir, (T*)C->val, err, flt,
+          units_h, rmap, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, rm_cols, cpC, C->ir, (T*)C->val, err, flt,
           cfg.unit_xcd_group);
     else if (hu[1])
       k_num_units<K, T, kHeavyNT, 4, heavy_k<K, T>(), kHeavyRB, 4><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
-          units_h, B->cp, bpos, valB, A->cp, rowsA, valA, P, S, cpC, C->ir, (T*)C->val, err, flt, cfg.unit_xcd_group);
+          units_h, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, cpC, C->ir, (T*)C->val, err, flt, cfg.unit_xcd_group);
     if (hu[0])
       k_num_units<K, T, kLightNT, 4, kLightK, kLightRB, 2><<<(unsigned)hu[0], kLightNT, 0, s>>>(
-          units_l, B->cp, bpos, valB, A->cp, rowsA, valA, P, S, cpC, C->ir, (T*)C->val, err, flt, cfg.unit_xcd_group);
+          units_l, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, cpC, C->ir, (T*)C->val, err, flt, cfg.unit_xcd_group);
     if (hu[2])
       k_num_list<K, T, kLightNT, 4, kLightK><<<(unsigned)hu[2], kLightNT, 0, s>>>(
-          ul.units, ul.lists, ul.off, ul.bcnt, B->cp, bpos, valB, A->cp, rowsA, valA, P, S, cpC, C->ir, (T*)C->val,
+          ul.units, ul.lists, ul.off, ul.bcnt, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, cpC, C->ir, (T*)C->val,
           err, flt, cfg.unit_xcd_group);
   } else if (n_dense) {
     k_num_dense<K, T, kDenseNT><<<(unsigned)n_dense, kDenseNT, 0, s>>>(order_s, 0, B->cp, bpos, valB, A->cp, rowsA,
