@@ -36,16 +36,29 @@ inline dim3 wave_grid(int64_t nwaves, int bs = 256) {
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & (kWave - 1)); }
 __device__ __forceinline__ int wave_id() { return (int)(threadIdx.x >> 6); }
 
-// Inclusive prefix sum over the 64 lanes of a wave.
+// v + the value of the lane that the DPP control names (0 where it names none
+// or the row mask leaves the lane out).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+
+// Inclusive prefix sum over the 64 lanes of a wave (all must be active): row
+// shifts by 1, 2, 4 and 8 within rows of 16 lanes, then the rows' last lanes
+// broadcast to the rows after them.  Six VALU instructions; shuffles went
+// through LDS and a compare each step.
 __device__ __forceinline__ int wave_incl_scan(int v) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    int t = __shfl_up(v, d, kWave);
-    if (lane >= d) v += t;
-  }
+  v = dpp_add<0x111, 0xf>(v);
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);
+  v = dpp_add<0x143, 0xc>(v);
   return v;
 }
+
+// The wave's index in its workgroup, in a scalar register.
+__device__ __forceinline__ int wave_id_uniform() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
 __device__ __forceinline__ long long wave_sum_ll(long long v) {
 #pragma unroll
@@ -59,48 +72,51 @@ __device__ __forceinline__ long long wave_sum_ll(long long v) {
 template <int NT>
 __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int& total) {
   constexpr int NW = NT / kWave;
-  const int lane = lane_id(), w = wave_id();
+  const int lane = lane_id(), w = wave_id_uniform();
   const int inc = wave_incl_scan(v);
   if (lane == kWave - 1) wsum[w] = inc;
   __syncthreads();
-  if (w == 0) {
-    int x = lane < NW ? wsum[lane] : 0;
-    x = wave_incl_scan(x);
-    if (lane < NW) wsum[lane] = x;
-  }
-  __syncthreads();
-  const int base = w ? wsum[w - 1] : 0;
-  total = wsum[NW - 1];
+  const int x = wave_incl_scan(lane < NW ? wsum[lane] : 0);  // every wave scans the waves' sums
+  const int base = w ? __builtin_amdgcn_readlane(x, w - 1) : 0;
+  total = __builtin_amdgcn_readlane(x, NW - 1);
   __syncthreads();
   return base + inc - v;
 }
 
+template <int CTRL, int ROWS>
+__device__ __forceinline__ long long dpp_add_ll(long long v) {
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, ROWS, 0xf, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xf, false);
+  return v + (long long)(((unsigned long long)hi << 32) | lo);
+}
+
 __device__ __forceinline__ long long wave_incl_scan_ll(long long v) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    long long t = __shfl_up(v, d, kWave);
-    if (lane >= d) v += t;
-  }
+  v = dpp_add_ll<0x111, 0xf>(v);
+  v = dpp_add_ll<0x112, 0xf>(v);
+  v = dpp_add_ll<0x114, 0xf>(v);
+  v = dpp_add_ll<0x118, 0xf>(v);
+  v = dpp_add_ll<0x142, 0xa>(v);
+  v = dpp_add_ll<0x143, 0xc>(v);
   return v;
+}
+
+__device__ __forceinline__ long long readlane_ll(long long v, int lane) {
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), lane);
+  return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
 // 64-bit exclusive prefix sum over a block of NT threads (wsum: NT/64 slots).
 template <int NT>
 __device__ __forceinline__ long long block_excl_scan_ll(long long v, long long* wsum, long long& total) {
   constexpr int NW = NT / kWave;
-  const int lane = lane_id(), w = wave_id();
+  const int lane = lane_id(), w = wave_id_uniform();
   const long long inc = wave_incl_scan_ll(v);
   if (lane == kWave - 1) wsum[w] = inc;
   __syncthreads();
-  if (w == 0) {
-    long long x = lane < NW ? wsum[lane] : 0;
-    x = wave_incl_scan_ll(x);
-    if (lane < NW) wsum[lane] = x;
-  }
-  __syncthreads();
-  const long long base = w ? wsum[w - 1] : 0;
-  total = wsum[NW - 1];
+  const long long x = wave_incl_scan_ll(lane < NW ? wsum[lane] : 0);
+  const long long base = w ? readlane_ll(x, w - 1) : 0;
+  total = readlane_ll(x, NW - 1);
   __syncthreads();
   return base + inc - v;
 }

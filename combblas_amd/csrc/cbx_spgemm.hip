@@ -1266,19 +1266,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
   constexpr int BMW = IBLK * kBRW;     // bitmap words of one sub-pass
   static_assert(BPP % IBLK == 0, "sub-passes tile the cutting pass");
   static_assert(IBLK <= kWave, "a wave scans the block counts of a sub-pass");
-  static_assert(sizeof(SegStage<uint8_t, NT>) >= BPP * sizeof(Unit), "list units are staged in the gather stage");
   __shared__ uint32_t bits[BMW];
   __shared__ int bpre[BPP];           // block counts, then their inclusive prefix
-  __shared__ SegStage<uint8_t, NT> st;
-  __shared__ long long wsum[NT / kWave];
+  __shared__ FlatStage<uint8_t, NT, false> st;
   __shared__ int s_nu, s_slot, s_ns, s_sslot;
   // the units of a pass, staged while it is cut: in the bitmap, which every
   // thread has finished reading (barrier) and the next pass clears only after
   // the end-of-pass barrier
-  static_assert(sizeof(uint32_t) * BMW >= BPP * sizeof(Unit), "the bitmap holds a pass's units");
+  static_assert(sizeof(uint32_t) * BMW >= 2 * BPP * sizeof(Unit), "the bitmap holds a pass's units");
   Unit* su = reinterpret_cast<Unit*>(bits);
   __shared__ unsigned long long s_dense[BPP / kWave];  // blocks of the pass above kListBlockMax outputs
-  Unit* su2 = reinterpret_cast<Unit*>(&st);  // list units of a pass (the stage is idle while cutting)
+  Unit* su2 = su + BPP;  // list units of a pass
   const int col = order[first + blockIdx.x];
   const int64_t b0 = cpB[col], b1 = cpB[col + 1];
   const int npass = (S + BPP - 1) / BPP;
@@ -1289,6 +1287,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
     region = list_off[blockIdx.x + 1] - list_base;
   }
   int64_t colcnt = 0;
+  int par = 0;
+  flat_init(st);
   int unit_off = 0;  // meaningful in thread 0 only
   for (int sp = 0; sp < npass; ++sp) {
     const int t_lo = sp * BPP, t_hi = min(S, t_lo + BPP), nblk = t_hi - t_lo;
@@ -1305,9 +1305,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         uint8_t dummy;
         load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, P, i_lo, i_hi, whole, nullptr, base, len,
                                  dummy);
-        int nseg;
-        const int tot = stage_chunk<uint8_t, NT>(st, wsum, base, len, 0, nseg);
-        visit_staged<uint8_t, NT, U>(st, nseg, tot, [&](const int64_t(&idx)[U], const uint8_t(&)[U]) {
+        const FlatSeg me = flat_stage<uint8_t, NT, false>(st, (int32_t)base, len, 0);
+        flat_chunk<uint8_t, NT, false, U>(st, me, par, [&](const int32_t(&idx)[U], const uint8_t(&)[U]) {
           int32_t r[U];
 #pragma unroll
           for (int u = 0; u < U; ++u) r[u] = idx[u] >= 0 ? rowsA[idx[u]] - row0 : -1;
@@ -1467,8 +1466,7 @@ __global__ __launch_bounds__(NT) void k_sym_band(const int32_t* __restrict__ ord
                                                  uint32_t* __restrict__ rmap, int64_t rm_cols) {
   constexpr int BMW = IBLK * kBRW;  // bitmap words of one band
   __shared__ uint32_t bits[BMW];
-  __shared__ SegStage<uint8_t, NT> st;
-  __shared__ long long wsum[NT / kWave];
+  __shared__ FlatStage<uint8_t, NT, false> st;
   const int64_t slot = blockIdx.x;  // the column's position in the launch
   const int col = order[first + slot];
   const int i_lo = (int)blockIdx.y * IBLK, i_hi = min(S, i_lo + IBLK), inb = i_hi - i_lo;
@@ -1477,14 +1475,15 @@ __global__ __launch_bounds__(NT) void k_sym_band(const int32_t* __restrict__ ord
   const bool whole = S <= IBLK;  // one band covers every row: no tile look-ups
   for (int i = threadIdx.x; i < inb * kBRW; i += NT) bits[i] = 0u;
   // (the staging barrier below orders the clear before any insertion)
+  int par = 0;
+  flat_init(st);
   for (int64_t eb = b0; eb < b1; eb += NT) {
     int64_t base;
     int len;
     uint8_t dummy;
     load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, P, i_lo, i_hi, whole, nullptr, base, len, dummy);
-    int nseg;
-    const int tot = stage_chunk<uint8_t, NT>(st, wsum, base, len, 0, nseg);
-    visit_staged<uint8_t, NT, U>(st, nseg, tot, [&](const int64_t(&idx)[U], const uint8_t(&)[U]) {
+    const FlatSeg me = flat_stage<uint8_t, NT, false>(st, (int32_t)base, len, 0);
+    flat_chunk<uint8_t, NT, false, U>(st, me, par, [&](const int32_t(&idx)[U], const uint8_t(&)[U]) {
       int32_t r[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) r[u] = idx[u] >= 0 ? rowsA[idx[u]] - row0 : -1;
@@ -1713,7 +1712,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
   __shared__ Acc vals[KMAX];
   __shared__ uint32_t bits[NW32];
   __shared__ uint16_t pre[NW64];
-  __shared__ SegStage<T, NT> st;
+  __shared__ FlatStage<T, NT, true> st;
   __shared__ long long wsum[NT / kWave];
   const Unit un = units[xcd_unit((int)blockIdx.x, (int)gridDim.x, xg)];
   const int col = un.col;
@@ -1732,11 +1731,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
     return;
   }
   const int ninit = direct ? (t_hi - t_lo) * kBR : cnt;
+  flat_init(st);
   for (int i = threadIdx.x; i < ninit; i += NT) vals[i] = SR::ident();
   const int nw32 = (t_hi - t_lo) * kBRW;
   for (int i = threadIdx.x; i < nw32; i += NT) bits[i] = 0u;
 
-  auto set_bits = [&](const int64_t(&idx)[U], const T(&)[U]) {
+  auto set_bits = [&](const int32_t(&idx)[U], const T(&)[U]) {
     int32_t r[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) r[u] = idx[u] >= 0 ? rowsA[idx[u]] - row0 : -1;
@@ -1749,7 +1749,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
     const uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
     return (int)pre[w] + __popcll(word & ((1ull << b) - 1ull));
   };
-  auto accumulate = [&](const int64_t(&idx)[U], const T(&bvs)[U]) {
+  auto accumulate = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
     int32_t r[U];
     T a[U];
 #pragma unroll
@@ -1770,64 +1770,65 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
 
   int32_t crow[CR][U];
   Acc cprod[CR][U];
-  int tot = 0, nseg = 0;
-  if (single_chunk) {
+  int par = 0;
+  FlatSeg me{};
+  FlatTile ft{};
+  bool cached = false;  // the only chunk is one tile: its first CR rounds stay in registers
+  auto acc_direct = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
+    int32_t r[U];
+    T a[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      r[u] = -1;
+      if (idx[u] >= 0) {
+        r[u] = rowsA[idx[u]] - row0;
+        a[u] = valA[idx[u]];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (r[u] >= 0) {
+        atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
+        SR::acc(&vals[r[u]], SR::mul(a[u], bvs[u]));
+      }
+  };
+  // sweep 1 (the staging barrier orders the initialisation before any insertion)
+  for (int64_t eb = b0; eb < b1; eb += NT) {
     int64_t base;
     int len;
     T bv;
-    load_seg<T, true>(b0 + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
-    tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
-    // sweep 1, cached rounds
+    load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
+    me = flat_stage<T, NT, true>(st, (int32_t)base, len, bv);
+    cached = single_chunk && me.total <= kTileProducts;
+    if (cached) {
+      ft = flat_tile(st, me, 0, 0, par);
+      par ^= 1;
 #pragma unroll
-    for (int rr = 0; rr < CR; ++rr) {
-      int64_t idx[U];
-      T bvs[U];
-      fill_round<T, NT, U>(st, nseg, tot, (rr * NT + (int)threadIdx.x) * U, idx, bvs);
-      T a[U];
+      for (int rr = 0; rr < CR; ++rr) {
+        int32_t idx[U];
+        T bvs[U];
+        flat_round<T, NT, true, U>(st, ft, me.total, rr, idx, bvs);
+        T a[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        crow[rr][u] = -1;
-        if (idx[u] >= 0) {
-          crow[rr][u] = rowsA[idx[u]] - row0;
-          a[u] = valA[idx[u]];
+        for (int u = 0; u < U; ++u) {
+          crow[rr][u] = -1;
+          if (idx[u] >= 0) {
+            crow[rr][u] = rowsA[idx[u]] - row0;
+            a[u] = valA[idx[u]];
+          }
         }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (crow[rr][u] >= 0) {
+            atomicOr(&bits[crow[rr][u] >> 5], 1u << (crow[rr][u] & 31));
+            cprod[rr][u] = SR::mul(a[u], bvs[u]);
+          }
       }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (crow[rr][u] >= 0) {
-          atomicOr(&bits[crow[rr][u] >> 5], 1u << (crow[rr][u] & 31));
-          cprod[rr][u] = SR::mul(a[u], bvs[u]);
-        }
-    }
-    visit_staged<T, NT, U>(st, nseg, tot, set_bits, CR);
-  } else {
-    auto acc_direct = [&](const int64_t(&idx)[U], const T(&bvs)[U]) {
-      int32_t r[U];
-      T a[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        r[u] = -1;
-        if (idx[u] >= 0) {
-          r[u] = rowsA[idx[u]] - row0;
-          a[u] = valA[idx[u]];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (r[u] >= 0) {
-          atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
-          SR::acc(&vals[r[u]], SR::mul(a[u], bvs[u]));
-        }
-    };
-    if (direct) __syncthreads();  // the value window is initialised before anyone accumulates
-    for (int64_t eb = b0; eb < b1; eb += NT) {
-      int64_t base;
-      int len;
-      T bv;
-      load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
-      tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
-      if (direct) visit_staged<T, NT, U>(st, nseg, tot, acc_direct);
-      else visit_staged<T, NT, U>(st, nseg, tot, set_bits);
+      flat_visit<T, NT, true, U>(st, ft, me.total, set_bits, CR);
+    } else if (direct) {
+      flat_chunk<T, NT, true, U>(st, me, par, acc_direct);
+    } else {
+      flat_chunk<T, NT, true, U>(st, me, par, set_bits);
     }
   }
   __syncthreads();
@@ -1859,7 +1860,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
     return;
   }
   // sweep 2: accumulate values at their ranks
-  if (single_chunk) {
+  if (cached) {
 #pragma unroll
     for (int rr = 0; rr < CR; ++rr)
 #pragma unroll
@@ -1868,16 +1869,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
           const int rank = rank_of(crow[rr][u]);
           if (rank < cnt) SR::acc(&vals[rank], cprod[rr][u]);
         }
-    visit_staged<T, NT, U>(st, nseg, tot, accumulate, CR);
+    flat_visit<T, NT, true, U>(st, ft, me.total, accumulate, CR);
   } else {
     for (int64_t eb = b0; eb < b1; eb += NT) {
       int64_t base;
       int len;
       T bv;
       load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
-      int ns2;
-      const int t2 = stage_chunk<T, NT>(st, wsum, base, len, bv, ns2);
-      visit_staged<T, NT, U>(st, ns2, t2, accumulate);
+      me = flat_stage<T, NT, true>(st, (int32_t)base, len, bv);
+      flat_chunk<T, NT, true, U>(st, me, par, accumulate);
     }
   }
   __syncthreads();
@@ -1907,7 +1907,7 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
   __shared__ Acc vals[KMAX];
   __shared__ uint32_t bits[NW32];
   __shared__ uint16_t pre[NW64];
-  __shared__ SegStage<T, NT> st;
+  __shared__ FlatStage<T, NT, true> st;
   __shared__ long long wsum[NT / kWave];
   const Unit un = units[xcd_unit((int)blockIdx.x, (int)gridDim.x, xg)];
   const int col = un.col;
@@ -1922,6 +1922,7 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
     return;
   }
   const int ninit = direct ? (t_hi - t_lo) * kBR : cnt;
+  flat_init(st);
   for (int i = threadIdx.x; i < ninit; i += NT) vals[i] = SR::ident();
   const int nw32 = (t_hi - t_lo) * kBRW;
   const uint32_t* src = rmap + (int64_t)un.slot * S * kBRW + (int64_t)t_lo * kBRW;
@@ -1953,7 +1954,7 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
     const uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
     return (int)pre[w] + __popcll(word & ((1ull << b) - 1ull));
   };
-  auto accumulate = [&](const int64_t(&idx)[U], const T(&bvs)[U]) {
+  auto accumulate = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
     int32_t r[U];
     T a[U];
 #pragma unroll
@@ -1971,14 +1972,14 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
       if (q < (direct ? ninit : cnt)) SR::acc(&vals[q], SR::mul(a[u], bvs[u]));
     }
   };
+  int par = 0;
   for (int64_t eb = b0; eb < b1; eb += NT) {
     int64_t base;
     int len;
     T bv;
     load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
-    int nseg;
-    const int tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
-    visit_staged<T, NT, U>(st, nseg, tot, accumulate);
+    const FlatSeg me = flat_stage<T, NT, true>(st, (int32_t)base, len, bv);
+    flat_chunk<T, NT, true, U>(st, me, par, accumulate);
   }
   __syncthreads();
   unit_emit<K, T, NT>(direct, ninit, cnt, nw64, bits, pre, vals, row0, out, irC, valC, flt, col,
@@ -2009,7 +2010,7 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
   __shared__ Acc vals[KMAX];
   __shared__ uint16_t lst[KMAX];
   __shared__ int dir[BPP + 1];  // list position of each block's first row; dir[nb] = cnt
-  __shared__ SegStage<T, NT> st;
+  __shared__ FlatStage<T, NT, true> st;
   __shared__ long long wsum[NT / kWave];
   const Unit un = units[xcd_unit((int)blockIdx.x, (int)gridDim.x, xg)];
   const int col = un.col;
@@ -2022,6 +2023,7 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
     if (threadIdx.x == 0) atomicOr(err, 64);
     return;
   }
+  flat_init(st);
   const uint16_t* src = lists + list_off[un.slot] + un.off;
   for (int i = threadIdx.x; i < cnt; i += NT) {
     lst[i] = src[i];
@@ -2038,7 +2040,7 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
     if (threadIdx.x <= nb) dir[threadIdx.x] = ex;
   }
   __syncthreads();
-  auto accumulate = [&](const int64_t(&idx)[U], const T(&bvs)[U]) {
+  auto accumulate = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
     int32_t r[U];
     T a[U];
 #pragma unroll
@@ -2065,14 +2067,14 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
       else atomicOr(err, 4);  // symbolic and numeric agree; guard anyway
     }
   };
+  int par = 0;
   for (int64_t eb = b0; eb < b1; eb += NT) {
     int64_t base;
     int len;
     T bv;
     load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
-    int nseg;
-    const int tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
-    visit_staged<T, NT, U>(st, nseg, tot, accumulate);
+    const FlatSeg me = flat_stage<T, NT, true>(st, (int32_t)base, len, bv);
+    flat_chunk<T, NT, true, U>(st, me, par, accumulate);
   }
   __syncthreads();
   auto row_of = [&](int i) {  // the block holding list position i: largest b with dir[b] <= i
@@ -2320,7 +2322,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   // exclusive prefix counts: 16 bits while 64 * NW64 <= 65536
   using PreT = typename std::conditional<(64 * NW64 <= 65536), uint16_t, int32_t>::type;
   __shared__ PreT pre[NW64];
-  __shared__ SegStage<T, NT> st;
+  __shared__ FlatStage<T, NT, true> st;
   __shared__ long long wsum[NT / kWave];
   __shared__ int s_t;
   __shared__ long long s_excl;
@@ -2335,7 +2337,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   const int nw32 = min(t_hi - t_lo, RBLK) * kBRW;
   for (int i = threadIdx.x; i < nw32; i += NT) bits[i] = 0u;
 
-  auto set_bits = [&](const int64_t(&idx)[U], const T(&)[U]) {
+  auto set_bits = [&](const int32_t(&idx)[U], const T(&)[U]) {
     int32_t r[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) r[u] = idx[u] >= 0 ? rowsA[idx[u]] - row0 : -1;
@@ -2349,7 +2351,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
     return (int)pre[w] + __popcll(word & ((1ull << b) - 1ull));
   };
   int q0 = 0;  // first rank of the current value window
-  auto accumulate = [&](const int64_t(&idx)[U], const T(&bvs)[U]) {
+  auto accumulate = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
     int32_t r[U];
     T a[U];
 #pragma unroll
@@ -2370,7 +2372,11 @@ __global__ __launch_bounds__(NT) void k_num_learned(
 
   int32_t crow[CR][U];
   Acc cprod[CR][U];
-  int tot = 0, nseg = 0;
+  int par = 0;
+  FlatSeg me{};
+  FlatTile ft{};
+  bool cached = false;  // the only chunk is one tile: its first CR rounds stay in registers
+  flat_init(st);
   const bool valid = (t_hi - t_lo) <= RBLK;
   if (!valid && threadIdx.x == 0) atomicOr(err, 64);
   // A unit whose rows fit the value window accumulates at its rows in a
@@ -2380,7 +2386,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   if (direct) {
     for (int i = threadIdx.x; i < ndirect; i += NT) vals[i] = SR::ident();
     // (the staging barriers below order the window's initialisation before any accumulation)
-    auto acc_direct = [&](const int64_t(&idx)[U], const T(&bvs)[U]) {
+    auto acc_direct = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
       int32_t r[U];
       T a[U];
 #pragma unroll
@@ -2403,38 +2409,9 @@ __global__ __launch_bounds__(NT) void k_num_learned(
       int len;
       T bv;
       load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
-      tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
-      visit_staged<T, NT, U>(st, nseg, tot, acc_direct);
+      me = flat_stage<T, NT, true>(st, (int32_t)base, len, bv);
+      flat_chunk<T, NT, true, U>(st, me, par, acc_direct);
     }
-  } else if (single_chunk) {
-    int64_t base;
-    int len;
-    T bv;
-    load_seg<T, true>(b0 + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
-    if (!valid) len = 0;
-    tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
-#pragma unroll
-    for (int rr = 0; rr < CR; ++rr) {
-      int64_t idx[U];
-      T bvs[U];
-      fill_round<T, NT, U>(st, nseg, tot, (rr * NT + (int)threadIdx.x) * U, idx, bvs);
-      T a[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        crow[rr][u] = -1;
-        if (idx[u] >= 0) {
-          crow[rr][u] = rowsA[idx[u]] - row0;
-          a[u] = valA[idx[u]];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (crow[rr][u] >= 0) {
-          atomicOr(&bits[crow[rr][u] >> 5], 1u << (crow[rr][u] & 31));
-          cprod[rr][u] = SR::mul(a[u], bvs[u]);
-        }
-    }
-    visit_staged<T, NT, U>(st, nseg, tot, set_bits, CR);
   } else {
     for (int64_t eb = b0; eb < b1; eb += NT) {
       int64_t base;
@@ -2442,8 +2419,36 @@ __global__ __launch_bounds__(NT) void k_num_learned(
       T bv;
       load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
       if (!valid) len = 0;
-      tot = stage_chunk<T, NT>(st, wsum, base, len, bv, nseg);
-      visit_staged<T, NT, U>(st, nseg, tot, set_bits);
+      me = flat_stage<T, NT, true>(st, (int32_t)base, len, bv);
+      cached = single_chunk && me.total <= kTileProducts;
+      if (!cached) {
+        flat_chunk<T, NT, true, U>(st, me, par, set_bits);
+        continue;
+      }
+      ft = flat_tile(st, me, 0, 0, par);
+      par ^= 1;
+#pragma unroll
+      for (int rr = 0; rr < CR; ++rr) {
+        int32_t idx[U];
+        T bvs[U];
+        flat_round<T, NT, true, U>(st, ft, me.total, rr, idx, bvs);
+        T a[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          crow[rr][u] = -1;
+          if (idx[u] >= 0) {
+            crow[rr][u] = rowsA[idx[u]] - row0;
+            a[u] = valA[idx[u]];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (crow[rr][u] >= 0) {
+            atomicOr(&bits[crow[rr][u] >> 5], 1u << (crow[rr][u] & 31));
+            cprod[rr][u] = SR::mul(a[u], bvs[u]);
+          }
+      }
+      flat_visit<T, NT, true, U>(st, ft, me.total, set_bits, CR);
     }
   }
   __syncthreads();
@@ -2527,7 +2532,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
     const int wn = min(KMAX, cnt - q0);
     for (int i = threadIdx.x; i < wn; i += NT) vals[i] = SR::ident();
     __syncthreads();
-    if (single_chunk) {
+    if (cached) {
 #pragma unroll
       for (int rr = 0; rr < CR; ++rr)
 #pragma unroll
@@ -2536,7 +2541,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
             const int q = rank_of(crow[rr][u]) - q0;
             if (q >= 0 && q < KMAX) SR::acc(&vals[q], cprod[rr][u]);
           }
-      visit_staged<T, NT, U>(st, nseg, tot, accumulate, CR);
+      flat_visit<T, NT, true, U>(st, ft, me.total, accumulate, CR);
     } else {
       for (int64_t eb = b0; eb < b1; eb += NT) {
         int64_t base;
@@ -2544,9 +2549,8 @@ __global__ __launch_bounds__(NT) void k_num_learned(
         T bv;
         load_seg<T, true>(eb + threadIdx.x, b1, bpos, cpA, P, t_lo, t_hi, false, valB, base, len, bv);
         if (!valid) len = 0;
-        int ns2;
-        const int t2 = stage_chunk<T, NT>(st, wsum, base, len, bv, ns2);
-        visit_staged<T, NT, U>(st, ns2, t2, accumulate);
+        me = flat_stage<T, NT, true>(st, (int32_t)base, len, bv);
+        flat_chunk<T, NT, true, U>(st, me, par, accumulate);
       }
     }
     __syncthreads();
