@@ -89,6 +89,21 @@ __device__ __forceinline__ void visit_staged(const SegStage<T, NT>& st, int nseg
   }
 }
 
+// Holds v in a register at this point, so that a load of v (and of what its
+// address comes from) is issued before it even where v is only used under a
+// condition: the compiler otherwise sinks the load into the branch, and a
+// lane's independent loads then wait for each other.
+template <class T>
+__device__ __forceinline__ void pin(T& v) {
+  if constexpr (sizeof(T) < 4) {
+    uint32_t x = (uint32_t)v;
+    asm volatile("" : "+v"(x));
+    v = (T)x;
+  } else {
+    asm volatile("" : "+v"(v));
+  }
+}
+
 // ------------------------------------------------------------- bit-flattened
 // Flattening by a bitmap of segment starts.  Product x of a chunk lies in
 // segment k(x) = the number of segments (after the first) that start at or
@@ -194,44 +209,59 @@ __device__ __forceinline__ FlatTile flat_tile(FlatStage<T, NT, VAL>& st, const F
   return ft;
 }
 
-// A-entry index (-1 past the chunk's end) and multiplier of this lane's
-// product in words (round * U + u) * NW + wave, u < U.  No barriers.
+// A-entry index and multiplier of this lane's product in words
+// (round * U + u) * NW + wave, u < U, and whether there is one: past the end
+// the lane has the chunk's last product again, ok false, so that the caller
+// loads what the indices name without a branch (a branch around each load
+// would wait for it before the next is issued).  The round's first word must
+// hold products; rounds do not straddle the tile's halves.  No barriers.
 template <class T, int NT, bool VAL, int U>
 __device__ __forceinline__ void flat_round(const FlatStage<T, NT, VAL>& st, const FlatTile& ft, int total, int round,
-                                           int32_t (&idx)[U], T (&bvs)[U]) {
+                                           int32_t (&idx)[U], T (&bvs)[U], bool (&ok)[U]) {
   constexpr int NW = NT / kWave;
-  const int w = wave_id_uniform();
+  static_assert(kWave % (U * NW) == 0 || U * NW == kWave, "a round lies in one half of the tile");
+  const int j0 = round * U * NW + wave_id_uniform();
+  const bool low = j0 < kWave;  // uniform
+  const unsigned wl = low ? (unsigned)ft.w0 : (unsigned)ft.w1;
+  const unsigned wh = low ? (unsigned)(ft.w0 >> 32) : (unsigned)(ft.w1 >> 32);
+  const int pp = low ? ft.p0 : ft.p1;
   const int end = min(total - ft.base, kTileProducts);
+  int k[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int j = (round * U + u) * NW + w;  // scalar
-    const unsigned long long ww = j < kWave ? ft.w0 : ft.w1;
-    const int pp = j < kWave ? ft.p0 : ft.p1;
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)ww, j & (kWave - 1));
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(ww >> 32), j & (kWave - 1));
-    const unsigned kb = (unsigned)__builtin_amdgcn_readlane(pp, j & (kWave - 1));
-    const int k = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, kb));
-    const int x = j * kWave + lane_id();
-    idx[u] = -1;
-    bvs[u] = T{};
-    if (x < end) {
-      idx[u] = ft.base + x + st.delta[k];
-      if constexpr (VAL) bvs[u] = st.bval[k];
-    }
+    const int j = (j0 + u * NW) & (kWave - 1);  // scalar
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)wl, j);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)wh, j);
+    const unsigned kb = (unsigned)__builtin_amdgcn_readlane(pp, j);
+    k[u] = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, kb));
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int x = (j0 + u * NW) * kWave + lane_id();
+    ok[u] = x < end;
+    idx[u] = ft.base + min(x, end - 1) + st.delta[k[u]];
+    if constexpr (VAL) bvs[u] = st.bval[k[u]];
+    else bvs[u] = T{};
   }
 }
 
-// f(idx, bvs) for every round of the tile from first_round on.
+// The words of the tile that hold products.
+__device__ __forceinline__ int flat_words(const FlatTile& ft, int total) {
+  return (min(total - ft.base, kTileProducts) + 63) >> 6;
+}
+
+// f(idx, bvs, ok) for every round of the tile from first_round on.
 template <class T, int NT, bool VAL, int U, class F>
 __device__ __forceinline__ void flat_visit(const FlatStage<T, NT, VAL>& st, const FlatTile& ft, int total, F&& f,
                                            int first_round = 0) {
   constexpr int NW = NT / kWave;
-  const int words = (min(total - ft.base, kTileProducts) + 63) >> 6;
-  for (int r = first_round; r * U * NW + wave_id_uniform() < words; ++r) {
+  const int words = flat_words(ft, total) - wave_id_uniform();
+  for (int r = first_round; r * U * NW < words; ++r) {
     int32_t idx[U];
     T bvs[U];
-    flat_round<T, NT, VAL, U>(st, ft, total, r, idx, bvs);
-    f(idx, bvs);
+    bool ok[U];
+    flat_round<T, NT, VAL, U>(st, ft, total, r, idx, bvs, ok);
+    f(idx, bvs, ok);
   }
 }
 

@@ -205,6 +205,36 @@ __device__ __forceinline__ void load_seg(int64_t e, int64_t b1, const int32_t* _
   }
 }
 
+// Rows (less row0) and values of U entries of A, all loads in flight together.
+template <int U>
+__device__ __forceinline__ void load_rows(const int32_t* __restrict__ rowsA, int32_t row0, const int32_t (&idx)[U],
+                                          int32_t (&r)[U]) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) r[u] = rowsA[idx[u]];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    pin(r[u]);
+    r[u] -= row0;
+  }
+}
+template <class T, int U>
+__device__ __forceinline__ void load_entries(const int32_t* __restrict__ rowsA, const T* __restrict__ valA,
+                                             int32_t row0, const int32_t (&idx)[U], T (&bvs)[U], int32_t (&r)[U],
+                                             T (&a)[U]) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    r[u] = rowsA[idx[u]];
+    a[u] = valA[idx[u]];
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    pin(r[u]);
+    pin(a[u]);
+    pin(bvs[u]);
+    r[u] -= row0;
+  }
+}
+
 // ------------------------------------------------------------------ setup
 __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -1306,13 +1336,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, P, i_lo, i_hi, whole, nullptr, base, len,
                                  dummy);
         const FlatSeg me = flat_stage<uint8_t, NT, false>(st, (int32_t)base, len, 0);
-        flat_chunk<uint8_t, NT, false, U>(st, me, par, [&](const int32_t(&idx)[U], const uint8_t(&)[U]) {
+        flat_chunk<uint8_t, NT, false, U>(st, me, par, [&](const int32_t(&idx)[U], uint8_t(&)[U], const bool(&ok)[U]) {
           int32_t r[U];
-#pragma unroll
-          for (int u = 0; u < U; ++u) r[u] = idx[u] >= 0 ? rowsA[idx[u]] - row0 : -1;
+          load_rows(rowsA, row0, idx, r);
 #pragma unroll
           for (int u = 0; u < U; ++u)
-            if (r[u] >= 0) atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
+            if (ok[u]) atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
         });
       }
       __syncthreads();
@@ -1483,13 +1512,12 @@ __global__ __launch_bounds__(NT) void k_sym_band(const int32_t* __restrict__ ord
     uint8_t dummy;
     load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, P, i_lo, i_hi, whole, nullptr, base, len, dummy);
     const FlatSeg me = flat_stage<uint8_t, NT, false>(st, (int32_t)base, len, 0);
-    flat_chunk<uint8_t, NT, false, U>(st, me, par, [&](const int32_t(&idx)[U], const uint8_t(&)[U]) {
+    flat_chunk<uint8_t, NT, false, U>(st, me, par, [&](const int32_t(&idx)[U], uint8_t(&)[U], const bool(&ok)[U]) {
       int32_t r[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) r[u] = idx[u] >= 0 ? rowsA[idx[u]] - row0 : -1;
+      load_rows(rowsA, row0, idx, r);
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        if (r[u] >= 0) atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
+        if (ok[u]) atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
     });
   }
   __syncthreads();
@@ -1686,13 +1714,13 @@ __device__ __forceinline__ void unit_emit(bool direct, int ninit, int cnt, int n
 // accumulates every product at its row's rank.  When the column's B entries
 // fit one chunk, the first CR rounds of products (row, product value) stay in
 // registers between the sweeps, so sweep 2 re-reads nothing for them.
-// Waves per SIMD the small-unit kernel asks for: eight where its LDS allows
-// four 512-thread workgroups per CU (a value window of at most 16 KB: 4-byte
-// accumulators), which then caps it at 64 VGPRs; otherwise the compiler's
-// choice (the LDS limits 8-byte windows to six waves anyway).
+// Waves per SIMD the small-unit kernel asks for, as many as its LDS allows:
+// eight for a value window of at most 16 KB (4-byte accumulators; 64 VGPRs),
+// else six (three 512-thread workgroups of 51 KB; 80 VGPRs).  Left alone, the
+// compiler keeps 81, and a third workgroup stays out.
 template <class Acc, int NT, int KMAX>
 struct UnitWaves {
-  static constexpr int value = (NT == 512 && sizeof(Acc) * KMAX <= 16384) ? 8 : 1;
+  static constexpr int value = NT != 512 ? 1 : sizeof(Acc) * KMAX <= 16384 ? 8 : 6;
 };
 
 template <int K, class T, int NT, int U, int KMAX, int RBLK, int CR>
@@ -1736,36 +1764,33 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
   const int nw32 = (t_hi - t_lo) * kBRW;
   for (int i = threadIdx.x; i < nw32; i += NT) bits[i] = 0u;
 
-  auto set_bits = [&](const int32_t(&idx)[U], const T(&)[U]) {
+  auto set_bits = [&](const int32_t(&idx)[U], T(&)[U], const bool(&ok)[U]) {
     int32_t r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) r[u] = idx[u] >= 0 ? rowsA[idx[u]] - row0 : -1;
+    load_rows(rowsA, row0, idx, r);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (r[u] >= 0) atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
+      if (ok[u]) atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
   };
   auto rank_of = [&](int32_t r) {
     const int w = r >> 6, b = r & 63;
     const uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
     return (int)pre[w] + __popcll(word & ((1ull << b) - 1ull));
   };
-  auto accumulate = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
+  auto ranks_of = [&](const int32_t(&r)[U], int(&rank)[U]) {  // all the LDS reads in flight together
+#pragma unroll
+    for (int u = 0; u < U; ++u) rank[u] = rank_of(r[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) pin(rank[u]);
+  };
+  auto accumulate = [&](const int32_t(&idx)[U], T(&bvs)[U], const bool(&ok)[U]) {
     int32_t r[U];
     T a[U];
+    load_entries(rowsA, valA, row0, idx, bvs, r, a);
+    int rank[U];
+    ranks_of(r, rank);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      r[u] = -1;
-      if (idx[u] >= 0) {
-        r[u] = rowsA[idx[u]] - row0;
-        a[u] = valA[idx[u]];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (r[u] < 0) continue;
-      const int rank = rank_of(r[u]);
-      if (rank < cnt) SR::acc(&vals[rank], SR::mul(a[u], bvs[u]));
-    }
+    for (int u = 0; u < U; ++u)
+      if (ok[u] && rank[u] < cnt) SR::acc(&vals[rank[u]], SR::mul(a[u], bvs[u]));
   };
 
   int32_t crow[CR][U];
@@ -1774,20 +1799,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
   FlatSeg me{};
   FlatTile ft{};
   bool cached = false;  // the only chunk is one tile: its first CR rounds stay in registers
-  auto acc_direct = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
+  unsigned cok = 0;     // which of them are products
+  auto acc_direct = [&](const int32_t(&idx)[U], T(&bvs)[U], const bool(&ok)[U]) {
     int32_t r[U];
     T a[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      r[u] = -1;
-      if (idx[u] >= 0) {
-        r[u] = rowsA[idx[u]] - row0;
-        a[u] = valA[idx[u]];
-      }
-    }
+    load_entries(rowsA, valA, row0, idx, bvs, r, a);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (r[u] >= 0) {
+      if (ok[u]) {
         atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
         SR::acc(&vals[r[u]], SR::mul(a[u], bvs[u]));
       }
@@ -1805,24 +1824,22 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
       par ^= 1;
 #pragma unroll
       for (int rr = 0; rr < CR; ++rr) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) crow[rr][u] = 0;
+        if (rr * U * (NT / kWave) + wave_id_uniform() >= flat_words(ft, me.total)) continue;
         int32_t idx[U];
-        T bvs[U];
-        flat_round<T, NT, true, U>(st, ft, me.total, rr, idx, bvs);
-        T a[U];
+        T bvs[U], a[U];
+        bool ok[U];
+        flat_round<T, NT, true, U>(st, ft, me.total, rr, idx, bvs, ok);
+        load_entries(rowsA, valA, row0, idx, bvs, crow[rr], a);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          crow[rr][u] = -1;
-          if (idx[u] >= 0) {
-            crow[rr][u] = rowsA[idx[u]] - row0;
-            a[u] = valA[idx[u]];
+          cprod[rr][u] = SR::mul(a[u], bvs[u]);
+          if (ok[u]) {
+            cok |= 1u << (rr * U + u);
+            atomicOr(&bits[crow[rr][u] >> 5], 1u << (crow[rr][u] & 31));
           }
         }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (crow[rr][u] >= 0) {
-            atomicOr(&bits[crow[rr][u] >> 5], 1u << (crow[rr][u] & 31));
-            cprod[rr][u] = SR::mul(a[u], bvs[u]);
-          }
       }
       flat_visit<T, NT, true, U>(st, ft, me.total, set_bits, CR);
     } else if (direct) {
@@ -1862,13 +1879,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
   // sweep 2: accumulate values at their ranks
   if (cached) {
 #pragma unroll
-    for (int rr = 0; rr < CR; ++rr)
+    for (int rr = 0; rr < CR; ++rr) {
+      int rank[U];
+      ranks_of(crow[rr], rank);
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        if (crow[rr][u] >= 0) {
-          const int rank = rank_of(crow[rr][u]);
-          if (rank < cnt) SR::acc(&vals[rank], cprod[rr][u]);
-        }
+        if ((cok >> (rr * U + u) & 1u) && rank[u] < cnt) SR::acc(&vals[rank[u]], cprod[rr][u]);
+    }
     flat_visit<T, NT, true, U>(st, ft, me.total, accumulate, CR);
   } else {
     for (int64_t eb = b0; eb < b1; eb += NT) {
@@ -1954,23 +1971,26 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
     const uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
     return (int)pre[w] + __popcll(word & ((1ull << b) - 1ull));
   };
-  auto accumulate = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
+  auto ranks_of = [&](const int32_t(&r)[U], int(&rank)[U]) {  // all the LDS reads in flight together
+#pragma unroll
+    for (int u = 0; u < U; ++u) rank[u] = rank_of(r[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) pin(rank[u]);
+  };
+  auto accumulate = [&](const int32_t(&idx)[U], T(&bvs)[U], const bool(&ok)[U]) {
     int32_t r[U];
     T a[U];
+    load_entries(rowsA, valA, row0, idx, bvs, r, a);
+    int q[U];
+    if (direct) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      r[u] = -1;
-      if (idx[u] >= 0) {
-        r[u] = rowsA[idx[u]] - row0;
-        a[u] = valA[idx[u]];
-      }
+      for (int u = 0; u < U; ++u) q[u] = r[u];
+    } else {
+      ranks_of(r, q);
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (r[u] < 0) continue;
-      const int q = direct ? r[u] : rank_of(r[u]);
-      if (q < (direct ? ninit : cnt)) SR::acc(&vals[q], SR::mul(a[u], bvs[u]));
-    }
+    for (int u = 0; u < U; ++u)
+      if (ok[u] && q[u] < (direct ? ninit : cnt)) SR::acc(&vals[q[u]], SR::mul(a[u], bvs[u]));
   };
   int par = 0;
   for (int64_t eb = b0; eb < b1; eb += NT) {
@@ -2009,6 +2029,7 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
   static_assert(NT > BPP, "one block count per thread, plus the total");
   __shared__ Acc vals[KMAX];
   __shared__ uint16_t lst[KMAX];
+  __shared__ int s_full[NT / kWave];  // each wave's blocks: none with 16 outputs, some with 16, some with 64
   __shared__ int dir[BPP + 1];  // list position of each block's first row; dir[nb] = cnt
   __shared__ FlatStage<T, NT, true> st;
   __shared__ long long wsum[NT / kWave];
@@ -2038,32 +2059,42 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
       return;
     }
     if (threadIdx.x <= nb) dir[threadIdx.x] = ex;
+    const unsigned long long wide = __ballot(c >= 16), wider = __ballot(c >= 64);
+    if (lane_id() == 0) s_full[wave_id()] = wider ? 2 : wide ? 1 : 0;
   }
   __syncthreads();
-  auto accumulate = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
+  int top = 8;  // the search's first step: half the power of two above the fullest block's count
+#pragma unroll
+  for (int i = 0; i < NT / kWave; ++i) top = max(top, s_full[i] == 2 ? 128 : s_full[i] == 1 ? 32 : 8);
+  auto accumulate = [&](const int32_t(&idx)[U], T(&bvs)[U], const bool(&ok)[U]) {
     int32_t r[U];
     T a[U];
+    load_entries(rowsA, valA, row0, idx, bvs, r, a);
+    // first position in the row's block with an offset not below the row's:
+    // all U searches step together, with as many steps as the unit's fullest
+    // block needs
+    int pos[U], end[U], off[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      r[u] = -1;
-      if (idx[u] >= 0) {
-        r[u] = rowsA[idx[u]] - row0;
-        a[u] = valA[idx[u]];
-      }
+      const int b = r[u] >> 12;  // kBR = 4096 rows per block
+      off[u] = r[u] & (kBR - 1);
+      pos[u] = dir[b];
+      end[u] = dir[b + 1];
+    }
+    for (int step = top; step > 0; step >>= 1) {
+      int v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = (int)lst[min(pos[u] + step, end[u]) - 1];
+#pragma unroll
+      for (int u = 0; u < U; ++u) pin(v[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (pos[u] + step <= end[u] && v[u] < off[u]) pos[u] += step;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (r[u] < 0) continue;
-      const int b = r[u] >> 12;  // kBR = 4096 rows per block
-      const uint16_t o = (uint16_t)(r[u] & (kBR - 1));
-      const int end = dir[b + 1];
-      int lo = dir[b], hi = end;  // first position in the block with offset >= o
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (lst[mid] < o) lo = mid + 1;
-        else hi = mid;
-      }
-      if (lo < end && lst[lo] == o) SR::acc(&vals[lo], SR::mul(a[u], bvs[u]));
+      if (!ok[u]) continue;
+      if (pos[u] < end[u] && lst[pos[u]] == off[u]) SR::acc(&vals[pos[u]], SR::mul(a[u], bvs[u]));
       else atomicOr(err, 4);  // symbolic and numeric agree; guard anyway
     }
   };
@@ -2337,37 +2368,34 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   const int nw32 = min(t_hi - t_lo, RBLK) * kBRW;
   for (int i = threadIdx.x; i < nw32; i += NT) bits[i] = 0u;
 
-  auto set_bits = [&](const int32_t(&idx)[U], const T(&)[U]) {
+  auto set_bits = [&](const int32_t(&idx)[U], T(&)[U], const bool(&ok)[U]) {
     int32_t r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) r[u] = idx[u] >= 0 ? rowsA[idx[u]] - row0 : -1;
+    load_rows(rowsA, row0, idx, r);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (r[u] >= 0) atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
+      if (ok[u]) atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
   };
   auto rank_of = [&](int32_t r) {
     const int w = r >> 6, b = r & 63;
     const uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
     return (int)pre[w] + __popcll(word & ((1ull << b) - 1ull));
   };
+  auto ranks_of = [&](const int32_t(&r)[U], int(&rank)[U]) {  // all the LDS reads in flight together
+#pragma unroll
+    for (int u = 0; u < U; ++u) rank[u] = rank_of(r[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) pin(rank[u]);
+  };
   int q0 = 0;  // first rank of the current value window
-  auto accumulate = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
+  auto accumulate = [&](const int32_t(&idx)[U], T(&bvs)[U], const bool(&ok)[U]) {
     int32_t r[U];
     T a[U];
+    load_entries(rowsA, valA, row0, idx, bvs, r, a);
+    int q[U];
+    ranks_of(r, q);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      r[u] = -1;
-      if (idx[u] >= 0) {
-        r[u] = rowsA[idx[u]] - row0;
-        a[u] = valA[idx[u]];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (r[u] < 0) continue;
-      const int q = rank_of(r[u]) - q0;
-      if (q >= 0 && q < KMAX) SR::acc(&vals[q], SR::mul(a[u], bvs[u]));
-    }
+    for (int u = 0; u < U; ++u)
+      if (ok[u] && q[u] >= q0 && q[u] < q0 + KMAX) SR::acc(&vals[q[u] - q0], SR::mul(a[u], bvs[u]));
   };
 
   int32_t crow[CR][U];
@@ -2376,6 +2404,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   FlatSeg me{};
   FlatTile ft{};
   bool cached = false;  // the only chunk is one tile: its first CR rounds stay in registers
+  unsigned cok = 0;     // which of them are products
   flat_init(st);
   const bool valid = (t_hi - t_lo) <= RBLK;
   if (!valid && threadIdx.x == 0) atomicOr(err, 64);
@@ -2386,20 +2415,13 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   if (direct) {
     for (int i = threadIdx.x; i < ndirect; i += NT) vals[i] = SR::ident();
     // (the staging barriers below order the window's initialisation before any accumulation)
-    auto acc_direct = [&](const int32_t(&idx)[U], const T(&bvs)[U]) {
+    auto acc_direct = [&](const int32_t(&idx)[U], T(&bvs)[U], const bool(&ok)[U]) {
       int32_t r[U];
       T a[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        r[u] = -1;
-        if (idx[u] >= 0) {
-          r[u] = rowsA[idx[u]] - row0;
-          a[u] = valA[idx[u]];
-        }
-      }
+      load_entries(rowsA, valA, row0, idx, bvs, r, a);
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        if (r[u] >= 0) {
+        if (ok[u]) {
           atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
           SR::acc(&vals[r[u]], SR::mul(a[u], bvs[u]));
         }
@@ -2429,24 +2451,22 @@ __global__ __launch_bounds__(NT) void k_num_learned(
       par ^= 1;
 #pragma unroll
       for (int rr = 0; rr < CR; ++rr) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) crow[rr][u] = 0;
+        if (rr * U * (NT / kWave) + wave_id_uniform() >= flat_words(ft, me.total)) continue;
         int32_t idx[U];
-        T bvs[U];
-        flat_round<T, NT, true, U>(st, ft, me.total, rr, idx, bvs);
-        T a[U];
+        T bvs[U], a[U];
+        bool ok[U];
+        flat_round<T, NT, true, U>(st, ft, me.total, rr, idx, bvs, ok);
+        load_entries(rowsA, valA, row0, idx, bvs, crow[rr], a);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          crow[rr][u] = -1;
-          if (idx[u] >= 0) {
-            crow[rr][u] = rowsA[idx[u]] - row0;
-            a[u] = valA[idx[u]];
+          cprod[rr][u] = SR::mul(a[u], bvs[u]);
+          if (ok[u]) {
+            cok |= 1u << (rr * U + u);
+            atomicOr(&bits[crow[rr][u] >> 5], 1u << (crow[rr][u] & 31));
           }
         }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (crow[rr][u] >= 0) {
-            atomicOr(&bits[crow[rr][u] >> 5], 1u << (crow[rr][u] & 31));
-            cprod[rr][u] = SR::mul(a[u], bvs[u]);
-          }
       }
       flat_visit<T, NT, true, U>(st, ft, me.total, set_bits, CR);
     }
@@ -2534,13 +2554,13 @@ __global__ __launch_bounds__(NT) void k_num_learned(
     __syncthreads();
     if (cached) {
 #pragma unroll
-      for (int rr = 0; rr < CR; ++rr)
+      for (int rr = 0; rr < CR; ++rr) {
+        int q[U];
+        ranks_of(crow[rr], q);
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          if (crow[rr][u] >= 0) {
-            const int q = rank_of(crow[rr][u]) - q0;
-            if (q >= 0 && q < KMAX) SR::acc(&vals[q], cprod[rr][u]);
-          }
+          if ((cok >> (rr * U + u) & 1u) && q[u] >= q0 && q[u] < q0 + KMAX) SR::acc(&vals[q[u] - q0], cprod[rr][u]);
+      }
       flat_visit<T, NT, true, U>(st, ft, me.total, accumulate, CR);
     } else {
       for (int64_t eb = b0; eb < b1; eb += NT) {
