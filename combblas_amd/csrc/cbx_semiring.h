@@ -8,10 +8,13 @@
 //              which saturates at numeric_limits<T>::max().
 //   SelectMax  Semirings.h:165-190  add max, multiply a*b.
 //
-// Accumulation happens in LDS with atomics.  `Acc` is the LDS accumulator
-// type and `ident()` a true identity of `add` for it, so an accumulator slot
-// that starts at ident() and receives the products x1..xk holds
-// x1 (+) ... (+) xk exactly as the reference's first-insert-then-add does:
+// Accumulation happens in LDS with atomics.  `Acc` is the accumulator type and
+// `ident()` a true identity of `add` for it, so an accumulator slot that starts
+// at ident() and receives the products x1..xk holds x1 (+) ... (+) xk exactly
+// as the reference's first-insert-then-add does.  `Lds` (lident, lout) is its
+// type in LDS: the same, but double for FP32 sums, which are then rounded once
+// (ds_add_f32 takes 193 cycles a wave instruction at random addresses,
+// ds_add_f64 21, ds_add_u64 11).  Identities:
 //   PlusTimes integers 0; floating point -0.0 (so a lone -0.0 stays -0.0);
 //   MinPlus   max();
 //   SelectMax lowest() (the reference's id() of -1 is not an identity of max
@@ -31,6 +34,14 @@ enum SemiringKind : int { kPlusTimes = 0, kMinPlus = 1, kSelectMax = 2 };
 
 template <int K, class T>
 struct Sem;
+
+// Lds, lident and lout of a semiring that accumulates in LDS as in registers.
+template <class SR, class S, class A>
+struct LdsAsAcc {
+  using Lds = A;
+  static __device__ __forceinline__ Lds lident() { return SR::ident(); }
+  static __device__ __forceinline__ S lout(Lds a) { return SR::out(a); }
+};
 
 // -------------------------------------------------------------- helpers
 template <class A>
@@ -66,7 +77,7 @@ __device__ __forceinline__ void lds_cas_minmax(F* p, F v, bool is_min) {
 
 // -------------------------------------------------------------- PlusTimes
 template <>
-struct Sem<kPlusTimes, int64_t> {
+struct Sem<kPlusTimes, int64_t> : LdsAsAcc<Sem<kPlusTimes, int64_t>, int64_t, unsigned long long> {
   using S = int64_t;
   using Acc = unsigned long long;  // two's-complement wrap like the reference
   static __device__ __forceinline__ Acc ident() { return 0ull; }
@@ -76,7 +87,7 @@ struct Sem<kPlusTimes, int64_t> {
   static __device__ __forceinline__ S out(Acc a) { return (S)a; }
 };
 template <>
-struct Sem<kPlusTimes, double> {
+struct Sem<kPlusTimes, double> : LdsAsAcc<Sem<kPlusTimes, double>, double, double> {
   using S = double;
   using Acc = double;
   static __device__ __forceinline__ Acc ident() { return -0.0; }
@@ -89,14 +100,17 @@ template <>
 struct Sem<kPlusTimes, float> {
   using S = float;
   using Acc = float;
+  using Lds = double;
+  static __device__ __forceinline__ Lds lident() { return -0.0; }
+  static __device__ __forceinline__ S lout(Lds a) { return (float)a; }
   static __device__ __forceinline__ Acc ident() { return -0.0f; }
   static __device__ __forceinline__ Acc mul(S a, S b) { return a * b; }
-  static __device__ __forceinline__ void acc(Acc* p, Acc v) { lds_add(p, v); }
+  static __device__ __forceinline__ void acc(Lds* p, Acc v) { lds_add(p, (Lds)v); }
   static __device__ __forceinline__ Acc add(Acc a, Acc b) { return a + b; }
   static __device__ __forceinline__ S out(Acc a) { return a; }
 };
 template <>
-struct Sem<kPlusTimes, uint8_t> {  // bool: OR / AND
+struct Sem<kPlusTimes, uint8_t> : LdsAsAcc<Sem<kPlusTimes, uint8_t>, uint8_t, uint32_t> {  // bool: OR / AND
   using S = uint8_t;
   using Acc = uint32_t;
   static __device__ __forceinline__ Acc ident() { return 0u; }
@@ -116,7 +130,7 @@ __device__ __forceinline__ T inf_plus(T a, T b) {
   return a + b;
 }
 template <>
-struct Sem<kMinPlus, int64_t> {
+struct Sem<kMinPlus, int64_t> : LdsAsAcc<Sem<kMinPlus, int64_t>, int64_t, int64_t> {
   using S = int64_t;
   using Acc = int64_t;
   static __device__ __forceinline__ Acc ident() { return std::numeric_limits<int64_t>::max(); }
@@ -130,17 +144,17 @@ struct Sem<kMinPlus, int64_t> {
   static __device__ __forceinline__ S out(Acc a) { return a; }
 };
 template <>
-struct Sem<kMinPlus, double> {
+struct Sem<kMinPlus, double> : LdsAsAcc<Sem<kMinPlus, double>, double, double> {
   using S = double;
   using Acc = double;
   static __device__ __forceinline__ Acc ident() { return std::numeric_limits<double>::max(); }
   static __device__ __forceinline__ Acc mul(S a, S b) { return inf_plus(a, b); }
-  static __device__ __forceinline__ void acc(Acc* p, Acc v) { lds_cas_minmax<double, unsigned long long>(p, v, true); }
+  static __device__ __forceinline__ void acc(Acc* p, Acc v) { lds_min(p, v); }
   static __device__ __forceinline__ Acc add(Acc a, Acc b) { return b < a ? b : a; }
   static __device__ __forceinline__ S out(Acc a) { return a; }
 };
 template <>
-struct Sem<kMinPlus, float> {
+struct Sem<kMinPlus, float> : LdsAsAcc<Sem<kMinPlus, float>, float, float> {
   using S = float;
   using Acc = float;
   static __device__ __forceinline__ Acc ident() { return std::numeric_limits<float>::max(); }
@@ -152,7 +166,7 @@ struct Sem<kMinPlus, float> {
 
 // -------------------------------------------------------------- SelectMax
 template <>
-struct Sem<kSelectMax, int64_t> {
+struct Sem<kSelectMax, int64_t> : LdsAsAcc<Sem<kSelectMax, int64_t>, int64_t, int64_t> {
   using S = int64_t;
   using Acc = int64_t;
   static __device__ __forceinline__ Acc ident() { return std::numeric_limits<int64_t>::lowest(); }
@@ -162,17 +176,17 @@ struct Sem<kSelectMax, int64_t> {
   static __device__ __forceinline__ S out(Acc a) { return a; }
 };
 template <>
-struct Sem<kSelectMax, double> {
+struct Sem<kSelectMax, double> : LdsAsAcc<Sem<kSelectMax, double>, double, double> {
   using S = double;
   using Acc = double;
   static __device__ __forceinline__ Acc ident() { return -std::numeric_limits<double>::infinity(); }
   static __device__ __forceinline__ Acc mul(S a, S b) { return a * b; }
-  static __device__ __forceinline__ void acc(Acc* p, Acc v) { lds_cas_minmax<double, unsigned long long>(p, v, false); }
+  static __device__ __forceinline__ void acc(Acc* p, Acc v) { lds_max(p, v); }
   static __device__ __forceinline__ Acc add(Acc a, Acc b) { return a < b ? b : a; }
   static __device__ __forceinline__ S out(Acc a) { return a; }
 };
 template <>
-struct Sem<kSelectMax, float> {
+struct Sem<kSelectMax, float> : LdsAsAcc<Sem<kSelectMax, float>, float, float> {
   using S = float;
   using Acc = float;
   static __device__ __forceinline__ Acc ident() { return -std::numeric_limits<float>::infinity(); }

@@ -168,6 +168,45 @@ __device__ __forceinline__ void filter_add_run(const Filter<T>& f, int64_t src, 
   }
 }
 
+// Writes the kept ones (!(v < thr)) of the items i in [0, n) that item(i, v)
+// has, in order and with their rows row_of(i), at `out` (at most cap of them),
+// and appends the range to the run list.  Every wave takes one contiguous share of the
+// items and goes over it twice, counting and then writing, with one barrier
+// between.  `isum`: LDS that no thread still reads.
+template <class T, int NT, class G, class R>
+__device__ __forceinline__ void emit_filtered(int n, int cap, G&& item, R&& row_of, int64_t out, int64_t* __restrict__ irC,
+                                              T* __restrict__ valC, const Filter<T>& flt, int col, int* isum,
+                                              int* err) {
+  constexpr int NW = NT / kWave;
+  const int w = wave_id_uniform(), lane = lane_id();
+  const int share = (n + NT - 1) / NT * kWave;
+  const int i0 = w * share, i1 = min(n, i0 + share);
+  int count = 0;
+  for (int i = i0; i < i1; i += kWave) {
+    T v{};
+    const bool keep = i + lane < i1 && item(i + lane, v) && !(v < flt.thr);
+    count += __popcll(__ballot(keep));
+  }
+  if (lane == 0) isum[w] = count;
+  __syncthreads();
+  const int incl = wave_incl_scan(lane < NW ? isum[lane] : 0);
+  int pos = w ? __builtin_amdgcn_readlane(incl, w - 1) : 0;
+  const int total = __builtin_amdgcn_readlane(incl, NW - 1);
+  if (count)
+    for (int i = i0; i < i1; i += kWave) {
+      T v{};
+      const bool keep = i + lane < i1 && item(i + lane, v) && !(v < flt.thr);
+      const unsigned long long m = __ballot(keep);
+      const int at = pos + __popcll(m & ((1ull << lane) - 1ull));
+      if (keep && at < cap) {
+        irC[out + at] = row_of(i + lane);
+        valC[out + at] = v;
+      }
+      pos += __popcll(m);
+    }
+  if (threadIdx.x == 0) filter_add_run(flt, out, min(total, cap), col, err);
+}
+
 // Tile pointers of the unit tier: at[t * ncols + p] is the index of the first
 // entry of A's p-th stored column with row >= t * kBR (t = 0 .. S; the index
 // runs over all of A's entries).  Tile-major: the units in flight share a few
@@ -732,7 +771,7 @@ __global__ __launch_bounds__(256) void k_tiny_h(const int32_t* __restrict__ orde
   constexpr int kLgHash = 9;
   static_assert((1 << kLgHash) == kTinyHash, "table size");
   __shared__ int32_t s_key[kTinyWaves][kTinyHash];
-  __shared__ Acc s_val[SYM ? 1 : kTinyWaves][SYM ? 1 : kTinyHash];
+  __shared__ typename SR::Lds s_val[SYM ? 1 : kTinyWaves][SYM ? 1 : kTinyHash];
   __shared__ __align__(16) int32_t s_row[kTinyWaves][kTinyMax + 4];  // compacted rows, kNone-padded
   __shared__ uint16_t s_slot[SYM ? 1 : kTinyWaves][SYM ? 1 : kTinyMax];
   const int lane = lane_id(), w = wave_id();
@@ -750,7 +789,7 @@ __global__ __launch_bounds__(256) void k_tiny_h(const int32_t* __restrict__ orde
 #pragma unroll
     for (int q = 0; q < kSPL; ++q) {
       hk[q * kWave + lane] = kEmpty;
-      if constexpr (!SYM) s_val[w][q * kWave + lane] = SR::ident();
+      if constexpr (!SYM) s_val[w][q * kWave + lane] = SR::lident();
     }
     wave_lds_sync();
     // insert: every product finds its row's slot (linear probing)
@@ -829,7 +868,7 @@ __global__ __launch_bounds__(256) void k_tiny_h(const int32_t* __restrict__ orde
           const int e = r * kWave + lane;
           if (r < nc && e < D && rank[r] < have) {
             irC[out + rank[r]] = mine[r];
-            valC[out + rank[r]] = SR::out(s_val[w][s_slot[w][e]]);
+            valC[out + rank[r]] = SR::lout(s_val[w][s_slot[w][e]]);
           }
         }
       } else {  // the fused threshold: a kept row's place is the kept rows below it
@@ -840,7 +879,7 @@ __global__ __launch_bounds__(256) void k_tiny_h(const int32_t* __restrict__ orde
           const int e = r * kWave + lane;
           keep[r] = false;
           if (r < nc && e < D) {
-            v[r] = SR::out(s_val[w][s_slot[w][e]]);
+            v[r] = SR::lout(s_val[w][s_slot[w][e]]);
             keep[r] = !(v[r] < flt.thr);
           }
         }
@@ -985,7 +1024,7 @@ __global__ __launch_bounds__(NT) void k_num_sort(const int32_t* __restrict__ ord
   static_assert((1 << kDigit) * NW == 2 * NT, "one pair of counters per thread");
   union Window {
     SegStage<T, NT> st;  // while the products are gathered
-    Acc vals[CAP];       // once their ranks are known
+    typename SR::Lds vals[CAP];  // once their ranks are known
   };
   __shared__ __align__(16) uint32_t keys[CAP];
   __shared__ __align__(8) uint16_t pay[CAP];  // product numbers, then the products' ranks
@@ -1152,7 +1191,7 @@ __global__ __launch_bounds__(NT) void k_num_sort(const int32_t* __restrict__ ord
     if (head[u]) keys[rk] = key[u];  // the output rows
     pay[num[u]] = (uint16_t)rk;
   }
-  for (int i = tid; i < cnt; i += NT) win.vals[i] = SR::ident();
+  for (int i = tid; i < cnt; i += NT) win.vals[i] = SR::lident();
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < U; ++u)
@@ -1165,24 +1204,15 @@ __global__ __launch_bounds__(NT) void k_num_sort(const int32_t* __restrict__ ord
   if (!flt.on) {
     for (int i = tid; i < cnt; i += NT) {
       irC[out + i] = (int64_t)keys[i];
-      valC[out + i] = SR::out(win.vals[i]);
+      valC[out + i] = SR::lout(win.vals[i]);
     }
     return;
   }
-  int kept = 0;  // the fused threshold: the kept entries, in order, at out
-  for (int c0 = 0; c0 < cnt; c0 += NT) {
-    const int i = c0 + tid;
-    const T v = i < cnt ? SR::out(win.vals[i]) : T{};
-    const bool keep = i < cnt && !(v < flt.thr);
-    long long tot;
-    const int ex = (int)block_excl_scan_ll<NT>(keep ? 1 : 0, wsum, tot);
-    if (keep) {
-      irC[out + kept + ex] = (int64_t)keys[i];
-      valC[out + kept + ex] = v;
-    }
-    kept += (int)tot;
-  }
-  if (tid == 0) filter_add_run(flt, out, kept, col, err);
+  auto item = [&](int i, T& v) {  // the fused threshold
+    v = SR::lout(win.vals[i]);
+    return true;
+  };
+  emit_filtered<T, NT>(cnt, cnt, item, [&](int i) { return (int64_t)keys[i]; }, out, irC, valC, flt, col, isum, err);
 }
 
 // --------------------------------------------------------- numeric: dense
@@ -1199,14 +1229,14 @@ __global__ __launch_bounds__(NT) void k_num_dense(const int32_t* __restrict__ or
   using SR = Sem<K, T>;
   using Acc = typename SR::Acc;
   constexpr int TR = 32 * NT;
-  __shared__ Acc acc[TR];
+  __shared__ typename SR::Lds acc[TR];
   __shared__ uint32_t bits[NT];
   __shared__ int wsum[NT / kWave];
   const int col = order[first + blockIdx.x];
   const int64_t b0 = cpB[col], b1 = cpB[col + 1];
   int64_t out = cpC[col];
   const int64_t out_end = cpC[col + 1];
-  for (int i = threadIdx.x; i < TR; i += NT) acc[i] = SR::ident();
+  for (int i = threadIdx.x; i < TR; i += NT) acc[i] = SR::lident();
   bits[threadIdx.x] = 0u;
   __syncthreads();
   for (int s = 0; s < S; ++s) {
@@ -1243,11 +1273,11 @@ __global__ __launch_bounds__(NT) void k_num_dense(const int32_t* __restrict__ or
       const int r = threadIdx.x * 32 + b;
       if (o < out_end) {  // symbolic and numeric agree; guard anyway
         irC[o] = (int64_t)row0 + r;
-        valC[o] = SR::out(acc[r]);
+        valC[o] = SR::lout(acc[r]);
       } else {
         atomicOr(err, 4);
       }
-      acc[r] = SR::ident();
+      acc[r] = SR::lident();
       ++o;
     }
     bits[threadIdx.x] = 0u;
@@ -1439,7 +1469,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         }
         // a unit whose first blocks alone fill half the value window stops
         // at the window's rows, so the numeric pass handles it in one sweep
-        const int dl = kmax / kBR;
+        const int dl = max(kmax / kBR, 1);
         if (lo - start + 1 > dl && bpre[start + dl - 1] - before >= kmax / 2) lo = start + dl - 1;
         const int c = bpre[lo] - before;
         if (c > 0) {
@@ -1572,7 +1602,7 @@ __global__ __launch_bounds__(256) void k_sym_cut(const int32_t* __restrict__ ord
           if (bpre[mid] <= lim) lo = mid;
           else hi = mid - 1;
         }
-        const int dl = kmax / kBR;
+        const int dl = max(kmax / kBR, 1);
         if (lo - start + 1 > dl && bpre[start + dl - 1] - before >= kmax / 2) lo = start + dl - 1;
         const int cu = bpre[lo] - before;
         if (cu > 0) {
@@ -1607,106 +1637,87 @@ __global__ __launch_bounds__(256) void k_sym_cut(const int32_t* __restrict__ ord
   if (threadIdx.x == 0) nnzcol[col] = colcnt;
 }
 
-// Emission of a unit's cnt outputs at `out`, rows ascending.  direct: the
-// value of window row r sits at vals[r] (rows [0, ninit), presence in bits);
-// otherwise at vals[rank], with the rank of a row given by its bitmap word's
-// prefix count pre[] and the rows staged in rank order in the value array's
-// LDS after the values have left (every Acc is at least 4 bytes), so both
-// leave in full, coalesced lines.  With the filter on, only entries with
-// !(v < thr) are written, compacted at `out`, and the unit's range is
-// appended to the run list; `scratch` (LDS no longer needed by the caller,
-// cnt bits) holds the kept flags between the value and row passes.
-template <int K, class T, int NT>
-__device__ __forceinline__ void unit_emit(bool direct, int ninit, int cnt, int nw64, const uint32_t* bits,
-                                          const uint16_t* pre, typename Sem<K, T>::Acc* vals, int32_t row0,
+// A unit's accumulators: vals[row] for the DR rows of a direct unit (at most
+// DR / kBR blocks), or vals[rank] with the rows of its KMAX outputs at most
+// behind them (16 bits each: a unit spans at most 16 blocks).  Every product
+// leaves its row at its rank as it accumulates, so rows are emitted like
+// values; rebuilding them from the bitmap's words, as many steps as the
+// fullest of 64 words had outputs, took as long as a third of the unit.
+template <class Lds, int KMAX, int DR>
+struct UnitWindow {
+  static constexpr size_t bytes =
+      sizeof(Lds) * DR > (sizeof(Lds) + 2) * KMAX ? sizeof(Lds) * DR : (sizeof(Lds) + 2) * KMAX;
+  __align__(16) unsigned char mem[bytes];
+  __device__ __forceinline__ Lds* vals() { return reinterpret_cast<Lds*>(mem); }
+  __device__ __forceinline__ uint16_t* rows() { return reinterpret_cast<uint16_t*>(mem + sizeof(Lds) * KMAX); }
+};
+
+// pre[w] = outputs of the unit below bitmap word w, four words per thread and
+// step; returns their number.  Contains barriers.
+template <int NT, int NW32>
+__device__ __forceinline__ int unit_prefix(const uint32_t* bits, uint16_t* pre, int nw32, int* isum) {
+  static_assert(NW32 % 4 == 0 && NW32 <= 4 * NT, "one step");
+  const int w = threadIdx.x * 4;
+  uint4 q{0, 0, 0, 0};
+  if (w < nw32) q = *reinterpret_cast<const uint4*>(bits + w);
+  const int c0 = __popc(q.x), c1 = c0 + __popc(q.y), c2 = c1 + __popc(q.z), c3 = c2 + __popc(q.w);
+  int total;
+  const int ex = block_excl_scan<NT>(c3, isum, total);
+  if (w < nw32) {
+    const uint2 p{(uint32_t)ex | (uint32_t)(ex + c0) << 16, (uint32_t)(ex + c1) | (uint32_t)(ex + c2) << 16};
+    *reinterpret_cast<uint2*>(pre + w) = p;
+  }
+  __syncthreads();
+  return total;
+}
+
+// Emission of a unit's cnt outputs at `out`, rows ascending: from rows and
+// vals in rank order, or (direct) from the rows present in the window, a wave
+// per 64 rows.
+template <int K, class T, int NT, int KMAX, int DR>
+__device__ __forceinline__ void unit_emit(bool direct, int nw32, int cnt, const uint32_t* bits, const uint16_t* pre,
+                                          UnitWindow<typename Sem<K, T>::Lds, KMAX, DR>& win, int32_t row0,
                                           int64_t out, int64_t* __restrict__ irC, T* __restrict__ valC,
-                                          const Filter<T>& flt, int col, uint32_t* scratch, long long* wsum,
-                                          int* err) {
+                                          const Filter<T>& flt, int col, int* isum, int* err) {
   using SR = Sem<K, T>;
-  auto rank_of = [&](int32_t r) {
-    const int w = r >> 6, b = r & 63;
-    const uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
-    return (int)pre[w] + __popcll(word & ((1ull << b) - 1ull));
-  };
-  auto present = [&](int r) { return ((bits[r >> 5] >> (r & 31)) & 1u) != 0; };
+  constexpr int NW = NT / kWave;
+  auto* vals = win.vals();
+  const uint16_t* rows = win.rows();
+  if (flt.on) {
+    auto in_window = [&](int i, T& v) {
+      v = SR::lout(vals[i]);
+      return ((bits[i >> 5] >> (i & 31)) & 1u) != 0;
+    };
+    auto at_rank = [&](int i, T& v) {
+      v = SR::lout(vals[i]);
+      return true;
+    };
+    if (direct)
+      emit_filtered<T, NT>(nw32 * 32, cnt, in_window, [&](int i) { return (int64_t)row0 + i; }, out, irC, valC, flt,
+                           col, isum, err);
+    else
+      emit_filtered<T, NT>(cnt, cnt, at_rank, [&](int i) { return (int64_t)row0 + rows[i]; }, out, irC, valC, flt, col,
+                           isum, err);
+    return;
+  }
   if (direct) {
-    if (!flt.on) {  // one thread per row, stores stay coalesced
-      for (int r = threadIdx.x; r < ninit; r += NT) {
-        if (!present(r)) continue;
-        const int q = rank_of(r);
-        if (q < cnt) {
-          irC[out + q] = (int64_t)row0 + r;
-          valC[out + q] = SR::out(vals[r]);
-        }
+    for (int q = wave_id_uniform(); q < nw32 / 2; q += NW) {
+      const uint32_t lo = __builtin_amdgcn_readfirstlane(bits[2 * q]);
+      const uint32_t hi = __builtin_amdgcn_readfirstlane(bits[2 * q + 1]);
+      const uint32_t p = __builtin_amdgcn_readfirstlane((int)pre[2 * q]);
+      const int at = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, p));
+      const int r = q * 64 + lane_id();
+      if (((lane_id() < 32 ? lo : hi) >> (lane_id() & 31) & 1u) && at < cnt) {
+        irC[out + at] = (int64_t)row0 + r;
+        valC[out + at] = SR::lout(vals[r]);
       }
-      return;
     }
-    int kept = 0;
-    for (int c0 = 0; c0 < ninit; c0 += NT) {
-      const int r = c0 + threadIdx.x;
-      T v{};
-      bool keep = false;
-      if (r < ninit && present(r)) {
-        v = SR::out(vals[r]);
-        keep = !(v < flt.thr);
-      }
-      long long tot;
-      const int ex = (int)block_excl_scan_ll<NT>(keep ? 1 : 0, wsum, tot);
-      if (keep && kept + ex < cnt) {
-        irC[out + kept + ex] = (int64_t)row0 + r;
-        valC[out + kept + ex] = v;
-      }
-      kept += (int)tot;
-    }
-    if (threadIdx.x == 0) filter_add_run(flt, out, min(kept, cnt), col, err);
     return;
   }
-  int kept = 0;
-  if (!flt.on) {
-    for (int i = threadIdx.x; i < cnt; i += NT) valC[out + i] = SR::out(vals[i]);
-  } else {
-    for (int i = threadIdx.x; i <= cnt / 32; i += NT) scratch[i] = 0u;
-    __syncthreads();
-    for (int c0 = 0; c0 < cnt; c0 += NT) {
-      const int i = c0 + threadIdx.x;
-      const T v = i < cnt ? SR::out(vals[i]) : T{};
-      const bool keep = i < cnt && !(v < flt.thr);
-      long long tot;
-      const int ex = (int)block_excl_scan_ll<NT>(keep ? 1 : 0, wsum, tot);
-      if (keep) {
-        valC[out + kept + ex] = v;
-        atomicOr(&scratch[i >> 5], 1u << (i & 31));
-      }
-      kept += (int)tot;
-    }
+  for (int i = threadIdx.x; i < cnt; i += NT) {
+    irC[out + i] = (int64_t)row0 + rows[i];
+    valC[out + i] = SR::lout(vals[i]);
   }
-  __syncthreads();
-  uint32_t* rstage = reinterpret_cast<uint32_t*>(vals);
-  for (int w = threadIdx.x; w < nw64; w += NT) {
-    uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
-    int q = pre[w];
-    while (word) {
-      const int b = __ffsll((unsigned long long)word) - 1;
-      word &= word - 1;
-      if (q < cnt) rstage[q] = (uint32_t)(w * 64 + b);
-      ++q;
-    }
-  }
-  __syncthreads();
-  if (!flt.on) {
-    for (int i = threadIdx.x; i < cnt; i += NT) irC[out + i] = (int64_t)row0 + rstage[i];
-    return;
-  }
-  int kept2 = 0;
-  for (int c0 = 0; c0 < cnt; c0 += NT) {
-    const int i = c0 + threadIdx.x;
-    const bool keep = i < cnt && ((scratch[i >> 5] >> (i & 31)) & 1u);
-    long long tot;
-    const int ex = (int)block_excl_scan_ll<NT>(keep ? 1 : 0, wsum, tot);
-    if (keep) irC[out + kept2 + ex] = (int64_t)row0 + rstage[i];
-    kept2 += (int)tot;
-  }
-  if (threadIdx.x == 0) filter_add_run(flt, out, kept, col, err);
 }
 
 // Numeric pass of the unit tier: one workgroup per unit.  Sweep 1 sets the
@@ -1718,14 +1729,14 @@ __device__ __forceinline__ void unit_emit(bool direct, int ninit, int cnt, int n
 // eight for a value window of at most 16 KB (4-byte accumulators; 64 VGPRs),
 // else six (three 512-thread workgroups of 51 KB; 80 VGPRs).  Left alone, the
 // compiler keeps 81, and a third workgroup stays out.
-template <class Acc, int NT, int KMAX>
+template <class Lds, int NT, int DR>
 struct UnitWaves {
-  static constexpr int value = NT != 512 ? 1 : sizeof(Acc) * KMAX <= 16384 ? 8 : 6;
+  static constexpr int value = NT != 512 ? 1 : sizeof(Lds) * DR <= 16384 ? 8 : 6;
 };
 
-template <int K, class T, int NT, int U, int KMAX, int RBLK, int CR>
+template <int K, class T, int NT, int U, int KMAX, int DR, int RBLK, int CR>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
-    UnitWaves<typename Sem<K, T>::Acc, NT, KMAX>::value))) void k_num_units(const Unit* __restrict__ units,
+    UnitWaves<typename Sem<K, T>::Lds, NT, DR>::value))) void k_num_units(const Unit* __restrict__ units,
                                                                             const int64_t* __restrict__ cpB,
                                                   const int32_t* __restrict__ bpos, const T* __restrict__ valB,
                                                   const int64_t* __restrict__ cpA, const int32_t* __restrict__ rowsA,
@@ -1735,13 +1746,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
   using SR = Sem<K, T>;
   using Acc = typename SR::Acc;
   constexpr int NW32 = RBLK * kBRW;   // bitmap words
-  constexpr int NW64 = NW32 / 2;
-  constexpr int WPT = (NW64 + NT - 1) / NT;  // 64-bit words per thread in the prefix scan
-  __shared__ Acc vals[KMAX];
-  __shared__ uint32_t bits[NW32];
-  __shared__ uint16_t pre[NW64];
+  __shared__ UnitWindow<typename SR::Lds, KMAX, DR> win;
+  __shared__ __align__(16) uint32_t bits[NW32];
+  __shared__ __align__(8) uint16_t pre[NW32];
   __shared__ FlatStage<T, NT, true> st;
-  __shared__ long long wsum[NT / kWave];
+  __shared__ int isum[NT / kWave];
+  auto* vals = win.vals();
+  uint16_t* rows = win.rows();
   const Unit un = units[xcd_unit((int)blockIdx.x, (int)gridDim.x, xg)];
   const int col = un.col;
   const int t_lo = un.blk_lo, t_hi = un.blk_hi;
@@ -1752,15 +1763,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
   // A unit whose rows fit the value window (dense output) accumulates at
   // vals[row - row0] in a single sweep; the others count first and
   // accumulate at the rank in a second sweep.
-  const bool direct = (t_hi - t_lo) * kBR <= KMAX;
+  const bool direct = (t_hi - t_lo) * kBR <= DR;
   const bool single_chunk = !direct && (b1 - b0) <= NT;
-  if (cnt > KMAX || t_hi - t_lo > RBLK) {  // units are cut to fit; guard anyway
+  if ((!direct && cnt > KMAX) || t_hi - t_lo > RBLK) {  // units are cut to fit; guard anyway
     if (threadIdx.x == 0) atomicOr(err, 64);
     return;
   }
   const int ninit = direct ? (t_hi - t_lo) * kBR : cnt;
   flat_init(st);
-  for (int i = threadIdx.x; i < ninit; i += NT) vals[i] = SR::ident();
+  for (int i = threadIdx.x; i < ninit; i += NT) vals[i] = SR::lident();
   const int nw32 = (t_hi - t_lo) * kBRW;
   for (int i = threadIdx.x; i < nw32; i += NT) bits[i] = 0u;
 
@@ -1772,9 +1783,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
       if (ok[u]) atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
   };
   auto rank_of = [&](int32_t r) {
-    const int w = r >> 6, b = r & 63;
-    const uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
-    return (int)pre[w] + __popcll(word & ((1ull << b) - 1ull));
+    const int w = r >> 5;
+    return (int)pre[w] + __popc(__builtin_amdgcn_ubfe(bits[w], 0, r & 31));
   };
   auto ranks_of = [&](const int32_t(&r)[U], int(&rank)[U]) {  // all the LDS reads in flight together
 #pragma unroll
@@ -1790,7 +1800,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
     ranks_of(r, rank);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (ok[u] && rank[u] < cnt) SR::acc(&vals[rank[u]], SR::mul(a[u], bvs[u]));
+      if (ok[u] && rank[u] < cnt) {
+        SR::acc(&vals[rank[u]], SR::mul(a[u], bvs[u]));
+        rows[rank[u]] = (uint16_t)r[u];
+      }
   };
 
   int32_t crow[CR][U];
@@ -1849,31 +1862,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
     }
   }
   __syncthreads();
-  // exclusive prefix popcount per 64-bit word
-  const int nw64 = nw32 / 2;
-  {
-    int local[WPT];
-    int sum = 0;
-#pragma unroll
-    for (int q = 0; q < WPT; ++q) {
-      const int w = threadIdx.x * WPT + q;
-      const int c = w < nw64 ? __popc(bits[2 * w]) + __popc(bits[2 * w + 1]) : 0;
-      local[q] = sum;
-      sum += c;
-    }
-    long long total;
-    const int ex = (int)block_excl_scan_ll<NT>(sum, wsum, total);
-#pragma unroll
-    for (int q = 0; q < WPT; ++q) {
-      const int w = threadIdx.x * WPT + q;
-      if (w < nw64) pre[w] = (uint16_t)(ex + local[q]);
-    }
-    if (threadIdx.x == 0 && total != cnt) atomicOr(err, 128);
-  }
-  __syncthreads();
+  const int total = unit_prefix<NT, NW32>(bits, pre, nw32, isum);
+  if (threadIdx.x == 0 && total != cnt) atomicOr(err, 128);
   if (direct) {  // values already sit at their rows
-    unit_emit<K, T, NT>(true, ninit, cnt, nw64, bits, pre, vals, row0, out, irC, valC, flt, col,
-                        reinterpret_cast<uint32_t*>(&st), wsum, err);
+    unit_emit<K, T, NT, KMAX, DR>(true, nw32, cnt, bits, pre, win, row0, out, irC, valC, flt, col, isum, err);
     return;
   }
   // sweep 2: accumulate values at their ranks
@@ -1884,7 +1876,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
       ranks_of(crow[rr], rank);
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        if ((cok >> (rr * U + u) & 1u) && rank[u] < cnt) SR::acc(&vals[rank[u]], cprod[rr][u]);
+        if ((cok >> (rr * U + u) & 1u) && rank[u] < cnt) {
+          SR::acc(&vals[rank[u]], cprod[rr][u]);
+          rows[rank[u]] = (uint16_t)crow[rr][u];
+        }
     }
     flat_visit<T, NT, true, U>(st, ft, me.total, accumulate, CR);
   } else {
@@ -1898,8 +1893,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
     }
   }
   __syncthreads();
-  unit_emit<K, T, NT>(false, ninit, cnt, nw64, bits, pre, vals, row0, out, irC, valC, flt, col,
-                      reinterpret_cast<uint32_t*>(&st), wsum, err);
+  unit_emit<K, T, NT, KMAX, DR>(false, nw32, cnt, bits, pre, win, row0, out, irC, valC, flt, col, isum, err);
 }
 
 // Numeric pass of the unit tier with the symbolic pass's row map: the unit's
@@ -1907,7 +1901,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
 // its prefix popcounts, and one sweep gathers every product once and
 // accumulates it at its rank (at its row for a unit whose rows fit the value
 // window).
-template <int K, class T, int NT, int U, int KMAX, int RBLK>
+template <int K, class T, int NT, int U, int KMAX, int DR, int RBLK>
 __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ units, const uint32_t* __restrict__ rmap,
                                                      const int64_t* __restrict__ cpB, const int32_t* __restrict__ bpos,
                                                      const T* __restrict__ valB, const int64_t* __restrict__ cpA,
@@ -1919,13 +1913,13 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
   using SR = Sem<K, T>;
   using Acc = typename SR::Acc;
   constexpr int NW32 = RBLK * kBRW;
-  constexpr int NW64 = NW32 / 2;
-  constexpr int WPT = (NW64 + NT - 1) / NT;
-  __shared__ Acc vals[KMAX];
-  __shared__ uint32_t bits[NW32];
-  __shared__ uint16_t pre[NW64];
+  __shared__ UnitWindow<typename SR::Lds, KMAX, DR> win;
+  __shared__ __align__(16) uint32_t bits[NW32];
+  __shared__ __align__(8) uint16_t pre[NW32];
   __shared__ FlatStage<T, NT, true> st;
-  __shared__ long long wsum[NT / kWave];
+  __shared__ int isum[NT / kWave];
+  auto* vals = win.vals();
+  uint16_t* rows = win.rows();
   const Unit un = units[xcd_unit((int)blockIdx.x, (int)gridDim.x, xg)];
   const int col = un.col;
   const int t_lo = un.blk_lo, t_hi = un.blk_hi;
@@ -1933,43 +1927,23 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
   const int cnt = un.cnt;
   const int64_t out = cpC[col] + un.off;
   const int64_t b0 = cpB[col], b1 = cpB[col + 1];
-  const bool direct = (t_hi - t_lo) * kBR <= KMAX;
-  if (cnt > KMAX || t_hi - t_lo > RBLK || t_lo < 0 || t_hi > S || un.slot < 0 || un.slot >= rm_cols) {
+  const bool direct = (t_hi - t_lo) * kBR <= DR;
+  if ((!direct && cnt > KMAX) || t_hi - t_lo > RBLK || t_lo < 0 || t_hi > S || un.slot < 0 || un.slot >= rm_cols) {
     if (threadIdx.x == 0) atomicOr(err, 64);
     return;
   }
   const int ninit = direct ? (t_hi - t_lo) * kBR : cnt;
   flat_init(st);
-  for (int i = threadIdx.x; i < ninit; i += NT) vals[i] = SR::ident();
+  for (int i = threadIdx.x; i < ninit; i += NT) vals[i] = SR::lident();
   const int nw32 = (t_hi - t_lo) * kBRW;
   const uint32_t* src = rmap + (int64_t)un.slot * S * kBRW + (int64_t)t_lo * kBRW;
   for (int i = threadIdx.x; i < nw32; i += NT) bits[i] = src[i];
   __syncthreads();
-  const int nw64 = nw32 / 2;
-  {
-    int local[WPT];
-    int sum = 0;
-#pragma unroll
-    for (int q = 0; q < WPT; ++q) {
-      const int w = threadIdx.x * WPT + q;
-      const int c = w < nw64 ? __popc(bits[2 * w]) + __popc(bits[2 * w + 1]) : 0;
-      local[q] = sum;
-      sum += c;
-    }
-    long long total;
-    const int ex = (int)block_excl_scan_ll<NT>(sum, wsum, total);
-#pragma unroll
-    for (int q = 0; q < WPT; ++q) {
-      const int w = threadIdx.x * WPT + q;
-      if (w < nw64) pre[w] = (uint16_t)(ex + local[q]);
-    }
-    if (threadIdx.x == 0 && total != cnt) atomicOr(err, 128);
-  }
-  __syncthreads();
+  const int total = unit_prefix<NT, NW32>(bits, pre, nw32, isum);
+  if (threadIdx.x == 0 && total != cnt) atomicOr(err, 128);
   auto rank_of = [&](int32_t r) {
-    const int w = r >> 6, b = r & 63;
-    const uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
-    return (int)pre[w] + __popcll(word & ((1ull << b) - 1ull));
+    const int w = r >> 5;
+    return (int)pre[w] + __popc(__builtin_amdgcn_ubfe(bits[w], 0, r & 31));
   };
   auto ranks_of = [&](const int32_t(&r)[U], int(&rank)[U]) {  // all the LDS reads in flight together
 #pragma unroll
@@ -1990,7 +1964,10 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (ok[u] && q[u] < (direct ? ninit : cnt)) SR::acc(&vals[q[u]], SR::mul(a[u], bvs[u]));
+      if (ok[u] && q[u] < (direct ? ninit : cnt)) {
+        SR::acc(&vals[q[u]], SR::mul(a[u], bvs[u]));
+        if (!direct) rows[q[u]] = (uint16_t)r[u];
+      }
   };
   int par = 0;
   for (int64_t eb = b0; eb < b1; eb += NT) {
@@ -2002,8 +1979,7 @@ __global__ __launch_bounds__(NT) void k_num_units_rm(const Unit* __restrict__ un
     flat_chunk<T, NT, true, U>(st, me, par, accumulate);
   }
   __syncthreads();
-  unit_emit<K, T, NT>(direct, ninit, cnt, nw64, bits, pre, vals, row0, out, irC, valC, flt, col,
-                      reinterpret_cast<uint32_t*>(&st), wsum, err);
+  unit_emit<K, T, NT, KMAX, DR>(direct, nw32, cnt, bits, pre, win, row0, out, irC, valC, flt, col, isum, err);
 }
 
 // Numeric pass of the list units: at most KMAX outputs of one column over
@@ -2027,7 +2003,7 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
   using Acc = typename SR::Acc;
   constexpr int BPP = 256;  // blocks of one symbolic cutting pass
   static_assert(NT > BPP, "one block count per thread, plus the total");
-  __shared__ Acc vals[KMAX];
+  __shared__ typename SR::Lds vals[KMAX];
   __shared__ uint16_t lst[KMAX];
   __shared__ int s_full[NT / kWave];  // each wave's blocks: none with 16 outputs, some with 16, some with 64
   __shared__ int dir[BPP + 1];  // list position of each block's first row; dir[nb] = cnt
@@ -2048,7 +2024,7 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
   const uint16_t* src = lists + list_off[un.slot] + un.off;
   for (int i = threadIdx.x; i < cnt; i += NT) {
     lst[i] = src[i];
-    vals[i] = SR::ident();
+    vals[i] = SR::lident();
   }
   {
     const int c = threadIdx.x < nb ? (int)bcnt16[(int64_t)un.slot * S + t_lo + threadIdx.x] : 0;
@@ -2120,28 +2096,15 @@ __global__ __launch_bounds__(NT) void k_num_list(const Unit* __restrict__ units,
   if (!flt.on) {
     for (int i = threadIdx.x; i < cnt; i += NT) {
       irC[out + i] = row_of(i);
-      valC[out + i] = SR::out(vals[i]);
+      valC[out + i] = SR::lout(vals[i]);
     }
     return;
   }
-  int kept = 0;
-  for (int c0 = 0; c0 < cnt; c0 += NT) {
-    const int i = c0 + threadIdx.x;
-    T v{};
-    bool keep = false;
-    if (i < cnt) {
-      v = SR::out(vals[i]);
-      keep = !(v < flt.thr);
-    }
-    long long tot;
-    const int ex = (int)block_excl_scan_ll<NT>(keep ? 1 : 0, wsum, tot);
-    if (keep) {
-      irC[out + kept + ex] = row_of(i);
-      valC[out + kept + ex] = v;
-    }
-    kept += (int)tot;
-  }
-  if (threadIdx.x == 0) filter_add_run(flt, out, kept, col, err);
+  auto item = [&](int i, T& v) {
+    v = SR::lout(vals[i]);
+    return true;
+  };
+  emit_filtered<T, NT>(cnt, cnt, item, row_of, out, irC, valC, flt, col, s_full, err);
 }
 
 // Predictor features per stored column of B (one wave per column); see
@@ -2348,7 +2311,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   constexpr int NW32 = RBLK * kBRW;
   constexpr int NW64 = NW32 / 2;
   constexpr int WPT = (NW64 + NT - 1) / NT;
-  __shared__ Acc vals[KMAX];
+  __shared__ typename SR::Lds vals[KMAX];
   __shared__ uint32_t bits[NW32];
   // exclusive prefix counts: 16 bits while 64 * NW64 <= 65536
   using PreT = typename std::conditional<(64 * NW64 <= 65536), uint16_t, int32_t>::type;
@@ -2413,7 +2376,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   const bool direct = valid && (t_hi - t_lo) * kBR <= KMAX;
   const int ndirect = direct ? (t_hi - t_lo) * kBR : 0;
   if (direct) {
-    for (int i = threadIdx.x; i < ndirect; i += NT) vals[i] = SR::ident();
+    for (int i = threadIdx.x; i < ndirect; i += NT) vals[i] = SR::lident();
     // (the staging barriers below order the window's initialisation before any accumulation)
     auto acc_direct = [&](const int32_t(&idx)[U], T(&bvs)[U], const bool(&ok)[U]) {
       int32_t r[U];
@@ -2543,14 +2506,14 @@ __global__ __launch_bounds__(NT) void k_num_learned(
         if (!((bits[r >> 5] >> (r & 31)) & 1u)) continue;
         const int q = rank_of(r);
         irC[out + q] = (int64_t)row0 + r;
-        valC[out + q] = SR::out(vals[r]);
+        valC[out + q] = SR::lout(vals[r]);
       }
     return;
   }
   // values, in windows of KMAX ranks (one window unless the unit overflowed)
   for (q0 = 0; q0 < cnt; q0 += KMAX) {
     const int wn = min(KMAX, cnt - q0);
-    for (int i = threadIdx.x; i < wn; i += NT) vals[i] = SR::ident();
+    for (int i = threadIdx.x; i < wn; i += NT) vals[i] = SR::lident();
     __syncthreads();
     if (cached) {
 #pragma unroll
@@ -2575,7 +2538,7 @@ __global__ __launch_bounds__(NT) void k_num_learned(
     }
     __syncthreads();
     if (can_write)
-      for (int i = threadIdx.x; i < wn; i += NT) valC[out + q0 + i] = SR::out(vals[i]);
+      for (int i = threadIdx.x; i < wn; i += NT) valC[out + q0 + i] = SR::lout(vals[i]);
     __syncthreads();
   }
   if (can_write) {
@@ -2824,16 +2787,12 @@ constexpr int kSymRBW = 32768;                // bitmap words per symbolic pass 
 // unit tier
 constexpr int kSymUnitNT = 512, kSymUnitIBLK = 64;  // 32 KB bitmap: three workgroups per CU
 constexpr int kSymBandNT = 256;                     // banded symbolic pass
-// light units span at most 16 blocks: ~53 KB of LDS, three workgroups per CU
-constexpr int kLightNT = 512, kLightK = 4096, kLightRB = 16;    // <= 4096 outputs, <= 64K rows
-constexpr int kHeavyNT = 1024, kHeavyK = 16384, kHeavyRB = 16;  // <= 16384 outputs, <= 64K rows
-// The large units' value window: 16384 outputs, or 12288 for 4-byte
-// accumulators, whose large-unit kernel then takes about 76 KB of LDS
-// instead of 92 KB: two workgroups per CU, eight waves per SIMD, not four.
-template <int K, class T>
-constexpr int heavy_k() {
-  return sizeof(typename Sem<K, T>::Acc) <= 4 ? 12288 : kHeavyK;
-}
+// Light units: at most 16 blocks (64K rows) and 3264 outputs, whose 8-byte
+// accumulators and 16-bit rows share the 32 KB of a direct unit's 4096 rows:
+// 53 KB of LDS with the bitmap and its prefix, three workgroups per CU.
+// Heavy units: 13056 outputs or 16384 direct rows, 128 KB.
+constexpr int kLightNT = 512, kLightK = 3264, kLightDR = 4096, kLightRB = 16;
+constexpr int kHeavyNT = 1024, kHeavyK = 13056, kHeavyDR = 16384, kHeavyRB = 16;
 // learned units: one workgroup shape for all (512 threads, 4096-entry value
 // window, 32 row blocks), cut to target * 4096 predicted outputs
 constexpr int kLearnNT = 512, kLearnK = 4096, kLearnRB = 32, kLearnCR = 2;
@@ -3099,7 +3058,7 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
       CBX_TRY(alloc_unit_lists(hcols, flop, nheavy, S, cap_l, std::min<int64_t>(cfg.unit_split_nnz, m), hucnt + 2, tmp,
                                tmp_bytes, b_lsz, b_loff, b_lists, b_lbc, b_us, s, ul));
     CBX_TRY(launch_sym_units(cfg, hcols, nheavy, A, B, bpos, rowsA, P, S, nnzcol, units_l, hucnt, (int)cap_l, units_h,
-                             hucnt + 1, (int)cap_h, rm.p, rm_cols, err, b_bcnt, heavy_k<K, T>(), s, ul));
+                             hucnt + 1, (int)cap_h, rm.p, rm_cols, err, b_bcnt, kHeavyK, s, ul));
     CBX_HIP(hipGetLastError());
   }
   CBX_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, nnzcol, hcs, (int)(nzcB + 1), s));
@@ -3190,15 +3149,15 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
     if (hu[2] > 1) CBX_TRY(sort_units_by_block(ul.units, hu[2], S, s, b_us_sorted, &ul.units));
   }
   if (hu[1] && rm.p)
-    k_num_units_rm<K, T, kHeavyNT, 4, heavy_k<K, T>(), kHeavyRB><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
+    k_num_units_rm<K, T, kHeavyNT, 4, kHeavyK, kHeavyDR, kHeavyRB><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
         units_h, rm.p, B->cp, bpos, (const T*)B->val, A->cp, rowsA, (const T*)A->val, P, S, rm_cols, cpC, C->ir,
         (T*)C->val, err, Filter<T>{}, cfg.unit_xcd_group);
   else if (hu[1])
-    k_num_units<K, T, kHeavyNT, 4, heavy_k<K, T>(), kHeavyRB, 4><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
+    k_num_units<K, T, kHeavyNT, 4, kHeavyK, kHeavyDR, kHeavyRB, 4><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
         units_h, B->cp, bpos, (const T*)B->val, A->cp, rowsA, (const T*)A->val, P, S, cpC, C->ir, (T*)C->val, err,
         Filter<T>{}, cfg.unit_xcd_group);
   if (hu[0])
-    k_num_units<K, T, kLightNT, 4, kLightK, kLightRB, 2><<<(unsigned)hu[0], kLightNT, 0, s>>>(
+    k_num_units<K, T, kLightNT, 4, kLightK, kLightDR, kLightRB, 2><<<(unsigned)hu[0], kLightNT, 0, s>>>(
         units_l, B->cp, bpos, (const T*)B->val, A->cp, rowsA, (const T*)A->val, P, S, cpC, C->ir, (T*)C->val, err,
         Filter<T>{}, cfg.unit_xcd_group);
   if (hu[2])
@@ -3530,7 +3489,7 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
       if (ul.lists && lists_used) *lists_used = true;
     }
     CBX_TRY(launch_sym_units(cfg, order_s, n_dense, A, B, bpos, rowsA, tiles, S, nnzcol, units_l, ucnt, (int)cap_l, units_h,
-                             ucnt + 1, (int)cap_h, rmap, rm_cols, err, b_bcnt, heavy_k<K, T>(), s, ul));
+                             ucnt + 1, (int)cap_h, rmap, rm_cols, err, b_bcnt, kHeavyK, s, ul));
   } else if (n_dense) {
     k_sym_dense<kSymNT, kSymRBW><<<(unsigned)n_dense, kSymNT, 0, s>>>(order_s, 0, B->cp, bpos, A->cp, rowsA, P, S, G,
                                                                        TR, nnzcol);
@@ -3631,14 +3590,14 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
     // units keep the two-sweep kernel, whose second sweep mostly replays
     // registers
     if (hu[1] && rmap)
-      k_num_units_rm<K, T, kHeavyNT, 4, heavy_k<K, T>(), kHeavyRB><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
+      k_num_units_rm<K, T, kHeavyNT, 4, kHeavyK, kHeavyDR, kHeavyRB><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
           units_h, rmap, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, rm_cols, cpC, C->ir, (T*)C->val, err, flt,
           cfg.unit_xcd_group);
     else if (hu[1])
-      k_num_units<K, T, kHeavyNT, 4, heavy_k<K, T>(), kHeavyRB, 4><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
+      k_num_units<K, T, kHeavyNT, 4, kHeavyK, kHeavyDR, kHeavyRB, 4><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
           units_h, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, cpC, C->ir, (T*)C->val, err, flt, cfg.unit_xcd_group);
     if (hu[0])
-      k_num_units<K, T, kLightNT, 4, kLightK, kLightRB, 2><<<(unsigned)hu[0], kLightNT, 0, s>>>(
+      k_num_units<K, T, kLightNT, 4, kLightK, kLightDR, kLightRB, 2><<<(unsigned)hu[0], kLightNT, 0, s>>>(
           units_l, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, cpC, C->ir, (T*)C->val, err, flt, cfg.unit_xcd_group);
     if (hu[2])
       k_num_list<K, T, kLightNT, 4, kLightK><<<(unsigned)hu[2], kLightNT, 0, s>>>(

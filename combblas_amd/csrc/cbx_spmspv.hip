@@ -1085,7 +1085,7 @@ __global__ __launch_bounds__(kSvNT) void k_svb_accumulate(const int64_t* __restr
                                                           const int* __restrict__ malformed) {
   using SR = Sem<K, T>;
   using Acc = typename SR::Acc;
-  __shared__ Acc acc[kSvBR];
+  __shared__ typename SR::Lds acc[kSvBR];
   if (*malformed) return;  // y is left as it was
   const int64_t g = blockIdx.x;
   if (g >= cstart[nblk]) return;
@@ -1093,7 +1093,7 @@ __global__ __launch_bounds__(kSvNT) void k_svb_accumulate(const int64_t* __restr
   const int64_t lo = offs[(int64_t)b * ntiles], hi = b + 1 < nblk ? offs[(int64_t)(b + 1) * ntiles] : nnz;
   const int64_t c = g - cstart[b], nch = cstart[b + 1] - cstart[b];
   const int64_t i0 = lo + c * kSvChunk, i1 = min<int64_t>(hi, i0 + kSvChunk);
-  for (int r = threadIdx.x; r < kSvBR; r += kSvNT) acc[r] = SR::ident();
+  for (int r = threadIdx.x; r < kSvBR; r += kSvNT) acc[r] = SR::lident();
   __syncthreads();
   for (int64_t i = i0 + threadIdx.x; i < i1; i += kSvNT) SR::acc(&acc[brow[i]], (Acc)bval[i]);
   __syncthreads();
@@ -1101,7 +1101,7 @@ __global__ __launch_bounds__(kSvNT) void k_svb_accumulate(const int64_t* __restr
   using Bits = typename std::conditional<sizeof(Acc) == 8, unsigned long long, unsigned int>::type;
   const Bits id = __builtin_bit_cast(Bits, SR::ident());
   for (int r = threadIdx.x; r < kSvBR && row0 + r < m; r += kSvNT) {
-    const Acc a = acc[r];
+    const Acc a = (Acc)SR::lout(acc[r]);
     if (nch == 1) {
       y[row0 + r] = (T)SR::out(SR::add((Acc)y[row0 + r], a));
     } else if (__builtin_bit_cast(Bits, a) != id) {  // the identity changes nothing
