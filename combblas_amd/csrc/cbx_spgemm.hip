@@ -1326,7 +1326,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
   constexpr int BMW = IBLK * kBRW;     // bitmap words of one sub-pass
   static_assert(BPP % IBLK == 0, "sub-passes tile the cutting pass");
   static_assert(IBLK <= kWave, "a wave scans the block counts of a sub-pass");
-  __shared__ uint32_t bits[BMW];
+  __shared__ __align__(16) uint32_t bits[BMW];
   __shared__ int bpre[BPP];           // block counts, then their inclusive prefix
   __shared__ FlatStage<uint8_t, NT, false> st;
   __shared__ int s_nu, s_slot, s_ns, s_sslot;
@@ -1357,7 +1357,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
     for (int i_lo = t_lo; i_lo < t_hi; i_lo += IBLK) {
       const int i_hi = min(t_hi, i_lo + IBLK), inb = i_hi - i_lo;
       const int32_t row0 = i_lo * kBR;
-      for (int i = threadIdx.x; i < inb * kBRW; i += NT) bits[i] = 0u;
+      for (int i = threadIdx.x * 4; i < inb * kBRW; i += NT * 4) *reinterpret_cast<uint4*>(bits + i) = uint4{0, 0, 0, 0};
       // (the staging barrier below orders the clear before any insertion)
       for (int64_t eb = b0; eb < b1; eb += NT) {
         int64_t base;
@@ -1384,10 +1384,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         for (int i = threadIdx.x; i < inb * kBRW; i += NT) dst[i] = bits[i];
       }
       // per-block counts: one wave per block, two words per lane
-      for (int b = wave_id(); b < inb; b += NT / kWave) {
-        const uint32_t* w = bits + b * kBRW;
-        int c = __popc(w[lane_id()]) + __popc(w[lane_id() + kWave]);
-        c = (int)wave_sum_ll(c);
+      for (int b = wave_id_uniform(); b < inb; b += NT / kWave) {
+        const uint2 x = reinterpret_cast<const uint2*>(bits + b * kBRW)[lane_id()];
+        const int c = __builtin_amdgcn_readlane(wave_incl_scan(__popc(x.x) + __popc(x.y)), kWave - 1);
         if (lane_id() == 0) {
           bpre[i_lo - t_lo + b] = c;
           if (lists) bcnt16[(int64_t)blockIdx.x * S + i_lo + b] = (uint16_t)c;
@@ -1406,19 +1405,22 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
         const int64_t have = colcnt + run;
         listok = listok && have + sub_total <= region;
         if (listok) {
-          for (int b = wave_id(); b < inb; b += NT / kWave) {
-            const int boff = __shfl(bincl - bc, b, kWave);
-            if (__shfl(bc, b, kWave) > kListBlockMax) continue;  // dense block: its units use the bitmap
-            const uint32_t* w = bits + b * kBRW;
-            uint64_t x = (uint64_t)w[2 * lane_id()] | ((uint64_t)w[2 * lane_id() + 1] << 32);
-            const int c = __popcll(x);
-            const int ex = wave_incl_scan(c) - c;
-            uint16_t* dst = lists + list_base + have + boff + ex;
-            int k = 0;
-            while (x) {
-              const int bit = __ffsll((unsigned long long)x) - 1;
-              x &= x - 1;
-              dst[k++] = (uint16_t)(lane_id() * 64 + bit);
+          for (int b = wave_id_uniform(); b < inb; b += NT / kWave) {
+            const int nb = __builtin_amdgcn_readlane(bc, b);
+            if (nb == 0 || nb > kListBlockMax) continue;  // dense block: its units use the bitmap
+            const int boff = __builtin_amdgcn_readlane(bincl, b) - nb;
+            uint2 x = reinterpret_cast<const uint2*>(bits + b * kBRW)[lane_id()];
+            const int c = __popc(x.x) + __popc(x.y);
+            uint16_t* dst = lists + list_base + have + boff + (wave_incl_scan(c) - c);
+            int row = lane_id() * 64;
+            while (x.x) {
+              *dst++ = (uint16_t)(row + __builtin_ctz(x.x));
+              x.x &= x.x - 1;
+            }
+            row += 32;
+            while (x.y) {
+              *dst++ = (uint16_t)(row + __builtin_ctz(x.y));
+              x.y &= x.y - 1;
             }
           }
         }
@@ -2298,8 +2300,9 @@ constexpr unsigned long long kAggFlag = 1ull << 62, kInclFlag = 2ull << 62, kVal
 
 // One workgroup per unit, units taken in order through a ticket counter so
 // that every predecessor of a unit is already resident when it waits on it.
-template <int K, class T, int NT, int U, int KMAX, int RBLK, int CR>
-__global__ __launch_bounds__(NT) void k_num_learned(
+template <int K, class T, int NT, int U, int KMAX, int DR, int RBLK, int CR>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
+    UnitWaves<typename Sem<K, T>::Lds, NT, DR>::value))) void k_num_learned(
     const UnitL* __restrict__ units, int* __restrict__ ticket, unsigned long long* __restrict__ status,
     const int64_t* __restrict__ hcs, const int64_t* __restrict__ cpB, const int32_t* __restrict__ bpos,
     const T* __restrict__ valB, const int64_t* __restrict__ cpA, const int32_t* __restrict__ rowsA,
@@ -2309,15 +2312,13 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   using SR = Sem<K, T>;
   using Acc = typename SR::Acc;
   constexpr int NW32 = RBLK * kBRW;
-  constexpr int NW64 = NW32 / 2;
-  constexpr int WPT = (NW64 + NT - 1) / NT;
-  __shared__ typename SR::Lds vals[KMAX];
-  __shared__ uint32_t bits[NW32];
-  // exclusive prefix counts: 16 bits while 64 * NW64 <= 65536
-  using PreT = typename std::conditional<(64 * NW64 <= 65536), uint16_t, int32_t>::type;
-  __shared__ PreT pre[NW64];
+  __shared__ UnitWindow<typename SR::Lds, KMAX, DR> win;
+  __shared__ __align__(16) uint32_t bits[NW32];
+  __shared__ __align__(8) uint16_t pre[NW32];
   __shared__ FlatStage<T, NT, true> st;
-  __shared__ long long wsum[NT / kWave];
+  __shared__ int isum[NT / kWave];
+  auto* vals = win.vals();
+  uint16_t* rows = win.rows();
   __shared__ int s_t;
   __shared__ long long s_excl;
   if (threadIdx.x == 0) s_t = atomicAdd(ticket, 1);
@@ -2339,9 +2340,8 @@ __global__ __launch_bounds__(NT) void k_num_learned(
       if (ok[u]) atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
   };
   auto rank_of = [&](int32_t r) {
-    const int w = r >> 6, b = r & 63;
-    const uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
-    return (int)pre[w] + __popcll(word & ((1ull << b) - 1ull));
+    const int w = r >> 5;
+    return (int)pre[w] + __popc(__builtin_amdgcn_ubfe(bits[w], 0, r & 31));
   };
   auto ranks_of = [&](const int32_t(&r)[U], int(&rank)[U]) {  // all the LDS reads in flight together
 #pragma unroll
@@ -2358,7 +2358,10 @@ __global__ __launch_bounds__(NT) void k_num_learned(
     ranks_of(r, q);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (ok[u] && q[u] >= q0 && q[u] < q0 + KMAX) SR::acc(&vals[q[u] - q0], SR::mul(a[u], bvs[u]));
+      if (ok[u] && q[u] >= q0 && q[u] < q0 + KMAX) {
+        SR::acc(&vals[q[u] - q0], SR::mul(a[u], bvs[u]));
+        rows[q[u] - q0] = (uint16_t)r[u];
+      }
   };
 
   int32_t crow[CR][U];
@@ -2373,11 +2376,10 @@ __global__ __launch_bounds__(NT) void k_num_learned(
   if (!valid && threadIdx.x == 0) atomicOr(err, 64);
   // A unit whose rows fit the value window accumulates at its rows in a
   // single sweep (its size, known after that sweep, never exceeds the window)
-  const bool direct = valid && (t_hi - t_lo) * kBR <= KMAX;
-  const int ndirect = direct ? (t_hi - t_lo) * kBR : 0;
+  const bool direct = valid && (t_hi - t_lo) * kBR <= DR;
+  // the first window (the staging barrier orders it and the bitmap before any insertion)
+  for (int i = threadIdx.x; i < (direct ? (t_hi - t_lo) * kBR : KMAX); i += NT) vals[i] = SR::lident();
   if (direct) {
-    for (int i = threadIdx.x; i < ndirect; i += NT) vals[i] = SR::lident();
-    // (the staging barriers below order the window's initialisation before any accumulation)
     auto acc_direct = [&](const int32_t(&idx)[U], T(&bvs)[U], const bool(&ok)[U]) {
       int32_t r[U];
       T a[U];
@@ -2435,86 +2437,71 @@ __global__ __launch_bounds__(NT) void k_num_learned(
     }
   }
   __syncthreads();
-  const int nw64 = nw32 / 2;
-  int cnt;
-  {
-    int local[WPT];
-    int sum = 0;
-#pragma unroll
-    for (int q = 0; q < WPT; ++q) {
-      const int w = threadIdx.x * WPT + q;
-      const int c = w < nw64 ? __popc(bits[2 * w]) + __popc(bits[2 * w + 1]) : 0;
-      local[q] = sum;
-      sum += c;
-    }
-    long long total;
-    const int ex = (int)block_excl_scan_ll<NT>(sum, wsum, total);
-#pragma unroll
-    for (int q = 0; q < WPT; ++q) {
-      const int w = threadIdx.x * WPT + q;
-      if (w < nw64) pre[w] = (PreT)(ex + local[q]);
-    }
-    cnt = (int)total;
-  }
-  // publish the size, then look back for the offset with the whole first
-  // wave: 64 predecessors per step, summing back to the nearest one that
-  // holds an inclusive prefix (bounded wait on predecessors still counting).
-  // A status word carries its flag and value together and no other data is
-  // passed between units, so the atomics are relaxed: at agent scope an
-  // acquire or release would invalidate or write back this XCD's whole L2.
-  if (threadIdx.x < kWave) {
-    const int lane = (int)threadIdx.x;
-    if (lane == 0)
-      __hip_atomic_store(&status[t], kAggFlag | (unsigned long long)cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    long long excl = 0;
-    int spins = 0;
-    for (int i = t - 1; i >= 0;) {
-      const int j = i - lane;
-      const unsigned long long v =
-          j >= 0 ? __hip_atomic_load(&status[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kInclFlag;
-      const unsigned long long incl = __ballot((v >> 62) == 2);
-      const unsigned long long none = __ballot((v >> 62) == 0);
-      const int first = incl ? __ffsll((unsigned long long)incl) - 1 : kWave;  // nearest inclusive prefix
-      const unsigned long long need = first >= kWave - 1 ? ~0ull : ((2ull << first) - 1ull);
-      if (none & need) {  // a predecessor in range has not published yet
-        if (++spins > (1 << 22)) {
-          if (lane == 0) atomicOr(err, 256);
-          break;
+  const int cnt = unit_prefix<NT, NW32>(bits, pre, nw32, isum);
+  // publish the size; the offset is looked for once the first window's values
+  // are accumulated, when most predecessors have published theirs
+  if (threadIdx.x == 0)
+    __hip_atomic_store(&status[t], kAggFlag | (unsigned long long)cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // Output offset of the unit: look back with the whole first wave, 64
+  // predecessors per step, summing back to the nearest one that holds an
+  // inclusive prefix (bounded wait on predecessors still counting).  A status
+  // word carries its flag and value together and no other data is passed
+  // between units, so the atomics are relaxed: at agent scope an acquire or
+  // release would invalidate or write back this XCD's whole L2.
+  auto look_back = [&]() {
+    if (threadIdx.x < kWave) {
+      const int lane = (int)threadIdx.x;
+      long long excl = 0;
+      int spins = 0;
+      for (int i = t - 1; i >= 0;) {
+        const int j = i - lane;
+        const unsigned long long v =
+            j >= 0 ? __hip_atomic_load(&status[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kInclFlag;
+        const unsigned long long incl = __ballot((v >> 62) == 2);
+        const unsigned long long none = __ballot((v >> 62) == 0);
+        const int first = incl ? __ffsll((unsigned long long)incl) - 1 : kWave;  // nearest inclusive prefix
+        const unsigned long long need = first >= kWave - 1 ? ~0ull : ((2ull << first) - 1ull);
+        if (none & need) {  // a predecessor in range has not published yet
+          if (++spins > (1 << 22)) {
+            if (lane == 0) atomicOr(err, 256);
+            break;
+          }
+          __builtin_amdgcn_s_sleep(2);
+          continue;
         }
-        __builtin_amdgcn_s_sleep(2);
-        continue;
+        excl += wave_sum_ll(lane <= first ? (long long)(v & kValMask) : 0ll);
+        if (first < kWave) break;
+        i -= kWave;
       }
-      excl += wave_sum_ll(lane <= first ? (long long)(v & kValMask) : 0ll);
-      if (first < kWave) break;
-      i -= kWave;
-    }
-    if (lane == 0) {
-      __hip_atomic_store(&status[t], kInclFlag | (unsigned long long)(excl + cnt), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-      s_excl = excl;
-      if (cnt) atomicAdd(&col_total[col], (unsigned long long)cnt);
-      if (cnt > KMAX) atomicAdd(ovf_units, 1);
-    }
-  }
-  __syncthreads();
-  const int64_t out = s_excl + hcs[col];
-  const bool can_write = out + cnt <= cap;
-  if (!can_write && threadIdx.x == 0) atomicOr(err, 512);
-  if (direct) {  // values sit at their rows: one thread per row, stores stay coalesced
-    if (can_write)
-      for (int r = threadIdx.x; r < ndirect; r += NT) {
-        if (!((bits[r >> 5] >> (r & 31)) & 1u)) continue;
-        const int q = rank_of(r);
-        irC[out + q] = (int64_t)row0 + r;
-        valC[out + q] = SR::lout(vals[r]);
+      if (lane == 0) {
+        __hip_atomic_store(&status[t], kInclFlag | (unsigned long long)(excl + cnt), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        s_excl = excl;
+        if (cnt) atomicAdd(&col_total[col], (unsigned long long)cnt);
+        if (cnt > (direct ? DR : KMAX)) atomicAdd(ovf_units, 1);
       }
+    }
+    __syncthreads();
+    const int64_t out = s_excl + hcs[col];
+    if (out + cnt > cap && threadIdx.x == 0) atomicOr(err, 512);
+    return out;
+  };
+  if (direct) {
+    const int64_t out = look_back();
+    if (out + cnt <= cap)
+      unit_emit<K, T, NT, KMAX, DR>(true, nw32, cnt, bits, pre, win, row0, out, irC, valC, Filter<T>{}, col, isum, err);
     return;
   }
   // values, in windows of KMAX ranks (one window unless the unit overflowed)
+  int64_t out = 0;
+  if (cnt == 0) look_back();
   for (q0 = 0; q0 < cnt; q0 += KMAX) {
     const int wn = min(KMAX, cnt - q0);
-    for (int i = threadIdx.x; i < wn; i += NT) vals[i] = SR::lident();
-    __syncthreads();
+    if (q0) {
+      __syncthreads();  // the previous window has been written
+      for (int i = threadIdx.x; i < wn; i += NT) vals[i] = SR::lident();
+      __syncthreads();
+    }
     if (cached) {
 #pragma unroll
       for (int rr = 0; rr < CR; ++rr) {
@@ -2522,7 +2509,10 @@ __global__ __launch_bounds__(NT) void k_num_learned(
         ranks_of(crow[rr], q);
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          if ((cok >> (rr * U + u) & 1u) && q[u] >= q0 && q[u] < q0 + KMAX) SR::acc(&vals[q[u] - q0], cprod[rr][u]);
+          if ((cok >> (rr * U + u) & 1u) && q[u] >= q0 && q[u] < q0 + KMAX) {
+            SR::acc(&vals[q[u] - q0], cprod[rr][u]);
+            rows[q[u] - q0] = (uint16_t)crow[rr][u];
+          }
       }
       flat_visit<T, NT, true, U>(st, ft, me.total, accumulate, CR);
     } else {
@@ -2537,30 +2527,12 @@ __global__ __launch_bounds__(NT) void k_num_learned(
       }
     }
     __syncthreads();
-    if (can_write)
-      for (int i = threadIdx.x; i < wn; i += NT) valC[out + q0 + i] = SR::lout(vals[i]);
-    __syncthreads();
-  }
-  if (can_write) {
-    // rows in rank order; staged in the value array's LDS when they fit in
-    // one window (the common case), so that they leave in coalesced lines
-    const bool staged = cnt <= KMAX;
-    uint32_t* rstage = reinterpret_cast<uint32_t*>(vals);
-    for (int w = threadIdx.x; w < nw64; w += NT) {
-      uint64_t word = (uint64_t)bits[2 * w] | ((uint64_t)bits[2 * w + 1] << 32);
-      int q = pre[w];
-      while (word) {
-        const int b = __ffsll((unsigned long long)word) - 1;
-        word &= word - 1;
-        if (staged) rstage[q] = (uint32_t)(w * 64 + b);
-        else irC[out + q] = (int64_t)row0 + w * 64 + b;
-        ++q;
+    if (q0 == 0) out = look_back();
+    if (out + cnt <= cap)
+      for (int i = threadIdx.x; i < wn; i += NT) {
+        irC[out + q0 + i] = (int64_t)row0 + rows[i];
+        valC[out + q0 + i] = SR::lout(vals[i]);
       }
-    }
-    if (staged) {
-      __syncthreads();
-      for (int i = threadIdx.x; i < cnt; i += NT) irC[out + i] = (int64_t)row0 + rstage[i];
-    }
   }
 }
 
@@ -2793,9 +2765,9 @@ constexpr int kSymBandNT = 256;                     // banded symbolic pass
 // Heavy units: 13056 outputs or 16384 direct rows, 128 KB.
 constexpr int kLightNT = 512, kLightK = 3264, kLightDR = 4096, kLightRB = 16;
 constexpr int kHeavyNT = 1024, kHeavyK = 13056, kHeavyDR = 16384, kHeavyRB = 16;
-// learned units: one workgroup shape for all (512 threads, 4096-entry value
-// window, 32 row blocks), cut to target * 4096 predicted outputs
-constexpr int kLearnNT = 512, kLearnK = 4096, kLearnRB = 32, kLearnCR = 2;
+// learned units: the light units' workgroup shape and window, cut to
+// target * 3264 predicted outputs
+constexpr int kLearnNT = 512, kLearnK = kLightK, kLearnRB = kLightRB, kLearnCR = 2;
 constexpr int kLearnFlopCap = 131072;  // expected products per learned unit
 constexpr int64_t kLearnChunk = 1 << 21;  // workgroups per learned launch
 // Tiny tier launch: `waves` columns (one wave each) per workgroup, grid-stride
@@ -3112,7 +3084,7 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   // units look back into statuses the earlier launches completed
   for (int64_t done = 0; done < nunits; done += kLearnChunk) {
     const int64_t nb = std::min<int64_t>(kLearnChunk, nunits - done);
-    k_num_learned<K, T, kLearnNT, 4, kLearnK, kLearnRB, kLearnCR><<<(unsigned)nb, kLearnNT, 0, s>>>(
+    k_num_learned<K, T, kLearnNT, 4, kLearnK, kLightDR, kLearnRB, kLearnCR><<<(unsigned)nb, kLearnNT, 0, s>>>(
         units, ticket, status, hcs, B->cp, bpos, (const T*)B->val, A->cp, rowsA, (const T*)A->val, P, S, cap, C->ir,
         (T*)C->val, col_total, ovf, err);
   }
