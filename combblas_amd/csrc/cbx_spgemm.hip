@@ -1676,16 +1676,16 @@ __device__ __forceinline__ int unit_prefix(const uint32_t* bits, uint16_t* pre, 
 // Emission of a unit's cnt outputs at `out`, rows ascending: from rows and
 // vals in rank order, or (direct) from the rows present in the window, a wave
 // per 64 rows.
-template <int K, class T, int NT, int KMAX, int DR>
+template <int K, class T, int NT, int KMAX, int DR, class R>
 __device__ __forceinline__ void unit_emit(bool direct, int nw32, int cnt, const uint32_t* bits, const uint16_t* pre,
                                           UnitWindow<typename Sem<K, T>::Lds, KMAX, DR>& win, int32_t row0,
-                                          int64_t out, int64_t* __restrict__ irC, T* __restrict__ valC,
+                                          int64_t out, R* __restrict__ irC, T* __restrict__ valC,
                                           const Filter<T>& flt, int col, int* isum, int* err) {
   using SR = Sem<K, T>;
   constexpr int NW = NT / kWave;
   auto* vals = win.vals();
   const uint16_t* rows = win.rows();
-  if (flt.on) {
+  if (sizeof(R) == 8 && flt.on) {
     auto in_window = [&](int i, T& v) {
       v = SR::lout(vals[i]);
       return ((bits[i >> 5] >> (i & 31)) & 1u) != 0;
@@ -1695,10 +1695,10 @@ __device__ __forceinline__ void unit_emit(bool direct, int nw32, int cnt, const 
       return true;
     };
     if (direct)
-      emit_filtered<T, NT>(nw32 * 32, cnt, in_window, [&](int i) { return (int64_t)row0 + i; }, out, irC, valC, flt,
+      emit_filtered<T, NT>(nw32 * 32, cnt, in_window, [&](int i) { return (int64_t)row0 + i; }, out, (int64_t*)irC, valC, flt,
                            col, isum, err);
     else
-      emit_filtered<T, NT>(cnt, cnt, at_rank, [&](int i) { return (int64_t)row0 + rows[i]; }, out, irC, valC, flt, col,
+      emit_filtered<T, NT>(cnt, cnt, at_rank, [&](int i) { return (int64_t)row0 + rows[i]; }, out, (int64_t*)irC, valC, flt, col,
                            isum, err);
     return;
   }
@@ -1710,14 +1710,14 @@ __device__ __forceinline__ void unit_emit(bool direct, int nw32, int cnt, const 
       const int at = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, p));
       const int r = q * 64 + lane_id();
       if (((lane_id() < 32 ? lo : hi) >> (lane_id() & 31) & 1u) && at < cnt) {
-        irC[out + at] = (int64_t)row0 + r;
+        irC[out + at] = (R)(row0 + r);
         valC[out + at] = SR::lout(vals[r]);
       }
     }
     return;
   }
   for (int i = threadIdx.x; i < cnt; i += NT) {
-    irC[out + i] = (int64_t)row0 + rows[i];
+    irC[out + i] = (R)(row0 + rows[i]);
     valC[out + i] = SR::lout(vals[i]);
   }
 }
@@ -2154,10 +2154,17 @@ __global__ void k_features(const int64_t* __restrict__ cpB, int64_t nzcB, const 
 }
 
 // ============================================================ learned tier
-// Single pass: units are cut from predicted column sizes, and each unit's
-// exact size (from its presence bitmap) is published to a decoupled
-// look-back chain that yields its output offset before its values are
-// accumulated and written.
+// Single pass: units are cut from predicted column sizes; a unit counts its
+// outputs from its bitmap, takes room for them from a running total, writes
+// them there (32-bit rows) and moves on.  Once all sizes are known a copy puts
+// every unit's outputs at its place.
+//
+// The copy (24 B per output more than writing in place) buys units that wait
+// for nobody.  With their places taken from a look-back over the units before
+// them, units retired in order: a unit that waits keeps its workgroup's LDS,
+// and a hub's dense blocks, of up to 1e5 products, held up the 768 units in
+// flight again and again.  At 2^17 vertices, edge factor 16, that kernel took
+// 13.2 ms with its VALU 18 % busy.
 struct UnitL {
   int32_t col;
   int32_t blk_lo;
@@ -2214,8 +2221,7 @@ __global__ void k_col_blocks(const int64_t* __restrict__ cpB, int64_t nzcB, cons
 // own (its rows fit the value window: one sweep, no counting sweep).  Other
 // units close when their expected outputs would pass `target`, their
 // expected products would pass `fcap`, or their span would pass rblk blocks.
-// Capping the products keeps every unit's counting sweep short, so no unit
-// holds its successors' look-back for long.  Pass 1 counts (out == null),
+// Capping the products keeps the units' work even.  Pass 1 counts (out == null),
 // pass 2 writes at `base`.
 __device__ __forceinline__ float distinct_rows(float flop, float wb) {
   return (float)kBR * (1.f - __expf(-flop * wb * (1.f / (float)kBR)));
@@ -2296,18 +2302,26 @@ __global__ void k_learned_units(const int64_t* __restrict__ flop, int64_t nzcB, 
   }
 }
 
-constexpr unsigned long long kAggFlag = 1ull << 62, kInclFlag = 2ull << 62, kValMask = (1ull << 62) - 1;
+// What the learned units write: sizes and places in the staging arrays, and
+// the arrays with the running total of what is taken.
+template <class T>
+struct LearnedStage {
+  int64_t* cnt;
+  int64_t* at;
+  unsigned long long* taken;
+  int64_t cap;
+  int32_t* rows;
+  T* vals;
+};
 
-// One workgroup per unit, units taken in order through a ticket counter so
-// that every predecessor of a unit is already resident when it waits on it.
+// One workgroup per unit, units first + blockIdx.x.
 template <int K, class T, int NT, int U, int KMAX, int DR, int RBLK, int CR>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
     UnitWaves<typename Sem<K, T>::Lds, NT, DR>::value))) void k_num_learned(
-    const UnitL* __restrict__ units, int* __restrict__ ticket, unsigned long long* __restrict__ status,
-    const int64_t* __restrict__ hcs, const int64_t* __restrict__ cpB, const int32_t* __restrict__ bpos,
-    const T* __restrict__ valB, const int64_t* __restrict__ cpA, const int32_t* __restrict__ rowsA,
-    const T* __restrict__ valA, const Tiles P, int S, int64_t cap, int64_t* __restrict__ irC,
-    T* __restrict__ valC, unsigned long long* __restrict__ col_total, int* __restrict__ ovf_units,
+    const UnitL* __restrict__ units, int64_t first, const int64_t* __restrict__ cpB,
+    const int32_t* __restrict__ bpos, const T* __restrict__ valB, const int64_t* __restrict__ cpA,
+    const int32_t* __restrict__ rowsA, const T* __restrict__ valA, const Tiles P, int S,
+    const LearnedStage<T> out, unsigned long long* __restrict__ col_total, int* __restrict__ ovf_units,
     int* __restrict__ err) {
   using SR = Sem<K, T>;
   using Acc = typename SR::Acc;
@@ -2317,13 +2331,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
   __shared__ __align__(8) uint16_t pre[NW32];
   __shared__ FlatStage<T, NT, true> st;
   __shared__ int isum[NT / kWave];
+  __shared__ long long s_at;
   auto* vals = win.vals();
   uint16_t* rows = win.rows();
-  __shared__ int s_t;
-  __shared__ long long s_excl;
-  if (threadIdx.x == 0) s_t = atomicAdd(ticket, 1);
-  __syncthreads();
-  const int t = s_t;
+  const int64_t t = first + blockIdx.x;
   const UnitL un = units[t];
   const int col = un.col, t_lo = un.blk_lo, t_hi = un.blk_hi;
   const int32_t row0 = t_lo * kBR;
@@ -2438,63 +2449,23 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
   }
   __syncthreads();
   const int cnt = unit_prefix<NT, NW32>(bits, pre, nw32, isum);
-  // publish the size; the offset is looked for once the first window's values
-  // are accumulated, when most predecessors have published theirs
-  if (threadIdx.x == 0)
-    __hip_atomic_store(&status[t], kAggFlag | (unsigned long long)cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  // Output offset of the unit: look back with the whole first wave, 64
-  // predecessors per step, summing back to the nearest one that holds an
-  // inclusive prefix (bounded wait on predecessors still counting).  A status
-  // word carries its flag and value together and no other data is passed
-  // between units, so the atomics are relaxed: at agent scope an acquire or
-  // release would invalidate or write back this XCD's whole L2.
-  auto look_back = [&]() {
-    if (threadIdx.x < kWave) {
-      const int lane = (int)threadIdx.x;
-      long long excl = 0;
-      int spins = 0;
-      for (int i = t - 1; i >= 0;) {
-        const int j = i - lane;
-        const unsigned long long v =
-            j >= 0 ? __hip_atomic_load(&status[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kInclFlag;
-        const unsigned long long incl = __ballot((v >> 62) == 2);
-        const unsigned long long none = __ballot((v >> 62) == 0);
-        const int first = incl ? __ffsll((unsigned long long)incl) - 1 : kWave;  // nearest inclusive prefix
-        const unsigned long long need = first >= kWave - 1 ? ~0ull : ((2ull << first) - 1ull);
-        if (none & need) {  // a predecessor in range has not published yet
-          if (++spins > (1 << 22)) {
-            if (lane == 0) atomicOr(err, 256);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(2);
-          continue;
-        }
-        excl += wave_sum_ll(lane <= first ? (long long)(v & kValMask) : 0ll);
-        if (first < kWave) break;
-        i -= kWave;
-      }
-      if (lane == 0) {
-        __hip_atomic_store(&status[t], kInclFlag | (unsigned long long)(excl + cnt), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-        s_excl = excl;
-        if (cnt) atomicAdd(&col_total[col], (unsigned long long)cnt);
-        if (cnt > (direct ? DR : KMAX)) atomicAdd(ovf_units, 1);
-      }
-    }
-    __syncthreads();
-    const int64_t out = s_excl + hcs[col];
-    if (out + cnt > cap && threadIdx.x == 0) atomicOr(err, 512);
-    return out;
-  };
+  if (threadIdx.x == 0) {
+    const long long at = (long long)atomicAdd(out.taken, (unsigned long long)cnt);
+    s_at = at;
+    out.cnt[t] = cnt;
+    out.at[t] = at;
+    if (cnt) atomicAdd(&col_total[col], (unsigned long long)cnt);
+    if (cnt > (direct ? DR : KMAX)) atomicAdd(ovf_units, 1);
+    if (at + cnt > out.cap) atomicOr(err, 512);
+  }
   if (direct) {
-    const int64_t out = look_back();
-    if (out + cnt <= cap)
-      unit_emit<K, T, NT, KMAX, DR>(true, nw32, cnt, bits, pre, win, row0, out, irC, valC, Filter<T>{}, col, isum, err);
+    __syncthreads();  // s_at
+    if (s_at + cnt <= out.cap)
+      unit_emit<K, T, NT, KMAX, DR, int32_t>(true, nw32, cnt, bits, pre, win, row0, s_at, out.rows, out.vals,
+                                             Filter<T>{}, col, isum, err);
     return;
   }
   // values, in windows of KMAX ranks (one window unless the unit overflowed)
-  int64_t out = 0;
-  if (cnt == 0) look_back();
   for (q0 = 0; q0 < cnt; q0 += KMAX) {
     const int wn = min(KMAX, cnt - q0);
     if (q0) {
@@ -2527,12 +2498,28 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
       }
     }
     __syncthreads();
-    if (q0 == 0) out = look_back();
-    if (out + cnt <= cap)
+    const int64_t at = s_at;
+    if (at + cnt <= out.cap)
       for (int i = threadIdx.x; i < wn; i += NT) {
-        irC[out + q0 + i] = (int64_t)row0 + rows[i];
-        valC[out + q0 + i] = SR::lout(vals[i]);
+        out.rows[at + q0 + i] = row0 + rows[i];
+        out.vals[at + q0 + i] = SR::lout(vals[i]);
       }
+  }
+}
+
+// A learned unit's outputs from the staging arrays into place: after the units
+// before it (upto, the scan of the sizes) and the exactly sized columns before
+// its own (hcs).  One workgroup per unit.
+template <class T>
+__global__ __launch_bounds__(256) void k_learned_place(const UnitL* __restrict__ units, int64_t first,
+                                                       const LearnedStage<T> in, const int64_t* __restrict__ upto,
+                                                       const int64_t* __restrict__ hcs, int64_t* __restrict__ irC,
+                                                       T* __restrict__ valC) {
+  const int64_t t = first + blockIdx.x;
+  const int64_t n = in.cnt[t], src = in.at[t], dst = upto[t] + hcs[units[t].col];
+  for (int64_t i = threadIdx.x; i < n; i += 256) {
+    irC[dst + i] = in.rows[src + i];
+    valC[dst + i] = in.vals[src + i];
   }
 }
 
@@ -2907,7 +2894,7 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
                                   int S, int64_t* nnzcol, int64_t* cpC, void* tmp, size_t tmp_bytes, cbx_dcsc* C,
                                   int* err, LearnedInfo& info) {
   const int64_t nzcB = B->nzc, m = A->m;
-  DevBuf b_feat, b_lp, b_hist, b_w, b_blo, b_bhi, b_uc, b_ub, b_pn, b_units, b_status, b_tick, b_ct, b_ovf, b_hcs, b_sum,
+  DevBuf b_feat, b_lp, b_hist, b_w, b_blo, b_bhi, b_uc, b_ub, b_pn, b_units, b_cnt, b_at, b_upto, b_taken, b_srow, b_sval, b_ct, b_ovf, b_hcs, b_sum,
       b_hflag, b_hcols, b_nh, b_hu;
   CachedBuf b_ul, b_uh, b_us;
   DevBuf b_bcnt, b_lsz, b_loff, b_lists, b_lbc;
@@ -2918,10 +2905,10 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   int* hucnt;
   Unit *units_l = nullptr, *units_h = nullptr;
   float *feats, *logpred, *w, *pred_nnz;
-  unsigned long long *hist, *status, *col_total;
+  unsigned long long *hist, *col_total;
   int32_t *blo, *bhi;
   int64_t *ucount, *ubase, *hcs;
-  int *ticket, *ovf;
+  int* ovf;
   double* dsum;
   UnitL* units;
   CBX_TRY(dalloc(b_feat, nzcB * CBX_MLP_FEATURES, s, &feats));
@@ -2935,7 +2922,6 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   CBX_TRY(dalloc(b_pn, nzcB, s, &pred_nnz));
   CBX_TRY(dalloc(b_hcs, nzcB + 1, s, &hcs));
   CBX_TRY(dalloc(b_sum, 2, s, &dsum));
-  CBX_TRY(dalloc(b_tick, 2, s, &ticket));
   CBX_TRY(dalloc(b_ovf, 2, s, &ovf));
   CBX_TRY(dalloc(b_ct, nzcB, s, &col_total));
   CBX_TRY(dalloc(b_hflag, nzcB, s, &heavy_flag));
@@ -2974,7 +2960,7 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   CBX_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, ucount, ubase, (int)(nzcB + 1), s));
   // columns predicted heavy: exact sizes from the symbolic unit pass (their
   // units then go through the two-phase unit kernels), so the single pass
-  // covers the many light columns and its look-back sees the heavy columns'
+  // covers the many light columns and its outputs are placed around the heavy columns'
   // sizes up front, like the hash tier's
   int64_t hash_only = 0;
   {
@@ -3047,46 +3033,33 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   info.hash_total = hash_only;
   info.exact_total = hash_total - hash_only;
   CBX_TRY(dalloc(b_units, std::max<int64_t>(nunits, 1), s, &units));
-  CBX_TRY(dalloc(b_status, std::max<int64_t>(nunits, 1), s, &status));
   if (nunits)
     k_learned_units<<<nblk(nzcB, 256), 256, 0, s>>>(flop, nzcB, cfg.small_flop_max, logpred, blo, bhi, w, target,
                                                     heavy_pred, fcap, kLearnRB, direct_flop, m, ubase, nullptr,
                                                     units, nullptr, nullptr);
-  // output capacity from the predictions (plus the exact hash-tier sizes)
-  const int64_t cap = hash_total + (int64_t)(pred_sum * (1.0 + cfg.capacity_margin)) + (1 << 20);
-  auto alloc_out = [&]() -> cbx_status {
-    if (!C->ir) CBX_TRY(dev_alloc((void**)&C->ir, sizeof(int64_t) * cap));
-    if (!C->val) CBX_TRY(dev_alloc(&C->val, sizeof(T) * cap));
-    return CBX_OK;
-  };
-  cbx_status ast = alloc_out();
-  if (ast != CBX_OK && rm.p) {  // give the row maps back; the large units then count in a sweep
-    CBX_HIP(hipStreamSynchronize(s));
-    dev_free(rm.p);
-    rm.p = nullptr;
-    release_cache();
-    ast = alloc_out();
-  }
-  if (ast == CBX_ERR_NOMEM) {  // predicted capacity does not fit: the exact two-phase path sizes the output
+  // staging capacity from the predictions; where it does not fit, the exact
+  // two-phase path computes the product
+  LearnedStage<T> stage;
+  stage.cap = (int64_t)(pred_sum * (1.0 + cfg.capacity_margin)) + (1 << 20);
+  int64_t* upto;
+  if (dalloc(b_cnt, nunits + 1, s, &stage.cnt) != CBX_OK || dalloc(b_at, nunits + 1, s, &stage.at) != CBX_OK ||
+      dalloc(b_upto, nunits + 1, s, &upto) != CBX_OK || dalloc(b_taken, 1, s, &stage.taken) != CBX_OK ||
+      dalloc(b_srow, stage.cap, s, &stage.rows) != CBX_OK || dalloc(b_sval, stage.cap, s, &stage.vals) != CBX_OK) {
     info.over_capacity = true;
     return CBX_OK;
   }
-  CBX_TRY(ast);
-  CBX_HIP(hipMemsetAsync(status, 0, sizeof(unsigned long long) * std::max<int64_t>(nunits, 1), s));
-  CBX_HIP(hipMemsetAsync(ticket, 0, sizeof(int) * 2, s));
+  CBX_HIP(hipMemsetAsync(stage.cnt + nunits, 0, sizeof(int64_t), s));
+  CBX_HIP(hipMemsetAsync(stage.taken, 0, sizeof(unsigned long long), s));
   CBX_HIP(hipMemsetAsync(ovf, 0, sizeof(int) * 2, s));
   CBX_HIP(hipMemsetAsync(col_total, 0, sizeof(unsigned long long) * nzcB, s));
   hipEvent_t kev[3] = {nullptr, nullptr, nullptr};
   for (auto& e : kev) (void)hipEventCreate(&e);
   (void)hipEventRecord(kev[0], s);
-  // launches of at most 2^21 workgroups (a dispatch holds fewer than 2^32
-  // work-items); the ticket counter runs on across them, and a later launch's
-  // units look back into statuses the earlier launches completed
+  // launches of at most 2^21 workgroups (a dispatch holds fewer than 2^32 work-items)
   for (int64_t done = 0; done < nunits; done += kLearnChunk) {
     const int64_t nb = std::min<int64_t>(kLearnChunk, nunits - done);
     k_num_learned<K, T, kLearnNT, 4, kLearnK, kLightDR, kLearnRB, kLearnCR><<<(unsigned)nb, kLearnNT, 0, s>>>(
-        units, ticket, status, hcs, B->cp, bpos, (const T*)B->val, A->cp, rowsA, (const T*)A->val, P, S, cap, C->ir,
-        (T*)C->val, col_total, ovf, err);
+        units, done, B->cp, bpos, (const T*)B->val, A->cp, rowsA, (const T*)A->val, P, S, stage, col_total, ovf, err);
   }
   (void)hipEventRecord(kev[1], s);
   CBX_HIP(hipGetLastError());
@@ -3099,16 +3072,56 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   CBX_HIP(hipStreamSynchronize(s));
   info.overflow_units = hovf;
   (void)hipEventElapsedTime(&info.kernel_ms, kev[0], kev[1]);
-  info.over_capacity = (herr & 512) != 0 || info.nnzC > cap;
-  if (herr & ~512 || info.over_capacity || !nheavy) {
+  info.over_capacity = (herr & 512) != 0;
+  if (herr & ~512 || info.over_capacity) {
     for (auto& e : kev) (void)hipEventDestroy(e);
     if (herr & ~512) return set_error(CBX_ERR_HIP, "cbx_spgemm: learned pass inconsistency (flag %d)", herr);
+    return CBX_OK;
+  }
+  auto alloc_out = [&]() -> cbx_status {
+    if (!C->ir) CBX_TRY(dev_alloc((void**)&C->ir, sizeof(int64_t) * std::max<int64_t>(info.nnzC, 1)));
+    if (!C->val) CBX_TRY(dev_alloc(&C->val, sizeof(T) * std::max<int64_t>(info.nnzC, 1)));
+    return CBX_OK;
+  };
+  cbx_status ast = alloc_out();
+  if (ast != CBX_OK && rm.p) {  // give the row maps back; the large units then count in a sweep
+    dev_free(rm.p);             // (the stream is idle)
+    rm.p = nullptr;
+    release_cache();
+    ast = alloc_out();
+  }
+  if (ast != CBX_OK) {  // the exact path has the staging arrays' room too
+    for (auto& e : kev) (void)hipEventDestroy(e);
+    if (ast != CBX_ERR_NOMEM) return ast;
+    info.over_capacity = true;
+    return CBX_OK;
+  }
+  (void)hipEventRecord(kev[2], s);  // the copy into place, and the numeric pass of the heavy columns
+  if (nunits) {
+    size_t need = 0;
+    CBX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, need, stage.cnt, upto, (int)(nunits + 1), s));
+    DevBuf b_t4;
+    void* t4 = tmp;
+    if (need > tmp_bytes) CBX_TRY(dalloc(b_t4, need, s, (uint8_t**)&t4));
+    need = std::max(need, tmp_bytes);
+    CBX_HIP(hipcub::DeviceScan::ExclusiveSum(t4, need, stage.cnt, upto, (int)(nunits + 1), s));
+    for (int64_t done = 0; done < nunits; done += kLearnChunk)
+      k_learned_place<T><<<(unsigned)std::min<int64_t>(kLearnChunk, nunits - done), 256, 0, s>>>(
+          units, done, stage, upto, hcs, C->ir, (T*)C->val);
+    CBX_HIP(hipGetLastError());
+  }
+  if (!nheavy) {
+    (void)hipEventRecord(kev[1], s);
+    CBX_HIP(hipStreamSynchronize(s));
+    float place_ms = 0;
+    (void)hipEventElapsedTime(&place_ms, kev[2], kev[1]);
+    info.kernel_ms += place_ms;
+    for (auto& e : kev) (void)hipEventDestroy(e);
     return CBX_OK;
   }
   // the heavy columns' values, at the offsets the scan above fixed
   int hu[3] = {0, 0, 0};  // small (bitmap), large, and small list units
   CBX_HIP(hipMemcpy(hu, hucnt, sizeof(hu), hipMemcpyDeviceToHost));
-  (void)hipEventRecord(kev[2], s);  // numeric of the heavy columns, after the offsets
   CBX_RETURN_IF(hu[0] > cap_l || hu[1] > cap_h || hu[2] > cap_l, CBX_ERR_HIP, "cbx_spgemm: unit list overflow");
   CBX_RETURN_IF((int64_t)hu[0] * kLightNT >= (1ll << 32) || (int64_t)hu[1] * kHeavyNT >= (1ll << 32) ||
                     (int64_t)hu[2] * kLightNT >= (1ll << 32),

@@ -166,9 +166,10 @@ enum {
   CBX_SPGEMM_UNSORTED = 1,
   /* Learned single pass: the installed nnz predictor (cbx_spgemm_set_predictor)
    * replaces the symbolic pass of the large columns; each row-range unit's
-   * exact size comes from its own presence bitmap and its output offset from
-   * a decoupled look-back, units larger than predicted are re-run exactly,
-   * and an exceeded output capacity falls back to the two-phase path.
+   * exact size comes from its own presence bitmap, its outputs go to a staging
+   * area and from there into place once all sizes are known; units larger than
+   * predicted are re-run exactly, and an exceeded staging capacity falls back
+   * to the two-phase path.
    * Output identical to CBX_SPGEMM_TWO_PHASE. */
   CBX_SPGEMM_LEARNED = 2
 };
