@@ -152,11 +152,12 @@ __device__ __forceinline__ void flat_init(FlatStage<T, NT, VAL>& st) {
   for (int i = threadIdx.x; i < 2 * kTileWords; i += NT) (&st.starts[0][0])[i] = 0ull;
 }
 
-// Stages one chunk, at most one segment per thread.  One barrier; the caller's
+// Stages one chunk, at most one segment per thread; its products are numbered
+// from x0 on (0 where flat_chunk visits them).  One barrier; the caller's
 // earlier writes to LDS are visible after it, and the previous chunk must have
 // been visited by each wave when it calls.
 template <class T, int NT, bool VAL>
-__device__ __forceinline__ FlatSeg flat_stage(FlatStage<T, NT, VAL>& st, int32_t base, int len, T bv) {
+__device__ __forceinline__ FlatSeg flat_stage(FlatStage<T, NT, VAL>& st, int32_t base, int len, T bv, int x0 = 0) {
   constexpr int NW = NT / kWave;
   const int lane = lane_id(), w = wave_id_uniform();
   const unsigned long long some = __ballot(len > 0);
@@ -172,7 +173,7 @@ __device__ __forceinline__ FlatSeg flat_stage(FlatStage<T, NT, VAL>& st, int32_t
   const int l0 = w ? __builtin_amdgcn_readlane(wl, w - 1) : 0;
   FlatSeg me;
   me.total = __builtin_amdgcn_readlane(wl, NW - 1);
-  me.start = l0 + incl - len;
+  me.start = x0 + l0 + incl - len;
   me.k = -1;
   if (len > 0) {
     me.k = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(some >> 32),

@@ -394,7 +394,6 @@ SpgemmConfig cbx::current_config() {
     c.row_map_share = g_config.row_map_share;
     c.tiny_wg_waves = g_config.tiny_wg_waves;
     c.unit_order = g_config.unit_order;
-    c.tiny_algo = g_config.tiny_algo;
     c.sym_band = g_config.sym_band;
     c.mcl_fuse = g_config.mcl_fuse != 0;
     c.unit_lists = g_config.unit_lists;

@@ -48,8 +48,6 @@ struct SpgemmConfig {
   // Exactly sized (two-phase) units in the symbolic pass's order (0) or
   // sorted by first row block (1).
   int unit_order = 1;
-  // Tiny tier: register bitonic sort (0) or per-wave LDS hash table (1).
-  int tiny_algo = 0;
   // Symbolic pass of the unit tier: per column (0) or in bands of 16 / 64
   // row blocks dispatched band by band.
   int sym_band = 0;

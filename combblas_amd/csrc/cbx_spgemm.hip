@@ -443,28 +443,28 @@ __global__ __launch_bounds__(NT) void k_sym_hash(const int32_t* __restrict__ ord
                                                  int* __restrict__ err) {
   __shared__ int32_t keys[HMAX];
   __shared__ long long wsum[NT / kWave];
-  __shared__ SegStage<uint8_t, NT> st;
+  __shared__ FlatStage<uint8_t, NT, false> st;
   const int col = order[first + blockIdx.x];
   const int lg = min(ceil_log2_dev(max(2 * flop[col], 64ll)), ceil_log2_dev(HMAX));
   const int H = 1 << lg;
   for (int i = threadIdx.x; i < H; i += NT) keys[i] = -1;
   __syncthreads();
-  long long cnt = 0;
+  flat_init(st);
+  int cnt = 0, par = 0;
   const int64_t b0 = cpB[col], b1 = cpB[col + 1];
   for (int64_t eb = b0; eb < b1; eb += NT) {
     int64_t base;
-    int len, nseg;
+    int len;
     uint8_t dummy;
     load_seg<uint8_t, false>(eb + threadIdx.x, b1, bpos, cpA, Tiles{}, 0, 0, true, nullptr, base, len, dummy);
-    const int tot = stage_chunk<uint8_t, NT>(st, wsum, base, len, 0, nseg);
-    visit_staged<uint8_t, NT, 4>(st, nseg, tot, [&](const int64_t(&idx)[4], const uint8_t(&)[4]) {
+    const FlatSeg me = flat_stage<uint8_t, NT, false>(st, (int32_t)base, len, 0);
+    flat_chunk<uint8_t, NT, false, 4>(st, me, par, [&](const int32_t(&idx)[4], uint8_t(&)[4], const bool(&ok)[4]) {
       int32_t rr[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) rr[u] = idx[u] >= 0 ? rowsA[idx[u]] : -1;
+      load_rows(rowsA, 0, idx, rr);
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int32_t r = rr[u];
-        if (r < 0) continue;
+        if (!ok[u]) continue;
         uint32_t h = hash_slot(r, lg);
         int probe = 0;
         for (; probe < H; ++probe) {  // the table is at least twice the column's flops
@@ -483,185 +483,73 @@ __global__ __launch_bounds__(NT) void k_sym_hash(const int32_t* __restrict__ ord
 
 // ------------------------------------------------------------ tiny tier
 // Columns with at most 256 products (most columns of multigrid triple
-// products, and the sparsest R-MAT columns): one wave per column, no LDS.
-// Lane l holds elements e = u*64 + l (u < 4).  The products are gathered with
-// a wave scan of the B entries' A-segment lengths and a 6-step binary search
-// over it by shuffles; a bitonic network sorts the 256 (row, value) pairs in
-// registers (partners in another lane through shuffles, in another register
-// of the same lane by swaps); equal rows are then adjacent, a segmented scan
-// in element order reduces each run, and the run's last element writes the
-// output at its rank.  SYM only counts the distinct rows.
+// products, and the sparsest R-MAT columns): one wave per column.
+//
+// The products are gathered into registers, element e = u * 64 + lane in
+// register u, their segments found by bit counts as in FlatStage.  Each then
+// finds its row's slot in a per-wave hash table (linear probing, at most half
+// full); the lanes whose products came first to their slots hold the distinct
+// rows, which are compacted by ballots and sorted: up to 64 by counting the
+// rows below each (broadcast reads of four), more by the digit passes of
+// k_num_sort on one wave.  The row's rank replaces its key in the table, and
+// every product accumulates at its slot's rank, so rows and values leave in
+// order.  SYM only counts the distinct rows.
+//
+// A bitonic network over the 256 elements in registers took some 430
+// cross-lane moves through LDS a column whatever its distinct rows: 4.0 ms for
+// the two products of 16 Galerkin blocks (4.1e5 columns each of 216 and 64
+// products, FP64); this takes 1.45 ms.  Bound by LDS latency at seven waves per
+// SIMD (23 KB for four waves).
 constexpr int kTinyMax = 256;
+constexpr int kTinyHash = 2 * kTinyMax;  // slots per wave at most
+constexpr int kTinyWaves = 4;            // waves per workgroup at most (launch bound 256)
+constexpr int kTinyDigit = 7;            // bits per digit pass: two 16-bit counters per lane
 
-template <class X>
-__device__ __forceinline__ X shfl_x(X v, int src) {
-  if constexpr (sizeof(X) < 4) return (X)__shfl((int)v, src, kWave);
-  else return __shfl(v, src, kWave);
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Sort, reduce and emit the first NR registers (NR * 64 elements) of a tiny
-// column; elements beyond them are empty (row kNone).
-template <int K, class T, bool SYM, int NR>
-__device__ __forceinline__ void tiny_finish(int32_t (&key)[kTinyMax / kWave],
-                                            typename Sem<K, T>::Acc (&val)[kTinyMax / kWave], int lane, int col,
-                                            int64_t* __restrict__ nnzcol, const int64_t* __restrict__ cpC,
-                                            int64_t* __restrict__ irC, T* __restrict__ valC, int* __restrict__ err,
-                                            const int64_t* __restrict__ stage_off, int64_t slot,
-                                            const Filter<T>& flt) {
-  using SR = Sem<K, T>;
-  using Acc = typename SR::Acc;
-  constexpr int32_t kNone = 0x7fffffff;
-  // bitonic sort of NR*64 elements, ascending by row
-#pragma unroll
-  for (int k = 2; k <= NR * kWave; k <<= 1) {
-#pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j >= kWave) {
-        const int du = j / kWave;
-#pragma unroll
-        for (int u = 0; u < NR; ++u) {
-          const int u2 = u ^ du;
-          if (u2 > u) {
-            const bool asc = (((u * kWave + lane) & k) == 0);
-            if ((key[u] > key[u2]) == asc && key[u] != key[u2]) {
-              const int32_t tk = key[u];
-              key[u] = key[u2];
-              key[u2] = tk;
-              if constexpr (!SYM) {
-                const Acc tv = val[u];
-                val[u] = val[u2];
-                val[u2] = tv;
-              }
-            }
-          }
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < NR; ++u) {
-          const int e = u * kWave + lane;
-          const bool asc = ((e & k) == 0);
-          const bool lower = (lane & j) == 0;
-          const int32_t pk = __shfl_xor(key[u], j, kWave);
-          Acc pv{};
-          if constexpr (!SYM) pv = __shfl_xor(val[u], j, kWave);
-          const bool take = lower == asc ? pk < key[u] : pk > key[u];
-          if (take) {
-            key[u] = pk;
-            if constexpr (!SYM) val[u] = pv;
-          }
-        }
-      }
-    }
+template <class T, class Lds, bool SYM>
+struct TinyLds {
+  __align__(16) int32_t keys[kTinyHash];  // rows, then their ranks
+  __align__(16) int32_t rows[kTinyMax + 4];
+  uint16_t slot[kTinyMax];  // of each compacted row
+  Lds vals[SYM ? 1 : kTinyMax];
+  uint32_t hist[SYM ? 1 : kWave];
+  unsigned long long starts[kTinyMax / 64];
+  int32_t delta[kWave];
+  T bval[SYM ? 1 : kWave];
+};
+
+// Lanes of the wave with the same value of the low `width` bits of d, among
+// `valid` ones.
+__device__ __forceinline__ unsigned long long wave_match(uint32_t d, int width, unsigned long long valid) {
+  unsigned long long same = valid;
+  for (int b = 0; b < width; ++b) {
+    const bool bit = (d >> b) & 1u;
+    const unsigned long long m = __ballot(bit);
+    same &= bit ? m : ~m;
   }
-  // run heads (first element of each distinct row)
-  bool head[NR];
-  unsigned long long hm[NR];
-  int count = 0;
-#pragma unroll
-  for (int u = 0; u < NR; ++u) {
-    int32_t prev = __shfl_up(key[u], 1, kWave);
-    const int32_t carry = u > 0 ? __shfl(key[u > 0 ? u - 1 : 0], kWave - 1, kWave) : kNone;
-    if (lane == 0) prev = u > 0 ? carry : -1;
-    head[u] = key[u] != kNone && key[u] != prev;
-    hm[u] = __ballot(head[u]);
-    count += __popcll(hm[u]);
-  }
-  if constexpr (SYM) {
-    if (lane == 0) nnzcol[col] = count;
-  } else {
-    // the column's allocation from the symbolic pass; or, staged (no symbolic
-    // pass), its slot of flop_j entries in the staging buffer, and the count
-    // is recorded for the copy into place
-    int64_t have, out;
-    if (stage_off) {
-      out = stage_off[slot];
-      have = stage_off[slot + 1] - out;
-      if (lane == 0) nnzcol[col] = count;
-      if (lane == 0 && count > have) atomicOr(err, 8);
-    } else {
-      have = nnzcol[col];
-      if (lane == 0 && count != have) atomicOr(err, 8);
-      out = cpC[col];
-    }
-    Acc carry = SR::ident();
-    bool open = false;  // a run continues from the previous register
-    int before = 0;     // heads in earlier registers
-    int kept = 0;       // entries written (filter on)
-#pragma unroll
-    for (int u = 0; u < NR; ++u) {
-      // segmented inclusive scan in element order
-      Acc x = val[u];
-      bool f = head[u];
-#pragma unroll
-      for (int d = 1; d < kWave; d <<= 1) {
-        const Acc y = __shfl_up(x, d, kWave);
-        const bool g = __shfl_up((int)f, d, kWave) != 0;
-        if (lane >= d) {
-          if (!f) x = SR::add(y, x);
-          f = f || g;
-        }
-      }
-      if (!f && open) x = SR::add(carry, x);
-      // the last element of a run writes it at its rank
-      int32_t next = __shfl_down(key[u], 1, kWave);
-      const int32_t nfirst = u + 1 < NR ? __shfl(key[u + 1 < NR ? u + 1 : u], 0, kWave) : kNone;
-      if (lane == kWave - 1) next = nfirst;
-      const bool end = key[u] != kNone && next != key[u];
-      if (!flt.on) {
-        if (end) {
-          const int rank = before + __popcll(hm[u] & ((2ull << lane) - 1ull)) - 1;
-          if (rank < have) {
-            irC[out + rank] = key[u];
-            valC[out + rank] = SR::out(x);
-          }
-        }
-      } else {  // the fused threshold: kept entries, in row order, at out
-        const T v = SR::out(x);
-        const bool keep = end && !(v < flt.thr);
-        const uint64_t km = __ballot(keep);
-        if (keep) {
-          const int rank = kept + __popcll(km & ((1ull << lane) - 1ull));
-          if (rank < have) {
-            irC[out + rank] = key[u];
-            valC[out + rank] = v;
-          }
-        }
-        kept += __popcll(km);
-      }
-      carry = __shfl(x, kWave - 1, kWave);
-      open = __shfl((int)(key[u] != kNone), kWave - 1, kWave) != 0;
-      before += __popcll(hm[u]);
-    }
-    if (flt.on) {  // staged: the kept count sizes the column; else its range joins the runs
-      if (stage_off) {
-        if (lane == 0) {
-          nnzcol[col] = kept;
-          if (count > kept) atomicAdd(flt.dropped, (unsigned long long)(count - kept));
-        }
-      } else if (lane == 0) {
-        filter_add_run(flt, out, kept, col, err);
-      }
-    }
-  }
+  return same;
 }
 
-// The products of one tiny column (at most kTinyMax of them) gathered into
-// the wave's registers: element e = u * 64 + lane sits in key[u] (its row)
-// and val[u] (its product); elements past the column's products hold kNone.
-// Returns the number of products (wave-uniform).  All lanes must call it.
-template <int K, class T, bool SYM>
-__device__ __forceinline__ int tiny_gather(int64_t b0, int64_t b1, const int32_t* __restrict__ bpos,
+// The products of one tiny column gathered into the wave's registers: rows
+// and products of elements u * 64 + lane.  Returns their number
+// (wave-uniform; above kTinyMax the rest is left out).
+template <int K, class T, bool SYM, class L>
+__device__ __forceinline__ int tiny_gather(L& ws, int64_t b0, int64_t b1, const int32_t* __restrict__ bpos,
                                            const T* __restrict__ valB, const int64_t* __restrict__ cpA,
                                            const int32_t* __restrict__ rowsA, const T* __restrict__ valA,
                                            int32_t (&key)[kTinyMax / kWave],
                                            typename Sem<K, T>::Acc (&val)[kTinyMax / kWave]) {
   using SR = Sem<K, T>;
   constexpr int kE = kTinyMax / kWave;
-  constexpr int32_t kNone = 0x7fffffff;
   const int lane = lane_id();
 #pragma unroll
   for (int u = 0; u < kE; ++u) {
-    key[u] = kNone;
+    key[u] = 0;
     val[u] = SR::ident();
   }
   int filled = 0;  // wave-uniform
@@ -670,40 +558,116 @@ __device__ __forceinline__ int tiny_gather(int64_t b0, int64_t b1, const int32_t
     int len;
     T bv;
     load_seg<T, !SYM>(eb + lane, b1, bpos, cpA, Tiles{}, 0, 0, true, valB, base, len, bv);
-    const int inc = wave_incl_scan(len);
-    const int off = filled + inc - len;  // first element of this lane's segment
-    const int total = __shfl(inc, kWave - 1, kWave);
-    // lanes that hold B entries in this chunk, and the search's first step:
-    // the largest power of two below that count (all wave-uniform)
-    const int nb = (int)(b1 - eb < kWave ? b1 - eb : kWave);
-    int top = 0;
-    if (nb > 1) top = 1 << (31 - __clz(nb - 1));
+    const unsigned long long some = __ballot(len > 0);
+    if (!some) continue;
+    const int incl = wave_incl_scan(len);
+    const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
+    const int k = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(some >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)some, 0));
+    const int start = filled + incl - len;
+    if (lane < kE) ws.starts[lane] = 0ull;
+    wave_lds_sync();
+    if (len > 0) {
+      ws.delta[k] = (int32_t)(base - start);
+      if constexpr (!SYM) ws.bval[k] = bv;
+      const int at = start - 1;  // one bit per segment after the first, before its first product
+      if (k > 0 && at < kTinyMax)
+        __hip_atomic_fetch_or(&ws.starts[at >> 6], 1ull << (at & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    wave_lds_sync();
+    const int end = min(filled + total, kTinyMax);
+    int before = 0;
 #pragma unroll
     for (int u = 0; u < kE; ++u) {
+      const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)ws.starts[u]);
+      const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(ws.starts[u] >> 32));
       // registers whose 64 elements miss this chunk's range stay as they are
-      if ((u + 1) * kWave <= filled || u * kWave >= filled + total) continue;
-      const int e = u * kWave + lane;
-      // last lane s < nb with off_s <= e (segments of length 0 share
-      // offsets; the search lands on the one that holds e when e is in this
-      // chunk)
-      int lo = 0;
-      for (int step = top; step > 0; step >>= 1) {
-        const int o = __shfl(off, lo + step, kWave);
-        if (lo + step < nb && o <= e) lo += step;
+      if ((u + 1) * kWave > filled && u * kWave < end) {
+        const int e = u * kWave + lane;
+        const int s = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, (unsigned)before));
+        // lanes outside repeat the chunk's first or last product
+        const int32_t idx = min(max(e, filled), end - 1) + ws.delta[s];
+        int32_t r = rowsA[idx];
+        pin(r);
+        const bool mine = e >= filled && e < end;
+        if constexpr (!SYM) {
+          T a = valA[idx], b = ws.bval[s];
+          pin(a);
+          if (mine) val[u] = SR::mul(a, b);
+        }
+        if (mine) key[u] = r;
       }
-      const int o = __shfl(off, lo, kWave);
-      const int l = __shfl(len, lo, kWave);
-      const int64_t bs = shfl_x(base, lo);
-      const T bval = shfl_x(bv, lo);
-      if (e >= filled && e < filled + total && e - o < l) {
-        const int64_t idx = bs + (e - o);
-        key[u] = rowsA[idx];
-        if constexpr (!SYM) val[u] = SR::mul(valA[idx], bval);
-      }
+      before += __popc(lo) + __popc(hi);
     }
     filled += total;
+    wave_lds_sync();  // the chunk's segments have been read
   }
   return filled;
+}
+
+// Sorts rows[0..D) and slot[0..D) by row, D in (64, 256], with wave ballots:
+// least significant digit first, over the bits in which the rows differ.
+template <class L>
+__device__ __forceinline__ void tiny_sort(L& ws, int D) {
+  constexpr int kE = kTinyMax / kWave;
+  const int lane = lane_id();
+  uint32_t key[kE], slot[kE];
+  const uint32_t first = (uint32_t)ws.rows[0];
+  uint32_t diff = 0;
+#pragma unroll
+  for (int u = 0; u < kE; ++u) {
+    const int e = u * kWave + lane;
+    key[u] = (uint32_t)ws.rows[min(e, D - 1)];
+    slot[u] = ws.slot[min(e, D - 1)];
+    diff |= key[u] ^ first;
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) diff |= (uint32_t)__shfl_xor((int)diff, d, kWave);
+  const int nbits = 32 - __clz((int)__builtin_amdgcn_readfirstlane((int)diff));  // at least 7: the rows are distinct
+  const int npass = (nbits + kTinyDigit - 1) / kTinyDigit;
+  const int width = (nbits + npass - 1) / npass;
+  uint16_t* hist = reinterpret_cast<uint16_t*>(ws.hist);
+  for (int p = 0, shift = 0; p < npass; ++p, shift += width) {
+    ws.hist[lane] = 0;
+    wave_lds_sync();
+    int rank[kE];
+#pragma unroll
+    for (int u = 0; u < kE; ++u) {
+      rank[u] = -1;
+      if (u * kWave >= D) continue;  // uniform
+      const bool valid = u * kWave + lane < D;
+      const uint32_t d = (key[u] >> shift) & ((1u << width) - 1u);
+      const unsigned long long same = wave_match(d, width, __ballot(valid));
+      const int before = __popcll(same & ((1ull << lane) - 1ull));
+      int seen = 0;
+      if (valid) seen = hist[d];
+      wave_lds_sync();
+      if (valid && before == 0) hist[d] = (uint16_t)(seen + __popcll(same));
+      wave_lds_sync();
+      if (valid) rank[u] = seen + before;
+    }
+    const uint32_t pair = ws.hist[lane];
+    const int c0 = (int)(pair & 0xffffu), c1 = (int)(pair >> 16);
+    const int ex = wave_incl_scan(c0 + c1) - c0 - c1;
+    ws.hist[lane] = (uint32_t)ex | (uint32_t)(ex + c0) << 16;
+    wave_lds_sync();
+#pragma unroll
+    for (int u = 0; u < kE; ++u)
+      if (rank[u] >= 0) {
+        const int at = (int)hist[(key[u] >> shift) & ((1u << width) - 1u)] + rank[u];
+        ws.rows[at] = (int32_t)key[u];
+        ws.slot[at] = (uint16_t)slot[u];
+      }
+    wave_lds_sync();
+    if (p + 1 < npass) {
+#pragma unroll
+      for (int u = 0; u < kE; ++u) {
+        const int e = min(u * kWave + lane, D - 1);
+        key[u] = (uint32_t)ws.rows[e];
+        slot[u] = ws.slot[e];
+      }
+      wave_lds_sync();
+    }
+  }
 }
 
 template <int K, class T, bool SYM>
@@ -716,128 +680,88 @@ __global__ __launch_bounds__(256) void k_tiny(const int32_t* __restrict__ order,
                                               const int64_t* __restrict__ stage_off = nullptr, Filter<T> flt = {}) {
   using SR = Sem<K, T>;
   using Acc = typename SR::Acc;
-  constexpr int kE = kTinyMax / kWave;  // 4 elements per lane
-  constexpr int32_t kNone = 0x7fffffff;
-  const int lane = lane_id();
-  const int64_t waves = (int64_t)gridDim.x * (blockDim.x / kWave);
-  for (int64_t i = (int64_t)blockIdx.x * (blockDim.x / kWave) + wave_id(); i < ncols; i += waves) {
-    const int col = order[first + i];
-    const int64_t b0 = cpB[col], b1 = cpB[col + 1];
-    int32_t key[kE];
-    Acc val[kE];
-    const int filled = tiny_gather<K, T, SYM>(b0, b1, bpos, valB, cpA, rowsA, valA, key, val);
-    if (filled > kTinyMax && lane == 0) atomicOr(err, 4);
-    // sort only as many registers as the column fills (wave-uniform)
-    if (filled <= kWave) tiny_finish<K, T, SYM, 1>(key, val, lane, col, nnzcol, cpC, irC, valC, err, stage_off, i, flt);
-    else if (filled <= 2 * kWave)
-      tiny_finish<K, T, SYM, 2>(key, val, lane, col, nnzcol, cpC, irC, valC, err, stage_off, i, flt);
-    else tiny_finish<K, T, SYM, 4>(key, val, lane, col, nnzcol, cpC, irC, valC, err, stage_off, i, flt);
-  }
-}
-
-// LDS form of the tiny tier: one wave per column, no sort.  The column's
-// products (gathered into registers as above) are inserted into a per-wave
-// linear-probing table of kTinyHash slots keyed by row (at most half full),
-// accumulating each product into its row's slot with the semiring's LDS
-// atomic; the occupied slots are compacted, and each distinct row's rank (its
-// position in the sorted column) is the number of distinct rows below it,
-// counted against the compacted rows read back four at a time (every lane
-// reads the same address).  Cross-lane traffic per column: a few dozen LDS
-// instructions against the several hundred lane shuffles of the register
-// bitonic sort.
-constexpr int kTinyHash = 2 * kTinyMax;  // slots per wave
-constexpr int kTinyWaves = 4;            // waves per workgroup at most (launch bound 256)
-
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-template <int K, class T, bool SYM>
-__global__ __launch_bounds__(256) void k_tiny_h(const int32_t* __restrict__ order, int64_t first, int64_t ncols,
-                                                const int64_t* __restrict__ cpB, const int32_t* __restrict__ bpos,
-                                                const T* __restrict__ valB, const int64_t* __restrict__ cpA,
-                                                const int32_t* __restrict__ rowsA, const T* __restrict__ valA,
-                                                int64_t* __restrict__ nnzcol, const int64_t* __restrict__ cpC,
-                                                int64_t* __restrict__ irC, T* __restrict__ valC,
-                                                int* __restrict__ err, const int64_t* __restrict__ stage_off = nullptr,
-                                                Filter<T> flt = {}) {
-  using SR = Sem<K, T>;
-  using Acc = typename SR::Acc;
   constexpr int kE = kTinyMax / kWave;
-  constexpr int kSPL = kTinyHash / kWave;  // table slots owned by a lane in the compaction
   constexpr int32_t kNone = 0x7fffffff, kEmpty = -1;
-  constexpr int kLgHash = 9;
-  static_assert((1 << kLgHash) == kTinyHash, "table size");
-  __shared__ int32_t s_key[kTinyWaves][kTinyHash];
-  __shared__ typename SR::Lds s_val[SYM ? 1 : kTinyWaves][SYM ? 1 : kTinyHash];
-  __shared__ __align__(16) int32_t s_row[kTinyWaves][kTinyMax + 4];  // compacted rows, kNone-padded
-  __shared__ uint16_t s_slot[SYM ? 1 : kTinyWaves][SYM ? 1 : kTinyMax];
-  const int lane = lane_id(), w = wave_id();
-  int32_t* hk = s_key[w];
-  int32_t* crow = s_row[w];
+  __shared__ TinyLds<T, typename SR::Lds, SYM> s_ws[kTinyWaves];
+  const int lane = lane_id(), w = wave_id_uniform();
+  auto& ws = s_ws[w];
   const int64_t waves = (int64_t)gridDim.x * (blockDim.x / kWave);
   for (int64_t i = (int64_t)blockIdx.x * (blockDim.x / kWave) + w; i < ncols; i += waves) {
     const int col = order[first + i];
-    const int64_t b0 = cpB[col], b1 = cpB[col + 1];
     int32_t key[kE];
     Acc val[kE];
-    const int filled = tiny_gather<K, T, SYM>(b0, b1, bpos, valB, cpA, rowsA, valA, key, val);
-    if (filled > kTinyMax && lane == 0) atomicOr(err, 4);
-    const int nr = (min(filled, kTinyMax) + kWave - 1) / kWave;  // registers in use (wave-uniform)
-#pragma unroll
-    for (int q = 0; q < kSPL; ++q) {
-      hk[q * kWave + lane] = kEmpty;
-      if constexpr (!SYM) s_val[w][q * kWave + lane] = SR::lident();
+    int filled = tiny_gather<K, T, SYM>(ws, cpB[col], cpB[col + 1], bpos, valB, cpA, rowsA, valA, key, val);
+    if (filled > kTinyMax) {  // the tier's bound keeps it below; guard anyway
+      if (lane == 0) atomicOr(err, 4);
+      filled = kTinyMax;
     }
+    int lg = 6;  // 64 slots at least, and twice the products
+    while ((1 << lg) < 2 * filled) ++lg;
+    const int H = 1 << lg;
+    for (int q = lane * 4; q < H; q += kWave * 4)
+      *reinterpret_cast<int4*>(ws.keys + q) = int4{kEmpty, kEmpty, kEmpty, kEmpty};
     wave_lds_sync();
-    // insert: every product finds its row's slot (linear probing)
+    // every product finds its row's slot; the first to come owns it
     int slot[kE];
+    int D = 0;  // distinct rows
 #pragma unroll
     for (int u = 0; u < kE; ++u) {
-      slot[u] = -1;
-      if (u < nr && key[u] != kNone) {
-        uint32_t h = hash_slot(key[u], kLgHash);
+      if (u * kWave >= filled) continue;  // uniform
+      bool owner = false;
+      slot[u] = 0;
+      if (u * kWave + lane < filled) {
+        uint32_t h = hash_slot(key[u], lg);
         while (true) {
-          const int32_t old = atomicCAS(&hk[h], kEmpty, key[u]);
-          if (old == kEmpty || old == key[u]) break;
-          h = (h + 1) & (kTinyHash - 1);
+          const int32_t old = atomicCAS(&ws.keys[h], kEmpty, key[u]);
+          owner = old == kEmpty;
+          if (owner || old == key[u]) break;
+          h = (h + 1) & (H - 1);
         }
         slot[u] = (int)h;
       }
+      const unsigned long long om = __ballot(owner);
+      if (!SYM && owner) {
+        const int at = D + __popcll(om & ((1ull << lane) - 1ull));
+        ws.rows[at] = key[u];
+        ws.slot[at] = (uint16_t)slot[u];
+      }
+      D += __popcll(om);
     }
-    if constexpr (!SYM) {
-#pragma unroll
-      for (int u = 0; u < kE; ++u)
-        if (slot[u] >= 0) SR::acc(&s_val[w][slot[u]], val[u]);
-    }
-    wave_lds_sync();
-    // compaction of the occupied slots (lane owns slots lane*kSPL ..)
-    int32_t kk[kSPL];
-    int occ = 0;
-#pragma unroll
-    for (int q = 0; q < kSPL; ++q) {
-      kk[q] = hk[lane * kSPL + q];
-      occ += kk[q] != kEmpty;
-    }
-    const int incl = wave_incl_scan(occ);
-    const int D = __shfl(incl, kWave - 1, kWave);  // distinct rows of the column
     if constexpr (SYM) {
       if (lane == 0) nnzcol[col] = D;
-    } else {
-      int pos = incl - occ;
-#pragma unroll
-      for (int q = 0; q < kSPL; ++q)
-        if (kk[q] != kEmpty) {
-          crow[pos] = kk[q];
-          s_slot[w][pos] = (uint16_t)(lane * kSPL + q);
-          ++pos;
-        }
-      if (lane < 4) crow[D + lane] = kNone;  // padding for the four-wide reads
       wave_lds_sync();
+      continue;
+    } else {
+      if (D <= kWave) {  // rank of every distinct row: the distinct rows below it
+        if (lane < 4) ws.rows[D + lane] = kNone;  // padding for the four-wide reads
+        wave_lds_sync();
+        const int32_t mine = lane < D ? ws.rows[lane] : kNone;
+        const int at = ws.slot[min(lane, max(D - 1, 0))];
+        int rank = 0;
+        for (int j = 0; j < D; j += 4) {
+          const int4 q = *reinterpret_cast<const int4*>(ws.rows + j);
+          rank += (q.x < mine) + (q.y < mine) + (q.z < mine) + (q.w < mine);
+        }
+        wave_lds_sync();
+        if (lane < D) {
+          ws.rows[rank] = mine;
+          ws.keys[at] = rank;
+        }
+      } else {
+        wave_lds_sync();
+        tiny_sort(ws, D);
+        for (int e = lane; e < D; e += kWave) ws.keys[ws.slot[e]] = e;
+      }
+      for (int e = lane; e < D; e += kWave) ws.vals[e] = SR::lident();
+      wave_lds_sync();
+#pragma unroll
+      for (int u = 0; u < kE; ++u)
+        if (u * kWave + lane < filled) SR::acc(&ws.vals[ws.keys[slot[u]]], val[u]);
+      // the column's allocation from the symbolic pass; or, staged (no symbolic
+      // pass), its slot of flop_j entries in the staging buffer, and the count
+      // is recorded for the copy into place
       int64_t have, out;
-      if (stage_off) {  // staged (no symbolic pass): its slot of flop_j entries; the count goes to nnzcol
+      if (stage_off) {
         out = stage_off[i];
         have = stage_off[i + 1] - out;
         if (lane == 0) nnzcol[col] = D;
@@ -847,64 +771,25 @@ __global__ __launch_bounds__(256) void k_tiny_h(const int32_t* __restrict__ orde
         if (lane == 0 && D != have) atomicOr(err, 8);
         out = cpC[col];
       }
-      // rank of every distinct row: the distinct rows below it
-      const int nc = (D + kWave - 1) / kWave;  // compacted entries per lane (wave-uniform)
-      int32_t mine[kE];
-      int rank[kE];
-#pragma unroll
-      for (int r = 0; r < kE; ++r) {
-        mine[r] = r < nc && r * kWave + lane < D ? crow[r * kWave + lane] : kNone;
-        rank[r] = 0;
-      }
-      for (int j = 0; j < D; j += 4) {
-        const int4 q4 = *reinterpret_cast<const int4*>(crow + j);
-#pragma unroll
-        for (int r = 0; r < kE; ++r)
-          if (r < nc) rank[r] += (q4.x < mine[r]) + (q4.y < mine[r]) + (q4.z < mine[r]) + (q4.w < mine[r]);
-      }
+      wave_lds_sync();
       if (!flt.on) {
-#pragma unroll
-        for (int r = 0; r < kE; ++r) {
-          const int e = r * kWave + lane;
-          if (r < nc && e < D && rank[r] < have) {
-            irC[out + rank[r]] = mine[r];
-            valC[out + rank[r]] = SR::lout(s_val[w][s_slot[w][e]]);
-          }
+        for (int e = lane; e < D && e < have; e += kWave) {
+          irC[out + e] = ws.rows[e];
+          valC[out + e] = SR::lout(ws.vals[e]);
         }
-      } else {  // the fused threshold: a kept row's place is the kept rows below it
-        T v[kE];
-        bool keep[kE];
-#pragma unroll
-        for (int r = 0; r < kE; ++r) {
-          const int e = r * kWave + lane;
-          keep[r] = false;
-          if (r < nc && e < D) {
-            v[r] = SR::lout(s_val[w][s_slot[w][e]]);
-            keep[r] = !(v[r] < flt.thr);
-          }
-        }
-        wave_lds_sync();
-#pragma unroll
-        for (int r = 0; r < kE; ++r)  // kept rows replace the compacted rows (others: kNone)
-          if (r < nc && r * kWave + lane < D) crow[r * kWave + lane] = keep[r] ? mine[r] : kNone;
-        wave_lds_sync();
-        int kr[kE];
-#pragma unroll
-        for (int r = 0; r < kE; ++r) kr[r] = 0;
-        for (int j = 0; j < D; j += 4) {
-          const int4 q4 = *reinterpret_cast<const int4*>(crow + j);
-#pragma unroll
-          for (int r = 0; r < kE; ++r)
-            if (r < nc) kr[r] += (q4.x < mine[r]) + (q4.y < mine[r]) + (q4.z < mine[r]) + (q4.w < mine[r]);
-        }
+      } else {  // the fused threshold: kept entries, in row order, at out
         int kept = 0;
-#pragma unroll
-        for (int r = 0; r < kE; ++r) {
-          kept += __popcll(__ballot(keep[r]));
-          if (keep[r] && kr[r] < have) {
-            irC[out + kr[r]] = mine[r];
-            valC[out + kr[r]] = v[r];
+        for (int e0 = 0; e0 < D; e0 += kWave) {
+          const int e = e0 + lane;
+          const T v = e < D ? SR::lout(ws.vals[e]) : T{};
+          const bool keep = e < D && !(v < flt.thr);
+          const unsigned long long km = __ballot(keep);
+          const int at = kept + __popcll(km & ((1ull << lane) - 1ull));
+          if (keep && at < have) {
+            irC[out + at] = ws.rows[e];
+            valC[out + at] = v;
           }
+          kept += __popcll(km);
         }
         if (lane == 0) {
           if (stage_off) {
@@ -915,8 +800,8 @@ __global__ __launch_bounds__(256) void k_tiny_h(const int32_t* __restrict__ orde
           }
         }
       }
+      wave_lds_sync();  // the next column reuses the wave's LDS
     }
-    wave_lds_sync();  // the next column reuses the wave's table
   }
 }
 
@@ -1003,7 +888,7 @@ __global__ __launch_bounds__(NT) void k_sym_dense(const int32_t* __restrict__ or
 // A digit pass ranks 64 keys at a time by wave ballots: every wave counts its
 // own 256 keys, so the pass needs one block scan over (digit, wave) and no
 // atomics.  At R-MAT s19 ef16 (int64) the columns of 1025 to 4096 products
-// take 3.2 ms and the smaller ones 0.35 ms; a hash table with LDS compaction
+// take 1.9 ms and the smaller ones 0.32 ms; a hash table with LDS compaction
 // and a bitonic sort took 17.3 ms (one 119 KB workgroup per CU, 78 barriers a
 // sort) and 1.2 ms.  Bound by VALU (the ballots) and LDS; 60 KB at 1024
 // threads: two workgroups per CU, all 32 waves.  The workgroup has a quarter
@@ -1021,76 +906,74 @@ __global__ __launch_bounds__(NT) void k_num_sort(const int32_t* __restrict__ ord
   using Acc = typename SR::Acc;
   constexpr int U = 4, CAP = U * NT, NW = NT / kWave;
   constexpr int kDigit = 7;  // bits per pass at most: 128 * NW 16-bit counters, two per thread
+  constexpr int kRow = (1 << kDigit) + 2;  // a wave's counters, padded so that equal digits differ in bank
   static_assert((1 << kDigit) * NW == 2 * NT, "one pair of counters per thread");
   union Window {
-    SegStage<T, NT> st;  // while the products are gathered
+    FlatStage<T, NT, true> st;  // while the products are gathered
     typename SR::Lds vals[CAP];  // once their ranks are known
   };
   __shared__ __align__(16) uint32_t keys[CAP];
   __shared__ __align__(8) uint16_t pay[CAP];  // product numbers, then the products' ranks
-  __shared__ uint32_t hist32[NT];
+  __shared__ __align__(8) uint16_t hist[kRow * NW];
   __shared__ __align__(16) unsigned char window_mem[sizeof(Window)];
   __shared__ long long wsum[NW];
   __shared__ int isum[NW];
   Window& win = *reinterpret_cast<Window*>(window_mem);
-  uint16_t* hist = reinterpret_cast<uint16_t*>(hist32);
-  const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
+  const int tid = threadIdx.x, lane = lane_id(), w = wave_id_uniform();
+  // where position p of the sorted order is kept: a pass's stores come 4096 /
+  // 128 positions apart where a segment's rows are dense, one bank without it
+  auto place = [](int p) { return p ^ ((p >> 6) & 63); };
+  auto clear_hist = [&]() {
+    for (int i = tid; i < kRow * NW / 2; i += NT) reinterpret_cast<uint32_t*>(hist)[i] = 0;
+  };
   const int col = order[first + blockIdx.x];
   const int64_t b0 = cpB[col], b1 = cpB[col + 1];
-  // products tid * U .. tid * U + U - 1 of the column
+  // products (u * NW + w) * 64 + lane of the column
   uint32_t key[U], num[U];
   Acc prod[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     key[u] = 0;
-    num[u] = (uint32_t)(tid * U + u);
+    num[u] = (uint32_t)((u * NW + w) * kWave + lane);
     prod[u] = SR::ident();
   }
-  int total = 0;
+  int total = 0, par = 0;
+  flat_init(win.st);
   for (int64_t eb = b0; eb < b1; eb += NT) {
     int64_t base;
-    int len, nseg;
+    int len;
     T bv;
     load_seg<T, true>(eb + tid, b1, bpos, cpA, Tiles{}, 0, 0, true, valB, base, len, bv);
-    const int tot = stage_chunk<T, NT>(win.st, wsum, base, len, bv, nseg);
-    const int x0 = tid * U - total;  // this chunk's number of the thread's first product
-    if (x0 + U > 0 && x0 < tot) {
-      const int xf = max(x0, 0);
-      int lo = 0, hi = nseg;  // largest k with off[k] <= xf
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (win.st.off[mid] <= xf) lo = mid;
-        else hi = mid;
-      }
-      int k = lo, cur = win.st.off[k], nxt = win.st.off[k + 1];
-      int64_t idx[U];
-      T bvs[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int x = x0 + u;
-        idx[u] = -1;
-        if (x >= 0 && x < tot) {
-          if (x >= nxt) {
-            ++k;
-            cur = nxt;
-            nxt = win.st.off[k + 1];
-          }
-          idx[u] = win.st.base[k] + (x - cur);
-          bvs[u] = win.st.bval[k];
-        }
-      }
-      T a[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (idx[u] >= 0) {
-          key[u] = (uint32_t)rowsA[idx[u]];
-          a[u] = valA[idx[u]];
-        }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (idx[u] >= 0) prod[u] = SR::mul(a[u], bvs[u]);
+    const FlatSeg me = flat_stage<T, NT, true>(win.st, (int32_t)base, len, bv, total);
+    if (me.total == 0 || total >= CAP) {  // (uniform)
+      total += me.total;
+      __syncthreads();  // every wave has read the counts before the next chunk's are written
+      continue;
     }
-    total += tot;
+    const FlatTile ft = flat_tile(win.st, me, 0, 0, par);
+    par ^= 1;
+    const int end = min(total + me.total, CAP);
+    int32_t idx[U], r[U];
+    T a[U], bvs[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int wd = u * NW + w;  // at most 63: the tile's first half
+      const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)ft.w0, wd);
+      const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(ft.w0 >> 32), wd);
+      const unsigned kb = (unsigned)__builtin_amdgcn_readlane(ft.p0, wd);
+      const int k = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, kb));
+      // products of other chunks repeat this one's first or last
+      idx[u] = min(max((int)num[u], total), end - 1) + win.st.delta[k];
+      bvs[u] = win.st.bval[k];
+    }
+    load_entries(rowsA, valA, 0, idx, bvs, r, a);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if ((int)num[u] >= total && (int)num[u] < end) {
+        key[u] = (uint32_t)r[u];
+        prod[u] = SR::mul(a[u], bvs[u]);
+      }
+    total += me.total;
   }
   if (total > CAP) {  // the tier's bound keeps it below; guard anyway (uniform)
     if (tid == 0) atomicOr(err, 2);
@@ -1103,12 +986,12 @@ __global__ __launch_bounds__(NT) void k_num_sort(const int32_t* __restrict__ ord
   uint32_t diff = 0;
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    if (tid * U + u < total) diff |= key[u] ^ key0;
+    if ((int)num[u] < total) diff |= key[u] ^ key0;
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) diff |= (uint32_t)__shfl_xor((int)diff, d, kWave);
   __syncthreads();
   if (lane == 0) isum[w] = (int)diff;
-  hist32[tid] = 0;
+  clear_hist();
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NW; ++i) diff |= (uint32_t)isum[i];
@@ -1121,16 +1004,11 @@ __global__ __launch_bounds__(NT) void k_num_sort(const int32_t* __restrict__ ord
     int rank[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const bool valid = p == 0 ? tid * U + u < total : (w * U + u) * kWave + lane < total;
+      const bool valid = (p == 0 ? (int)num[u] : (w * U + u) * kWave + lane) < total;
       const uint32_t d = (key[u] >> shift) & dmask;
-      unsigned long long same = __ballot(valid);
-      for (int b = 0; b < width; ++b) {
-        const bool bit = (d >> b) & 1u;
-        const unsigned long long m = __ballot(bit);
-        same &= bit ? m : ~m;
-      }
+      const unsigned long long same = wave_match(d, width, __ballot(valid));
       const int before = __popcll(same & ((1ull << lane) - 1ull));
-      uint16_t* h = &hist[d * NW + w];
+      uint16_t* h = &hist[w * kRow + d];
       int seen = 0;
       if (valid) seen = *h;
       wave_lds_sync();
@@ -1140,41 +1018,43 @@ __global__ __launch_bounds__(NT) void k_num_sort(const int32_t* __restrict__ ord
     }
     __syncthreads();
     {
-      const uint32_t pair = hist32[tid];
-      const int c0 = (int)(pair & 0xffffu), c1 = (int)(pair >> 16);
+      // counters 2 tid and 2 tid + 1 in (digit, wave) order
+      uint16_t* h = &hist[2 * tid % NW * kRow + 2 * tid / NW];
+      const int c0 = h[0], c1 = h[kRow];
       int all;
       const int ex = block_excl_scan<NT>(c0 + c1, isum, all);
-      hist32[tid] = (uint32_t)ex | ((uint32_t)(ex + c0) << 16);
+      h[0] = (uint16_t)ex;
+      h[kRow] = (uint16_t)(ex + c0);
     }
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (rank[u] >= 0) {
-        const int at = (int)hist[((key[u] >> shift) & dmask) * NW + w] + rank[u];
+        const int at = place((int)hist[w * kRow + ((key[u] >> shift) & dmask)] + rank[u]);
         keys[at] = key[u];
         pay[at] = (uint16_t)num[u];
       }
     __syncthreads();
     if (p + 1 < npass) {
-      hist32[tid] = 0;
+      clear_hist();
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int e = (w * U + u) * kWave + lane;
-        key[u] = e < total ? keys[e] : 0u;
+        const int e = place((w * U + u) * kWave + lane);
+        key[u] = keys[e];  // (past the end: never counted)
         num[u] = pay[e];
       }
       __syncthreads();
     }
   }
   // heads of equal rows among the thread's four sorted positions, and their numbers
-  uint32_t prev = tid > 0 && tid * U - 1 < total ? keys[tid * U - 1] : 0u;
+  uint32_t prev = tid > 0 ? keys[place(tid * U - 1)] : 0u;
   bool head[U];
   int heads = 0;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int e = tid * U + u;
-    key[u] = e < total ? keys[e] : 0u;
-    num[u] = pay[e];
+    key[u] = keys[place(e)];
+    num[u] = pay[place(e)];
     head[u] = e < total && (e == 0 || key[u] != prev);
     prev = key[u];
     heads += head[u];
@@ -1195,8 +1075,8 @@ __global__ __launch_bounds__(NT) void k_num_sort(const int32_t* __restrict__ ord
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    if (tid * U + u < total) {
-      const int q = pay[tid * U + u];
+    if ((u * NW + w) * kWave + lane < total) {
+      const int q = pay[(u * NW + w) * kWave + lane];
       if (q < cnt) SR::acc(&win.vals[q], prod[u]);
     }
   __syncthreads();
@@ -2763,20 +2643,15 @@ inline unsigned tiny_grid(int64_t ncols, int waves) {
   return (unsigned)std::min<int64_t>((ncols + waves - 1) / waves, (int64_t)262144 / waves);
 }
 
-// The tiny tier in the configured form (register sort or LDS table) and
-// workgroup shape.
+// The tiny tier in the configured workgroup shape.
 template <int K, class T, bool SYM>
 void launch_tiny(const SpgemmConfig& cfg, const int32_t* order, int64_t first, int64_t ncols, const int64_t* cpB,
                  const int32_t* bpos, const T* valB, const int64_t* cpA, const int32_t* rowsA, const T* valA,
                  int64_t* nnzcol, const int64_t* cpC, int64_t* irC, T* valC, int* err, const int64_t* stage_off,
                  hipStream_t s, const Filter<T>& flt = {}) {
   const dim3 g(tiny_grid(ncols, cfg.tiny_wg_waves)), b(kWave * cfg.tiny_wg_waves);
-  if (cfg.tiny_algo == 1)
-    k_tiny_h<K, T, SYM><<<g, b, 0, s>>>(order, first, ncols, cpB, bpos, valB, cpA, rowsA, valA, nnzcol, cpC, irC,
-                                        valC, err, stage_off, flt);
-  else
-    k_tiny<K, T, SYM><<<g, b, 0, s>>>(order, first, ncols, cpB, bpos, valB, cpA, rowsA, valA, nnzcol, cpC, irC, valC,
-                                      err, stage_off, flt);
+  k_tiny<K, T, SYM><<<g, b, 0, s>>>(order, first, ncols, cpB, bpos, valB, cpA, rowsA, valA, nnzcol, cpC, irC, valC, err,
+                                    stage_off, flt);
 }
 
 // Row lists of the small units (k_sym_units); lists == nullptr: none.

@@ -198,8 +198,8 @@ typedef struct cbx_spgemm_config {
   int32_t unit_order;      /* order of the exactly sized row-range units in the numeric pass: 0 as the symbolic
                               pass cut them (column by column), 1 by first row block (the units in flight then
                               gather from a narrow band of A's rows, which the L2 caches hold) */
-  int32_t tiny_algo;       /* tiny tier: 0 sorts a column's products in registers (bitonic network across lanes),
-                              1 merges them in a per-wave LDS hash table and ranks the distinct rows */
+  int32_t tiny_algo;       /* tiny tier: 0 or 1, both the per-wave LDS hash table with sorted distinct rows (0 was a
+                              bitonic sort in registers, slower at every size) */
   int32_t sym_band;        /* symbolic pass of the row-range units: 0 one workgroup per column over all its rows;
                               16 or 64 one workgroup per (column, band of that many 4096-row blocks), dispatched
                               band by band so the gathers in flight stay in one band of A's rows */
@@ -207,7 +207,7 @@ typedef struct cbx_spgemm_config {
                               into the product's emission (only entries that can survive the epilogue are
                               written; same result), 0 writes the whole product first */
   int32_t unit_lists;      /* two-phase mode with sym_band 0: 1 lets the symbolic pass write the sorted rows of the
-                              columns that form 4096-output units (2 bytes per output, when they fit a fifth of
+                              columns that form 3264-output units (2 bytes per output, when they fit a fifth of
                               the free memory), so those columns are cut by output count alone, over any number
                               of row blocks, and each such unit gathers its products once; 0 cuts them at 16
                               blocks and counts each unit's rows in a first sweep */
