@@ -9,6 +9,7 @@
 #include <map>
 #include <mutex>
 #include <unordered_map>
+#include <vector>
 
 #include "cbx_device.h"
 #include "cbx_spgemm.h"
@@ -129,6 +130,62 @@ size_t cache_idle_bytes() {
   return c.idle_bytes;
 }
 
+namespace {
+struct Slots {
+  std::mutex mu;
+  std::vector<CallSlot*> idle;
+};
+Slots& slots() {
+  static Slots* p = new Slots();  // never destroyed: outlives static teardown order
+  return *p;
+}
+void destroy_slot(CallSlot* p) {
+  if (p->host) (void)hipHostFree(p->host);
+  for (hipEvent_t e : p->ev)
+    if (e) (void)hipEventDestroy(e);
+  delete p;
+}
+}  // namespace
+
+CallSlot* slot_acquire() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  {
+    std::lock_guard<std::mutex> g(slots().mu);
+    auto& v = slots().idle;
+    for (size_t i = v.size(); i-- > 0;)
+      if (v[i]->device == dev) {
+        CallSlot* p = v[i];
+        v.erase(v.begin() + (ptrdiff_t)i);
+        return p;
+      }
+  }
+  CallSlot* p = new CallSlot();
+  p->device = dev;
+  bool ok = hipHostMalloc(&p->host, 4096, hipHostMallocDefault) == hipSuccess;
+  for (int i = 0; ok && i < CallSlot::kEvents; ++i) ok = hipEventCreate(&p->ev[i]) == hipSuccess;
+  if (!ok) {
+    (void)hipGetLastError();
+    destroy_slot(p);
+    return nullptr;
+  }
+  return p;
+}
+
+void slot_release(CallSlot* p) {
+  std::lock_guard<std::mutex> g(slots().mu);
+  slots().idle.push_back(p);
+}
+
+void release_slots() {
+  std::vector<CallSlot*> v;
+  {
+    std::lock_guard<std::mutex> g(slots().mu);
+    v.swap(slots().idle);
+  }
+  for (CallSlot* p : v) destroy_slot(p);
+}
+
 void release_cache() {
   Cache& c = cache();
   {
@@ -149,28 +206,9 @@ void release_cache() {
 
 using namespace cbx;
 
-extern "C" void cbx_release_cached_memory(void) { release_cache(); }
-
-cbx_status cbx::scratch_alloc(void** p, size_t bytes, hipStream_t s) {
-  bytes = std::max<size_t>(bytes, 256);
-  if (bytes >= kScratchCacheMin) return dev_alloc(p, bytes);
-  const hipError_t e = hipMallocAsync(p, bytes, s);
-  if (e != hipSuccess) {
-    *p = nullptr;
-    (void)hipGetLastError();
-    return set_error(CBX_ERR_NOMEM, "device allocation of %zu bytes failed: %s", bytes, hipGetErrorString(e));
-  }
-  return CBX_OK;
-}
-
-void cbx::scratch_free(void* p, size_t bytes, hipStream_t s) {
-  if (!p) return;
-  if (std::max<size_t>(bytes, 256) >= kScratchCacheMin) {
-    (void)hipStreamSynchronize(s);  // the stream's kernels may still read it
-    dev_free(p);
-  } else {
-    (void)hipFreeAsync(p, s);
-  }
+extern "C" void cbx_release_cached_memory(void) {
+  release_cache();
+  release_slots();
 }
 
 extern "C" int32_t cbx_device_count(void) {

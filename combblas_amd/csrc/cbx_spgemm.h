@@ -3,7 +3,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <utility>
 #include <vector>
 
 #include "cbx_internal.h"
@@ -89,26 +88,16 @@ void dev_free(void* p);
 void release_cache();
 size_t cache_idle_bytes();  // bytes held by the cache and free for reuse
 
-// Scratch of one call on stream s.  Blocks of kScratchCacheMin bytes or more
-// come from the caching allocator above (plain hipMalloc on a miss, which is
-// fast); smaller ones from the stream-ordered pool.  Growing the pool by
-// gigabytes has taken up to 1.5 s per allocation, and hipFreeAsync of pool
-// blocks of a few megabytes 2-4 ms of host time each (7 ms per R-MAT s20
-// product at a 64 MB bound), so all but the smallest scratch stays out of
-// it.  scratch_free waits for s before it caches a block.
-constexpr size_t kScratchCacheMin = (size_t)1 << 20;
-cbx_status scratch_alloc(void** p, size_t bytes, hipStream_t s);
-void scratch_free(void* p, size_t bytes, hipStream_t s);
-
-// The scratch blocks of one call, released together (at the latest when the
-// set goes out of scope).  Requests of up to 64 KB are carved (256-byte
-// aligned) from 1 MB chunks of the caching allocator: counters, verdicts and
-// scan storage then cost no stream-pool call each (a pool free has taken
-// 10-20 us of host time, several per call).
+// The scratch blocks of one call, from the caching allocator above, released
+// together once the stream's kernels are done (at the latest when the set goes
+// out of scope).  Requests of up to 64 KB are carved (256-byte aligned) from
+// 1 MB chunks.  The stream-ordered pool is not used: its frees took 10-20 us of
+// host time each (blocks of a few megabytes 2-4 ms), some thirty a product,
+// and growing it by gigabytes up to 1.5 s.
 struct ScratchSet {
   static constexpr size_t kSmall = (size_t)64 << 10, kChunk = (size_t)1 << 20;
   hipStream_t s;
-  std::vector<std::pair<void*, size_t>> blocks;
+  std::vector<void*> blocks;
   uint8_t* chunk = nullptr;
   size_t chunk_used = 0;
   explicit ScratchSet(hipStream_t st) : s(st) {}
@@ -119,8 +108,8 @@ struct ScratchSet {
     if (bytes <= kSmall) {
       if (!chunk || chunk_used + bytes > kChunk) {
         void* c = nullptr;
-        if (scratch_alloc(&c, kChunk, s) != CBX_OK) return false;
-        blocks.emplace_back(c, kChunk);
+        if (dev_alloc(&c, kChunk) != CBX_OK) return false;
+        blocks.push_back(c);
         chunk = (uint8_t*)c;
         chunk_used = 0;
       }
@@ -128,8 +117,8 @@ struct ScratchSet {
       chunk_used += bytes;
       return true;
     }
-    if (scratch_alloc(p, bytes, s) != CBX_OK) return false;
-    blocks.emplace_back(*p, bytes);
+    if (dev_alloc(p, bytes) != CBX_OK) return false;
+    blocks.push_back(*p);
     return true;
   }
   template <class X>
@@ -140,12 +129,35 @@ struct ScratchSet {
     return ok;
   }
   void release() {
-    for (auto& b : blocks) scratch_free(b.first, b.second, s);
+    if (!blocks.empty()) (void)hipStreamSynchronize(s);  // the stream's kernels may still read them
+    for (void* b : blocks) dev_free(b);
     blocks.clear();
     chunk = nullptr;
     chunk_used = 0;
   }
   ~ScratchSet() { release(); }
+};
+
+// What one call at a time holds beside device memory: a page of pinned host
+// memory that its kernels report into, and events for its timings.  Kept in a
+// list of idle ones, as many as calls ran at once on a device, and given back
+// by cbx_release_cached_memory.
+struct CallSlot {
+  static constexpr int kEvents = 9;
+  int device = 0;
+  void* host = nullptr;  // 4096 bytes
+  hipEvent_t ev[kEvents] = {};
+};
+CallSlot* slot_acquire();  // null: no memory
+void slot_release(CallSlot* slot);
+struct SlotHold {
+  CallSlot* p;
+  SlotHold() : p(slot_acquire()) {}
+  ~SlotHold() {
+    if (p) slot_release(p);
+  }
+  SlotHold(const SlotHold&) = delete;
+  SlotHold& operator=(const SlotHold&) = delete;
 };
 
 // Shared front-door helpers (cbx_runtime.hip).

@@ -274,49 +274,449 @@ __device__ __forceinline__ void load_entries(const int32_t* __restrict__ rowsA, 
   }
 }
 
+// Lanes of the wave with the same value of the low `width` bits of d, among
+// `valid` ones.
+__device__ __forceinline__ unsigned long long wave_match(uint32_t d, int width, unsigned long long valid) {
+  unsigned long long same = valid;
+  for (int b = 0; b < width; ++b) {
+    const bool bit = (d >> b) & 1u;
+    const unsigned long long m = __ballot(bit);
+    same &= bit ? m : ~m;
+  }
+  return same;
+}
+
 // ------------------------------------------------------------------ setup
 __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
 
-__global__ void k_iota_i32(int32_t* p, int64_t n) {
-  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) p[i] = (int32_t)i;
+// Input validation (the reference's preconditions, mtSpGEMM.h / dcsc.h):
+// cp starts at 0, ends at nnz and never decreases (empty columns allowed); jc
+// strictly increasing and below ncols; rows of every column strictly
+// increasing and below nrows.  One fully parallel pass: per entry, rows in
+// range and every adjacent descent ir[e+1] <= ir[e] counted; per column, cp
+// and jc, and the descents at the positions where a column begins (each
+// distinct start counted once).  With cp valid those are the only places a
+// descent is allowed, so the rows ascend within columns iff the two counts
+// agree.  cnt[0] violations, cnt[1] descents, cnt[2] descents at starts.
+// With rows32 the pass also writes the rows as 32-bit (garbage where a row is
+// out of range; nothing uses it then): one reading of ir instead of two.
+constexpr int kValNT = 256, kValBlocks = 1024;
+
+__global__ __launch_bounds__(kValNT) void k_validate(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc,
+                                                     const int64_t* __restrict__ ir, int64_t nzc, int64_t nnz,
+                                                     int64_t nrows, int64_t ncols, int eblocks,
+                                                     int32_t* __restrict__ rows32,
+                                                     unsigned long long* __restrict__ cnt) {
+  long long bad = 0, desc = 0;
+  if ((int)blockIdx.x < eblocks) {  // entries
+    const int64_t stride = (int64_t)eblocks * kValNT;
+    for (int64_t e = blockIdx.x * (int64_t)kValNT + threadIdx.x; e < nnz; e += stride) {
+      const int64_t r = ir[e];
+      const int64_t next = ir[min(e + 1, nnz - 1)];
+      bad += r < 0 || r >= nrows;
+      desc += e + 1 < nnz && next <= r;
+      if (rows32) rows32[e] = (int32_t)r;
+    }
+    block_add_counts<kValNT>(bad, desc, &cnt[0], &cnt[1]);
+  } else {  // columns
+    const int64_t stride = (int64_t)(gridDim.x - eblocks) * kValNT;
+    for (int64_t q = ((int64_t)blockIdx.x - eblocks) * kValNT + threadIdx.x; q < nzc; q += stride) {
+      const int64_t b = cp[q], e = cp[q + 1], j = jc[q];
+      bool err = b < 0 || e < b || e > nnz || j < 0 || j >= ncols;
+      if (q + 1 < nzc) err |= jc[q + 1] <= j;
+      if (q == 0) err |= b != 0;
+      if (q == nzc - 1) err |= e != nnz;
+      bad += err;
+      if (!err && q > 0 && b > 0 && b < nnz && cp[q - 1] < b) desc += ir[b] <= ir[b - 1];
+    }
+    block_add_counts<kValNT>(bad, desc, &cnt[0], &cnt[2]);
+  }
 }
 
-// colmap[jcA[p]] = p  (dense lookup replacing Dcsc::ConstructAux/FillColInds,
-// dcsc.cpp:1042-1070 and :1361-1423)
-__global__ void k_colmap(const int64_t* __restrict__ jc, int64_t nzc, int32_t* __restrict__ colmap) {
-  int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (p < nzc) colmap[jc[p]] = (int32_t)p;
+__device__ __forceinline__ bool counts_valid(const unsigned long long* cnt) {
+  return cnt[0] == 0 && cnt[1] == cnt[2];
 }
 
+__global__ void k_validate_flag(const unsigned long long* __restrict__ cnt, int flagbit, int* __restrict__ err) {
+  if (threadIdx.x == 0 && !counts_valid(cnt)) atomicOr(err, 1 << flagbit);
+}
+
+// Launches the validation of X on s; cnt: 3 device counters, cleared before.
+static cbx_status launch_validate(const cbx_dcsc* X, int32_t* rows32, unsigned long long* cnt, hipStream_t s) {
+  auto blocks = [](int64_t n) {
+    return (unsigned)std::min<int64_t>(std::max<int64_t>((n + kValNT - 1) / kValNT, 1), kValBlocks);
+  };
+  const unsigned eb = blocks(X->nnz);
+  k_validate<<<eb + blocks(X->nzc), kValNT, 0, s>>>(X->cp, X->jc, X->ir, X->nzc, X->nnz, X->m, X->n, (int)eb, rows32,
+                                                    cnt);
+  CBX_HIP(hipGetLastError());
+  return CBX_OK;
+}
+
+// 32-bit rows alone, for operands that need no validation.
 __global__ void k_rows32(const int64_t* __restrict__ ir, int64_t nnz, int32_t* __restrict__ out) {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < nnz) out[i] = (int32_t)ir[i];
 }
 
-// bpos[e] = stored-column position in A of B's row index irB[e] (-1 if A(:,k) is empty).
-__global__ void k_bpos(const int64_t* __restrict__ irB, int64_t nnzB, const int32_t* __restrict__ colmap,
-                       int32_t* __restrict__ bpos) {
-  int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (e < nnzB) bpos[e] = colmap[irB[e]];
+// Columns by their products, largest class first: 0 beyond unit_split_nnz
+// (large units possible), 1 the other unit-tier columns, 2..4 the sort tier's
+// three workgroup sizes, 5 tiny, 6 empty.
+struct FlopClasses {
+  int64_t split, small, s4k, mid, tiny;  // lower bounds (exclusive) of classes 0 .. 4
+  int64_t list_cap;                      // row-list region of a unit-tier column: min(flop, list_cap)
+};
+constexpr int kClasses = 7, kDigits = kClasses * 32;
+
+// The column's class and, within it, 32 steps by size: the sort digit, small
+// for large columns.
+__device__ __forceinline__ int flop_digit(const FlopClasses& c, int64_t f) {
+  auto octaves = [](int64_t f, int64_t lo) {  // half octaves above lo
+    const int l = 63 - __clzll((unsigned long long)f), l0 = 63 - __clzll((unsigned long long)(lo | 1));
+    return min(31, max(0, 2 * (l - l0) + (int)((f >> max(l - 1, 0)) & 1)));
+  };
+  int cls, sub = 0;
+  if (f > c.split) cls = 0, sub = octaves(f, c.split);
+  else if (f > c.small) cls = 1, sub = octaves(f, c.small);
+  else if (f > c.s4k) cls = 2, sub = (int)(f >> 7);
+  else if (f > c.mid) cls = 3, sub = (int)(f >> 6);
+  else if (f > c.tiny) cls = 4, sub = (int)(f >> 5);
+  else if (f > 0) cls = 5, sub = (int)(f >> 3);
+  else cls = 6;
+  return cls * 32 + 31 - min(31, sub);
 }
 
-// flop_j (estimateFLOP, mtSpGEMM.h:1112-1130): one wave per column of B.
-__global__ void k_flop(const int64_t* __restrict__ cpB, int64_t nzcB, const int32_t* __restrict__ bpos,
-                       const int64_t* __restrict__ cpA, int64_t* __restrict__ flop) {
-  const int64_t col = global_wave();
-  if (col >= nzcB) return;
-  const int lane = lane_id();
-  long long f = 0;
-  for (int64_t e = cpB[col] + lane; e < cpB[col + 1]; e += kWave) {
-    const int32_t p = bpos[e];
-    if (p >= 0) f += cpA[p + 1] - cpA[p];
+// Device-side counters of one product, cleared together before it starts.
+struct Counters {
+  int err;
+  int units[3];                     // small (bitmap), large, and small list units
+  unsigned long long val[6];        // validation of A and of B
+  unsigned int digits[kDigits];     // columns of each sort digit
+  unsigned int cursor[kDigits];     // of them placed so far
+  unsigned long long flops, tiny_flops, list_rows;  // totals: products, those of tiny columns, list regions
+  unsigned long long tiny_at, list_at;              // of the latter two, handed out so far
+  unsigned long long main_nnz;                      // outputs of the unit-tier columns
+  unsigned long long dropped;                       // fused threshold: entries the staged tiny tier left out
+  int runs;                                         // fused threshold: ranges appended
+};
+
+// What the host waits for, written by a kernel into pinned memory: after the
+// setup, after the symbolic pass, at the end.
+struct Report {
+  int err, units[3];
+  int64_t columns[kClasses];
+  int64_t flops, tiny_flops, list_rows;
+  int64_t nnz, nzc, main_nnz, dropped;
+};
+
+__global__ __launch_bounds__(256) void k_init(Counters* __restrict__ c, int32_t* __restrict__ colmap, int64_t n,
+                                              int64_t* __restrict__ flop, int64_t* __restrict__ nnzcol, int64_t nzcB) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x, t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  for (int64_t i = t; i < (int64_t)(sizeof(Counters) / 4); i += stride) reinterpret_cast<uint32_t*>(c)[i] = 0;
+  if (colmap)
+    for (int64_t i = t; i < n; i += stride) colmap[i] = -1;
+  for (int64_t i = t; i <= nzcB; i += stride) {
+    flop[i] = 0;
+    nnzcol[i] = 0;
   }
-  f = wave_sum_ll(f);
-  if (lane == 0) flop[col] = f;
+}
+
+// colmap[jcA[p]] = p  (dense lookup replacing Dcsc::ConstructAux/FillColInds,
+// dcsc.cpp:1042-1070 and :1361-1423)
+__global__ void k_colmap(const int64_t* __restrict__ jc, int64_t nzc, const Counters* __restrict__ c,
+                         int32_t* __restrict__ colmap) {
+  if (c && !counts_valid(c->val)) return;
+  int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (p < nzc) colmap[jc[p]] = (int32_t)p;
+}
+
+// bpos[e] = stored-column position in A of B's row index irB[e] (-1 if A(:,k)
+// is empty; the row itself where A stores every column, colmap null), and the
+// columns' products flop_j (estimateFLOP, mtSpGEMM.h:1112-1130; flop cleared
+// before).  One workgroup per 1024 consecutive entries: their A-column lengths
+// are summed by a block scan, and every column takes the difference of two
+// prefixes, so a hub column of 1e5 entries is shared by a hundred workgroups
+// (a wave per column took 0.20 ms at R-MAT s19, this 0.04 with the positions).
+constexpr int kFlopNT = 256, kFlopTile = 4 * kFlopNT;
+__global__ __launch_bounds__(kFlopNT) void k_flops(const int64_t* __restrict__ cpB, const int64_t* __restrict__ irB,
+                                                   int64_t nzcB, int64_t nnzB, const int32_t* __restrict__ colmap,
+                                                   const int64_t* __restrict__ cpA, const Counters* __restrict__ c,
+                                                   int32_t* __restrict__ bpos, int64_t* __restrict__ flop) {
+  __shared__ int len[kFlopTile];
+  __shared__ long long pre[kFlopTile + 1];
+  __shared__ long long wsum[kFlopNT / kWave];
+  if (c && !(counts_valid(c->val) && counts_valid(c->val + 3))) return;
+  const int64_t t0 = blockIdx.x * (int64_t)kFlopTile;
+  const int n = (int)min((int64_t)kFlopTile, nnzB - t0);
+  int32_t p[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int64_t k = irB[t0 + min(u * kFlopNT + (int)threadIdx.x, n - 1)];
+    p[u] = colmap ? colmap[k] : (int32_t)k;
+    pin(p[u]);
+  }
+  int l[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int32_t q = max(p[u], 0);
+    l[u] = (int)(cpA[q + 1] - cpA[q]);
+    pin(l[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int i = u * kFlopNT + threadIdx.x;
+    if (i < n) bpos[t0 + i] = p[u];
+    len[i] = i < n && p[u] >= 0 ? l[u] : 0;
+  }
+  __syncthreads();
+  const int4 v = reinterpret_cast<const int4*>(len)[threadIdx.x];
+  const long long s0 = v.x, s1 = s0 + v.y, s2 = s1 + v.z, s3 = s2 + v.w;
+  long long total;
+  const long long ex = block_excl_scan_ll<kFlopNT>(s3, wsum, total);
+  const int i4 = threadIdx.x * 4;
+  pre[i4] = ex;
+  pre[i4 + 1] = ex + s0;
+  pre[i4 + 2] = ex + s1;
+  pre[i4 + 3] = ex + s2;
+  if (threadIdx.x == kFlopNT - 1) pre[kFlopTile] = total;
+  // the column of the tile's first entry: last c with cp[c] <= t0, 256 probes a step
+  int64_t lo = 0, hi = nzcB;
+  while (hi - lo > 1) {
+    const int64_t step = (hi - lo + kFlopNT - 1) / kFlopNT;
+    const int64_t at = lo + (int64_t)threadIdx.x * step;
+    const int below = __syncthreads_count(at < hi && cpB[min(at, hi - 1)] <= t0);
+    lo += (int64_t)(below - 1) * step;
+    hi = min(hi, lo + step);
+  }
+  __syncthreads();
+  for (int64_t q = lo + threadIdx.x; q < nzcB; q += kFlopNT) {
+    const int64_t b = cpB[q], e = cpB[q + 1];
+    if (b >= t0 + n) break;
+    const int64_t from = max(b, t0), to = min(e, t0 + n);
+    if (to <= from) continue;
+    const long long f = pre[to - t0] - pre[from - t0];
+    if (b >= t0 && e <= t0 + n) flop[q] = f;
+    else if (f) atomicAdd((unsigned long long*)&flop[q], (unsigned long long)f);
+  }
+}
+
+// Counts of the sort digits, and totals.  One workgroup per 1024 columns.
+constexpr int kColTile = 1024;
+__global__ __launch_bounds__(256) void k_count_digits(const int64_t* __restrict__ flop, int64_t nzcB,
+                                                      const FlopClasses cls, Counters* __restrict__ c) {
+  __shared__ unsigned int h[kDigits];
+  for (int i = threadIdx.x; i < kDigits; i += 256) h[i] = 0;
+  __syncthreads();
+  long long all = 0, tiny = 0, list = 0;
+#pragma unroll
+  for (int u = 0; u < kColTile / 256; ++u) {
+    const int64_t q = blockIdx.x * (int64_t)kColTile + u * 256 + threadIdx.x;
+    const bool ok = q < nzcB;
+    const int64_t f = ok ? flop[q] : 0;
+    const int d = flop_digit(cls, f);
+    const unsigned long long same = wave_match((uint32_t)d, 8, __ballot(ok));
+    if (ok && __popcll(same & ((1ull << lane_id()) - 1ull)) == 0) atomicAdd(&h[d], (unsigned)__popcll(same));
+    all += f;
+    if (d / 32 == 5) tiny += f;
+    if (d / 32 < 2) list += min(f, cls.list_cap);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kDigits; i += 256)
+    if (h[i]) atomicAdd(&c->digits[i], h[i]);
+  block_add_counts<256>(all, tiny, &c->flops, &c->tiny_flops);
+  list = wave_sum_ll(list);
+  if (lane_id() == 0 && list) atomicAdd(&c->list_rows, (unsigned long long)list);
+}
+
+// Columns in digit order (within a digit, tiles of 1024 columns stay together,
+// nearly in column order): order and flop_s; the tiny columns' staging slots of
+// flop_j entries (tiny_off, by position after the classes before) and the
+// unit-tier columns' row-list regions (list_off, by position).  Two launches of
+// one pass each; a full radix sort of (flop, column) took 0.45 ms at R-MAT s19
+// and seven launches at 2^14 vertices.  The first workgroup reports the counts.
+__global__ __launch_bounds__(256) void k_order_columns(const int64_t* __restrict__ flop, int64_t nzcB,
+                                                       const FlopClasses cls, Counters* __restrict__ c,
+                                                       int32_t* __restrict__ order, int64_t* __restrict__ flop_s,
+                                                       int64_t* __restrict__ tiny_off, int64_t* __restrict__ list_off,
+                                                       Report* __restrict__ rep) {
+  constexpr int PT = kColTile / 256;
+  __shared__ int base[256];  // first position of each digit
+  __shared__ unsigned int h[kDigits], at[kDigits];
+  __shared__ long long wsum[256 / kWave];
+  __shared__ int isum[256 / kWave];
+  __shared__ long long s_at[2];
+  const int tid = threadIdx.x, lane = lane_id();
+  const bool bad_a = !counts_valid(c->val), bad_b = !counts_valid(c->val + 3);
+  if (blockIdx.x == 0 && tid == 0) {
+    rep->err = (bad_a ? 16 : 0) | (bad_b ? 32 : 0);
+    rep->flops = (int64_t)c->flops;
+    rep->tiny_flops = (int64_t)c->tiny_flops;
+    rep->list_rows = (int64_t)c->list_rows;
+    for (int k = 0; k < kClasses; ++k) {
+      int64_t n = 0;
+      for (int i = 0; i < 32; ++i) n += c->digits[k * 32 + i];
+      rep->columns[k] = n;
+    }
+  }
+  if (bad_a || bad_b) return;
+  int total;
+  const int count = tid < kDigits ? (int)c->digits[tid] : 0;
+  base[tid] = block_excl_scan<256>(count, isum, total);
+  for (int i = tid; i < kDigits; i += 256) h[i] = 0;
+  __syncthreads();
+  int64_t f[PT];
+  int d[PT];
+  unsigned rank[PT];
+  long long tiny = 0, list = 0;
+#pragma unroll
+  for (int u = 0; u < PT; ++u) {
+    const int64_t q = blockIdx.x * (int64_t)kColTile + u * 256 + tid;
+    const bool ok = q < nzcB;
+    f[u] = ok ? flop[q] : 0;
+    d[u] = flop_digit(cls, f[u]);
+    const unsigned long long same = wave_match((uint32_t)d[u], 8, __ballot(ok));
+    const int before = __popcll(same & ((1ull << lane) - 1ull));
+    unsigned first = 0;
+    if (ok && before == 0) first = atomicAdd(&h[d[u]], (unsigned)__popcll(same));
+    first = (unsigned)__shfl((int)first, __ffsll((unsigned long long)same) - 1, kWave);
+    rank[u] = first + before;
+    if (d[u] / 32 == 5) tiny += f[u];
+    if (ok && d[u] / 32 < 2) list += min(f[u], cls.list_cap);
+  }
+  __syncthreads();
+  for (int i = tid; i < kDigits; i += 256) at[i] = h[i] ? atomicAdd(&c->cursor[i], h[i]) : 0;
+  long long tiny_all, list_all;
+  long long t_at = block_excl_scan_ll<256>(tiny, wsum, tiny_all);
+  long long l_at = block_excl_scan_ll<256>(list, wsum, list_all);
+  if (tid == 0) {
+    s_at[0] = tiny_all ? (long long)atomicAdd(&c->tiny_at, (unsigned long long)tiny_all) : 0;
+    s_at[1] = list_all ? (long long)atomicAdd(&c->list_at, (unsigned long long)list_all) : 0;
+  }
+  __syncthreads();
+  t_at += s_at[0];
+  l_at += s_at[1];
+#pragma unroll
+  for (int u = 0; u < PT; ++u) {
+    const int64_t q = blockIdx.x * (int64_t)kColTile + u * 256 + tid;
+    if (q >= nzcB) continue;
+    const int pos = base[d[u]] + (int)(at[d[u]] + rank[u]);
+    order[pos] = (int32_t)q;
+    flop_s[pos] = f[u];
+    if (d[u] / 32 == 5) {
+      tiny_off[pos - base[5 * 32]] = t_at;
+      t_at += f[u];
+    }
+    if (d[u] / 32 < 2) {
+      list_off[pos] = l_at;
+      l_at += min(f[u], cls.list_cap);
+    }
+  }
+}
+
+// Output offsets and the product's DCSC columns from the columns' sizes:
+// sums of each 1024 columns, then (a scan of the sums in between where they
+// are many and) offsets cpC, and the non-empty columns' starts and ids
+// compacted into cp and jc.  The last workgroup reports the totals.
+struct ColSum {
+  long long nnz, cols;
+};
+
+__global__ __launch_bounds__(256) void k_col_sums(const int64_t* __restrict__ nnzcol, int64_t nzcB,
+                                                  const int64_t* __restrict__ flop, int64_t main_above,
+                                                  ColSum* __restrict__ sums, Counters* __restrict__ c) {
+  __shared__ long long wsum[256 / kWave];
+  long long nnz = 0, cols = 0, mine = 0;
+#pragma unroll
+  for (int u = 0; u < kColTile / 256; ++u) {
+    const int64_t q = blockIdx.x * (int64_t)kColTile + u * 256 + threadIdx.x;
+    const int64_t v = q < nzcB ? nnzcol[q] : 0;
+    nnz += v;
+    cols += v > 0;
+    if (flop && v && flop[q] > main_above) mine += v;
+  }
+  nnz = block_sum_ll<256>(nnz, wsum);
+  cols = block_sum_ll<256>(cols, wsum);
+  mine = wave_sum_ll(mine);
+  if (lane_id() == 0 && mine) atomicAdd(&c->main_nnz, (unsigned long long)mine);
+  if (threadIdx.x == 0) sums[blockIdx.x] = ColSum{nnz, cols};
+}
+
+// sums[0..n) replaced by their exclusive prefixes (one workgroup).
+__global__ __launch_bounds__(1024) void k_scan_sums(ColSum* __restrict__ sums, int64_t n) {
+  __shared__ long long wsum[1024 / kWave];
+  long long nnz = 0, cols = 0;
+  for (int64_t i0 = 0; i0 < n; i0 += 1024) {
+    const int64_t i = i0 + threadIdx.x;
+    const ColSum v = i < n ? sums[i] : ColSum{0, 0};
+    long long a, b;
+    const long long ea = block_excl_scan_ll<1024>(v.nnz, wsum, a), eb = block_excl_scan_ll<1024>(v.cols, wsum, b);
+    if (i < n) sums[i] = ColSum{nnz + ea, cols + eb};
+    nnz += a;
+    cols += b;
+  }
+}
+
+__global__ __launch_bounds__(256) void k_col_offsets(const int64_t* __restrict__ nnzcol, int64_t nzcB,
+                                                     const ColSum* __restrict__ sums, int scanned,
+                                                     const int64_t* __restrict__ jcB, const Counters* __restrict__ c,
+                                                     int64_t* __restrict__ cpC, int64_t* __restrict__ cp,
+                                                     int64_t* __restrict__ jc, Report* __restrict__ rep) {
+  constexpr int PT = kColTile / 256;
+  __shared__ long long wsum[256 / kWave];
+  const int tid = threadIdx.x;
+  long long nnz0 = 0, cols0 = 0;  // before this workgroup's columns
+  if (scanned) {
+    nnz0 = sums[blockIdx.x].nnz;
+    cols0 = sums[blockIdx.x].cols;
+  } else {
+    for (int i = tid; i < (int)blockIdx.x; i += 256) {
+      nnz0 += sums[i].nnz;
+      cols0 += sums[i].cols;
+    }
+    nnz0 = block_sum_ll<256>(nnz0, wsum);
+    cols0 = block_sum_ll<256>(cols0, wsum);
+  }
+  const int64_t q0 = blockIdx.x * (int64_t)kColTile + tid * PT;
+  int64_t v[PT];
+  long long nnz = 0, cols = 0;
+#pragma unroll
+  for (int u = 0; u < PT; ++u) {
+    v[u] = q0 + u < nzcB ? nnzcol[q0 + u] : 0;
+    nnz += v[u];
+    cols += v[u] > 0;
+  }
+  long long all_nnz, all_cols;
+  long long at = nnz0 + block_excl_scan_ll<256>(nnz, wsum, all_nnz);
+  long long col = cols0 + block_excl_scan_ll<256>(cols, wsum, all_cols);
+#pragma unroll
+  for (int u = 0; u < PT; ++u)
+    if (q0 + u < nzcB) {
+      cpC[q0 + u] = at;
+      if (v[u] > 0 && cp) {
+        cp[col] = at;
+        jc[col] = jcB[q0 + u];
+        ++col;
+      }
+      at += v[u];
+    }
+  if (blockIdx.x == gridDim.x - 1 && tid == 0) {
+    const long long n = nnz0 + all_nnz, k = cols0 + all_cols;
+    cpC[nzcB] = n;
+    if (cp) cp[k] = n;
+    rep->nnz = n;
+    rep->nzc = k;
+    rep->main_nnz = (int64_t)c->main_nnz;
+    rep->dropped = (int64_t)c->dropped;
+    rep->err = c->err;
+    for (int i = 0; i < 3; ++i) rep->units[i] = c->units[i];
+  }
+}
+
+__global__ void k_report_err(const int* __restrict__ err, Report* __restrict__ rep) {
+  if (threadIdx.x == 0) rep->err = *err;
 }
 
 // Tile pointers: P[p*(S+1)+s] = number of entries of A's p-th stored column
@@ -334,102 +734,6 @@ __global__ void k_ptable(const int64_t* __restrict__ cpA, int64_t nzcA, const in
     while (t <= tile) out[t++] = i;
   }
   while (t <= S) out[t++] = len;
-}
-
-// Class boundaries over columns sorted by flop descending:
-// bounds[c] = number of columns with flop > thr[c].
-__global__ void k_class_bounds(const int64_t* __restrict__ flop_sorted, int64_t n, const int64_t* thr, int nthr,
-                               int64_t* bounds) {
-  const int c = threadIdx.x;
-  if (c >= nthr) return;
-  int64_t lo = 0, hi = n;  // first index with flop <= thr[c]
-  while (lo < hi) {
-    int64_t mid = (lo + hi) / 2;
-    if (flop_sorted[mid] > thr[c]) lo = mid + 1;
-    else hi = mid;
-  }
-  bounds[c] = lo;
-}
-
-__global__ void k_cp_finish(int64_t* nnzcol, int64_t nzcB) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) nnzcol[nzcB] = 0;
-}
-
-// sum of nnzcol over order[0..n) (outputs of the unit-tier columns)
-__global__ void k_sum_ordered(const int32_t* __restrict__ order, int64_t n, const int64_t* __restrict__ nnzcol,
-                              unsigned long long* __restrict__ out) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  long long v = i < n ? nnzcol[order[i]] : 0;
-  v = wave_sum_ll(v);
-  if (lane_id() == 0 && v) atomicAdd(out, (unsigned long long)v);
-}
-
-__global__ void k_nonempty_flags(const int64_t* __restrict__ nnzcol, int64_t n, uint8_t* __restrict__ flags) {
-  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) flags[i] = nnzcol[i] > 0;
-}
-
-__global__ void k_set_last(int64_t* cp, const int64_t* nsel, const int64_t* total_src, int64_t total_idx) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) cp[*nsel] = total_src[total_idx];
-}
-
-// Input validation (the reference's preconditions, mtSpGEMM.h / dcsc.h):
-// cp starts at 0, ends at nnz and never decreases (empty columns allowed); jc
-// strictly increasing and below ncols; rows of every column strictly
-// increasing and below nrows.  Two fully parallel passes: per entry, rows in
-// range and every adjacent descent ir[e+1] <= ir[e] counted; per column, cp
-// and jc, and the descents at the positions where a column begins (each
-// distinct start counted once).  With cp valid those are the only places a
-// descent is allowed, so the rows ascend within columns iff the two counts
-// agree.  cnt[0] violations, cnt[1] descents, cnt[2] descents at starts;
-// k_validate_flag then sets bit `flagbit` of *err.
-constexpr int kValNT = 256, kValBlocks = 1024;
-
-__global__ __launch_bounds__(kValNT) void k_validate_cols(const int64_t* __restrict__ cp,
-                                                          const int64_t* __restrict__ jc,
-                                                          const int64_t* __restrict__ ir, int64_t nzc, int64_t nnz,
-                                                          int64_t ncols, unsigned long long* __restrict__ cnt) {
-  long long bad = 0, desc = 0;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < nzc; q += stride) {
-    const int64_t b = cp[q], e = cp[q + 1], j = jc[q];
-    bool err = b < 0 || e < b || e > nnz || j < 0 || j >= ncols;
-    if (q + 1 < nzc) err |= jc[q + 1] <= j;
-    if (q == 0) err |= b != 0;
-    if (q == nzc - 1) err |= e != nnz;
-    bad += err;
-    if (!err && q > 0 && b > 0 && b < nnz && cp[q - 1] < b) desc += ir[b] <= ir[b - 1];
-  }
-  block_add_counts<kValNT>(bad, desc, &cnt[0], &cnt[2]);
-}
-
-__global__ __launch_bounds__(kValNT) void k_validate_entries(const int64_t* __restrict__ ir, int64_t nnz,
-                                                             int64_t nrows, unsigned long long* __restrict__ cnt) {
-  long long bad = 0, desc = 0;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nnz; e += stride) {
-    const int64_t r = ir[e];
-    bad += r < 0 || r >= nrows;
-    if (e + 1 < nnz) desc += ir[e + 1] <= r;
-  }
-  block_add_counts<kValNT>(bad, desc, &cnt[0], &cnt[1]);
-}
-
-__global__ void k_validate_flag(const unsigned long long* __restrict__ cnt, int flagbit, int* __restrict__ err) {
-  if (threadIdx.x == 0 && (cnt[0] || cnt[1] != cnt[2])) atomicOr(err, 1 << flagbit);
-}
-
-// Launches the validation of X on s; cnt: 3 device counters (cleared here).
-static cbx_status launch_validate(const cbx_dcsc* X, int flagbit, unsigned long long* cnt, int* err, hipStream_t s) {
-  auto blocks = [](int64_t n) {
-    return (unsigned)std::min<int64_t>(std::max<int64_t>((n + kValNT - 1) / kValNT, 1), kValBlocks);
-  };
-  CBX_HIP(hipMemsetAsync(cnt, 0, 3 * sizeof(unsigned long long), s));
-  k_validate_cols<<<blocks(X->nzc), kValNT, 0, s>>>(X->cp, X->jc, X->ir, X->nzc, X->nnz, X->n, cnt);
-  k_validate_entries<<<blocks(X->nnz), kValNT, 0, s>>>(X->ir, X->nnz, X->m, cnt);
-  k_validate_flag<<<1, 64, 0, s>>>(cnt, flagbit, err);
-  CBX_HIP(hipGetLastError());
-  return CBX_OK;
 }
 
 // --------------------------------------------------------- symbolic: hash
@@ -522,18 +826,6 @@ struct TinyLds {
   int32_t delta[kWave];
   T bval[SYM ? 1 : kWave];
 };
-
-// Lanes of the wave with the same value of the low `width` bits of d, among
-// `valid` ones.
-__device__ __forceinline__ unsigned long long wave_match(uint32_t d, int width, unsigned long long valid) {
-  unsigned long long same = valid;
-  for (int b = 0; b < width; ++b) {
-    const bool bit = (d >> b) & 1u;
-    const unsigned long long m = __ballot(bit);
-    same &= bit ? m : ~m;
-  }
-  return same;
-}
 
 // The products of one tiny column gathered into the wave's registers: rows
 // and products of elements u * 64 + lane.  Returns their number
@@ -677,7 +969,8 @@ __global__ __launch_bounds__(256) void k_tiny(const int32_t* __restrict__ order,
                                               const int32_t* __restrict__ rowsA, const T* __restrict__ valA,
                                               int64_t* __restrict__ nnzcol, const int64_t* __restrict__ cpC,
                                               int64_t* __restrict__ irC, T* __restrict__ valC, int* __restrict__ err,
-                                              const int64_t* __restrict__ stage_off = nullptr, Filter<T> flt = {}) {
+                                              const int64_t* __restrict__ stage_off = nullptr,
+                                              const int64_t* __restrict__ stage_flop = nullptr, Filter<T> flt = {}) {
   using SR = Sem<K, T>;
   using Acc = typename SR::Acc;
   constexpr int kE = kTinyMax / kWave;
@@ -763,7 +1056,7 @@ __global__ __launch_bounds__(256) void k_tiny(const int32_t* __restrict__ order,
       int64_t have, out;
       if (stage_off) {
         out = stage_off[i];
-        have = stage_off[i + 1] - out;
+        have = stage_flop[first + i];
         if (lane == 0) nnzcol[col] = D;
         if (lane == 0 && D > have) atomicOr(err, 8);
       } else {
@@ -1175,7 +1468,7 @@ __global__ __launch_bounds__(NT) void k_num_dense(const int32_t* __restrict__ or
 // With `lists`, the column's sorted output rows in blocks of at most
 // kListBlockMax outputs are also written, as 12-bit offsets within their
 // 4096-row blocks, at their output positions in the column's region
-// lists[list_off[slot] .. list_off[slot + 1]) (slot = the workgroup), and its
+// of min(flop_j, region_cap) entries from lists[list_off[slot]] on (slot = the workgroup), and its
 // per-block counts into bcnt16[slot * S ..].  The small units of a pass whose
 // rows fit the region are then cut by output count alone over runs of such
 // blocks: those wider than rblk_l blocks go to units_s, whose numeric pass
@@ -1199,6 +1492,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
                                                   int64_t rm_cols, int* __restrict__ err,
                                                   uint16_t* __restrict__ lists = nullptr,
                                                   const int64_t* __restrict__ list_off = nullptr,
+                                                  const int64_t* __restrict__ flop = nullptr, int64_t region_cap = 0,
                                                   uint16_t* __restrict__ bcnt16 = nullptr,
                                                   Unit* __restrict__ units_s = nullptr, int* __restrict__ n_s = nullptr,
                                                   int cap_s = 0) {
@@ -1224,7 +1518,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
   int64_t list_base = 0, region = 0;
   if (lists) {
     list_base = list_off[blockIdx.x];
-    region = list_off[blockIdx.x + 1] - list_base;
+    region = min(flop[col], region_cap);
   }
   int64_t colcnt = 0;
   int par = 0;
@@ -2462,29 +2756,6 @@ __global__ void k_sum_f32(const float* __restrict__ v, int64_t n, double* __rest
 // ------------------------------------------------------------------ driver
 namespace {
 
-struct DevBuf {
-  void* p = nullptr;
-  size_t bytes = 0;
-  hipStream_t s = nullptr;
-  ~DevBuf() { scratch_free(p, bytes, s); }
-};
-
-// Large per-call arrays whose size repeats from product to product (the unit
-// lists) come from the caching allocator: a stream-pool allocation of several
-// GB has, now and then, taken over a second when the pool had to grow.  The
-// block returns to the cache at scope exit, once the stream's kernels that
-// read it are done (the synchronisation is free on the normal path, which
-// has already synchronised; an early error return waits for them).
-struct CachedBuf {
-  void* p = nullptr;
-  hipStream_t s = nullptr;
-  ~CachedBuf() {
-    if (!p) return;
-    (void)hipStreamSynchronize(s);
-    dev_free(p);
-  }
-};
-
 // Row maps of the symbolic pass (from the caching allocator): returned to
 // the cache once the stream's unit kernels that read them are done.
 struct RowMap {
@@ -2498,28 +2769,19 @@ struct RowMap {
 };
 
 template <class X>
-cbx_status calloc_cached(CachedBuf& b, size_t count, hipStream_t s, X** out) {
-  b.s = s;
-  const cbx_status st = dev_alloc(&b.p, std::max<size_t>(count * sizeof(X), 256));
-  if (st != CBX_OK) {
-    b.p = nullptr;
-    return st;
-  }
-  *out = (X*)b.p;
-  return CBX_OK;
+cbx_status dalloc(ScratchSet& ws, size_t count, X** out) {
+  if (ws.take(out, count)) return CBX_OK;
+  *out = nullptr;
+  return CBX_ERR_NOMEM;
 }
 
-template <class X>
-cbx_status dalloc(DevBuf& b, size_t count, hipStream_t s, X** out) {
-  b.s = s;
-  b.bytes = std::max<size_t>(count * sizeof(X), 256);
-  const cbx_status st = scratch_alloc(&b.p, b.bytes, s);
-  if (st != CBX_OK) {
-    b.p = nullptr;
-    return st;
-  }
-  *out = (X*)b.p;
-  return CBX_OK;
+// Whether `bytes` fit a share of the free memory (the library's idle blocks
+// included).  Up to 64 MB do without asking the driver, which costs more than
+// a small product's kernels.
+bool fits(double bytes, double share) {
+  if (bytes <= 64.0 * (1 << 20) && share > 0.0) return true;
+  size_t freeb = 0, totb = 0;
+  return hipMemGetInfo(&freeb, &totb) == hipSuccess && bytes <= share * (double)(freeb + cache_idle_bytes());
 }
 
 #define CBX_TRY(x)                 \
@@ -2559,37 +2821,36 @@ __global__ void k_gather_flop(const int32_t* __restrict__ cols, int64_t n, const
 // Reorders cols[0..n) by descending flop (into `keep`, returned in *out), so a
 // per-column launch over them starts its longest columns first, as the
 // two-phase path's flop-sorted order does.
-cbx_status sort_cols_by_flop(const int32_t* cols, int64_t n, const int64_t* flop, hipStream_t s, DevBuf& keep,
-                             int32_t** out) {
-  DevBuf b_k, b_k2, b_t;
+cbx_status sort_cols_by_flop(const int32_t* cols, int64_t n, const int64_t* flop, ScratchSet& ws, int32_t** out) {
+  hipStream_t s = ws.s;
   int64_t *k1, *k2;
   uint8_t* t;
-  CBX_TRY(dalloc(b_k, n, s, &k1));
-  CBX_TRY(dalloc(b_k2, n, s, &k2));
-  CBX_TRY(dalloc(keep, n, s, out));
+  CBX_TRY(dalloc(ws, n, &k1));
+  CBX_TRY(dalloc(ws, n, &k2));
+  CBX_TRY(dalloc(ws, n, out));
   size_t tb = 0;
   CBX_HIP(hipcub::DeviceRadixSort::SortPairsDescending(nullptr, tb, k1, k2, cols, *out, (int)n, 0, 64, s));
-  CBX_TRY(dalloc(b_t, std::max<size_t>(tb, 16), s, &t));
+  CBX_TRY(dalloc(ws, std::max<size_t>(tb, 16), &t));
   k_gather_flop<<<nblk(n, 256), 256, 0, s>>>(cols, n, flop, k1);
   CBX_HIP(hipcub::DeviceRadixSort::SortPairsDescending(t, tb, k1, k2, cols, *out, (int)n, 0, 64, s));
   CBX_HIP(hipGetLastError());
   return CBX_OK;
 }
 
-cbx_status sort_units_by_block(const Unit* units, int n, int S, hipStream_t s, DevBuf& keep, Unit** out) {
-  DevBuf b_k, b_k2, b_i, b_i2, b_t;
+cbx_status sort_units_by_block(const Unit* units, int n, int S, ScratchSet& ws, Unit** out) {
+  hipStream_t s = ws.s;
   int32_t *k1, *k2, *i1, *i2;
   uint8_t* t;
-  CBX_TRY(dalloc(b_k, n, s, &k1));
-  CBX_TRY(dalloc(b_k2, n, s, &k2));
-  CBX_TRY(dalloc(b_i, n, s, &i1));
-  CBX_TRY(dalloc(b_i2, n, s, &i2));
-  CBX_TRY(dalloc(keep, n, s, out));
+  CBX_TRY(dalloc(ws, n, &k1));
+  CBX_TRY(dalloc(ws, n, &k2));
+  CBX_TRY(dalloc(ws, n, &i1));
+  CBX_TRY(dalloc(ws, n, &i2));
+  CBX_TRY(dalloc(ws, n, out));
   int bits = 1;
   while ((1 << bits) <= S) ++bits;
   size_t tb = 0;
   CBX_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k1, k2, i1, i2, n, 0, bits, s));
-  CBX_TRY(dalloc(b_t, std::max<size_t>(tb, 16), s, &t));
+  CBX_TRY(dalloc(ws, std::max<size_t>(tb, 16), &t));
   k_unit_keys<<<nblk(n, 256), 256, 0, s>>>(units, n, k1, i1);
   CBX_HIP(hipcub::DeviceRadixSort::SortPairs(t, tb, k1, k2, i1, i2, n, 0, bits, s));
   k_unit_permute<<<nblk(n, 256), 256, 0, s>>>(units, i2, n, *out);
@@ -2597,17 +2858,10 @@ cbx_status sort_units_by_block(const Unit* units, int n, int S, hipStream_t s, D
   return CBX_OK;
 }
 
+// Timings from a call's events (on: the caller asked for statistics).
 struct Timer {
-  hipEvent_t ev[6];
+  hipEvent_t* ev;
   bool on;
-  explicit Timer(bool enable) : on(enable) {
-    if (on)
-      for (auto& e : ev) (void)hipEventCreate(&e);
-  }
-  ~Timer() {
-    if (on)
-      for (auto& e : ev) (void)hipEventDestroy(e);
-  }
   void mark(int i, hipStream_t s) {
     if (on) (void)hipEventRecord(ev[i], s);
   }
@@ -2648,75 +2902,58 @@ template <int K, class T, bool SYM>
 void launch_tiny(const SpgemmConfig& cfg, const int32_t* order, int64_t first, int64_t ncols, const int64_t* cpB,
                  const int32_t* bpos, const T* valB, const int64_t* cpA, const int32_t* rowsA, const T* valA,
                  int64_t* nnzcol, const int64_t* cpC, int64_t* irC, T* valC, int* err, const int64_t* stage_off,
-                 hipStream_t s, const Filter<T>& flt = {}) {
+                 const int64_t* stage_flop, hipStream_t s, const Filter<T>& flt = {}) {
   const dim3 g(tiny_grid(ncols, cfg.tiny_wg_waves)), b(kWave * cfg.tiny_wg_waves);
   k_tiny<K, T, SYM><<<g, b, 0, s>>>(order, first, ncols, cpB, bpos, valB, cpA, rowsA, valA, nnzcol, cpC, irC, valC, err,
-                                    stage_off, flt);
+                                    stage_off, stage_flop, flt);
 }
 
 // Row lists of the small units (k_sym_units); lists == nullptr: none.
 struct UnitLists {
   uint16_t* lists = nullptr;
-  int64_t* off = nullptr;  // per symbolic slot, ncols + 1 entries
+  int64_t* off = nullptr;         // first entry, per symbolic slot
+  const int64_t* flop = nullptr;  // per column; a region holds min(flop, region_cap)
+  int64_t region_cap = 0;
   uint16_t* bcnt = nullptr;
   Unit* units = nullptr;
   int* n = nullptr;
   int cap = 0;
 };
 
-// Region of symbolic slot i in the row lists: the column's outputs in the
-// small-unit passes are at most min(flop_j, unit_split_nnz, m).  Slot i is
-// column order[i] (flop indexed by column), or column i of flop when order
-// is null (flop already in slot order).
+// Region sizes of the symbolic slots order[0..n): a column's outputs in the
+// small-unit passes are at most min(flop_j, unit_split_nnz, m).
 __global__ void k_list_regions(const int32_t* __restrict__ order, const int64_t* __restrict__ flop, int64_t n,
                                int64_t cap, int64_t* __restrict__ sz) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < n) {
-    const int64_t f = flop[order ? order[i] : i];
+    const int64_t f = flop[order[i]];
     sz[i] = f < cap ? f : cap;
   } else if (i == n) {
     sz[i] = 0;
   }
 }
 
-// Region offsets, row lists, block counts and list-unit array for the
-// symbolic slots order[0..n) (order null: slot i is flop[i]), when they fit a
-// fifth of the free memory; otherwise ul.lists stays null.  The buffers are
-// owned by the caller's DevBufs / CachedBuf.
-static cbx_status alloc_unit_lists(const int32_t* order, const int64_t* flop, int64_t n, int S, int64_t cap_units,
-                                   int64_t region_cap, int* counter, void* tmp, size_t tmp_bytes, DevBuf& b_lsz,
-                                   DevBuf& b_loff, DevBuf& b_lists, DevBuf& b_lbc, CachedBuf& b_us, hipStream_t s,
-                                   UnitLists& ul) {
+// Row lists of `rows` entries, block counts and list-unit array for n symbolic
+// slots with region starts `off`, when they fit a fifth of the free memory;
+// otherwise ul.lists stays null.
+static void alloc_unit_lists(int64_t* off, const int64_t* flop, int64_t n, int64_t rows, int S, int64_t cap_units,
+                             int64_t region_cap, int* counter, ScratchSet& ws, UnitLists& ul) {
   ul = UnitLists{};
-  int64_t *lsz, *off;
-  CBX_TRY(dalloc(b_lsz, n + 1, s, &lsz));
-  CBX_TRY(dalloc(b_loff, n + 1, s, &off));
-  k_list_regions<<<nblk(n + 1, 256), 256, 0, s>>>(order, flop, n, region_cap, lsz);
-  size_t need = 0;
-  CBX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, need, lsz, off, (int)(n + 1), s));
-  DevBuf b_t3;
-  void* t3 = tmp;
-  if (need > tmp_bytes) CBX_TRY(dalloc(b_t3, need, s, (uint8_t**)&t3));
-  CBX_HIP(hipcub::DeviceScan::ExclusiveSum(t3, need, lsz, off, (int)(n + 1), s));
-  int64_t total = 0;
-  CBX_HIP(hipMemcpyAsync(&total, off + n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  CBX_HIP(hipStreamSynchronize(s));
-  size_t freeb = 0, totb = 0;
-  const double bytes = 2.0 * (double)total + 2.0 * (double)n * S + (double)sizeof(Unit) * cap_units;
+  const double bytes = 2.0 * (double)rows + 2.0 * (double)n * S + (double)sizeof(Unit) * cap_units;
   uint16_t *lists = nullptr, *bcnt = nullptr;
   Unit* units = nullptr;
-  if (hipMemGetInfo(&freeb, &totb) == hipSuccess && bytes <= 0.2 * (double)(freeb + cache_idle_bytes()) &&
-      dalloc(b_lists, std::max<int64_t>(total, 1), s, &lists) == CBX_OK &&
-      dalloc(b_lbc, n * (int64_t)S, s, &bcnt) == CBX_OK && calloc_cached(b_us, cap_units, s, &units) == CBX_OK) {
+  if (fits(bytes, 0.2) && dalloc(ws, std::max<int64_t>(rows, 1), &lists) == CBX_OK &&
+      dalloc(ws, n * (int64_t)S, &bcnt) == CBX_OK && dalloc(ws, cap_units, &units) == CBX_OK) {
     ul.lists = lists;
     ul.off = off;
+    ul.flop = flop;
+    ul.region_cap = region_cap;
     ul.bcnt = bcnt;
     ul.units = units;
     ul.n = counter;
     ul.cap = (int)cap_units;
   }
   (void)hipGetLastError();
-  return CBX_OK;
 }
 
 // The unit tier's symbolic pass: per column (sym_band 0, optionally with the
@@ -2725,17 +2962,18 @@ static cbx_status alloc_unit_lists(const int32_t* order, const int64_t* flop, in
 cbx_status launch_sym_units(const SpgemmConfig& cfg, const int32_t* order, int64_t ncols, const cbx_dcsc* A,
                             const cbx_dcsc* B, const int32_t* bpos, const int32_t* rowsA, const Tiles& P, int S,
                             int64_t* nnzcol, Unit* units_l, int* n_l, int cap_l, Unit* units_h, int* n_h, int cap_h,
-                            uint32_t* rmap, int64_t rm_cols, int* err, DevBuf& bcnt_buf, int kmax_h, hipStream_t s,
+                            uint32_t* rmap, int64_t rm_cols, int* err, int kmax_h, ScratchSet& ws,
                             const UnitLists& ul = {}) {
+  hipStream_t s = ws.s;
   if (cfg.sym_band == 0) {
     k_sym_units<kSymUnitNT, 4, kSymUnitIBLK><<<(unsigned)ncols, kSymUnitNT, 0, s>>>(
         order, 0, B->cp, bpos, A->cp, rowsA, P, S, kLightK, kLightRB, kmax_h, kHeavyRB, cfg.unit_split_nnz, nnzcol,
-        units_l, n_l, cap_l, units_h, n_h, cap_h, rmap, rm_cols, err, ul.lists, ul.off, ul.bcnt, ul.units, ul.n,
-        ul.cap);
+        units_l, n_l, cap_l, units_h, n_h, cap_h, rmap, rm_cols, err, ul.lists, ul.off, ul.flop,
+        ul.region_cap, ul.bcnt, ul.units, ul.n, ul.cap);
     return CBX_OK;
   }
   int32_t* bcnt;
-  CBX_TRY(dalloc(bcnt_buf, (size_t)ncols * S, s, &bcnt));
+  CBX_TRY(dalloc(ws, (size_t)ncols * S, &bcnt));
   const int band = cfg.sym_band;
   const dim3 g((unsigned)ncols, (unsigned)((S + band - 1) / band));  // band-major dispatch order
   if (band == 16)
@@ -2766,13 +3004,15 @@ struct LearnedInfo {
 template <int K, class T>
 static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const SpgemmConfig& cfg, hipStream_t s,
                                   const int32_t* rowsA, const int32_t* bpos, const int64_t* flop, const Tiles& P,
-                                  int S, int64_t* nnzcol, int64_t* cpC, void* tmp, size_t tmp_bytes, cbx_dcsc* C,
-                                  int* err, LearnedInfo& info) {
+                                  int S, int64_t* nnzcol, int64_t* cpC, cbx_dcsc* C, int* err, hipEvent_t* kev,
+                                  LearnedInfo& info) {
   const int64_t nzcB = B->nzc, m = A->m;
-  DevBuf b_feat, b_lp, b_hist, b_w, b_blo, b_bhi, b_uc, b_ub, b_pn, b_units, b_cnt, b_at, b_upto, b_taken, b_srow, b_sval, b_ct, b_ovf, b_hcs, b_sum,
-      b_hflag, b_hcols, b_nh, b_hu;
-  CachedBuf b_ul, b_uh, b_us;
-  DevBuf b_bcnt, b_lsz, b_loff, b_lists, b_lbc;
+  ScratchSet ws(s);
+  size_t tmp_bytes = 0;  // scans over up to nzcB + 1 columns
+  CBX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, nnzcol, cpC, (int)(nzcB + 1), s));
+  tmp_bytes = std::max<size_t>(tmp_bytes, 16);
+  void* tmp;
+  CBX_TRY(dalloc(ws, tmp_bytes, (uint8_t**)&tmp));
   UnitLists ul;
   uint8_t* heavy_flag;
   int32_t* hcols;
@@ -2786,30 +3026,29 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   int* ovf;
   double* dsum;
   UnitL* units;
-  CBX_TRY(dalloc(b_feat, nzcB * CBX_MLP_FEATURES, s, &feats));
-  CBX_TRY(dalloc(b_lp, nzcB, s, &logpred));
-  CBX_TRY(dalloc(b_hist, S, s, &hist));
-  CBX_TRY(dalloc(b_w, S, s, &w));
-  CBX_TRY(dalloc(b_blo, nzcB, s, &blo));
-  CBX_TRY(dalloc(b_bhi, nzcB, s, &bhi));
-  CBX_TRY(dalloc(b_uc, nzcB + 1, s, &ucount));
-  CBX_TRY(dalloc(b_ub, nzcB + 1, s, &ubase));
-  CBX_TRY(dalloc(b_pn, nzcB, s, &pred_nnz));
-  CBX_TRY(dalloc(b_hcs, nzcB + 1, s, &hcs));
-  CBX_TRY(dalloc(b_sum, 2, s, &dsum));
-  CBX_TRY(dalloc(b_ovf, 2, s, &ovf));
-  CBX_TRY(dalloc(b_ct, nzcB, s, &col_total));
-  CBX_TRY(dalloc(b_hflag, nzcB, s, &heavy_flag));
-  CBX_TRY(dalloc(b_hcols, nzcB, s, &hcols));
-  CBX_TRY(dalloc(b_nh, 1, s, &nh_dev));
-  CBX_TRY(dalloc(b_hu, 3, s, &hucnt));
+  CBX_TRY(dalloc(ws, nzcB * CBX_MLP_FEATURES, &feats));
+  CBX_TRY(dalloc(ws, nzcB, &logpred));
+  CBX_TRY(dalloc(ws, S, &hist));
+  CBX_TRY(dalloc(ws, S, &w));
+  CBX_TRY(dalloc(ws, nzcB, &blo));
+  CBX_TRY(dalloc(ws, nzcB, &bhi));
+  CBX_TRY(dalloc(ws, nzcB + 1, &ucount));
+  CBX_TRY(dalloc(ws, nzcB + 1, &ubase));
+  CBX_TRY(dalloc(ws, nzcB, &pred_nnz));
+  CBX_TRY(dalloc(ws, nzcB + 1, &hcs));
+  CBX_TRY(dalloc(ws, 2, &dsum));
+  CBX_TRY(dalloc(ws, 2, &ovf));
+  CBX_TRY(dalloc(ws, nzcB, &col_total));
+  CBX_TRY(dalloc(ws, nzcB, &heavy_flag));
+  CBX_TRY(dalloc(ws, nzcB, &hcols));
+  CBX_TRY(dalloc(ws, 1, &nh_dev));
+  CBX_TRY(dalloc(ws, 3, &hucnt));
   // prediction: the network on the columns' features, or (without it) the
   // min-hash estimates of estimateNNZ_sampling
   if (cfg.sampling_rounds > 0) {
-    DevBuf b_samp, b_est;
     float *samp, *est;
-    CBX_TRY(dalloc(b_samp, sampling_scratch_floats(A, cfg.sampling_rounds), s, &samp));
-    CBX_TRY(dalloc(b_est, nzcB, s, &est));
+    CBX_TRY(dalloc(ws, sampling_scratch_floats(A, cfg.sampling_rounds), &samp));
+    CBX_TRY(dalloc(ws, nzcB, &est));
     CBX_TRY(sampling_estimate_launch(A, B, cfg.sampling_rounds, rowsA, bpos, samp, est, s));
     k_log2p1<<<nblk(nzcB, 256), 256, 0, s>>>(est, nzcB, logpred);
   } else {
@@ -2844,9 +3083,8 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
     CBX_HIP(hipcub::DeviceSelect::Flagged(nullptr, need2, hipcub::CountingInputIterator<int32_t>(0), heavy_flag,
                                           hcols, nh_dev, (int)nzcB, s));
     need = std::max(need, need2);
-    DevBuf b_tmp2;
     void* t2 = tmp;
-    if (need > tmp_bytes) CBX_TRY(dalloc(b_tmp2, need, s, (uint8_t**)&t2));
+    if (need > tmp_bytes) CBX_TRY(dalloc(ws, need, (uint8_t**)&t2));
     const size_t tb = std::max(need, tmp_bytes);
     size_t tb1 = tb, tb2 = tb;
     CBX_HIP(hipcub::DeviceReduce::Sum(t2, tb1, nnzcol, nh_dev, (int)nzcB, s));
@@ -2865,33 +3103,39 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   RowMap rm;
   rm.s = s;
   int64_t rm_cols = 0;
-  DevBuf b_hsorted;
   if (nheavy > 1) {  // longest columns first
     int32_t* hs = nullptr;
-    CBX_TRY(sort_cols_by_flop(hcols, nheavy, flop, s, b_hsorted, &hs));
+    CBX_TRY(sort_cols_by_flop(hcols, nheavy, flop, ws, &hs));
     hcols = hs;
   }
   if (nheavy) {
     cap_l = std::max<int64_t>(1, std::min<int64_t>(nheavy * (int64_t)S, 1ll << 30));
     cap_h = cap_l;
-    CBX_TRY(calloc_cached(b_ul, cap_l, s, &units_l));
-    CBX_TRY(calloc_cached(b_uh, cap_h, s, &units_h));
+    CBX_TRY(dalloc(ws, cap_l, &units_l));
+    CBX_TRY(dalloc(ws, cap_h, &units_h));
     CBX_HIP(hipMemsetAsync(hucnt, 0, 3 * sizeof(int), s));
     if (cfg.row_map_share > 0.0f) {
       const int64_t rm_words = nheavy * (int64_t)S * kBRW;
-      size_t freeb = 0, totb = 0;
-      if (hipMemGetInfo(&freeb, &totb) == hipSuccess &&
-          4.0 * (double)rm_words <= (double)cfg.row_map_share * (double)(freeb + cache_idle_bytes()) &&
+      if (fits(4.0 * (double)rm_words, cfg.row_map_share) &&
           dev_alloc((void**)&rm.p, sizeof(uint32_t) * rm_words) == CBX_OK)
         rm_cols = nheavy;
       (void)hipGetLastError();
     }
     // the small units' row lists, as in the two-phase path
-    if (cfg.unit_lists && cfg.sym_band == 0)
-      CBX_TRY(alloc_unit_lists(hcols, flop, nheavy, S, cap_l, std::min<int64_t>(cfg.unit_split_nnz, m), hucnt + 2, tmp,
-                               tmp_bytes, b_lsz, b_loff, b_lists, b_lbc, b_us, s, ul));
+    if (cfg.unit_lists && cfg.sym_band == 0) {
+      const int64_t region = std::min<int64_t>(cfg.unit_split_nnz, m);
+      int64_t *lsz, *loff;
+      CBX_TRY(dalloc(ws, nheavy + 1, &lsz));
+      CBX_TRY(dalloc(ws, nheavy + 1, &loff));
+      k_list_regions<<<nblk(nheavy + 1, 256), 256, 0, s>>>(hcols, flop, nheavy, region, lsz);
+      CBX_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, lsz, loff, (int)(nheavy + 1), s));
+      int64_t rows = 0;
+      CBX_HIP(hipMemcpyAsync(&rows, loff + nheavy, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+      CBX_HIP(hipStreamSynchronize(s));
+      alloc_unit_lists(loff, flop, nheavy, rows, S, cap_l, region, hucnt + 2, ws, ul);
+    }
     CBX_TRY(launch_sym_units(cfg, hcols, nheavy, A, B, bpos, rowsA, P, S, nnzcol, units_l, hucnt, (int)cap_l, units_h,
-                             hucnt + 1, (int)cap_h, rm.p, rm_cols, err, b_bcnt, kHeavyK, s, ul));
+                             hucnt + 1, (int)cap_h, rm.p, rm_cols, err, kHeavyK, ws, ul));
     CBX_HIP(hipGetLastError());
   }
   CBX_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, nnzcol, hcs, (int)(nzcB + 1), s));
@@ -2907,7 +3151,7 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   info.pred_sum = pred_sum;
   info.hash_total = hash_only;
   info.exact_total = hash_total - hash_only;
-  CBX_TRY(dalloc(b_units, std::max<int64_t>(nunits, 1), s, &units));
+  CBX_TRY(dalloc(ws, std::max<int64_t>(nunits, 1), &units));
   if (nunits)
     k_learned_units<<<nblk(nzcB, 256), 256, 0, s>>>(flop, nzcB, cfg.small_flop_max, logpred, blo, bhi, w, target,
                                                     heavy_pred, fcap, kLearnRB, direct_flop, m, ubase, nullptr,
@@ -2917,9 +3161,9 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   LearnedStage<T> stage;
   stage.cap = (int64_t)(pred_sum * (1.0 + cfg.capacity_margin)) + (1 << 20);
   int64_t* upto;
-  if (dalloc(b_cnt, nunits + 1, s, &stage.cnt) != CBX_OK || dalloc(b_at, nunits + 1, s, &stage.at) != CBX_OK ||
-      dalloc(b_upto, nunits + 1, s, &upto) != CBX_OK || dalloc(b_taken, 1, s, &stage.taken) != CBX_OK ||
-      dalloc(b_srow, stage.cap, s, &stage.rows) != CBX_OK || dalloc(b_sval, stage.cap, s, &stage.vals) != CBX_OK) {
+  if (dalloc(ws, nunits + 1, &stage.cnt) != CBX_OK || dalloc(ws, nunits + 1, &stage.at) != CBX_OK ||
+      dalloc(ws, nunits + 1, &upto) != CBX_OK || dalloc(ws, 1, &stage.taken) != CBX_OK ||
+      dalloc(ws, stage.cap, &stage.rows) != CBX_OK || dalloc(ws, stage.cap, &stage.vals) != CBX_OK) {
     info.over_capacity = true;
     return CBX_OK;
   }
@@ -2927,8 +3171,6 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   CBX_HIP(hipMemsetAsync(stage.taken, 0, sizeof(unsigned long long), s));
   CBX_HIP(hipMemsetAsync(ovf, 0, sizeof(int) * 2, s));
   CBX_HIP(hipMemsetAsync(col_total, 0, sizeof(unsigned long long) * nzcB, s));
-  hipEvent_t kev[3] = {nullptr, nullptr, nullptr};
-  for (auto& e : kev) (void)hipEventCreate(&e);
   (void)hipEventRecord(kev[0], s);
   // launches of at most 2^21 workgroups (a dispatch holds fewer than 2^32 work-items)
   for (int64_t done = 0; done < nunits; done += kLearnChunk) {
@@ -2949,7 +3191,6 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   (void)hipEventElapsedTime(&info.kernel_ms, kev[0], kev[1]);
   info.over_capacity = (herr & 512) != 0;
   if (herr & ~512 || info.over_capacity) {
-    for (auto& e : kev) (void)hipEventDestroy(e);
     if (herr & ~512) return set_error(CBX_ERR_HIP, "cbx_spgemm: learned pass inconsistency (flag %d)", herr);
     return CBX_OK;
   }
@@ -2966,7 +3207,6 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
     ast = alloc_out();
   }
   if (ast != CBX_OK) {  // the exact path has the staging arrays' room too
-    for (auto& e : kev) (void)hipEventDestroy(e);
     if (ast != CBX_ERR_NOMEM) return ast;
     info.over_capacity = true;
     return CBX_OK;
@@ -2975,9 +3215,8 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   if (nunits) {
     size_t need = 0;
     CBX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, need, stage.cnt, upto, (int)(nunits + 1), s));
-    DevBuf b_t4;
     void* t4 = tmp;
-    if (need > tmp_bytes) CBX_TRY(dalloc(b_t4, need, s, (uint8_t**)&t4));
+    if (need > tmp_bytes) CBX_TRY(dalloc(ws, need, (uint8_t**)&t4));
     need = std::max(need, tmp_bytes);
     CBX_HIP(hipcub::DeviceScan::ExclusiveSum(t4, need, stage.cnt, upto, (int)(nunits + 1), s));
     for (int64_t done = 0; done < nunits; done += kLearnChunk)
@@ -2991,7 +3230,6 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
     float place_ms = 0;
     (void)hipEventElapsedTime(&place_ms, kev[2], kev[1]);
     info.kernel_ms += place_ms;
-    for (auto& e : kev) (void)hipEventDestroy(e);
     return CBX_OK;
   }
   // the heavy columns' values, at the offsets the scan above fixed
@@ -3002,11 +3240,10 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
                     (int64_t)hu[2] * kLightNT >= (1ll << 32),
                 CBX_ERR_LIMIT, "cbx_spgemm: too many units for a single launch");
   info.heavy_units = hu[0] + hu[1] + hu[2];
-  DevBuf b_ul_sorted, b_uh_sorted, b_us_sorted;
   if (cfg.unit_order == 1) {
-    if (hu[0] > 1) CBX_TRY(sort_units_by_block(units_l, hu[0], S, s, b_ul_sorted, &units_l));
-    if (hu[1] > 1) CBX_TRY(sort_units_by_block(units_h, hu[1], S, s, b_uh_sorted, &units_h));
-    if (hu[2] > 1) CBX_TRY(sort_units_by_block(ul.units, hu[2], S, s, b_us_sorted, &ul.units));
+    if (hu[0] > 1) CBX_TRY(sort_units_by_block(units_l, hu[0], S, ws, &units_l));
+    if (hu[1] > 1) CBX_TRY(sort_units_by_block(units_h, hu[1], S, ws, &units_h));
+    if (hu[2] > 1) CBX_TRY(sort_units_by_block(ul.units, hu[2], S, ws, &ul.units));
   }
   if (hu[1] && rm.p)
     k_num_units_rm<K, T, kHeavyNT, 4, kHeavyK, kHeavyDR, kHeavyRB><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
@@ -3031,7 +3268,6 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   float heavy_ms = 0;
   (void)hipEventElapsedTime(&heavy_ms, kev[2], kev[1]);
   info.kernel_ms += heavy_ms;
-  for (auto& e : kev) (void)hipEventDestroy(e);
   if (herr) return set_error(CBX_ERR_HIP, "cbx_spgemm: learned pass, large columns inconsistent (flag %d)", herr);
   return CBX_OK;
 }
@@ -3069,30 +3305,28 @@ __global__ void k_iota32(int32_t* __restrict__ p, int n) {
 
 // The product after a fused threshold: the runs the numeric kernels appended
 // (sorted by start, which is column then row order in the unfiltered layout)
-// gathered into new arrays; nnzcol and cpC become the kept counts and their
-// scan.  C keeps its other fields.
+// gathered into new arrays; nnzcol becomes the kept counts.  C keeps its other fields.
 template <class T>
-static cbx_status filter_compact(const Filter<T>& flt, int64_t nzcB, int64_t* nnzcol, int64_t* cpC, void* tmp,
-                                 size_t tmp_bytes, cbx_dcsc* C, hipStream_t s) {
+static cbx_status filter_compact(const Filter<T>& flt, int64_t nzcB, int64_t* nnzcol, cbx_dcsc* C, ScratchSet& ws) {
+  hipStream_t s = ws.s;
   int nrun = 0;
   CBX_HIP(hipMemcpyAsync(&nrun, flt.run_count, sizeof(int), hipMemcpyDeviceToHost, s));
   CBX_HIP(hipStreamSynchronize(s));
   CBX_RETURN_IF(nrun > flt.run_cap, CBX_ERR_HIP, "cbx_spgemm: run list overflow (%d > %d)", nrun, flt.run_cap);
-  DevBuf b_k2, b_i, b_i2, b_ks, b_dst, b_t;
   int64_t *k2, *ks, *dst;
   int32_t *i1, *i2;
   uint8_t* t;
   const int nr = std::max(nrun, 1);
-  CBX_TRY(dalloc(b_k2, nr, s, &k2));
-  CBX_TRY(dalloc(b_i, nr, s, &i1));
-  CBX_TRY(dalloc(b_i2, nr, s, &i2));
-  CBX_TRY(dalloc(b_ks, nr + 1, s, &ks));
-  CBX_TRY(dalloc(b_dst, nr + 1, s, &dst));
+  CBX_TRY(dalloc(ws, nr, &k2));
+  CBX_TRY(dalloc(ws, nr, &i1));
+  CBX_TRY(dalloc(ws, nr, &i2));
+  CBX_TRY(dalloc(ws, nr + 1, &ks));
+  CBX_TRY(dalloc(ws, nr + 1, &dst));
   size_t tb = 0, tb2 = 0;
   CBX_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, flt.run_src, k2, i1, i2, nr, 0, 64, s));
   CBX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb2, ks, dst, nr + 1, s));
   tb = std::max(tb, tb2);
-  CBX_TRY(dalloc(b_t, std::max<size_t>(tb, 16), s, &t));
+  CBX_TRY(dalloc(ws, std::max<size_t>(tb, 16), &t));
   CBX_HIP(hipMemsetAsync(nnzcol, 0, sizeof(int64_t) * (nzcB + 1), s));
   int64_t total = 0;
   if (nrun) {
@@ -3116,8 +3350,6 @@ static cbx_status filter_compact(const Filter<T>& flt, int64_t nzcB, int64_t* nn
   }
   if (nrun) k_run_copy<T><<<(unsigned)nrun, 256, 0, s>>>(i2, flt.run_src, flt.run_kept, dst, C->ir, (const T*)C->val,
                                                         ir2, (T*)val2);
-  size_t tb4 = tmp_bytes;
-  CBX_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tb4, nnzcol, cpC, (int)(nzcB + 1), s));
   CBX_HIP(hipGetLastError());
   CBX_HIP(hipStreamSynchronize(s));
   dev_free(C->ir);
@@ -3134,8 +3366,6 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
                                     int64_t* symbolic_out, bool* lists_used) {
   const int64_t m = A->m, n = B->n;
   const int64_t nzcA = A->nzc, nzcB = B->nzc, nnzA = A->nnz, nnzB = B->nnz;
-  Timer tm(stats != nullptr);
-  tm.mark(0, s);
 
   std::memset(C, 0, sizeof(*C));
   C->m = m;
@@ -3156,119 +3386,101 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
     return CBX_OK;
   }
 
+  // Three waits for the device per product: after the setup (the tiers' sizes),
+  // after the symbolic pass (the output's), at the end.  Kernels report into
+  // the slot's pinned page; counters are cleared together, and all scratch is
+  // taken from one set and returned after the last wait.
+  SlotHold slot;
+  CBX_RETURN_IF(!slot.p, CBX_ERR_NOMEM, "cbx_spgemm: no pinned host memory");
+  volatile Report* rep = (volatile Report*)slot.p->host;
+  Report* rep_dev = (Report*)slot.p->host;
+  ScratchSet ws(s);
+  Timer tm{slot.p->ev, stats != nullptr};
+  tm.mark(0, s);
+
   // Unit tier needs the tile-pointer table at kBR-row granularity; it is used
   // when that table stays modest, otherwise the streaming dense tier runs.
   const int S4 = (int)((m + kBR - 1) / kBR);
   const bool use_units = m <= (1ll << 24) && (double)nzcA * (S4 + 1) * 4.0 <= 8.0e9;
-  // the fused threshold (two-phase, unit or hash tiers; the streaming tier has no filtered emission)
-  Filter<T> flt;
-  flt.on = cfg.filter && mode == CBX_SPGEMM_TWO_PHASE && use_units && symbolic_out == nullptr;
-  flt.thr = (T)cfg.filter_thr;
-  DevBuf b_drop;
-  if (flt.on) {
-    CBX_TRY(dalloc(b_drop, 1, s, &flt.dropped));
-    CBX_HIP(hipMemsetAsync(flt.dropped, 0, sizeof(unsigned long long), s));
-  }
   const int TR = kDenseTR;
   const int S16 = (int)((m + TR - 1) / TR);
   const int S = use_units ? S4 : S16;
   const int G = kSymRBW * 32 / TR;  // tiles per symbolic pass of the streaming tier
 
-  DevBuf b_colmap, b_rows, b_bpos, b_flop, b_order, b_flop_s, b_order_s, b_P, b_nnz, b_cp, b_tmp, b_thr, b_bounds,
-      b_flags, b_nsel, b_err, b_vcnt, b_ucnt, b_soff, b_sir, b_sval, b_bcnt;
-  CachedBuf b_ul, b_uh, b_us;
-  int32_t *colmap, *rowsA, *bpos, *order, *order_s, *P;
-  int *err, *ucnt;
-  unsigned long long* vcnt;
-  int64_t *stage_off = nullptr, *stage_ir = nullptr;  // staged tiny tier (see the symbolic pass)
+  int32_t *colmap = nullptr, *rowsA, *bpos, *order_s, *P = nullptr;
+  Counters* ctr;
+  int64_t *stage_off, *stage_ir = nullptr;  // staged tiny tier (see the symbolic pass)
   T* stage_val = nullptr;
   bool tiny_staged = false;
-  int64_t *flop, *flop_s, *nnzcol, *cpC, *thr, *bounds, *nsel;
-  uint8_t* flags;
-  Unit *units_l = nullptr, *units_h = nullptr;
-  UnitLists ul;
-  DevBuf b_lsz, b_loff, b_lists, b_lbc;
-  CBX_TRY(dalloc(b_colmap, A->n, s, &colmap));
-  CBX_TRY(dalloc(b_rows, nnzA, s, &rowsA));
-  CBX_TRY(dalloc(b_bpos, nnzB, s, &bpos));
-  CBX_TRY(dalloc(b_flop, nzcB, s, &flop));
-  CBX_TRY(dalloc(b_flop_s, nzcB, s, &flop_s));
-  CBX_TRY(dalloc(b_order, nzcB, s, &order));
-  CBX_TRY(dalloc(b_order_s, nzcB, s, &order_s));
-  CBX_TRY(dalloc(b_nnz, nzcB + 1, s, &nnzcol));
-  CBX_TRY(dalloc(b_cp, nzcB + 1, s, &cpC));
-  CBX_TRY(dalloc(b_thr, 8, s, &thr));
-  CBX_TRY(dalloc(b_bounds, 8, s, &bounds));
-  CBX_TRY(dalloc(b_flags, nzcB, s, &flags));
-  CBX_TRY(dalloc(b_nsel, 2, s, &nsel));
-  CBX_TRY(dalloc(b_err, 1, s, &err));
-  CBX_TRY(dalloc(b_vcnt, 6, s, &vcnt));
-  CBX_TRY(dalloc(b_ucnt, 3, s, &ucnt));
-  CBX_HIP(hipMemsetAsync(err, 0, sizeof(int), s));
-  CBX_HIP(hipMemsetAsync(ucnt, 0, 3 * sizeof(int), s));
+  int64_t *flop, *flop_s, *nnzcol, *cpC, *list_off;
+  ColSum* sums;
+  const int64_t ctiles = (nzcB + kColTile - 1) / kColTile;
+  CBX_TRY(dalloc(ws, 1, &ctr));
+  if (nzcA != A->n) CBX_TRY(dalloc(ws, A->n, &colmap));
+  CBX_TRY(dalloc(ws, nnzA, &rowsA));
+  CBX_TRY(dalloc(ws, nnzB, &bpos));
+  CBX_TRY(dalloc(ws, nzcB + 1, &flop));
+  CBX_TRY(dalloc(ws, nzcB, &flop_s));
+  CBX_TRY(dalloc(ws, nzcB, &order_s));
+  CBX_TRY(dalloc(ws, nzcB + 1, &nnzcol));
+  CBX_TRY(dalloc(ws, nzcB + 1, &cpC));
+  CBX_TRY(dalloc(ws, nzcB, &stage_off));
+  CBX_TRY(dalloc(ws, nzcB, &list_off));
+  CBX_TRY(dalloc(ws, ctiles, &sums));
+  int* err = &ctr->err;
+  int* ucnt = ctr->units;
 
   const T* valA = (const T*)A->val;
   const T* valB = (const T*)B->val;
+  // the fused threshold (two-phase, unit or sort tiers; the streaming tier has no filtered emission)
+  Filter<T> flt;
+  flt.on = cfg.filter && mode == CBX_SPGEMM_TWO_PHASE && use_units && symbolic_out == nullptr;
+  flt.thr = (T)cfg.filter_thr;
+  flt.dropped = &ctr->dropped;
+  flt.run_count = &ctr->runs;
 
-  // --- validate both operands before any indexed access
-  if (!cfg.trusted_a) CBX_TRY(launch_validate(A, 4, vcnt, err, s));
-  if (!cfg.trusted_b) CBX_TRY(launch_validate(B, 5, vcnt + 3, err, s));
-  {
-    int herr = 0;
-    CBX_HIP(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, s));
-    CBX_HIP(hipStreamSynchronize(s));
-    if (herr)
-      return set_error(CBX_ERR_INVALID,
-                       "cbx_spgemm: %s is not a valid DCSC (cp/jc/ir out of range, or rows not strictly "
-                       "increasing within a column)", (herr & 16) ? "A" : "B");
-  }
-
-  // --- setup: column map, 32-bit rows, B->A positions, flops, tile pointers
-  k_fill_i32<<<nblk(A->n, 256), 256, 0, s>>>(colmap, A->n, -1);
-  k_colmap<<<nblk(nzcA, 256), 256, 0, s>>>(A->jc, nzcA, colmap);
-  k_rows32<<<nblk(nnzA, 256), 256, 0, s>>>(A->ir, nnzA, rowsA);
-  k_bpos<<<nblk(nnzB, 256), 256, 0, s>>>(B->ir, nnzB, colmap, bpos);
-  k_flop<<<wave_grid(nzcB), 256, 0, s>>>(B->cp, nzcB, bpos, A->cp, flop);
-  k_iota_i32<<<nblk(nzcB, 256), 256, 0, s>>>(order, nzcB);
-
-  // sort columns by flop, descending (largest work first)
-  size_t tmp_bytes = 0, tmp2 = 0;
-  CBX_HIP(hipcub::DeviceRadixSort::SortPairsDescending(nullptr, tmp_bytes, flop, flop_s, order, order_s, (int)nzcB, 0,
-                                                       64, s));
-  CBX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp2, nnzcol, cpC, (int)(nzcB + 1), s));
-  tmp_bytes = std::max(tmp_bytes, tmp2);
-  CBX_HIP(hipcub::DeviceSelect::Flagged(nullptr, tmp2, B->jc, flags, (int64_t*)nullptr, nsel, (int)nzcB, s));
-  tmp_bytes = std::max(tmp_bytes, tmp2);
-  CBX_HIP(hipcub::DeviceReduce::Sum(nullptr, tmp2, flop, bounds + 6, (int)nzcB, s));
-  tmp_bytes = std::max(tmp_bytes, tmp2);
-  void* tmp;
-  CBX_TRY(dalloc(b_tmp, tmp_bytes, s, (uint8_t**)&tmp));
-  CBX_HIP(hipcub::DeviceRadixSort::SortPairsDescending(tmp, tmp_bytes, flop, flop_s, order, order_s, (int)nzcB, 0, 64,
-                                                       s));
-  CBX_HIP(hipcub::DeviceReduce::Sum(tmp, tmp_bytes, flop, bounds + 6, (int)nzcB, s));
-
-  // class thresholds: units > small_max ; hash8k > mid ; hash2k > tiny ; tiny (one wave) > 0 ;
-  // large units possible > unit_split_nnz ; 1024-thread sort > 2048
-  int64_t hthr[6] = {cfg.small_flop_max, cfg.hash_mid_flop, cfg.tiny_flop, 0, cfg.unit_split_nnz, 2048};
-  CBX_HIP(hipMemcpyAsync(thr, hthr, sizeof(hthr), hipMemcpyHostToDevice, s));
-  k_class_bounds<<<1, 64, 0, s>>>(flop_s, nzcB, thr, 6, bounds);
-  int64_t hb[7];
-  CBX_HIP(hipMemcpyAsync(hb, bounds, sizeof(hb), hipMemcpyDeviceToHost, s));
-  CBX_HIP(hipMemsetAsync(nnzcol, 0, sizeof(int64_t) * (nzcB + 1), s));
+  // --- setup: both operands validated before any indexed access (kernels that
+  // index through them do nothing where the counts say they are malformed),
+  // column map, 32-bit rows, B->A positions, products and order of the columns
+  k_init<<<(unsigned)std::min<int64_t>(1024, nblk(std::max<int64_t>({colmap ? A->n : 1, nzcB + 1, 1024}), 256)), 256, 0,
+           s>>>(ctr, colmap, A->n, flop, nnzcol, nzcB);
+  if (cfg.trusted_a) k_rows32<<<nblk(nnzA, 256), 256, 0, s>>>(A->ir, nnzA, rowsA);
+  else CBX_TRY(launch_validate(A, rowsA, ctr->val, s));
+  const bool same = A->cp == B->cp && A->jc == B->jc && A->ir == B->ir && nzcA == nzcB && nnzA == nnzB &&
+                    A->m == B->m && A->n == B->n;  // A*A: one look will do
+  if (!cfg.trusted_b && !(same && !cfg.trusted_a)) CBX_TRY(launch_validate(B, nullptr, ctr->val + 3, s));
+  if (colmap) k_colmap<<<nblk(nzcA, 256), 256, 0, s>>>(A->jc, nzcA, ctr, colmap);
+  k_flops<<<nblk(nnzB, kFlopTile), kFlopNT, 0, s>>>(B->cp, B->ir, nzcB, nnzB, colmap, A->cp, ctr, bpos, flop);
+  FlopClasses cls;
+  cls.split = cfg.unit_split_nnz;
+  cls.small = cfg.small_flop_max;
+  cls.s4k = 2048;
+  cls.mid = cfg.hash_mid_flop;
+  cls.tiny = cfg.tiny_flop;
+  cls.list_cap = std::min<int64_t>(cfg.unit_split_nnz, m);
+  k_count_digits<<<(unsigned)ctiles, 256, 0, s>>>(flop, nzcB, cls, ctr);
+  k_order_columns<<<(unsigned)ctiles, 256, 0, s>>>(flop, nzcB, cls, ctr, order_s, flop_s, stage_off, list_off, rep_dev);
+  CBX_HIP(hipGetLastError());
   CBX_HIP(hipStreamSynchronize(s));
-  const int64_t n_dense = hb[0], n_h8 = hb[1] - hb[0], n_h2 = hb[2] - hb[1], n_h256 = hb[3] - hb[2];
-  const int64_t n_heavy_max = hb[4];  // columns whose flops (an upper bound of nnz) exceed unit_split_nnz
-  const int64_t total_flop = hb[6];
-  const int64_t n_s4k = std::min(n_h8, std::max<int64_t>(hb[5] - hb[0], 0));  // of n_h8, those above 2048 products
-  // one workgroup per column (hash tiers, symbolic units): a dispatch holds
+  if (rep->err)
+    return set_error(CBX_ERR_INVALID,
+                     "cbx_spgemm: %s is not a valid DCSC (cp/jc/ir out of range, or rows not strictly "
+                     "increasing within a column)", (rep->err & 16) ? "A" : "B");
+  // tiers in the order of order_s: units, sort tier (1024, 512, 256 threads), tiny (one wave)
+  const int64_t n_heavy_max = rep->columns[0];  // columns whose flops (an upper bound of nnz) exceed unit_split_nnz
+  const int64_t n_dense = n_heavy_max + rep->columns[1];
+  const int64_t n_s4k = rep->columns[2], n_h8 = n_s4k + rep->columns[3], n_h2 = rep->columns[4];
+  const int64_t n_h256 = rep->columns[5];
+  const int64_t hb[3] = {n_dense, n_dense + n_h8, n_dense + n_h8 + n_h2};  // tier ends
+  const int64_t total_flop = rep->flops, tiny_slots = rep->tiny_flops, list_rows = rep->list_rows;
+  // one workgroup per column (sort tier, symbolic units): a dispatch holds
   // fewer than 2^32 work-items
   CBX_RETURN_IF(n_dense * 1024 >= (1ll << 32) || n_h8 * 1024 >= (1ll << 32) || n_h2 * kHashNT >= (1ll << 32),
                 CBX_ERR_LIMIT, "cbx_spgemm: too many columns in one tier for a single launch");
-  // tile pointers only when some column is beyond the hash tier (the table is
+  // tile pointers only when some column is beyond the sort tier (the table is
   // nzc(A) x m/4096 entries, large for tall packed batches of small columns)
-  P = nullptr;
   if (n_dense) {
-    CBX_TRY(dalloc(b_P, (size_t)nzcA * (S + 1), s, &P));
+    CBX_TRY(dalloc(ws, (size_t)nzcA * (S + 1), &P));
     if (use_units)
       k_tiles<<<dim3(nblk(nzcA, 256), nblk(S + 1, kTileRun)), 256, 0, s>>>(A->cp, nzcA, rowsA, S, P);
     else
@@ -3277,23 +3489,47 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   const Tiles tiles{P, nzcA};
   tm.mark(1, s);
 
-  // --- learned single pass (unit-tier columns), with the exact hash-tier
+  // sizes of the output's columns to offsets and its DCSC columns, and the report
+  auto finish_columns = [&]() -> cbx_status {
+    k_col_sums<<<(unsigned)ctiles, 256, 0, s>>>(nnzcol, nzcB, n_dense ? flop : nullptr, cfg.small_flop_max, sums, ctr);
+    const int scanned = ctiles > 1024;
+    if (scanned) k_scan_sums<<<1, 1024, 0, s>>>(sums, ctiles);
+    k_col_offsets<<<(unsigned)ctiles, 256, 0, s>>>(nnzcol, nzcB, sums, scanned, B->jc, ctr, cpC, C->cp, C->jc, rep_dev);
+    CBX_HIP(hipGetLastError());
+    return CBX_OK;
+  };
+  auto alloc_columns = [&]() -> cbx_status {
+    CBX_TRY(dev_alloc((void**)&C->cp, sizeof(int64_t) * (nzcB + 1)));
+    CBX_TRY(dev_alloc((void**)&C->jc, sizeof(int64_t) * std::max<int64_t>(nzcB, 1)));
+    return CBX_OK;
+  };
+
+  auto launch_sym_small = [&]() {
+    if (n_h8)
+      k_sym_hash<8192, kHashNT><<<(unsigned)n_h8, kHashNT, 0, s>>>(order_s, hb[0], flop, B->cp, bpos, A->cp, rowsA,
+                                                                 nnzcol, err);
+    if (n_h2)
+      k_sym_hash<2048, kHashNT><<<(unsigned)n_h2, kHashNT, 0, s>>>(order_s, hb[1], flop, B->cp, bpos, A->cp, rowsA,
+                                                                 nnzcol, err);
+  };
+
+  // --- learned single pass (unit-tier columns), with the exact sort-tier
   //     symbolic for the small columns
   bool learned = mode == CBX_SPGEMM_LEARNED && use_units && n_dense > 0 &&
                  (cfg.predictor != nullptr || cfg.sampling_rounds > 0);
   bool learned_done = false;
   LearnedInfo linfo;
-  int64_t nnzC = 0, nnz_main = 0;
-  int hu[3] = {0, 0, 0}, herr = 0;  // small (bitmap), large, and small list units
+  int64_t nnzC = 0, nnz_main = 0, nzcC = 0;
+  int hu[3] = {0, 0, 0};  // small (bitmap), large, and small list units
   if (learned) {
-    if (n_h8) k_sym_hash<8192, kHashNT><<<(unsigned)n_h8, kHashNT, 0, s>>>(order_s, hb[0], flop, B->cp, bpos, A->cp, rowsA, nnzcol, err);
-    if (n_h2) k_sym_hash<2048, kHashNT><<<(unsigned)n_h2, kHashNT, 0, s>>>(order_s, hb[1], flop, B->cp, bpos, A->cp, rowsA, nnzcol, err);
+    launch_sym_small();
     if (n_h256)
       launch_tiny<K, T, true>(cfg, order_s, hb[2], n_h256, B->cp, bpos, valB, A->cp, rowsA, valA, nnzcol, nullptr,
-                              nullptr, nullptr, err, nullptr, s);
+                              nullptr, nullptr, err, nullptr, nullptr, s);
     tm.mark(2, s);
     tm.mark(3, s);
-    CBX_TRY((learned_numeric<K, T>(A, B, cfg, s, rowsA, bpos, flop, tiles, S, nnzcol, cpC, tmp, tmp_bytes, C, err, linfo)));
+    CBX_TRY((learned_numeric<K, T>(A, B, cfg, s, rowsA, bpos, flop, tiles, S, nnzcol, cpC, C, err, slot.p->ev + 6,
+                                   linfo)));
     if (linfo.over_capacity) {  // predictions too small overall: redo exactly
       dev_free(C->ir);
       dev_free(C->val);
@@ -3306,15 +3542,16 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
       nnzC = linfo.nnzC;
       nnz_main = linfo.nnzC - linfo.hash_total;
       C->nnz = nnzC;
-      CBX_TRY(dev_alloc((void**)&C->cp, sizeof(int64_t) * (nzcB + 1)));
-      CBX_TRY(dev_alloc((void**)&C->jc, sizeof(int64_t) * std::max<int64_t>(nzcB, 1)));
+      CBX_TRY(alloc_columns());
+      CBX_TRY(finish_columns());
       tm.mark(4, s);
     }
   }
   int64_t nnz_unfiltered = 0;
-  DevBuf b_rsrc, b_rkept, b_rcol, b_rcnt;  // the fused threshold's run list
   if (!learned_done) {
   // --- symbolic
+  Unit *units_l = nullptr, *units_h = nullptr;
+  UnitLists ul;
   int64_t cap_l = 0, cap_h = 0;
   // row maps (presence bitmaps, 512 B per 4096 rows) of the columns that can
   // form large units (flop above unit_split_nnz; they lead the flop order),
@@ -3328,9 +3565,7 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   const int64_t rm_cols = std::min<int64_t>(n_heavy_max, n_dense);
   if (use_units && rm_cols > 0 && cfg.row_map_share > 0.0f) {
     const int64_t rm_words = rm_cols * (int64_t)S * kBRW;
-    size_t freeb = 0, totb = 0;
-    if (hipMemGetInfo(&freeb, &totb) == hipSuccess &&
-        4.0 * (double)rm_words <= (double)cfg.row_map_share * (double)(freeb + cache_idle_bytes()) &&
+    if (fits(4.0 * (double)rm_words, cfg.row_map_share) &&
         dev_alloc((void**)&rmap, sizeof(uint32_t) * rm_words) != CBX_OK)
       rmap = nullptr;
     (void)hipGetLastError();
@@ -3338,86 +3573,71 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   if (use_units && n_dense) {
     cap_l = std::max<int64_t>(1, std::min<int64_t>(n_dense * (int64_t)S, 1ll << 30));
     cap_h = std::max<int64_t>(1, std::min<int64_t>(n_heavy_max * (int64_t)S, 1ll << 30));
-    CBX_TRY(calloc_cached(b_ul, cap_l, s, &units_l));
-    CBX_TRY(calloc_cached(b_uh, cap_h, s, &units_h));
+    CBX_TRY(dalloc(ws, cap_l, &units_l));
+    CBX_TRY(dalloc(ws, cap_h, &units_h));
     // the small units' row lists (per-column symbolic form only): one region
     // of min(flop_j, unit_split_nnz, m) 2-byte entries per column, plus the
     // per-block counts, when they fit a fifth of the free memory
     if (cfg.unit_lists && cfg.sym_band == 0 && symbolic_out == nullptr) {
-      CBX_TRY(alloc_unit_lists(nullptr, flop_s, n_dense, S, cap_l, std::min<int64_t>(cfg.unit_split_nnz, m), ucnt + 2,
-                               tmp, tmp_bytes, b_lsz, b_loff, b_lists, b_lbc, b_us, s, ul));
+      alloc_unit_lists(list_off, flop, n_dense, list_rows, S, cap_l, cls.list_cap, ucnt + 2, ws, ul);
       if (ul.lists && lists_used) *lists_used = true;
     }
-    CBX_TRY(launch_sym_units(cfg, order_s, n_dense, A, B, bpos, rowsA, tiles, S, nnzcol, units_l, ucnt, (int)cap_l, units_h,
-                             ucnt + 1, (int)cap_h, rmap, rm_cols, err, b_bcnt, kHeavyK, s, ul));
+    CBX_TRY(launch_sym_units(cfg, order_s, n_dense, A, B, bpos, rowsA, tiles, S, nnzcol, units_l, ucnt, (int)cap_l,
+                             units_h, ucnt + 1, (int)cap_h, rmap, rm_cols, err, kHeavyK, ws, ul));
   } else if (n_dense) {
     k_sym_dense<kSymNT, kSymRBW><<<(unsigned)n_dense, kSymNT, 0, s>>>(order_s, 0, B->cp, bpos, A->cp, rowsA, P, S, G,
                                                                        TR, nnzcol);
   }
-  if (n_h8) k_sym_hash<8192, kHashNT><<<(unsigned)n_h8, kHashNT, 0, s>>>(order_s, hb[0], flop, B->cp, bpos, A->cp, rowsA, nnzcol, err);
-  if (n_h2) k_sym_hash<2048, kHashNT><<<(unsigned)n_h2, kHashNT, 0, s>>>(order_s, hb[1], flop, B->cp, bpos, A->cp, rowsA, nnzcol, err);
+  launch_sym_small();
   // tiny tier: its numeric kernel runs now into a staging buffer (a slot of
   // flop_j entries per column) and records the exact counts; after the
   // output scan the entries are copied into place.  One gather and sort per
   // column instead of two (symbolic + numeric), when the slots fit a
   // quarter of the free memory.
   if (n_h256) {
-    CBX_TRY(dalloc(b_soff, n_h256 + 1, s, &stage_off));
-    CBX_HIP(hipMemsetAsync(stage_off, 0, sizeof(int64_t), s));
-    CBX_HIP(hipcub::DeviceScan::InclusiveSum(tmp, tmp_bytes, flop_s + hb[2], stage_off + 1, (int)n_h256, s));
-    int64_t slots = 0;
-    CBX_HIP(hipMemcpyAsync(&slots, stage_off + n_h256, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    CBX_HIP(hipStreamSynchronize(s));
-    size_t freeb = 0, totb = 0;
     // a symbolic-only call (symbolic_out) stages nothing: it counts rows
     // without reading values, so it runs for operands of any value type
-    if (symbolic_out == nullptr && hipMemGetInfo(&freeb, &totb) == hipSuccess &&
-        (double)slots * (sizeof(int64_t) + sizeof(T)) <= 0.25 * (double)(freeb + cache_idle_bytes()) &&
-        dalloc(b_sir, std::max<int64_t>(slots, 1), s, &stage_ir) == CBX_OK &&
-        dalloc(b_sval, std::max<int64_t>(slots, 1), s, &stage_val) == CBX_OK)
+    if (symbolic_out == nullptr && fits((double)tiny_slots * (sizeof(int64_t) + sizeof(T)), 0.25) &&
+        dalloc(ws, std::max<int64_t>(tiny_slots, 1), &stage_ir) == CBX_OK &&
+        dalloc(ws, std::max<int64_t>(tiny_slots, 1), &stage_val) == CBX_OK)
       tiny_staged = true;
     (void)hipGetLastError();
     if (tiny_staged)
       launch_tiny<K, T, false>(cfg, order_s, hb[2], n_h256, B->cp, bpos, valB, A->cp, rowsA, valA, nnzcol, nullptr,
-                               stage_ir, stage_val, err, stage_off, s, flt);
+                               stage_ir, stage_val, err, stage_off, flop_s, s, flt);
     else
-      launch_tiny<K, T, true>(cfg, order_s, hb[2], n_h256, B->cp, bpos, valB, A->cp, rowsA, valA, nnzcol, nullptr, nullptr, nullptr, err, nullptr, s);
+      launch_tiny<K, T, true>(cfg, order_s, hb[2], n_h256, B->cp, bpos, valB, A->cp, rowsA, valA, nnzcol, nullptr,
+                              nullptr, nullptr, err, nullptr, nullptr, s);
   }
-  CBX_HIP(hipGetLastError());
-  CBX_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, nnzcol, cpC, (int)(nzcB + 1), s));
-  if (n_dense) {
-    CBX_HIP(hipMemsetAsync(bounds + 7, 0, sizeof(int64_t), s));
-    k_sum_ordered<<<nblk(n_dense, 256), 256, 0, s>>>(order_s, n_dense, nnzcol, (unsigned long long*)(bounds + 7));
-    CBX_HIP(hipMemcpyAsync(&nnz_main, bounds + 7, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  }
-  CBX_HIP(hipMemcpyAsync(&nnzC, cpC + nzcB, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  CBX_HIP(hipMemcpyAsync(hu, ucnt, sizeof(hu), hipMemcpyDeviceToHost, s));
-  CBX_HIP(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, s));
+  if (!symbolic_out) CBX_TRY(alloc_columns());
+  CBX_TRY(finish_columns());
   tm.mark(2, s);
   if (symbolic_out) CBX_HIP(hipMemcpyAsync(symbolic_out, nnzcol, sizeof(int64_t) * nzcB, hipMemcpyDeviceToDevice, s));
   CBX_HIP(hipStreamSynchronize(s));
-  if (herr) return set_error(CBX_ERR_HIP, "cbx_spgemm: symbolic pass failed (flag %d)", herr);
+  if (rep->err) {
+    const int e = rep->err;
+    cbx_dcsc_free(C);
+    return set_error(CBX_ERR_HIP, "cbx_spgemm: symbolic pass failed (flag %d)", e);
+  }
   if (symbolic_out) return CBX_OK;
+  nnzC = rep->nnz;
+  nzcC = rep->nzc;
+  nnz_main = rep->main_nnz;
+  for (int i = 0; i < 3; ++i) hu[i] = rep->units[i];
   nnz_unfiltered = nnzC;
   if (flt.on) {
-    unsigned long long dropped = 0;
-    CBX_HIP(hipMemcpy(&dropped, flt.dropped, sizeof(dropped), hipMemcpyDeviceToHost));
-    nnz_unfiltered += (int64_t)dropped;
-    // one run per unit and per hash- or tiny-tier column at most
+    nnz_unfiltered += rep->dropped;
+    // one run per unit and per sort- or tiny-tier column at most
     const int64_t cap = (int64_t)hu[0] + hu[1] + hu[2] + nzcB + 16;
     CBX_RETURN_IF(cap >= (1ll << 31), CBX_ERR_LIMIT, "cbx_spgemm: too many output ranges for the fused threshold");
-    CBX_TRY(dalloc(b_rsrc, cap, s, &flt.run_src));
-    CBX_TRY(dalloc(b_rkept, cap, s, &flt.run_kept));
-    CBX_TRY(dalloc(b_rcol, cap, s, &flt.run_col));
-    CBX_TRY(dalloc(b_rcnt, 1, s, &flt.run_count));
-    CBX_HIP(hipMemsetAsync(flt.run_count, 0, sizeof(int), s));
+    CBX_TRY(dalloc(ws, cap, &flt.run_src));
+    CBX_TRY(dalloc(ws, cap, &flt.run_kept));
+    CBX_TRY(dalloc(ws, cap, &flt.run_col));
     flt.run_cap = (int)cap;
   }
 
   // --- output allocation (cached: repeated products reuse the arrays)
   auto alloc_out = [&]() -> cbx_status {
-    if (!C->cp) CBX_TRY(dev_alloc((void**)&C->cp, sizeof(int64_t) * (nzcB + 1)));
-    if (!C->jc) CBX_TRY(dev_alloc((void**)&C->jc, sizeof(int64_t) * std::max<int64_t>(nzcB, 1)));
     if (!C->ir) CBX_TRY(dev_alloc((void**)&C->ir, sizeof(int64_t) * std::max<int64_t>(nnzC, 1)));
     if (!C->val) CBX_TRY(dev_alloc(&C->val, sizeof(T) * std::max<int64_t>(nnzC, 1)));
     return CBX_OK;
@@ -3438,11 +3658,10 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   CBX_RETURN_IF((int64_t)hu[0] * kLightNT >= (1ll << 32) || (int64_t)hu[1] * kHeavyNT >= (1ll << 32) ||
                     (int64_t)hu[2] * kLightNT >= (1ll << 32),
                 CBX_ERR_LIMIT, "cbx_spgemm: too many units for a single launch");
-  DevBuf b_ul_sorted, b_uh_sorted, b_us_sorted;
   if (use_units && cfg.unit_order == 1) {
-    if (hu[0] > 1) CBX_TRY(sort_units_by_block(units_l, hu[0], S, s, b_ul_sorted, &units_l));
-    if (hu[1] > 1) CBX_TRY(sort_units_by_block(units_h, hu[1], S, s, b_uh_sorted, &units_h));
-    if (hu[2] > 1) CBX_TRY(sort_units_by_block(ul.units, hu[2], S, s, b_us_sorted, &ul.units));
+    if (hu[0] > 1) CBX_TRY(sort_units_by_block(units_l, hu[0], S, ws, &units_l));
+    if (hu[1] > 1) CBX_TRY(sort_units_by_block(units_h, hu[1], S, ws, &units_h));
+    if (hu[2] > 1) CBX_TRY(sort_units_by_block(ul.units, hu[2], S, ws, &ul.units));
   }
   if (use_units) {
     // large units: one sweep over the row map when it was kept (their
@@ -3455,10 +3674,12 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
           cfg.unit_xcd_group);
     else if (hu[1])
       k_num_units<K, T, kHeavyNT, 4, kHeavyK, kHeavyDR, kHeavyRB, 4><<<(unsigned)hu[1], kHeavyNT, 0, s>>>(
-          units_h, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, cpC, C->ir, (T*)C->val, err, flt, cfg.unit_xcd_group);
+          units_h, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, cpC, C->ir, (T*)C->val, err, flt,
+          cfg.unit_xcd_group);
     if (hu[0])
       k_num_units<K, T, kLightNT, 4, kLightK, kLightDR, kLightRB, 2><<<(unsigned)hu[0], kLightNT, 0, s>>>(
-          units_l, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, cpC, C->ir, (T*)C->val, err, flt, cfg.unit_xcd_group);
+          units_l, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, cpC, C->ir, (T*)C->val, err, flt,
+          cfg.unit_xcd_group);
     if (hu[2])
       k_num_list<K, T, kLightNT, 4, kLightK><<<(unsigned)hu[2], kLightNT, 0, s>>>(
           ul.units, ul.lists, ul.off, ul.bcnt, B->cp, bpos, valB, A->cp, rowsA, valA, tiles, S, cpC, C->ir, (T*)C->val,
@@ -3469,7 +3690,7 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   }
   tm.mark(4, s);
   }  // !learned_done
-  // hash-tier columns by the products that a workgroup holds (four per thread)
+  // sort-tier columns by the products that a workgroup holds (four per thread)
   if (n_s4k)
     k_num_sort<K, T, 1024><<<(unsigned)n_s4k, 1024, 0, s>>>(order_s, hb[0], nnzcol, B->cp, bpos, valB, A->cp, rowsA,
                                                             valA, cpC, C->ir, (T*)C->val, err, flt);
@@ -3485,30 +3706,26 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
                                                        stage_val, C->ir, (T*)C->val, flt, err);
   else if (n_h256)
     launch_tiny<K, T, false>(cfg, order_s, hb[2], n_h256, B->cp, bpos, valB, A->cp, rowsA, valA, nnzcol, cpC, C->ir,
-                             (T*)C->val, err, nullptr, s, flt);
+                             (T*)C->val, err, nullptr, nullptr, s, flt);
   CBX_HIP(hipGetLastError());
 
   if (flt.on) {  // the fused threshold's runs into the final arrays
-    CBX_HIP(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, s));
+    k_report_err<<<1, 64, 0, s>>>(err, rep_dev);
     CBX_HIP(hipStreamSynchronize(s));
-    if (herr) return set_error(CBX_ERR_HIP, "cbx_spgemm: numeric pass inconsistency (flag %d)", herr);
-    CBX_TRY(filter_compact<T>(flt, nzcB, nnzcol, cpC, tmp, tmp_bytes, C, s));
+    if (!rep->err) CBX_TRY(filter_compact<T>(flt, nzcB, nnzcol, C, ws));
+    if (!rep->err) CBX_TRY(finish_columns());  // (reports err as it is then)
     nnzC = C->nnz;
+  } else {
+    k_report_err<<<1, 64, 0, s>>>(err, rep_dev);
   }
-  // --- DCSC of C: keep the non-empty columns
-  k_nonempty_flags<<<nblk(nzcB, 256), 256, 0, s>>>(nnzcol, nzcB, flags);
-  CBX_HIP(hipcub::DeviceSelect::Flagged(tmp, tmp_bytes, B->jc, flags, C->jc, nsel, (int)nzcB, s));
-  CBX_HIP(hipcub::DeviceSelect::Flagged(tmp, tmp_bytes, cpC, flags, C->cp, nsel + 1, (int)nzcB, s));
-  k_set_last<<<1, 1, 0, s>>>(C->cp, nsel, cpC, nzcB);
-  int64_t nzcC = 0;
-  CBX_HIP(hipMemcpyAsync(&nzcC, nsel, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  CBX_HIP(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, s));
   tm.mark(5, s);
   CBX_HIP(hipStreamSynchronize(s));
+  if (learned_done || flt.on) nzcC = rep->nzc;
   C->nzc = nzcC;
-  if (herr) {
+  if (rep->err) {
+    const int e = rep->err;
     cbx_dcsc_free(C);
-    return set_error(CBX_ERR_HIP, "cbx_spgemm: numeric pass inconsistency (flag %d)", herr);
+    return set_error(CBX_ERR_HIP, "cbx_spgemm: numeric pass inconsistency (flag %d)", e);
   }
   if (stats) {
     stats->flops = total_flop;
@@ -3541,40 +3758,57 @@ static cbx_status spgemm_typed(const cbx_dcsc* A, const cbx_dcsc* B, cbx_spgemm_
                                int64_t* symbolic_out = nullptr) {
   bool lists_used = false;
   const cbx_status st = spgemm_typed_once<K, T>(A, B, mode, cfg, C, stats, s, symbolic_out, &lists_used);
+  if (st != CBX_OK) cbx_dcsc_free(C);
   if (st != CBX_ERR_NOMEM || !lists_used) return st;
   (void)hipStreamSynchronize(s);
-  cbx_dcsc_free(C);
   release_cache();
   SpgemmConfig plain = cfg;
   plain.unit_lists = 0;
   return spgemm_typed_once<K, T>(A, B, mode, plain, C, stats, s, symbolic_out, nullptr);
 }
 
-cbx_status spgemm_features(const cbx_dcsc* A, const cbx_dcsc* B, float* feats, hipStream_t s) {
-  const int64_t nzcA = A->nzc, nzcB = B->nzc, nnzA = A->nnz, nnzB = B->nnz;
-  if (nzcB == 0) return CBX_OK;
-  DevBuf b_colmap, b_rows, b_bpos, b_err;
-  int32_t *colmap, *rowsA, *bpos;
-  int* err;
-  CBX_TRY(dalloc(b_colmap, A->n, s, &colmap));
-  CBX_TRY(dalloc(b_rows, nnzA, s, &rowsA));
-  CBX_TRY(dalloc(b_bpos, nnzB, s, &bpos));
-  CBX_TRY(dalloc(b_err, 1, s, &err));
-  CBX_HIP(hipMemsetAsync(err, 0, sizeof(int), s));
-  DevBuf b_vcnt;
-  unsigned long long* vcnt;
-  CBX_TRY(dalloc(b_vcnt, 6, s, &vcnt));
-  CBX_TRY(launch_validate(A, 4, vcnt, err, s));
-  CBX_TRY(launch_validate(B, 5, vcnt + 3, err, s));
-  int herr = 0;
-  CBX_HIP(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, s));
+// The operands as the features and the sampling estimator read them: validated
+// (invalid: an error naming `who`), with A's rows as 32 bits and B's entries'
+// positions in A.
+static cbx_status index_operands(const cbx_dcsc* A, const cbx_dcsc* B, const char* who, ScratchSet& ws,
+                                 int32_t** rowsA, int32_t** bpos) {
+  hipStream_t s = ws.s;
+  SlotHold slot;
+  CBX_RETURN_IF(!slot.p, CBX_ERR_NOMEM, "%s: no pinned host memory", who);
+  Report* rep = (Report*)slot.p->host;
+  int32_t* colmap = nullptr;
+  int64_t *flop, *nnzcol;
+  Counters* ctr;
+  CBX_TRY(dalloc(ws, 1, &ctr));
+  if (A->nzc != A->n) CBX_TRY(dalloc(ws, A->n, &colmap));
+  CBX_TRY(dalloc(ws, std::max<int64_t>(A->nnz, 1), rowsA));
+  CBX_TRY(dalloc(ws, std::max<int64_t>(B->nnz, 1), bpos));
+  CBX_TRY(dalloc(ws, B->nzc + 1, &flop));
+  CBX_TRY(dalloc(ws, B->nzc + 1, &nnzcol));
+  k_init<<<256, 256, 0, s>>>(ctr, colmap, A->n, flop, nnzcol, B->nzc);
+  CBX_TRY(launch_validate(A, *rowsA, ctr->val, s));
+  CBX_TRY(launch_validate(B, nullptr, ctr->val + 3, s));
+  k_validate_flag<<<1, 64, 0, s>>>(ctr->val, 4, &ctr->err);
+  k_validate_flag<<<1, 64, 0, s>>>(ctr->val + 3, 5, &ctr->err);
+  k_report_err<<<1, 64, 0, s>>>(&ctr->err, rep);
   CBX_HIP(hipStreamSynchronize(s));
-  if (herr) return set_error(CBX_ERR_INVALID, "cbx_spgemm_features: operand is not a valid DCSC");
-  k_fill_i32<<<nblk(A->n, 256), 256, 0, s>>>(colmap, A->n, -1);
-  if (nzcA) k_colmap<<<nblk(nzcA, 256), 256, 0, s>>>(A->jc, nzcA, colmap);
-  if (nnzA) k_rows32<<<nblk(nnzA, 256), 256, 0, s>>>(A->ir, nnzA, rowsA);
-  if (nnzB) k_bpos<<<nblk(nnzB, 256), 256, 0, s>>>(B->ir, nnzB, colmap, bpos);
-  k_features<<<wave_grid(nzcB), 256, 0, s>>>(B->cp, nzcB, bpos, A->cp, rowsA, A->m, feats);
+  if (((volatile Report*)rep)->err) return set_error(CBX_ERR_INVALID, "%s: operand is not a valid DCSC", who);
+  if (colmap && A->nzc) k_colmap<<<nblk(A->nzc, 256), 256, 0, s>>>(A->jc, A->nzc, nullptr, colmap);
+  if (B->nnz && A->nzc)
+    k_flops<<<nblk(B->nnz, kFlopTile), kFlopNT, 0, s>>>(B->cp, B->ir, B->nzc, B->nnz, colmap, A->cp, nullptr, *bpos,
+                                                       flop);
+  else if (B->nnz)
+    k_fill_i32<<<nblk(B->nnz, 256), 256, 0, s>>>(*bpos, B->nnz, -1);
+  CBX_HIP(hipGetLastError());
+  return CBX_OK;
+}
+
+cbx_status spgemm_features(const cbx_dcsc* A, const cbx_dcsc* B, float* feats, hipStream_t s) {
+  if (B->nzc == 0) return CBX_OK;
+  ScratchSet ws(s);
+  int32_t *rowsA, *bpos;
+  CBX_TRY(index_operands(A, B, "cbx_spgemm_features", ws, &rowsA, &bpos));
+  k_features<<<wave_grid(B->nzc), 256, 0, s>>>(B->cp, B->nzc, bpos, A->cp, rowsA, A->m, feats);
   CBX_HIP(hipGetLastError());
   CBX_HIP(hipStreamSynchronize(s));
   return CBX_OK;
@@ -3582,35 +3816,18 @@ cbx_status spgemm_features(const cbx_dcsc* A, const cbx_dcsc* B, float* feats, h
 
 cbx_status spgemm_estimate_sampling(const cbx_dcsc* A, const cbx_dcsc* B, int rounds, float* est, double* total,
                                     hipStream_t s) {
-  const int64_t nzcA = A->nzc, nzcB = B->nzc, nnzA = A->nnz, nnzB = B->nnz;
+  const int64_t nzcB = B->nzc;
   if (total) *total = 0.0;
   if (nzcB == 0) return CBX_OK;
-  DevBuf b_colmap, b_rows, b_bpos, b_err, b_vcnt, b_samp, b_est, b_sum;
-  int32_t *colmap, *rowsA, *bpos;
-  int* err;
-  unsigned long long* vcnt;
+  ScratchSet ws(s);
+  int32_t *rowsA, *bpos;
   float *samp, *e;
   double* dsum;
-  CBX_TRY(dalloc(b_colmap, A->n, s, &colmap));
-  CBX_TRY(dalloc(b_rows, nnzA, s, &rowsA));
-  CBX_TRY(dalloc(b_bpos, nnzB, s, &bpos));
-  CBX_TRY(dalloc(b_err, 1, s, &err));
-  CBX_TRY(dalloc(b_vcnt, 6, s, &vcnt));
-  CBX_TRY(dalloc(b_samp, sampling_scratch_floats(A, rounds), s, &samp));
-  CBX_TRY(dalloc(b_sum, 1, s, &dsum));
+  CBX_TRY(index_operands(A, B, "cbx_spgemm_estimate_sampling", ws, &rowsA, &bpos));
+  CBX_TRY(dalloc(ws, sampling_scratch_floats(A, rounds), &samp));
+  CBX_TRY(dalloc(ws, 1, &dsum));
   e = est;
-  if (!e) CBX_TRY(dalloc(b_est, nzcB, s, &e));
-  CBX_HIP(hipMemsetAsync(err, 0, sizeof(int), s));
-  CBX_TRY(launch_validate(A, 4, vcnt, err, s));
-  CBX_TRY(launch_validate(B, 5, vcnt + 3, err, s));
-  int herr = 0;
-  CBX_HIP(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, s));
-  CBX_HIP(hipStreamSynchronize(s));
-  if (herr) return set_error(CBX_ERR_INVALID, "cbx_spgemm_estimate_sampling: operand is not a valid DCSC");
-  k_fill_i32<<<nblk(A->n, 256), 256, 0, s>>>(colmap, A->n, -1);
-  if (nzcA) k_colmap<<<nblk(nzcA, 256), 256, 0, s>>>(A->jc, nzcA, colmap);
-  if (nnzA) k_rows32<<<nblk(nnzA, 256), 256, 0, s>>>(A->ir, nnzA, rowsA);
-  if (nnzB) k_bpos<<<nblk(nnzB, 256), 256, 0, s>>>(B->ir, nnzB, colmap, bpos);
+  if (!e) CBX_TRY(dalloc(ws, nzcB, &e));
   CBX_TRY(sampling_estimate_launch(A, B, rounds, rowsA, bpos, samp, e, s));
   if (total) {
     CBX_HIP(hipMemsetAsync(dsum, 0, sizeof(double), s));
@@ -3625,16 +3842,22 @@ cbx_status spgemm_estimate_sampling(const cbx_dcsc* A, const cbx_dcsc* B, int ro
 cbx_status spgemm_flops(const cbx_dcsc* A, const cbx_dcsc* B, int64_t* flop_host, hipStream_t s) {
   const int64_t nzcA = A->nzc, nzcB = B->nzc, nnzB = B->nnz;
   if (nzcB == 0) return CBX_OK;
-  DevBuf b_colmap, b_bpos, b_flop;
-  int32_t *colmap, *bpos;
-  int64_t* flop;
-  CBX_TRY(dalloc(b_colmap, A->n, s, &colmap));
-  CBX_TRY(dalloc(b_bpos, nnzB, s, &bpos));
-  CBX_TRY(dalloc(b_flop, nzcB, s, &flop));
-  k_fill_i32<<<nblk(A->n, 256), 256, 0, s>>>(colmap, A->n, -1);
-  if (nzcA) k_colmap<<<nblk(nzcA, 256), 256, 0, s>>>(A->jc, nzcA, colmap);
-  if (nnzB) k_bpos<<<nblk(nnzB, 256), 256, 0, s>>>(B->ir, nnzB, colmap, bpos);
-  k_flop<<<wave_grid(nzcB), 256, 0, s>>>(B->cp, nzcB, bpos, A->cp, flop);
+  ScratchSet ws(s);
+  int32_t *colmap = nullptr, *bpos;
+  int64_t *flop, *nnzcol;
+  Counters* ctr;
+  CBX_TRY(dalloc(ws, 1, &ctr));
+  if (nzcA != A->n) CBX_TRY(dalloc(ws, A->n, &colmap));
+  CBX_TRY(dalloc(ws, std::max<int64_t>(nnzB, 1), &bpos));
+  CBX_TRY(dalloc(ws, nzcB + 1, &flop));
+  CBX_TRY(dalloc(ws, nzcB + 1, &nnzcol));
+  k_init<<<256, 256, 0, s>>>(ctr, colmap, A->n, flop, nnzcol, nzcB);
+  // a malformed operand has no products here; the product itself reports it
+  CBX_TRY(launch_validate(A, nullptr, ctr->val, s));
+  CBX_TRY(launch_validate(B, nullptr, ctr->val + 3, s));
+  if (colmap && nzcA) k_colmap<<<nblk(nzcA, 256), 256, 0, s>>>(A->jc, nzcA, ctr, colmap);
+  if (nnzB && nzcA)
+    k_flops<<<nblk(nnzB, kFlopTile), kFlopNT, 0, s>>>(B->cp, B->ir, nzcB, nnzB, colmap, A->cp, ctr, bpos, flop);
   CBX_HIP(hipGetLastError());
   CBX_HIP(hipMemcpyAsync(flop_host, flop, sizeof(int64_t) * nzcB, hipMemcpyDeviceToHost, s));
   CBX_HIP(hipStreamSynchronize(s));
