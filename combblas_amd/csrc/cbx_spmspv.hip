@@ -896,20 +896,37 @@ extern "C" void cbx_bfs_plan_destroy(cbx_bfs_plan_s* p) { bfs_plan_free(p); }
 // every stored entry, y accumulated in place; a boolean A contributes x[j]
 // itself.
 //
-// Bucketed form (m <= 2^24): the entries are cut into tiles of kSvTile; pass 1
-// counts each tile's entries per 4096-row block, a scan over (block, tile)
-// gives every tile a slot range per block, pass 2 writes each product with its
-// row offset into its block's bucket, and pass 3 accumulates each block's
-// bucket in LDS (chunks of kSvChunk entries per workgroup) and updates y once
+// Tiled form (m <= 2^24): the entries are cut into tiles of kSvTile.  One pass
+// over A forms a tile's products, orders them in LDS by the block of rows they
+// fall in and writes them, contiguous, to the tile's own place, with the
+// blocks' offsets in it; nothing has to be counted beforehand, and every write
+// is a full line.  A block's products are then the runs that the tiles hold of
+// it: k_svb_cut cuts each block's tiles into chunks of about equal numbers of
+// products, and k_svb_accumulate sums a chunk's runs in LDS and updates y once
 // per row: a plain read-modify-write when one workgroup owns the block, the
 // semiring's device atomic when a hot block is split over several.  Device
 // atomics per entry (the direct form below, kept for taller matrices and small
 // products) serialise on the hot rows of skewed matrices.
-constexpr int kSvLB = 12, kSvBR = 1 << kSvLB;  // rows per block
-constexpr int kSvMaxBlocks = 4096;            // bucketed form while m <= 2^24
-constexpr int kSvTile = 4096, kSvNT = 256;    // entries and threads per counting / scattering workgroup
-constexpr int64_t kSvChunk = 32768;           // bucket entries per accumulating workgroup
-constexpr int64_t kSvMinNnz = 1 << 16;        // below this the direct form is cheaper
+//
+// Blocks have 4096 rows up to m = 2^20 and 16384 above: a tile's run of one
+// block is then at least four products on average (256 and 1024 blocks), and
+// the block's sums still fit LDS.
+//
+// Counting the tiles' products per block first and scattering each product to
+// its block's bucket read the rows twice and wrote two scattered values per
+// entry, each with a search for its column and one load in flight at a time:
+// at 2^20 rows and 16 M entries (FP64) 0.49 ms a product, 0.36 of them in the
+// counting and scattering passes; now 0.21 ms, 0.095 in k_svb_tile (4.4 TB/s)
+// and 0.075 in k_svb_accumulate (2.1 TB/s: 40 us of loads, the rest the
+// rounds' barriers; chunks of half or twice the size and twice the loads in
+// flight measured 75 to 85).
+constexpr int kSvLB = 12, kSvLBTall = 14;           // log2 of the rows per block
+constexpr int64_t kSvShort = (int64_t)1 << 20;      // up to so many rows blocks have 2^kSvLB
+constexpr int kSvMaxBlocks = 1024;                  // tiled form while m <= 2^24
+constexpr int kSvTile = 4096, kSvNT = 256;          // entries and threads per tile
+constexpr int kSvPer = kSvTile / kSvNT;             // entries per thread
+constexpr int kSvChunkLog = 3;                      // log2 of the products per chunk and row of the block
+constexpr int64_t kSvMinNnz = 1 << 16;              // below this the direct form is cheaper
 
 template <int K, class T, bool BOOLA>
 __global__ void k_spmv_dense(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc,
@@ -927,182 +944,295 @@ __global__ void k_spmv_dense(const int64_t* __restrict__ cp, const int64_t* __re
   }
 }
 
-// pass 1: hist[b * ntiles + t] = entries of tile t in row block b.  It also
-// does the per-entry half of the structure check: part[2t] counts the tile's
-// rows outside [0, nrows) (only counted, never used as an index) and
-// part[2t+1] its descents ir[e+1] <= ir[e]; k_svb_verdict sums them (one slot
-// per tile: thousands of workgroups adding to one counter would serialise).
-__global__ __launch_bounds__(kSvNT) void k_svb_count(const int64_t* __restrict__ ir, int64_t nnz, int64_t nrows,
-                                                     int nblk, int64_t ntiles, int64_t* __restrict__ hist,
-                                                     long long* __restrict__ part) {
-  __shared__ int h[kSvMaxBlocks];
-  __shared__ long long ws[2][kSvNT / kWave];
-  const int64_t t = blockIdx.x;
-  for (int b = threadIdx.x; b < nblk; b += kSvNT) h[b] = 0;
-  __syncthreads();
-  const int64_t e0 = t * kSvTile, e1 = min<int64_t>(nnz, e0 + kSvTile);
-  long long bad = 0, desc = 0;
-  for (int64_t e = e0 + threadIdx.x; e < e1; e += kSvNT) {
-    const int64_t r = ir[e];
-    if (r < 0 || r >= nrows) ++bad;
-    else atomicAdd(&h[r >> kSvLB], 1);
-    if (e + 1 < nnz) desc += ir[e + 1] <= r;
-  }
-  bad = wave_sum_ll(bad);
-  desc = wave_sum_ll(desc);
-  if (lane_id() == 0) {
-    ws[0][wave_id()] = bad;
-    ws[1][wave_id()] = desc;
-  }
-  __syncthreads();  // (also orders the histogram before it is read)
-  if (threadIdx.x == 0) {
-    long long a = 0, d = 0;
-    for (int w = 0; w < kSvNT / kWave; ++w) {
-      a += ws[0][w];
-      d += ws[1][w];
-    }
-    part[2 * t] = a;
-    part[2 * t + 1] = d;
-  }
-  for (int b = threadIdx.x; b < nblk; b += kSvNT) hist[(int64_t)b * ntiles + t] = h[b];
+// What the passes report: the structure check's verdicts on columns and on
+// entries (a kernel that may find a fault stops only at those of the kernels
+// before it, so that a workgroup stops as a whole), and the chunks.
+struct SvFlags {
+  int bad_columns, bad_entries, nchunks;
+};
+
+__global__ void k_svb_begin(SvFlags* __restrict__ f) {
+  if (threadIdx.x == 0) *f = SvFlags{0, 0, 0};
 }
 
-// The structure check's verdict: *malformed = 1 when a column violates the
-// rules (cnt[0], from k_check_columns), a row is out of range, or the
-// descents differ from those at column starts (cnt[2]).  One workgroup.
-__global__ __launch_bounds__(kSvNT) void k_svb_verdict(const unsigned long long* __restrict__ cnt,
-                                                       const long long* __restrict__ part, int64_t ntiles,
-                                                       int* __restrict__ malformed) {
-  __shared__ long long ws[2][kSvNT / kWave];
-  long long bad = 0, desc = 0;
-  for (int64_t t = threadIdx.x; t < ntiles; t += kSvNT) {
-    bad += part[2 * t];
-    desc += part[2 * t + 1];
+// The structure check's per-column rules (those of cbx_dcsc_check), and the
+// column qs[t] that holds the first entry of tile t.  A column longer than m
+// is malformed (its rows could not ascend), so a thread writes at most m /
+// kSvTile + 1 of them.
+__global__ __launch_bounds__(256) void k_svb_columns(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc,
+                                                     int64_t nzc, int64_t nnz, int64_t m, int64_t n,
+                                                     int32_t* __restrict__ qs, SvFlags* __restrict__ f) {
+  const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (q >= nzc) return;
+  const int64_t b = cp[q], e = cp[q + 1], j = jc[q], jn = q + 1 < nzc ? jc[q + 1] : n;
+  const bool err = b < 0 || e <= b || e > nnz || e - b > m || j < 0 || jn <= j || (q == 0 && b != 0) ||
+                   (q == nzc - 1 && (e != nnz || j >= n));
+  if (err) {
+    f->bad_columns = 1;
+    return;
   }
-  bad = wave_sum_ll(bad);
-  desc = wave_sum_ll(desc);
-  if (lane_id() == 0) {
-    ws[0][wave_id()] = bad;
-    ws[1][wave_id()] = desc;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    long long a = 0, d = 0;
-    for (int w = 0; w < kSvNT / kWave; ++w) {
-      a += ws[0][w];
-      d += ws[1][w];
-    }
-    *malformed = (cnt[0] != 0 || a != 0 || (unsigned long long)d != cnt[2]) ? 1 : 0;
-  }
+  for (int64_t t = (b + kSvTile - 1) / kSvTile; t * kSvTile < e; ++t) qs[t] = (int32_t)q;
 }
 
-// largest q in [lo, hi] with c[q] <= e (c ascending, c[lo] <= e)
-template <class P>
-__device__ __forceinline__ int64_t last_le(const P* c, int64_t lo, int64_t hi, int64_t e) {
-  while (lo < hi) {
-    const int64_t mid = (lo + hi + 1) >> 1;
-    if (c[mid] <= e) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-
-// pass 2: products into their blocks' buckets (row offset in the block, value)
+// Products of one tile, ordered by row block: bval / brow (row in the block)
+// from the tile's first entry on, and tbl[b * ntiles + t] = the place of block
+// b's first one (b = nblk: the tile's end).  Also the structure check's rules
+// for entries: rows in range, ascending but for column starts.
+//
+// Bound by the bytes of A and of the products; each thread's 16 entries are
+// loaded before anything else.  A tile's columns' x values are gathered into
+// LDS once per column, and an entry finds its column by counting the column
+// starts before it (a bitmap, two mbcnt per entry); consecutive tiles go to
+// the same XCD, whose L2 then merges their neighbouring entries of tbl.
 template <int K, class T, bool BOOLA>
-__global__ __launch_bounds__(kSvNT) void k_svb_scatter(const int64_t* __restrict__ cp,
-                                                       const int64_t* __restrict__ jc,
-                                                       const int64_t* __restrict__ ir,
-                                                       const void* __restrict__ valA_, int64_t nzc, int64_t nnz,
-                                                       const T* __restrict__ x, int nblk, int64_t ntiles,
-                                                       const int64_t* __restrict__ offs, uint16_t* __restrict__ brow,
-                                                       T* __restrict__ bval, const int* __restrict__ malformed) {
+__global__ __launch_bounds__(kSvNT) void k_svb_tile(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc,
+                                                    const int64_t* __restrict__ ir, const void* __restrict__ valA_,
+                                                    int64_t nzc, int64_t nnz, int64_t m, const T* __restrict__ x,
+                                                    int lb, int nblk, int64_t ntiles,
+                                                    const int32_t* __restrict__ qs, uint16_t* __restrict__ tbl,
+                                                    uint16_t* __restrict__ brow, T* __restrict__ bval,
+                                                    SvFlags* __restrict__ f) {
   using SR = Sem<K, T>;
+  constexpr int U = kSvPer, NW = kSvNT / kWave;
+  static_assert(kSvTile == kWave * kWave, "one bitmap word per lane");
+  static_assert(kSvMaxBlocks % kSvNT == 0, "whole block counts per thread");
+  __shared__ T xs[kSvTile + 1];  // x of the tile's columns, then the ordered products
+  __shared__ uint16_t srow[kSvTile];
   __shared__ int h[kSvMaxBlocks];
-  __shared__ int64_t scp[kSvTile + 1];  // cp of the columns the tile spans (columns are non-empty)
-  __shared__ int64_t s_q[2];
-  if (*malformed) return;  // the structure check failed: cp, jc or ir cannot be trusted as indices
-  const int64_t t = blockIdx.x;
-  const int64_t e0 = t * kSvTile, e1 = min<int64_t>(nnz, e0 + kSvTile);
+  __shared__ unsigned long long starts[kWave];
+  __shared__ int wsum[NW];
+  if (f->bad_columns) return;  // cp, jc or qs cannot be trusted as indices
+  const int64_t per = (ntiles + 7) / 8;
+  const int64_t t = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (t >= ntiles) return;
+  const int64_t e0 = t * kSvTile;
+  const int cnt = (int)min<int64_t>(nnz - e0, kSvTile);
+  const int lane = lane_id(), w = wave_id_uniform();
+
+  int64_t r[U];
+  T a[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = min((w * U + u) * kWave + lane, cnt - 1);
+    r[u] = ir[e0 + i];
+    if constexpr (!BOOLA) a[u] = ((const T*)valA_)[e0 + i];
+  }
+  // the entry after this wave's last (its own last row + 1 where there is none)
+  const int last = (w + 1) * U * kWave;
+  const int64_t after = e0 + last < nnz ? ir[e0 + last] : 0;
+  const int64_t q0 = qs[t], q1 = t + 1 < ntiles ? qs[t + 1] : nzc - 1;
+  const int nq = (int)min<int64_t>(q1 - q0 + 1, kSvTile + 1);
   for (int b = threadIdx.x; b < nblk; b += kSvNT) h[b] = 0;
-  if (threadIdx.x < 2) s_q[threadIdx.x] = last_le(cp, 0, nzc - 1, threadIdx.x == 0 ? e0 : e1 - 1);
+  if (threadIdx.x < kWave) starts[threadIdx.x] = 0ull;
   __syncthreads();
-  const int64_t q0 = s_q[0], q1 = s_q[1];
-  const int nq = (int)(q1 - q0 + 2);  // <= kSvTile + 1
-  for (int i = threadIdx.x; i < nq; i += kSvNT) scp[i] = cp[q0 + i];
-  __syncthreads();
-  int64_t ql = 0;  // column of this thread's previous entry, relative to q0 (entries ascend)
-  for (int64_t e = e0 + threadIdx.x; e < e1; e += kSvNT) {
-    ql = last_le(scp, ql, nq - 2, e);
-    const T xj = x[jc[q0 + ql]];
-    T prod;
-    if constexpr (BOOLA) prod = xj;
-    else prod = (T)SR::out(SR::mul(((const T*)valA_)[e], xj));
-    const int64_t r = ir[e];
-    const int b = (int)(r >> kSvLB);
-    const int64_t pos = offs[(int64_t)b * ntiles + t] + atomicAdd(&h[b], 1);
-    brow[pos] = (uint16_t)(r & (kSvBR - 1));
-    bval[pos] = prod;
+  for (int i = threadIdx.x; i < nq; i += kSvNT) {
+    const int64_t s = cp[q0 + i] - e0, j = jc[q0 + i];
+    xs[i] = x[j];
+    // bit s - 1: the entries from s on lie past this column's start
+    if (i > 0 && s >= 1 && s <= kSvTile) atomicOr(&starts[(s - 1) >> 6], 1ull << ((s - 1) & 63));
   }
-}
-
-// chunk table: cstart[b] = chunks of the blocks before b (cstart[nblk] = all);
-// one workgroup, kSvChunkNT threads with kSvMaxBlocks / kSvChunkNT blocks each
-constexpr int kSvChunkNT = 1024, kSvChunkPT = kSvMaxBlocks / kSvChunkNT;
-__global__ __launch_bounds__(kSvChunkNT) void k_svb_chunks(const int64_t* __restrict__ offs, int nblk,
-                                                           int64_t ntiles, int64_t nnz,
-                                                           int64_t* __restrict__ cstart) {
-  __shared__ long long wsum[kSvChunkNT / kWave];
-  int64_t c[kSvChunkPT];
-  long long sum = 0;
 #pragma unroll
-  for (int k = 0; k < kSvChunkPT; ++k) {
-    const int b = threadIdx.x * kSvChunkPT + k;
-    c[k] = 0;
-    if (b < nblk) {
-      const int64_t lo = offs[(int64_t)b * ntiles], hi = b + 1 < nblk ? offs[(int64_t)(b + 1) * ntiles] : nnz;
-      c[k] = (hi - lo + kSvChunk - 1) / kSvChunk;
+  for (int u = 0; u < U; ++u) {
+    pin(r[u]);
+    if constexpr (!BOOLA) pin(a[u]);
+  }
+  __syncthreads();
+  const unsigned long long word = starts[lane];  // lane i: the starts in (64 i, 64 i + 64]
+  const int ones = __popcll(word);
+  const int before = wave_incl_scan(ones) - ones;
+
+  bool bad = false;
+  int rank[U];
+  T prod[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int j = w * U + u;
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)word, j);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(word >> 32), j);
+    const int k = (int)__builtin_amdgcn_mbcnt_hi(
+        hi, __builtin_amdgcn_mbcnt_lo(lo, (unsigned)__builtin_amdgcn_readlane(before, j)));
+    const int i = j * kWave + lane;
+    const bool live = i < cnt;
+    // descents: the next entry's row, unless a column starts there (bit i)
+    const int64_t nf = u + 1 < U ? readlane_ll(r[u + 1 < U ? u + 1 : u], 0) : after;
+    int64_t next = __shfl_down((long long)r[u], 1, kWave);
+    if (lane == kWave - 1) next = nf;
+    const bool start = ((((unsigned long long)hi << 32) | lo) >> lane) & 1u;
+    const bool in = r[u] >= 0 && r[u] < m;
+    bad |= live && (!in || (e0 + i + 1 < nnz && next <= r[u] && !start));
+    const T xj = xs[k];
+    if constexpr (BOOLA) prod[u] = xj;
+    else prod[u] = (T)SR::out(SR::mul(a[u], xj));
+    rank[u] = live && in ? atomicAdd(&h[r[u] >> lb], 1) : -1;
+  }
+  if (__ballot(bad) && lane == 0) f->bad_entries = 1;
+  __syncthreads();  // the blocks' counts; xs has been read
+  {
+    constexpr int PT = kSvMaxBlocks / kSvNT;
+    int c[PT], sum = 0;
+#pragma unroll
+    for (int k = 0; k < PT; ++k) {
+      const int b = threadIdx.x * PT + k;
+      c[k] = b < nblk ? h[b] : 0;
+      sum += c[k];
     }
-    sum += c[k];
-  }
-  long long total;
-  long long ex = block_excl_scan_ll<kSvChunkNT>(sum, wsum, total);
+    int total;
+    int ex = block_excl_scan<kSvNT>(sum, wsum, total);
 #pragma unroll
-  for (int k = 0; k < kSvChunkPT; ++k) {
-    const int b = threadIdx.x * kSvChunkPT + k;
-    if (b < nblk) cstart[b] = ex;
-    ex += c[k];
+    for (int k = 0; k < PT; ++k) {
+      const int b = threadIdx.x * PT + k;
+      if (b < nblk) h[b] = ex;
+      ex += c[k];
+    }
+    if (threadIdx.x == 0) tbl[(int64_t)nblk * ntiles + t] = (uint16_t)total;
   }
-  if (threadIdx.x == 0) cstart[nblk] = total;
+  __syncthreads();
+  for (int b = threadIdx.x; b < nblk; b += kSvNT) tbl[(int64_t)b * ntiles + t] = (uint16_t)h[b];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (rank[u] < 0) continue;
+    const int p = h[r[u] >> lb] + rank[u];
+    xs[p] = prod[u];
+    srow[p] = (uint16_t)(r[u] & ((1 << lb) - 1));
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < cnt; i += kSvNT) {
+    bval[e0 + i] = xs[i];
+    brow[e0 + i] = srow[i];
+  }
 }
 
-// pass 3: one workgroup per chunk of a block's bucket
-template <int K, class T>
-__global__ __launch_bounds__(kSvNT) void k_svb_accumulate(const int64_t* __restrict__ offs,
-                                                          const int64_t* __restrict__ cstart, int nblk,
-                                                          int64_t ntiles, int64_t nnz, int64_t m,
-                                                          const uint16_t* __restrict__ brow,
-                                                          const T* __restrict__ bval, T* __restrict__ y,
-                                                          const int* __restrict__ malformed) {
+// A chunk: the tiles [t0, t1) of a row block, one of n chunks of that block.
+struct SvChunk {
+  int32_t b, t0, t1, n;
+};
+
+// Cuts one row block's tiles into chunks (one workgroup per block): chunk c
+// starts at the first tile with at least c << lc products before it, so a
+// chunk has at most 2^lc + kSvTile products, and the numbers have no gaps
+// (2^lc >= kSvTile).  The chunks' places are taken with one atomic per block.
+constexpr int kSvCutNT = 256, kSvCutPer = 8;
+__global__ __launch_bounds__(kSvCutNT) void k_svb_cut(const uint16_t* __restrict__ tbl, int64_t ntiles, int lc,
+                                                      SvChunk* __restrict__ chunks, SvFlags* __restrict__ f) {
+  __shared__ long long wsum[kSvCutNT / kWave];
+  __shared__ int s_base;
+  if (f->bad_columns || f->bad_entries) return;
+  const int b = blockIdx.x;
+  const uint16_t* lo = tbl + (int64_t)b * ntiles;
+  const uint16_t* hi = lo + ntiles;
+  long long all = 0;
+  for (int64_t t0 = threadIdx.x; t0 < ntiles; t0 += kSvCutNT * kSvCutPer) {
+    uint16_t a[kSvCutPer], z[kSvCutPer];
+#pragma unroll
+    for (int k = 0; k < kSvCutPer; ++k) {
+      const int64_t t = min<int64_t>(t0 + k * kSvCutNT, ntiles - 1);
+      a[k] = lo[t];
+      z[k] = hi[t];
+    }
+#pragma unroll
+    for (int k = 0; k < kSvCutPer; ++k) {
+      pin(a[k]);
+      pin(z[k]);
+      if (t0 + k * kSvCutNT < ntiles) all += z[k] - a[k];
+    }
+  }
+  all = block_sum_ll<kSvCutNT>(all, wsum);
+  if (all == 0) return;
+  const int n = (int)((all - (hi[ntiles - 1] - lo[ntiles - 1])) >> lc) + 1;
+  if (threadIdx.x == 0) s_base = atomicAdd(&f->nchunks, n);
+  __syncthreads();
+  SvChunk* out = chunks + s_base;
+  long long done = 0;  // products before this round's tiles
+  for (int64_t t0 = 0; t0 < ntiles; t0 += kSvCutNT * kSvCutPer) {
+    const int64_t tb = t0 + threadIdx.x * kSvCutPer;
+    int len[kSvCutPer];
+    long long sum = 0;
+#pragma unroll
+    for (int k = 0; k < kSvCutPer; ++k) {
+      const int64_t t = min<int64_t>(tb + k, ntiles - 1);
+      len[k] = hi[t] - lo[t];
+      if (tb + k >= ntiles) len[k] = 0;
+      sum += len[k];
+    }
+    long long total;
+    long long p = done + block_excl_scan_ll<kSvCutNT>(sum, wsum, total);
+#pragma unroll
+    for (int k = 0; k < kSvCutPer; ++k) {
+      // the chunk after this tile's starts at the next tile
+      const int c = (int)(p >> lc), d = (int)((p + len[k]) >> lc);
+      const int64_t t = tb + k;
+      if (t == 0) {
+        out[0].b = b;
+        out[0].t0 = 0;
+        out[0].n = n;
+      }
+      if (t < ntiles && d != c && d < n) {
+        out[c].t1 = (int32_t)(t + 1);
+        out[d].b = b;
+        out[d].t0 = (int32_t)(t + 1);
+        out[d].n = n;
+      }
+      if (t == ntiles - 1) out[n - 1].t1 = (int32_t)ntiles;
+      p += len[k];
+    }
+    done += total;
+  }
+}
+
+// One workgroup per chunk: its runs, a tile per thread at a time, flattened.
+template <int K, class T, int LB, int NT, int U>
+__global__ __launch_bounds__(NT) void k_svb_accumulate(const SvChunk* __restrict__ chunks,
+                                                       const SvFlags* __restrict__ f,
+                                                       const uint16_t* __restrict__ tbl, int64_t ntiles, int64_t m,
+                                                       const uint16_t* __restrict__ brow,
+                                                       const T* __restrict__ bval, T* __restrict__ y) {
   using SR = Sem<K, T>;
   using Acc = typename SR::Acc;
-  __shared__ typename SR::Lds acc[kSvBR];
-  if (*malformed) return;  // y is left as it was
-  const int64_t g = blockIdx.x;
-  if (g >= cstart[nblk]) return;
-  const int b = (int)last_le(cstart, 0, nblk - 1, g);  // blocks without chunks share cstart with the next
-  const int64_t lo = offs[(int64_t)b * ntiles], hi = b + 1 < nblk ? offs[(int64_t)(b + 1) * ntiles] : nnz;
-  const int64_t c = g - cstart[b], nch = cstart[b + 1] - cstart[b];
-  const int64_t i0 = lo + c * kSvChunk, i1 = min<int64_t>(hi, i0 + kSvChunk);
-  for (int r = threadIdx.x; r < kSvBR; r += kSvNT) acc[r] = SR::lident();
+  constexpr int BR = 1 << LB;
+  __shared__ typename SR::Lds acc[BR];
+  __shared__ FlatStage<T, NT, false> st;
+  if (f->bad_columns || f->bad_entries || (int)blockIdx.x >= f->nchunks) return;  // malformed: y is left as it was
+  const SvChunk ch = chunks[blockIdx.x];
+  for (int r = threadIdx.x; r < BR; r += NT) acc[r] = SR::lident();
+  flat_init(st);
+  const uint16_t* lo = tbl + (int64_t)ch.b * ntiles;
+  const uint16_t* hi = lo + ntiles;
+  int par = 0;
+  const int tf = min(ch.t0 + (int)threadIdx.x, ch.t1 - 1);
+  uint16_t na = lo[tf], nz = hi[tf];  // the next round's run
+  for (int t0 = ch.t0; t0 < ch.t1; t0 += NT) {
+    const int a = na;
+    const int len = t0 + (int)threadIdx.x < ch.t1 ? nz - a : 0;
+    const int tn = min(t0 + NT + (int)threadIdx.x, ch.t1 - 1);
+    na = lo[tn];
+    nz = hi[tn];
+    const int64_t e0 = (int64_t)t0 * kSvTile;
+    const FlatSeg me = flat_stage<T, NT, false>(st, (int)threadIdx.x * kSvTile + a, len, T{});
+    flat_chunk<T, NT, false, U>(st, me, par, [&](const int32_t(&idx)[U], T(&)[U], const bool(&ok)[U]) {
+      uint16_t r[U];
+      T v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        r[u] = brow[e0 + idx[u]];
+        v[u] = bval[e0 + idx[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        pin(r[u]);
+        pin(v[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (ok[u]) SR::acc(&acc[r[u]], (Acc)v[u]);
+    });
+  }
   __syncthreads();
-  for (int64_t i = i0 + threadIdx.x; i < i1; i += kSvNT) SR::acc(&acc[brow[i]], (Acc)bval[i]);
-  __syncthreads();
-  const int64_t row0 = (int64_t)b * kSvBR;
+  const int64_t row0 = (int64_t)ch.b * BR;
   using Bits = typename std::conditional<sizeof(Acc) == 8, unsigned long long, unsigned int>::type;
   const Bits id = __builtin_bit_cast(Bits, SR::ident());
-  for (int r = threadIdx.x; r < kSvBR && row0 + r < m; r += kSvNT) {
+  for (int r = threadIdx.x; r < BR && row0 + r < m; r += NT) {
     const Acc a = (Acc)SR::lout(acc[r]);
-    if (nch == 1) {
+    if (ch.n == 1) {
       y[row0 + r] = (T)SR::out(SR::add((Acc)y[row0 + r], a));
     } else if (__builtin_bit_cast(Bits, a) != id) {  // the identity changes nothing
       GAcc<K, T>::acc(&y[row0 + r], (T)SR::out(a));
@@ -1114,7 +1244,8 @@ template <int K, class T>
 static cbx_status spmv_dense_typed(const cbx_dcsc* A, bool boolA, const T* x, T* y, hipStream_t s) {
   if (A->nzc == 0) return CBX_OK;
   const int64_t nnz = A->nnz, m = A->m;
-  const int64_t nblk64 = (m + kSvBR - 1) / kSvBR;
+  const int lb = m <= kSvShort ? kSvLB : kSvLBTall;
+  const int64_t nblk64 = (m + (1 << lb) - 1) >> lb;
   if (nnz < kSvMinNnz || nblk64 > kSvMaxBlocks) {
     {  // the structure check first: the kernel indexes y by A's rows and x by its columns
       ScratchSet cs(s);
@@ -1134,52 +1265,44 @@ static cbx_status spmv_dense_typed(const cbx_dcsc* A, bool boolA, const T* x, T*
   }
   const int nblk = (int)nblk64;
   const int64_t ntiles = (nnz + kSvTile - 1) / kSvTile;
-  const int64_t nh = (int64_t)nblk * ntiles;
-  const int64_t max_chunks = nnz / kSvChunk + nblk;
-  CBX_RETURN_IF(ntiles >= (1ll << 31) || max_chunks >= (1ll << 31) || nh >= (1ll << 31), CBX_ERR_LIMIT,
+  const int lc = lb + kSvChunkLog;
+  const int64_t max_chunks = (nnz >> lc) + nblk;
+  CBX_RETURN_IF(ntiles >= (1ll << 31) / nblk || max_chunks >= (1ll << 31), CBX_ERR_LIMIT,
                 "cbx_spmv_dense: matrix too large for one launch");
-  int64_t *hist = nullptr, *offs = nullptr, *cstart = nullptr;
-  uint16_t* brow = nullptr;
+  int32_t* qs = nullptr;
+  uint16_t *tbl = nullptr, *brow = nullptr;
   T* bval = nullptr;
-  void* tmp = nullptr;
-  unsigned long long* chk = nullptr;  // structure-check counters, then the device-side verdict
-  long long* part = nullptr;          // per-tile counts of the per-entry check
-  size_t tb = 0;
-  CBX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, hist, offs, (int)nh, s));
+  SvChunk* chunks = nullptr;
+  SvFlags* flags = nullptr;
   ScratchSet ws(s);
-  auto cleanup = [&]() { ws.release(); };
-  if (!ws.take(&hist, nh) || !ws.take(&offs, nh) || !ws.take(&cstart, nblk + 1) || !ws.take(&brow, nnz) ||
-      !ws.take(&bval, nnz) || !ws.take_bytes(&tmp, std::max<size_t>(tb, 16)) || !ws.take(&chk, 4) ||
-      !ws.take(&part, 2 * ntiles)) {
-    cleanup();
+  if (!ws.take(&qs, ntiles) || !ws.take(&tbl, (nblk + 1) * ntiles) || !ws.take(&brow, nnz) || !ws.take(&bval, nnz) ||
+      !ws.take(&chunks, max_chunks) || !ws.take(&flags, 1))
     return set_error(CBX_ERR_NOMEM, "cbx_spmv_dense: workspace allocation failed");
-  }
-  int* malformed = (int*)(chk + 3);
   // the structure check (the rules of cbx_dcsc_check) runs inside the
-  // launches: its per-column half here, the per-entry half in the counting
-  // pass, and the kernels that index by the structure wait for the verdict
-  dcsc_check_columns_launch(A, chk, s);
-  k_svb_count<<<(unsigned)ntiles, kSvNT, 0, s>>>(A->ir, nnz, m, nblk, ntiles, hist, part);
-  k_svb_verdict<<<1, kSvNT, 0, s>>>(chk, part, ntiles, malformed);
-  hipError_t e = hipcub::DeviceScan::ExclusiveSum(tmp, tb, hist, offs, (int)nh, s);
-  if (e == hipSuccess) {
-    if (boolA)
-      k_svb_scatter<K, T, true><<<(unsigned)ntiles, kSvNT, 0, s>>>(A->cp, A->jc, A->ir, A->val, A->nzc, nnz, x, nblk,
-                                                                 ntiles, offs, brow, bval, malformed);
-    else
-      k_svb_scatter<K, T, false><<<(unsigned)ntiles, kSvNT, 0, s>>>(A->cp, A->jc, A->ir, A->val, A->nzc, nnz, x,
-                                                                  nblk, ntiles, offs, brow, bval, malformed);
-    k_svb_chunks<<<1, kSvChunkNT, 0, s>>>(offs, nblk, ntiles, nnz, cstart);
-    k_svb_accumulate<K, T><<<(unsigned)max_chunks, kSvNT, 0, s>>>(offs, cstart, nblk, ntiles, nnz, m, brow, bval, y,
-                                                                 malformed);
-    e = hipGetLastError();
-  }
-  int bad = 0;
-  if (e == hipSuccess) e = hipMemcpyAsync(&bad, malformed, sizeof(int), hipMemcpyDeviceToHost, s);
+  // launches, and each stops at a verdict of those before it
+  k_svb_begin<<<1, 64, 0, s>>>(flags);
+  k_svb_columns<<<nb(A->nzc, 256), 256, 0, s>>>(A->cp, A->jc, A->nzc, nnz, m, A->n, qs, flags);
+  const unsigned g = (unsigned)((ntiles + 7) / 8 * 8);
+  if (boolA)
+    k_svb_tile<K, T, true><<<g, kSvNT, 0, s>>>(A->cp, A->jc, A->ir, A->val, A->nzc, nnz, m, x, lb, nblk, ntiles, qs,
+                                              tbl, brow, bval, flags);
+  else
+    k_svb_tile<K, T, false><<<g, kSvNT, 0, s>>>(A->cp, A->jc, A->ir, A->val, A->nzc, nnz, m, x, lb, nblk, ntiles, qs,
+                                               tbl, brow, bval, flags);
+  k_svb_cut<<<(unsigned)nblk, kSvCutNT, 0, s>>>(tbl, ntiles, lc, chunks, flags);
+  if (lb == kSvLB)
+    k_svb_accumulate<K, T, kSvLB, 512, 4><<<(unsigned)max_chunks, 512, 0, s>>>(chunks, flags, tbl, ntiles, m, brow,
+                                                                           bval, y);
+  else
+    k_svb_accumulate<K, T, kSvLBTall, 1024, 4><<<(unsigned)max_chunks, 1024, 0, s>>>(chunks, flags, tbl, ntiles, m,
+                                                                                 brow, bval, y);
+  hipError_t e = hipGetLastError();
+  SvFlags h{0, 0, 0};
+  if (e == hipSuccess) e = hipMemcpyAsync(&h, flags, sizeof(h), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  cleanup();
+  ws.release();
   if (e != hipSuccess) return set_error(CBX_ERR_HIP, "cbx_spmv_dense: %s", hipGetErrorString(e));
-  if (bad) return set_error(CBX_ERR_INVALID, "cbx_dcsc_check: malformed DCSC");
+  if (h.bad_columns || h.bad_entries) return set_error(CBX_ERR_INVALID, "cbx_dcsc_check: malformed DCSC");
   return CBX_OK;
 }
 
