@@ -18,8 +18,10 @@
 // fused per level into two kernels: expand (every frontier vertex k offers k to
 // each unvisited neighbour with an atomic max; the first offer appends the
 // neighbour to the next frontier) and finalize (parents = offers; mark
-// visited).  Each level is one captured hipGraph (two graphs alternate the
-// frontier buffers); the host reads only the next frontier's size.
+// visited).  Large frontiers of a symmetric pattern go bottom-up instead, from
+// and to a bitmap.  Each level is one captured hipGraph, whose last kernel
+// reports the next frontier's size and edges to the host's pinned memory (two
+// copies took longer than the small levels' kernels).
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -344,13 +346,25 @@ cbx_status spmspv_in_region(const cbx_dcsc* A, bool boolA, const int32_t* xind, 
 // ====================================================================== BFS
 namespace {
 
-__global__ void k_bfs_dense_cp(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc, int64_t nzc,
-                               int64_t n, int64_t* __restrict__ beg, int64_t* __restrict__ end) {
+// The rows of column j: [range[j].x, range[j].y) (empty: both 0).
+__global__ void k_bfs_ranges(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc, int64_t nzc,
+                             int2* __restrict__ range) {
   const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (p < nzc) {
-    beg[jc[p]] = cp[p];
-    end[jc[p]] = cp[p + 1];
-  }
+  if (p < nzc) range[jc[p]] = make_int2((int)cp[p], (int)cp[p + 1]);
+}
+
+// The vertices that no search reaches, as a bitmap: those without neighbours
+// in a symmetric pattern (in another a vertex without a column may have rows),
+// and the bits from n on.
+__global__ __launch_bounds__(256) void k_bfs_isolated(const int2* __restrict__ range, int64_t n, int64_t nw,
+                                                      bool symmetric, unsigned long long* __restrict__ isolated) {
+  const int64_t w = global_wave();
+  if (w >= nw) return;
+  const int64_t v = w * kWave + lane_id();
+  bool none = true;
+  if (v < n) none = symmetric && range[v].x == range[v].y;
+  const unsigned long long mask = __ballot(none);
+  if (lane_id() == 0) isolated[w] = mask;
 }
 
 // Number of positions where two int64 arrays differ (the symmetry check of
@@ -383,70 +397,145 @@ __device__ __forceinline__ void bfs_add_pieces(int32_t v, int64_t deg, int32_t* 
   for (int k = 0; k < np; ++k) pieces[b + k] = ((long long)v << 32) | k;
 }
 
+// What a level's workgroups count: vertices found and their edges, in slots a
+// line apart (thousands of workgroups adding to one counter would serialise).
+constexpr int kBfsSlots = 64;
+struct BfsSlot {
+  unsigned long long found, edges, pad[6];
+};
+
+// A search's state on the device; k_bfs_level_end brings it from level to level.
+struct BfsState {
+  BfsSlot slots[kBfsSlots];
+  int32_t listed[2], pieces[2];  // entries of the two frontier lists and of their hub pieces
+  int32_t size;                  // the current frontier
+  int32_t longs[2];              // vertices listed by k_bfs_bottom_up
+  unsigned long long levels, reached;
+};
+
+// What the host reads (pinned): the next frontier's size and edges, levels and
+// vertices reached so far.
+struct BfsReport {
+  unsigned long long size, edges, levels, reached;
+};
+
 __global__ void k_bfs_reset(int64_t n, int32_t* __restrict__ cand, int64_t* __restrict__ parents,
-                            uint32_t* __restrict__ visited, int64_t nw, int32_t* __restrict__ f0,
-                            int32_t* __restrict__ counts, int32_t* __restrict__ pcount,
-                            long long* __restrict__ pieces0, const int64_t* __restrict__ beg,
-                            const int64_t* __restrict__ end, unsigned long long* __restrict__ stat, int64_t root) {
+                            unsigned long long* __restrict__ visited,
+                            const unsigned long long* __restrict__ isolated, int64_t nw, int32_t* __restrict__ f0,
+                            long long* __restrict__ pieces0, const int2* __restrict__ range,
+                            BfsState* __restrict__ st, BfsReport* __restrict__ rep, int64_t root) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < n) {
     cand[i] = -1;
     parents[i] = -1;
   }
-  if (i < nw) visited[i] = 0u;
+  if (i < nw) visited[i] = isolated[i];
+  if (i < kBfsSlots) {
+    st->slots[i].found = 0ull;
+    st->slots[i].edges = 0ull;
+  }
   if (i == 0) {
     f0[0] = (int32_t)root;
-    counts[0] = 1;
-    counts[1] = 0;
-    pcount[0] = 0;
-    pcount[1] = 0;
-    stat[0] = 0ull;  // levels
-    stat[1] = 0ull;  // vertices reached
-    const int64_t deg = end[root] - beg[root];
-    if (deg > kBfsHub) bfs_add_pieces((int32_t)root, deg, pcount, pieces0);
+    st->listed[0] = 1;
+    st->listed[1] = 0;
+    st->pieces[0] = 0;
+    st->pieces[1] = 0;
+    st->size = 1;
+    st->levels = 0ull;
+    st->reached = 0ull;
+    st->longs[0] = 0;
+    st->longs[1] = 0;
+    const int64_t deg = range[root].y - range[root].x;
+    if (deg > kBfsHub) bfs_add_pieces((int32_t)root, deg, &st->pieces[0], pieces0);
+    rep->size = 1ull;
+    rep->edges = (unsigned long long)deg;
   }
 }
 
-// First kernel of a level: clears the next frontier's count and degree sum,
-// and counts the level if its frontier is not empty (a level graph launched
-// after the search ended changes nothing).
-__global__ void k_bfs_level_begin(const int32_t* __restrict__ cin, int32_t* __restrict__ c,
-                                  unsigned long long* __restrict__ edges, int32_t* __restrict__ pc,
-                                  unsigned long long* __restrict__ stat) {
-  if (threadIdx.x == 0) {
-    *c = 0;
-    *edges = 0ull;
-    *pc = 0;
-    if (*cin > 0) ++stat[0];
+// Last kernel of a level from frontier `par` to 1 - par: sums the slots, counts
+// the level if its frontier was not empty (a level launched after the search
+// ended changes nothing), clears what the next level counts in and reports to
+// the host.  A bottom-up level (bits) leaves its frontier as a bitmap, its list
+// empty.  One wave.
+__global__ __launch_bounds__(kWave) void k_bfs_level_end(BfsState* __restrict__ st, int par, bool bits,
+                                                         BfsReport* __restrict__ rep) {
+  BfsSlot& sl = st->slots[threadIdx.x];
+  const long long found = wave_sum_ll((long long)sl.found);
+  const long long edges = wave_sum_ll((long long)sl.edges);
+  sl.found = 0ull;
+  sl.edges = 0ull;
+  if (threadIdx.x) return;
+  const unsigned long long levels = st->levels + (st->size > 0), reached = st->reached + found;
+  st->levels = levels;
+  st->reached = reached;
+  st->size = (int32_t)found;
+  st->listed[par] = 0;
+  st->pieces[par] = 0;
+  if (bits) {
+    st->longs[0] = 0;
+    st->longs[1] = 0;
+    st->listed[1 - par] = 0;
+    st->pieces[1 - par] = 0;
   }
+  *rep = BfsReport{(unsigned long long)found, (unsigned long long)edges, levels, reached};
 }
 
-// A frontier vertex offers itself (k) to neighbour r: SelectMax keeps the
-// largest offer in cand[r]; the first offer appends r to the next frontier
-// (one atomic per wave for the appends of this step).  All lanes call it.
-__device__ __forceinline__ void bfs_offer(int32_t r, int32_t k, const uint32_t* __restrict__ visited,
-                                          int32_t* __restrict__ cand, int32_t* __restrict__ fout,
-                                          int32_t* __restrict__ fout_count) {
-  bool push = false;
-  if (r >= 0 && !((visited[r >> 5] >> (r & 31)) & 1u)) {
-    // Offers only grow cand, so a value read without the atomic (possibly
-    // stale, never above the true one) that already holds an offer at least
-    // this large makes the atomic a no-op: skip it.  Hubs receive thousands
-    // of offers per level and only the record-breaking ones reach the
-    // serialising atomic.
-    const int32_t seen = __hip_atomic_load(&cand[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (seen < k) {
-      const int32_t old = atomicMax(&cand[r], k);
-      push = old == -1;
-    }
+// A workgroup's counts into its slot.
+template <int NT>
+__device__ __forceinline__ void bfs_count(BfsState* st, long long found, long long edges) {
+  BfsSlot& sl = st->slots[blockIdx.x % kBfsSlots];
+  block_add_counts<NT>(found, edges, &sl.found, &sl.edges);
+}
+
+// Frontier vertices offer themselves (k[u]) to neighbours r[u] (ok[u]: there is
+// one): SelectMax keeps the largest offer in cand[r]; the first offer appends r
+// to the next frontier, one atomic per wave for the appends of this step.  The
+// U probes of a lane are in flight together.  All lanes call it.
+template <int U>
+__device__ __forceinline__ void bfs_offer(const int32_t (&r)[U], const int32_t (&k)[U], const bool (&ok)[U],
+                                          const uint32_t* __restrict__ visited, int32_t* __restrict__ cand,
+                                          int32_t* __restrict__ fout, int32_t* __restrict__ fout_count) {
+  uint32_t word[U];
+  int32_t seen[U], old[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) word[u] = visited[r[u] >> 5];
+#pragma unroll
+  for (int u = 0; u < U; ++u) pin(word[u]);
+  bool live[U];
+  // Offers only grow cand, so a value read without the atomic (possibly
+  // stale, never above the true one) that already holds an offer at least
+  // this large makes the atomic a no-op: skip it.  Hubs receive thousands
+  // of offers per level and only the record-breaking ones reach the
+  // serialising atomic.  (Lanes without an unvisited neighbour read cand[0].)
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    live[u] = ok[u] && !((word[u] >> (r[u] & 31)) & 1u);
+    seen[u] = __hip_atomic_load(&cand[live[u] ? r[u] : 0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  const uint64_t mask = __ballot(push);
-  if (mask) {
-    const int leader = __ffsll((unsigned long long)mask) - 1;
-    int basei = 0;
-    if (lane_id() == leader) basei = atomicAdd(fout_count, __popcll(mask));
-    basei = __shfl(basei, leader, kWave);
-    if (push) fout[basei + __popcll(mask & ((1ull << lane_id()) - 1ull))] = r;
+#pragma unroll
+  for (int u = 0; u < U; ++u) pin(seen[u]);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    old[u] = 0;
+    if (live[u] && seen[u] < k[u]) old[u] = atomicMax(&cand[r[u]], k[u]);
+  }
+  unsigned long long mask[U];
+  int total = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    mask[u] = __ballot(old[u] == -1);
+    total += __popcll(mask[u]);
+  }
+  if (!total) return;
+  int at = 0;
+  if (lane_id() == 0) at = atomicAdd(fout_count, total);
+  at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (old[u] == -1)
+      fout[at + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask[u] >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((unsigned)mask[u], 0u))] = r[u];
+    at += __popcll(mask[u]);
   }
 }
 
@@ -454,33 +543,35 @@ __device__ __forceinline__ void bfs_offer(int32_t r, int32_t k, const uint32_t* 
 // EWiseMult(exclude) filter: each frontier vertex k offers k to its unvisited
 // neighbours; cand[i] keeps the largest offer; the first offer appends i.
 template <int NT, int U>
-__global__ __launch_bounds__(NT) void k_bfs_expand(const int64_t* __restrict__ beg, const int64_t* __restrict__ end,
-                                                   const int32_t* __restrict__ rows, const int32_t* __restrict__ fin,
+__global__ __launch_bounds__(NT) void k_bfs_expand(const int2* __restrict__ range, const int32_t* __restrict__ rows,
+                                                   const int32_t* __restrict__ fin,
                                                    const int32_t* __restrict__ fin_count,
                                                    const uint32_t* __restrict__ visited, int32_t* __restrict__ cand,
                                                    int32_t* __restrict__ fout, int32_t* __restrict__ fout_count) {
-  __shared__ SegStage<int32_t, NT> st;
-  __shared__ long long wsum[NT / kWave];
+  __shared__ FlatStage<int32_t, NT, true> st;
   const int nf = *fin_count;
+  if ((int)blockIdx.x * NT >= nf) return;
+  flat_init(st);
+  int par = 0;
   for (int c0 = blockIdx.x * NT; c0 < nf; c0 += gridDim.x * NT) {
     const int t = c0 + threadIdx.x;
-    int64_t base = 0;
-    int len = 0;
+    int base = 0, len = 0;
     int32_t k = 0;
     if (t < nf) {
       k = fin[t];
-      base = beg[k];
-      len = (int)(end[k] - base);
+      const int2 rg = range[k];
+      base = rg.x;
+      len = rg.y - rg.x;
       if (len > kBfsHub) len = 0;  // a hub: k_bfs_expand_hubs takes its pieces
     }
-    int nseg;
-    const int tot = stage_chunk<int32_t, NT>(st, wsum, base, len, k, nseg);
-    visit_staged<int32_t, NT, U>(st, nseg, tot, [&](const int64_t(&idx)[U], const int32_t(&ks)[U]) {
+    const FlatSeg me = flat_stage<int32_t, NT, true>(st, base, len, k);
+    flat_chunk<int32_t, NT, true, U>(st, me, par, [&](const int32_t(&idx)[U], int32_t(&ks)[U], const bool(&ok)[U]) {
       int32_t r[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) r[u] = idx[u] >= 0 ? rows[idx[u]] : -1;
+      for (int u = 0; u < U; ++u) r[u] = rows[idx[u]];
 #pragma unroll
-      for (int u = 0; u < U; ++u) bfs_offer(r[u], ks[u], visited, cand, fout, fout_count);
+      for (int u = 0; u < U; ++u) pin(r[u]);
+      bfs_offer<U>(r, ks, ok, visited, cand, fout, fout_count);
     });
   }
 }
@@ -488,8 +579,7 @@ __global__ __launch_bounds__(NT) void k_bfs_expand(const int64_t* __restrict__ b
 // The hubs' pieces of the same level: one workgroup per piece of kBfsHub
 // consecutive edges (coalesced row reads, kBfsHub / NT edges per thread).
 template <int NT>
-__global__ __launch_bounds__(NT) void k_bfs_expand_hubs(const int64_t* __restrict__ beg,
-                                                        const int64_t* __restrict__ end,
+__global__ __launch_bounds__(NT) void k_bfs_expand_hubs(const int2* __restrict__ range,
                                                         const int32_t* __restrict__ rows,
                                                         const long long* __restrict__ pieces,
                                                         const int32_t* __restrict__ pcount,
@@ -497,138 +587,273 @@ __global__ __launch_bounds__(NT) void k_bfs_expand_hubs(const int64_t* __restric
                                                         int32_t* __restrict__ cand, int32_t* __restrict__ fout,
                                                         int32_t* __restrict__ fout_count) {
   static_assert(kBfsHub % NT == 0, "whole rounds per piece");
+  constexpr int U = kBfsHub / NT;
   const int np = *pcount;
   for (int p = blockIdx.x; p < np; p += gridDim.x) {
     const long long pc = pieces[p];
     const int32_t v = (int32_t)(pc >> 32);
-    const int64_t k = pc & 0xffffffffll;
-    const int64_t e0 = beg[v] + k * kBfsHub, e1 = min(end[v], e0 + kBfsHub);
+    const int2 rg = range[v];
+    const int e0 = rg.x + (int)((pc & 0xffffffffll) * kBfsHub);
+    int32_t r[U], ks[U];
+    bool ok[U];
 #pragma unroll
-    for (int64_t e = e0 + threadIdx.x; e < e0 + kBfsHub; e += NT)  // uniform trip count (ballots inside)
-      bfs_offer(e < e1 ? rows[e] : -1, v, visited, cand, fout, fout_count);
+    for (int u = 0; u < U; ++u) {
+      const int e = e0 + u * NT + (int)threadIdx.x;
+      ok[u] = e < rg.y;
+      ks[u] = v;
+      r[u] = rows[min(e, rg.y - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) pin(r[u]);
+    bfs_offer<U>(r, ks, ok, visited, cand, fout, fout_count);
   }
 }
 
 // parents.Set(fringe) (FullyDistVec.cpp:1036) and the visited mark; also
-// sums the new frontier's degrees (the host's direction choice), one atomic
-// per workgroup.
+// counts the new frontier and its edges (the host's direction choice).
 constexpr int kBfsFinNT = 256;
 __global__ __launch_bounds__(kBfsFinNT) void k_bfs_finalize(const int32_t* __restrict__ f,
                                                             const int32_t* __restrict__ count,
                                                             const int32_t* __restrict__ cand,
-                                                            const int64_t* __restrict__ beg,
-                                                            const int64_t* __restrict__ end,
+                                                            const int2* __restrict__ range,
                                                             int64_t* __restrict__ parents,
-                                                            uint32_t* __restrict__ visited,
-                                                            unsigned long long* __restrict__ edges,
-                                                            unsigned long long* __restrict__ reached,
+                                                            uint32_t* __restrict__ visited, BfsState* st,
                                                             int32_t* __restrict__ pcount,
                                                             long long* __restrict__ pieces) {
-  __shared__ long long ws[kBfsFinNT / kWave];
   const int nf = *count;
-  if (blockIdx.x == 0 && threadIdx.x == 0 && nf) atomicAdd(reached, (unsigned long long)nf);
+  if ((int)blockIdx.x * kBfsFinNT >= nf) return;
   long long deg = 0;
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nf; t += gridDim.x * blockDim.x) {
+  for (int t = blockIdx.x * kBfsFinNT + threadIdx.x; t < nf; t += gridDim.x * kBfsFinNT) {
     const int32_t i = f[t];
     parents[i] = cand[i];
     atomicOr(&visited[i >> 5], 1u << (i & 31));
-    const int64_t d = end[i] - beg[i];
+    const int2 rg = range[i];
+    const int d = rg.y - rg.x;
     deg += d;
     if (d > kBfsHub) bfs_add_pieces(i, d, pcount, pieces);  // the next level expands hubs in pieces
   }
-  deg = wave_sum_ll(deg);
-  if (lane_id() == 0) ws[wave_id()] = deg;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    long long d = 0;
-    for (int w = 0; w < kBfsFinNT / kWave; ++w) d += ws[w];
-    if (d) atomicAdd(edges, (unsigned long long)d);
-  }
+  bfs_count<kBfsFinNT>(st, blockIdx.x == 0 && threadIdx.x == 0 ? nf : 0, deg);
 }
 
-// Bottom-up form of the same level (for large frontiers): the frontier as a
-// bitmap, then every unvisited vertex scans its neighbours from the largest
-// index down and stops at the first one in the frontier -- the largest
-// frontier neighbour, the value SelectMax's atomic max gives top-down, so
-// both forms produce the same parents and next frontier.
-__global__ void k_bfs_fbits_clear(uint32_t* __restrict__ fbits, int64_t nw) {
+// A frontier between its two forms: the list as a bitmap, and back.
+__global__ void k_bfs_bits_clear(unsigned long long* __restrict__ bits, int64_t nw) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < nw) fbits[i] = 0u;
+  if (i < nw) bits[i] = 0ull;
 }
 
-__global__ void k_bfs_fbits_set(const int32_t* __restrict__ f, const int32_t* __restrict__ count,
-                                uint32_t* __restrict__ fbits) {
+__global__ void k_bfs_bits_set(const int32_t* __restrict__ f, const int32_t* __restrict__ count,
+                               uint32_t* __restrict__ bits) {
   const int nf = *count;
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nf; t += gridDim.x * blockDim.x)
-    atomicOr(&fbits[f[t] >> 5], 1u << (f[t] & 31));
+    atomicOr(&bits[f[t] >> 5], 1u << (f[t] & 31));
 }
 
-// Vertices of degree above kBfsSerialDeg are scanned by the whole wave, 64
-// neighbours per step from the top (hubs would stall a lane for thousands of
-// steps); the first step with a hit gives the largest frontier neighbour.
-constexpr int64_t kBfsSerialDeg = 64;
-
-__global__ __launch_bounds__(256) void k_bfs_bottom_up(const int64_t* __restrict__ beg,
-                                                       const int64_t* __restrict__ end,
-                                                       const int32_t* __restrict__ rows, int64_t n,
-                                                       const uint32_t* __restrict__ fbits,
-                                                       const uint32_t* __restrict__ visited,
-                                                       int32_t* __restrict__ cand, int32_t* __restrict__ fout,
-                                                       int32_t* __restrict__ fout_count) {
-  const int lane = lane_id();
-  for (int64_t v0 = blockIdx.x * (int64_t)blockDim.x; v0 < n; v0 += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t v = v0 + threadIdx.x;  // the loop bound is uniform per wave (ballots below)
-    bool push = false, heavy = false;
-    int64_t b = 0, e = 0;
-    if (v < n && !((visited[v >> 5] >> (v & 31)) & 1u)) {
-      b = beg[v];
-      e = end[v];
-      if (e - b > kBfsSerialDeg) {
-        heavy = true;
-      } else {
-        for (int64_t i = e - 1; i >= b; --i) {
-          const int32_t u = rows[i];
-          if ((fbits[u >> 5] >> (u & 31)) & 1u) {
-            cand[v] = u;
-            push = true;
-            break;
-          }
-        }
-      }
-    }
-    uint64_t hv = __ballot(heavy);
-    while (hv) {  // the wave's high-degree vertices, one at a time
-      const int h = __ffsll((unsigned long long)hv) - 1;
-      hv &= hv - 1;
-      const int64_t hb = __shfl(b, h, kWave), he = __shfl(e, h, kWave);
-      for (int64_t top = he; top > hb; top -= kWave) {
-        const int64_t i = top - 1 - lane;  // lane 0 holds the largest index of the step
-        int32_t u = -1;
-        if (i >= hb) {
-          u = rows[i];
-          if (!((fbits[u >> 5] >> (u & 31)) & 1u)) u = -1;
-        }
-        const uint64_t hit = __ballot(u >= 0);
-        if (hit) {
-          const int first = __ffsll((unsigned long long)hit) - 1;
-          const int32_t par = __shfl(u, first, kWave);
-          if (lane == h) {
-            cand[v] = par;
-            push = true;
-          }
-          break;
-        }
-      }
-    }
-    const uint64_t mask = __ballot(push);
-    if (mask) {
-      const int leader = __ffsll((unsigned long long)mask) - 1;
-      int basei = 0;
-      if (lane == leader) basei = atomicAdd(fout_count, __popcll(mask));
-      basei = __shfl(basei, leader, kWave);
-      if (push) fout[basei + __popcll(mask & ((1ull << lane) - 1ull))] = (int32_t)v;
+// (The frontiers that go back to a list are small: most words are empty.)
+__global__ __launch_bounds__(256) void k_bfs_bits_list(const unsigned long long* __restrict__ bits, int64_t nw,
+                                                       const int2* __restrict__ range, int32_t* __restrict__ f,
+                                                       int32_t* __restrict__ count, int32_t* __restrict__ pcount,
+                                                       long long* __restrict__ pieces) {
+  const int64_t w0 = global_wave() * kWave;
+  const int64_t i = w0 + lane_id();
+  const unsigned long long mine = i < nw ? bits[i] : 0ull;
+  unsigned long long some = __ballot(mine != 0ull);
+  while (some) {
+    const int j = __ffsll(some) - 1;
+    some &= some - 1;
+    const unsigned long long word = (unsigned long long)readlane_ll((long long)mine, j);
+    int at = 0;
+    if (lane_id() == 0) at = atomicAdd(count, __popcll(word));
+    at = __builtin_amdgcn_readfirstlane(at);
+    if ((word >> lane_id()) & 1ull) {
+      const int32_t v = (int32_t)((w0 + j) * kWave) + lane_id();
+      f[at + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(word >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)word, 0u))] = v;
+      const int2 rg = range[v];
+      if (rg.y - rg.x > kBfsHub) bfs_add_pieces(v, rg.y - rg.x, pcount, pieces);
     }
   }
+}
+
+// Eight consecutive rows from an address of any 4-byte alignment.
+struct __attribute__((packed, aligned(4))) BfsRows {
+  int32_t r[8];
+};
+constexpr int kBfsBatch = 8;
+
+// Bottom-up form of the same level (for large frontiers): every unvisited
+// vertex scans its neighbours from the largest index down and stops at the
+// first one in the frontier -- the largest frontier neighbour, the value
+// SelectMax's atomic max gives top-down, so both forms produce the same
+// parents and next frontier.
+//
+// A scan is a chain of two loads (a row, its bit) per step: bound by their
+// latency, and by the longest scan of the slowest wave, as vertices with many
+// neighbours lie next to each other in skewed graphs.  k_bfs_bottom_up gives a
+// vertex with at most kBfsSerialDeg neighbours to a lane, eight a step, and
+// lists the others; k_bfs_bottom_up_long spreads those evenly: sixteen lanes
+// and 128 neighbours a step, four vertices at once, up to kBfsWaveDeg (from the
+// list's front), the whole wave and 512 a step above (from its end).
+//
+// R-MAT s20, 31 M edges, the first bottom-up level: 386 us with one neighbour a
+// step per lane (64 for a wave above 64 neighbours), 164 with the batches alone
+// (the slowest waves then scanned 64 vertices of some 1000 neighbours), 36 + 46
+// with the list; a level that finds little 9 + 3.  Workgroups of 256 lose more
+// to their atomics on the list's ends (55 + 46) than those of 1024 to their
+// barriers (36 + 46, but 13 + 4); scan lengths of 16 and 64 for a lane gave
+// 32 + 49 and 60 + 34.  A copy of the frontier's bitmap in LDS did not pay: the
+// lookups are not what bounds it.
+constexpr int kBfsSerialDeg = 32, kBfsWaveDeg = 512;
+constexpr int kBfsUpNT = 512;
+constexpr unsigned kBfsUpGrid = 4096, kBfsLongGrid = 1024;
+
+// Which of a lane's neighbours r[u] are in the frontier.
+template <int U>
+__device__ __forceinline__ void bfs_lookup(const uint32_t* __restrict__ fin, const int32_t (&r)[U], bool (&in)[U]) {
+  uint32_t word[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) word[u] = fin[r[u] >> 5];
+#pragma unroll
+  for (int u = 0; u < U; ++u) pin(word[u]);
+#pragma unroll
+  for (int u = 0; u < U; ++u) in[u] = (word[u] >> (r[u] & 31)) & 1u;
+}
+
+// A wave has the 64 vertices of one word of the bitmaps: it marks what it found
+// visited, writes the next frontier's word and counts without atomics.
+__global__ __launch_bounds__(kBfsUpNT) void k_bfs_bottom_up(const int2* __restrict__ range,
+                                                            const int32_t* __restrict__ rows, int64_t n, int64_t nw,
+                                                            const uint32_t* __restrict__ fin,
+                                                            unsigned long long* __restrict__ fout,
+                                                            unsigned long long* __restrict__ visited,
+                                                            int64_t* __restrict__ parents,
+                                                            int32_t* __restrict__ longs, BfsState* st) {
+  constexpr int NW = kBfsUpNT / kWave;
+  __shared__ int wsum[NW];
+  __shared__ int s_at[2];
+  const int lane = lane_id();
+  long long found = 0, edges = 0;
+  for (int64_t w0 = (int64_t)blockIdx.x * NW; w0 < nw; w0 += (int64_t)gridDim.x * NW) {
+    const int64_t w = w0 + wave_id_uniform();
+    const unsigned long long vis = w < nw ? visited[w] : ~0ull;  // (vertices from n on count as visited)
+    const int64_t v = w * kWave + lane;
+    int b = 0, e = 0;
+    if (~vis) {
+      const int2 rg = range[min(v, n - 1)];
+      b = rg.x;
+      e = ((vis >> lane) & 1ull) ? rg.x : rg.y;
+    }
+    int32_t par = -1;
+    if (e - b <= kBfsSerialDeg) {
+      for (int i = e; i > b && par < 0; i -= kBfsBatch) {
+        const int s = max(i - kBfsBatch, 0);  // rows has kBfsBatch entries more than the matrix
+        const BfsRows a = *(const BfsRows*)(rows + s);
+        bool in[kBfsBatch];
+        bfs_lookup(fin, a.r, in);
+#pragma unroll
+        for (int j = 0; j < kBfsBatch; ++j)
+          if (s + j >= b && s + j < i && in[j]) par = a.r[j];
+      }
+    }
+    const unsigned long long next = __ballot(par >= 0);
+    if (par >= 0) {
+      parents[v] = par;
+      edges += e - b;
+    }
+    if (lane == 0 && w < nw) {
+      fout[w] = next;
+      if (next) visited[w] = vis | next;
+      found += __popcll(next);
+    }
+    // the vertices left to k_bfs_bottom_up_long
+    const int kind = e - b <= kBfsSerialDeg ? 0 : e - b <= kBfsWaveDeg ? 1 : 1 << 16;
+    int total;
+    const int at = block_excl_scan<kBfsUpNT>(kind, wsum, total);
+    if (total == 0) continue;
+    if (threadIdx.x == 0) {
+      s_at[0] = atomicAdd(&st->longs[0], total & 0xffff);
+      s_at[1] = total >> 16 ? atomicAdd(&st->longs[1], total >> 16) : 0;
+    }
+    __syncthreads();
+    if (kind == 1) longs[s_at[0] + (at & 0xffff)] = (int32_t)v;
+    if (kind > 1) longs[n - 1 - s_at[1] - (at >> 16)] = (int32_t)v;
+    __syncthreads();
+  }
+  bfs_count<kBfsUpNT>(st, found, edges);
+}
+
+__global__ __launch_bounds__(kBfsUpNT) void k_bfs_bottom_up_long(const int2* __restrict__ range,
+                                                                 const int32_t* __restrict__ rows, int64_t n,
+                                                                 const uint32_t* __restrict__ fin,
+                                                                 uint32_t* __restrict__ fout,
+                                                                 uint32_t* __restrict__ visited,
+                                                                 int64_t* __restrict__ parents,
+                                                                 const int32_t* __restrict__ longs, BfsState* st) {
+  constexpr int U = 8, G = 16;
+  const int nmid = st->longs[0], nbig = st->longs[1];
+  const int lane = lane_id(), g = lane / G;
+  const int nwaves = gridDim.x * (kBfsUpNT / kWave);
+  const int wave = wave_id_uniform() * gridDim.x + blockIdx.x;
+  long long found = 0, edges = 0;
+  auto set = [&](int32_t v, int32_t par, int deg) {
+    parents[v] = par;
+    atomicOr(&fout[v >> 5], 1u << (v & 31));
+    atomicOr(&visited[v >> 5], 1u << (v & 31));
+    ++found;
+    edges += deg;
+  };
+  // one vertex at a time
+  for (int i = wave; i < nbig; i += nwaves) {
+    const int32_t v = longs[n - 1 - i];
+    const int2 rg = range[v];
+    int32_t got = -1;
+    for (int top = rg.y; top > rg.x && got < 0; top -= U * kWave) {
+      int32_t u[U];
+      bool in[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) u[k] = rows[max(top - 1 - k * kWave - lane, rg.x)];
+#pragma unroll
+      for (int k = 0; k < U; ++k) pin(u[k]);
+      bfs_lookup(fin, u, in);
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const unsigned long long hits = __ballot(in[k]);
+        if (got < 0 && hits) got = __builtin_amdgcn_readlane(u[k], __ffsll(hits) - 1);
+      }
+    }
+    if (got >= 0 && lane == 0) set(v, got, rg.y - rg.x);
+  }
+  // four vertices at a time
+  for (int i = wave * 4; i < nmid; i += nwaves * 4) {
+    const bool mine = i + g < nmid;
+    const int32_t v = longs[min(i + g, nmid - 1)];
+    const int2 rg = range[v];
+    int top = mine ? rg.y : rg.x;
+    int32_t got = -1;
+    while (__ballot(top > rg.x)) {
+      int32_t u[U];
+      bool in[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) u[k] = rows[max(top - 1 - k * G - (lane & (G - 1)), rg.x)];
+#pragma unroll
+      for (int k = 0; k < U; ++k) pin(u[k]);
+      bfs_lookup(fin, u, in);
+      const bool live = top > rg.x;
+      int32_t first = -1;
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        // (past the list's end a lane has its first entry again)
+        const unsigned hits = (unsigned)(__ballot(live && in[k]) >> (g * G)) & 0xffffu;
+        const int32_t r = __shfl(u[k], g * G + (hits ? __ffs(hits) - 1 : 0), kWave);
+        if (first < 0 && hits) first = r;
+      }
+      top -= U * G;
+      if (first >= 0) {
+        got = first;
+        top = rg.x;
+      }
+    }
+    if (got >= 0 && (lane & (G - 1)) == 0) set(v, got, rg.y - rg.x);
+  }
+  bfs_count<kBfsUpNT>(st, found, edges);
 }
 
 }  // namespace
@@ -638,28 +863,25 @@ __global__ __launch_bounds__(256) void k_bfs_bottom_up(const int64_t* __restrict
 using namespace cbx;
 
 struct cbx_bfs_plan_s {
-  int64_t n = 0, nnz = 0, nw = 0;
+  int64_t n = 0, nnz = 0, nw = 0;  // nw: 64-bit words of a bitmap
   hipStream_t stream = nullptr;
-  int64_t *beg = nullptr, *end = nullptr, *parents = nullptr;
-  int32_t *rows = nullptr, *f[2] = {nullptr, nullptr}, *counts = nullptr;
-  int32_t* pcount = nullptr;                  // hub pieces of the two frontier buffers
-  long long* pieces[2] = {nullptr, nullptr};
+  hipEvent_t ev[2] = {nullptr, nullptr};  // around a run
+  int2* range = nullptr;
+  int64_t* parents = nullptr;
+  int32_t *rows = nullptr, *f[2] = {nullptr, nullptr};
+  long long* pieces[2] = {nullptr, nullptr};  // hub pieces of the two frontier lists
   int32_t* cand = nullptr;  // the largest offer per vertex (vertex ids fit 32 bits: n < 2^31)
-  uint32_t* visited = nullptr;
-  unsigned long long* edges = nullptr;  // degree sums of the two frontier buffers
-  uint32_t* fbits = nullptr;             // frontier bitmap of a bottom-up level
-  unsigned long long* stat = nullptr;  // device: levels, vertices reached
-  // pinned, 64 B: next frontier size; [2..3] its degree sum; [4..7] root's
-  // range; [8..11] the device statistics
-  int32_t* host_count = nullptr;
+  unsigned long long *visited = nullptr, *isolated = nullptr, *bits[2] = {nullptr, nullptr};
+  BfsState* state = nullptr;
+  BfsReport* report = nullptr;  // pinned
   int direction = CBX_BFS_DIRECTION_OPTIMIZING;
   // Pattern of A equal to that of its transpose.  Bottom-up levels scan column
   // v of A for frontier rows, which is row v only for a symmetric pattern, so
   // a plan over a directed graph runs every level top-down.
   bool symmetric = true;
-  // [direction (0 top-down, 1 bottom-up)][frontier parity]
-  hipGraph_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
-  hipGraphExec_t exec[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
+  // [the frontier comes as: 0 list, 1 bitmap][direction (0 top-down, 1 bottom-up)][frontier parity]
+  hipGraph_t graph[2][2][2] = {};
+  hipGraphExec_t exec[2][2][2] = {};
   // top-down only: kBfsTdLevels consecutive levels in one graph, launched
   // until the frontier is empty (levels after the last one do nothing)
   hipGraph_t td_graph = nullptr;
@@ -668,21 +890,19 @@ struct cbx_bfs_plan_s {
 
 static void bfs_plan_free(cbx_bfs_plan_s* p) {
   if (!p) return;
-  for (int d = 0; d < 2; ++d)
-    for (int i = 0; i < 2; ++i) {
-      if (p->exec[d][i]) (void)hipGraphExecDestroy(p->exec[d][i]);
-      if (p->graph[d][i]) (void)hipGraphDestroy(p->graph[d][i]);
-    }
+  for (int i = 0; i < 8; ++i) {
+    if (p->exec[i >> 2][(i >> 1) & 1][i & 1]) (void)hipGraphExecDestroy(p->exec[i >> 2][(i >> 1) & 1][i & 1]);
+    if (p->graph[i >> 2][(i >> 1) & 1][i & 1]) (void)hipGraphDestroy(p->graph[i >> 2][(i >> 1) & 1][i & 1]);
+  }
   if (p->td_exec) (void)hipGraphExecDestroy(p->td_exec);
   if (p->td_graph) (void)hipGraphDestroy(p->td_graph);
-  for (int i = 0; i < 2; ++i) {
-    if (p->f[i]) (void)hipFree(p->f[i]);
-    if (p->pieces[i]) (void)hipFree(p->pieces[i]);
-  }
-  for (void* q : {(void*)p->beg, (void*)p->end, (void*)p->parents, (void*)p->rows, (void*)p->counts, (void*)p->cand,
-                  (void*)p->visited, (void*)p->edges, (void*)p->fbits, (void*)p->stat, (void*)p->pcount})
+  for (void* q : {(void*)p->range, (void*)p->parents, (void*)p->rows, (void*)p->f[0], (void*)p->f[1],
+                  (void*)p->pieces[0], (void*)p->pieces[1], (void*)p->cand, (void*)p->visited, (void*)p->isolated,
+                  (void*)p->bits[0], (void*)p->bits[1], (void*)p->state})
     if (q) (void)hipFree(q);
-  if (p->host_count) (void)hipHostFree(p->host_count);
+  if (p->report) (void)hipHostFree(p->report);
+  for (hipEvent_t e : p->ev)
+    if (e) (void)hipEventDestroy(e);
   if (p->stream) (void)hipStreamDestroy(p->stream);
   delete p;
 }
@@ -692,6 +912,38 @@ constexpr unsigned kBfsGrid = 2048;
 constexpr unsigned kBfsHubGrid = 2048;  // workgroups over the hubs' pieces
 constexpr int64_t kBfsAlpha = 256;
 constexpr int kBfsTdLevels = 8;  // even: the frontier parity is 0 again after one top-down graph
+
+// One level from frontier `par` (a list, or a bitmap where `bits`) to 1 - par.
+static void bfs_level(cbx_bfs_plan_s* p, bool bits, bool bottom_up, int par, hipStream_t s) {
+  BfsState* st = p->state;
+  int32_t *cin = &st->listed[par], *cout = &st->listed[1 - par];
+  const unsigned words = nb(p->nw, 256);
+  if (bottom_up) {
+    if (!bits) {
+      k_bfs_bits_clear<<<words, 256, 0, s>>>(p->bits[par], p->nw);
+      k_bfs_bits_set<<<256, 256, 0, s>>>(p->f[par], cin, (uint32_t*)p->bits[par]);
+    }
+    const unsigned g = std::min(nb(p->nw * kWave, kBfsUpNT), kBfsUpGrid);
+    const uint32_t* fin = (const uint32_t*)p->bits[par];
+    int32_t* longs = p->f[1 - par];  // (free: the next frontier is a bitmap)
+    k_bfs_bottom_up<<<g, kBfsUpNT, 0, s>>>(p->range, p->rows, p->n, p->nw, fin, p->bits[1 - par], p->visited,
+                                           p->parents, longs, st);
+    k_bfs_bottom_up_long<<<kBfsLongGrid, kBfsUpNT, 0, s>>>(p->range, p->rows, p->n, fin, (uint32_t*)p->bits[1 - par],
+                                                           (uint32_t*)p->visited, p->parents, longs, st);
+  } else {
+    if (bits)
+      k_bfs_bits_list<<<words, 256, 0, s>>>(p->bits[par], p->nw, p->range, p->f[par], cin, &st->pieces[par],
+                                            p->pieces[par]);
+    k_bfs_expand<kBfsNT, 4><<<kBfsGrid, kBfsNT, 0, s>>>(p->range, p->rows, p->f[par], cin,
+                                                       (const uint32_t*)p->visited, p->cand, p->f[1 - par], cout);
+    k_bfs_expand_hubs<kBfsNT><<<kBfsHubGrid, kBfsNT, 0, s>>>(p->range, p->rows, p->pieces[par], &st->pieces[par],
+                                                             (const uint32_t*)p->visited, p->cand, p->f[1 - par],
+                                                             cout);
+    k_bfs_finalize<<<256, kBfsFinNT, 0, s>>>(p->f[1 - par], cout, p->cand, p->range, p->parents,
+                                             (uint32_t*)p->visited, st, &st->pieces[1 - par], p->pieces[1 - par]);
+  }
+  k_bfs_level_end<<<1, kWave, 0, s>>>(st, par, bottom_up, p->report);
+}
 
 extern "C" cbx_status cbx_bfs_plan_create(const cbx_dcsc* A, cbx_bfs_plan_s** out) {
   CBX_RETURN_IF(!A || !out, CBX_ERR_INVALID, "cbx_bfs_plan_create: null argument");
@@ -735,78 +987,45 @@ extern "C" cbx_status cbx_bfs_plan_create(const cbx_dcsc* A, cbx_bfs_plan_s** ou
   p->symmetric = symmetric;
   p->n = A->n;
   p->nnz = A->nnz;
-  p->nw = A->n / 32 + 1;
+  p->nw = A->n / kWave + 1;
   auto fail = [&](const char* what) {
     bfs_plan_free(p);
     return set_error(CBX_ERR_HIP, "cbx_bfs_plan_create: %s", what);
   };
-  if (hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking) != hipSuccess) return fail("stream");
+  if (hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking) != hipSuccess ||
+      hipEventCreate(&p->ev[0]) != hipSuccess || hipEventCreate(&p->ev[1]) != hipSuccess)
+    return fail("stream");
   const int64_t n = p->n;
   // every hub of a frontier contributes ceil(deg / kBfsHub) <= 2 deg / kBfsHub pieces
   const int64_t max_pieces = 2 * p->nnz / kBfsHub + 2;
-  if (hipMalloc(&p->beg, 8 * std::max<int64_t>(n, 1)) || hipMalloc(&p->end, 8 * std::max<int64_t>(n, 1)) ||
-      hipMalloc(&p->parents, 8 * std::max<int64_t>(n, 1)) || hipMalloc(&p->rows, 4 * std::max<int64_t>(p->nnz, 1)) ||
-      hipMalloc(&p->f[0], 4 * std::max<int64_t>(n, 1)) || hipMalloc(&p->f[1], 4 * std::max<int64_t>(n, 1)) ||
-      hipMalloc(&p->counts, 16) || hipMalloc(&p->cand, sizeof(int32_t) * std::max<int64_t>(n, 1)) ||
-      hipMalloc(&p->visited, 4 * p->nw) || hipMalloc(&p->edges, 2 * sizeof(unsigned long long)) ||
-      hipMalloc(&p->fbits, 4 * p->nw) || hipMalloc(&p->stat, 2 * sizeof(unsigned long long)) ||
-      hipMalloc(&p->pcount, 2 * sizeof(int32_t)) || hipMalloc(&p->pieces[0], 8 * max_pieces) ||
-      hipMalloc(&p->pieces[1], 8 * max_pieces) ||
-      hipHostMalloc(&p->host_count, 64, hipHostMallocDefault))
+  const int64_t n1 = std::max<int64_t>(n, 1);
+  if (hipMalloc(&p->range, 8 * n1) || hipMalloc(&p->parents, 8 * n1) ||
+      hipMalloc(&p->rows, 4 * (p->nnz + kBfsBatch)) || hipMalloc(&p->f[0], 4 * n1) || hipMalloc(&p->f[1], 4 * n1) ||
+      hipMalloc(&p->cand, 4 * n1) || hipMalloc(&p->visited, 8 * p->nw) || hipMalloc(&p->isolated, 8 * p->nw) ||
+      hipMalloc(&p->bits[0], 8 * p->nw) || hipMalloc(&p->bits[1], 8 * p->nw) ||
+      hipMalloc(&p->pieces[0], 8 * max_pieces) || hipMalloc(&p->pieces[1], 8 * max_pieces) ||
+      hipMalloc(&p->state, sizeof(BfsState)) || hipHostMalloc(&p->report, sizeof(BfsReport), hipHostMallocDefault))
     return fail("allocation");
   hipStream_t s = p->stream;
-  if (hipMemsetAsync(p->beg, 0, 8 * n, s) || hipMemsetAsync(p->end, 0, 8 * n, s)) return fail("memset");
-  k_bfs_dense_cp<<<nb(A->nzc, 256), 256, 0, s>>>(A->cp, A->jc, A->nzc, n, p->beg, p->end);
-  k_bfs_rows32<<<nb(A->nnz, 256), 256, 0, s>>>(A->ir, A->nnz, p->rows);
-  if (hipStreamSynchronize(s) != hipSuccess) return fail("setup kernels");
-  // one graph per (direction, frontier parity): clear the next count, the
-  // level's kernels, finalize, copy the next count and degree sum to pinned
-  // host memory
-  const unsigned bu_grid = (unsigned)std::min<int64_t>(std::max<int64_t>((n + 255) / 256, 1), 8192);
-  for (int dir = 0; dir < 2; ++dir)
-    for (int par = 0; par < 2; ++par) {
-      int32_t* cin = p->counts + par;
-      int32_t* cout = p->counts + (1 - par);
-      unsigned long long* eout = p->edges + (1 - par);
-      if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) return fail("capture begin");
-      k_bfs_level_begin<<<1, 64, 0, s>>>(cin, cout, eout, p->pcount + (1 - par), p->stat);
-      if (dir == 0) {
-        k_bfs_expand<kBfsNT, 4><<<kBfsGrid, kBfsNT, 0, s>>>(p->beg, p->end, p->rows, p->f[par], cin, p->visited,
-                                                           p->cand, p->f[1 - par], cout);
-        k_bfs_expand_hubs<kBfsNT><<<kBfsHubGrid, kBfsNT, 0, s>>>(p->beg, p->end, p->rows, p->pieces[par],
-                                                                 p->pcount + par, p->visited, p->cand,
-                                                                 p->f[1 - par], cout);
-      } else {
-        k_bfs_fbits_clear<<<nb(p->nw, 256), 256, 0, s>>>(p->fbits, p->nw);
-        k_bfs_fbits_set<<<256, 256, 0, s>>>(p->f[par], cin, p->fbits);
-        k_bfs_bottom_up<<<bu_grid, 256, 0, s>>>(p->beg, p->end, p->rows, n, p->fbits, p->visited, p->cand,
-                                                p->f[1 - par], cout);
-      }
-      k_bfs_finalize<<<256, kBfsFinNT, 0, s>>>(p->f[1 - par], cout, p->cand, p->beg, p->end, p->parents, p->visited,
-                                               eout, p->stat + 1, p->pcount + (1 - par), p->pieces[1 - par]);
-      (void)hipMemcpyAsync(p->host_count, cout, sizeof(int32_t), hipMemcpyDeviceToHost, s);
-      (void)hipMemcpyAsync(p->host_count + 2, eout, sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
-      if (hipStreamEndCapture(s, &p->graph[dir][par]) != hipSuccess) return fail("capture end");
-      if (hipGraphInstantiate(&p->exec[dir][par], p->graph[dir][par], nullptr, nullptr, 0) != hipSuccess)
-        return fail("graph instantiate");
-    }
+  if (hipMemsetAsync(p->range, 0, 8 * n, s) || hipMemsetAsync(p->rows + p->nnz, 0, 4 * kBfsBatch, s))
+    return fail("memset");
+  if (A->nzc) k_bfs_ranges<<<nb(A->nzc, 256), 256, 0, s>>>(A->cp, A->jc, A->nzc, p->range);
+  if (A->nnz) k_bfs_rows32<<<nb(A->nnz, 256), 256, 0, s>>>(A->ir, A->nnz, p->rows);
+  k_bfs_isolated<<<nb(p->nw, 4), 256, 0, s>>>(p->range, n, p->nw, symmetric, p->isolated);
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) return fail("setup kernels");
+  // one graph per form of the frontier, direction and parity
+  for (int i = 0; i < 8; ++i) {
+    const int from = i >> 2, dir = (i >> 1) & 1, par = i & 1;
+    if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) return fail("capture begin");
+    bfs_level(p, from, dir, par, s);
+    if (hipStreamEndCapture(s, &p->graph[from][dir][par]) != hipSuccess) return fail("capture end");
+    if (hipGraphInstantiate(&p->exec[from][dir][par], p->graph[from][dir][par], nullptr, nullptr, 0) != hipSuccess)
+      return fail("graph instantiate");
+  }
   // kBfsTdLevels top-down levels in one graph, no host round trip between
   // them; the host reads the frontier size once per graph
   if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) return fail("capture begin");
-  for (int l = 0; l < kBfsTdLevels; ++l) {
-    const int par = l & 1;
-    int32_t* cin = p->counts + par;
-    int32_t* cout = p->counts + (1 - par);
-    unsigned long long* eout = p->edges + (1 - par);
-    k_bfs_level_begin<<<1, 64, 0, s>>>(cin, cout, eout, p->pcount + (1 - par), p->stat);
-    k_bfs_expand<kBfsNT, 4><<<kBfsGrid, kBfsNT, 0, s>>>(p->beg, p->end, p->rows, p->f[par], cin, p->visited, p->cand,
-                                                       p->f[1 - par], cout);
-    k_bfs_expand_hubs<kBfsNT><<<kBfsHubGrid, kBfsNT, 0, s>>>(p->beg, p->end, p->rows, p->pieces[par], p->pcount + par,
-                                                             p->visited, p->cand, p->f[1 - par], cout);
-    k_bfs_finalize<<<256, kBfsFinNT, 0, s>>>(p->f[1 - par], cout, p->cand, p->beg, p->end, p->parents, p->visited,
-                                             eout, p->stat + 1, p->pcount + (1 - par), p->pieces[1 - par]);
-  }
-  (void)hipMemcpyAsync(p->host_count, p->counts, sizeof(int32_t), hipMemcpyDeviceToHost, s);
+  for (int l = 0; l < kBfsTdLevels; ++l) bfs_level(p, false, false, l & 1, s);
   if (hipStreamEndCapture(s, &p->td_graph) != hipSuccess) return fail("capture end");
   if (hipGraphInstantiate(&p->td_exec, p->td_graph, nullptr, nullptr, 0) != hipSuccess)
     return fail("graph instantiate");
@@ -818,13 +1037,11 @@ extern "C" cbx_status cbx_bfs_run(cbx_bfs_plan_s* p, int64_t root, int64_t* pare
   CBX_RETURN_IF(!p || !parents_dev, CBX_ERR_INVALID, "cbx_bfs_run: null argument");
   CBX_RETURN_IF(root < 0 || root >= p->n, CBX_ERR_INVALID, "cbx_bfs_run: root %lld out of range", (long long)root);
   hipStream_t s = p->stream;
-  hipEvent_t e0, e1;
-  CBX_HIP(hipEventCreate(&e0));
-  CBX_HIP(hipEventCreate(&e1));
-  CBX_HIP(hipEventRecord(e0, s));
-  k_bfs_reset<<<nb(std::max(p->n, p->nw), 256), 256, 0, s>>>(p->n, p->cand, p->parents, p->visited, p->nw, p->f[0],
-                                                             p->counts, p->pcount, p->pieces[0], p->beg, p->end,
-                                                             p->stat, root);
+  const volatile BfsReport* rep = p->report;
+  CBX_HIP(hipEventRecord(p->ev[0], s));
+  k_bfs_reset<<<nb(std::max<int64_t>(p->n, kBfsSlots), 256), 256, 0, s>>>(
+      p->n, p->cand, p->parents, p->visited, p->isolated, p->nw, p->f[0], p->pieces[0], p->range, p->state, p->report,
+      root);
   // direction per level: bottom-up while the frontier's edges exceed 1/256 of
   // the edges still unexplored.  (Beamer's rule compares the two with a factor
   // 14 for equal per-edge costs; here a top-down edge costs a device atomic on
@@ -836,42 +1053,37 @@ extern "C" cbx_status cbx_bfs_run(cbx_bfs_plan_s* p, int64_t root, int64_t* pare
     for (int64_t launched = 0;; launched += kBfsTdLevels) {
       CBX_HIP(hipGraphLaunch(p->td_exec, s));
       CBX_HIP(hipStreamSynchronize(s));
-      if (*(volatile int32_t*)p->host_count == 0 || launched > p->n + 1) break;
+      if (rep->size == 0 || launched > p->n + 1) break;
     }
   } else {
+    CBX_HIP(hipGetLastError());
+    CBX_HIP(hipStreamSynchronize(s));
     int levels = 0;
     int64_t mu = p->nnz;
-    int64_t* hdeg = reinterpret_cast<int64_t*>(p->host_count + 4);  // pinned: beg[root], end[root]
-    CBX_HIP(hipMemcpyAsync(hdeg, p->beg + root, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    CBX_HIP(hipMemcpyAsync(hdeg + 1, p->end + root, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    CBX_HIP(hipStreamSynchronize(s));
-    int64_t fe = hdeg[1] - hdeg[0];  // edges of the current frontier
-    bool bottom_up = p->direction == CBX_BFS_BOTTOM_UP;
+    int64_t fe = (int64_t)rep->edges;  // edges of the current frontier
+    bool bottom_up = p->direction == CBX_BFS_BOTTOM_UP, bits = false;
     for (int par = 0;; par ^= 1) {
       if (p->direction == CBX_BFS_DIRECTION_OPTIMIZING) bottom_up = fe > mu / kBfsAlpha;
-      CBX_HIP(hipGraphLaunch(p->exec[bottom_up ? 1 : 0][par], s));
+      CBX_HIP(hipGraphLaunch(p->exec[bits][bottom_up][par], s));
       CBX_HIP(hipStreamSynchronize(s));
       ++levels;
       bottom_up_levels += bottom_up;
-      const int32_t next = *(volatile int32_t*)p->host_count;
-      fe = (int64_t) * (volatile unsigned long long*)(p->host_count + 2);
+      bits = bottom_up;
+      fe = (int64_t)rep->edges;
       mu -= fe;
-      if (next == 0 || levels > p->n + 1) break;
+      if (rep->size == 0 || levels > p->n + 1) break;
     }
   }
-  unsigned long long* hstat = reinterpret_cast<unsigned long long*>(p->host_count + 8);
-  CBX_HIP(hipMemcpyAsync(hstat, p->stat, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+  const int64_t levels = (int64_t)rep->levels, reached = (int64_t)rep->reached;
   CBX_HIP(hipMemcpyAsync(parents_dev, p->parents, sizeof(int64_t) * p->n, hipMemcpyDeviceToDevice, s));
-  CBX_HIP(hipEventRecord(e1, s));
+  CBX_HIP(hipEventRecord(p->ev[1], s));
   CBX_HIP(hipStreamSynchronize(s));
   float ms = 0;
-  (void)hipEventElapsedTime(&ms, e0, e1);
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+  (void)hipEventElapsedTime(&ms, p->ev[0], p->ev[1]);
   if (stats) {
-    stats->levels = (int32_t)hstat[0];
+    stats->levels = (int32_t)levels;
     stats->bottom_up_levels = bottom_up_levels;
-    stats->reached = (int64_t)hstat[1];
+    stats->reached = reached;
     stats->ms = ms;
   }
   return CBX_OK;
