@@ -56,24 +56,39 @@ __global__ void k_col_checksum(const int64_t* __restrict__ cp, const int64_t* __
 // atomics serialise, so there are few of them (at most kCheckBlocks).
 constexpr int kCheckNT = 256, kCheckBlocks = 1024;
 
-__global__ __launch_bounds__(kCheckNT) void k_check_entries(const int64_t* __restrict__ ir, int64_t nnz, int64_t nrows,
-                                unsigned long long* __restrict__ cnt) {
-  long long bad = 0, desc = 0;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nnz; e += stride) {
-    const int64_t r = ir[e];
-    bad += r < 0 || r >= nrows;
-    if (e + 1 < nnz) desc += ir[e + 1] <= r;
+// Entries per thread and round; all of a round's loads are in flight together
+// (one at a time 64 MB of rows took 27 us).
+constexpr int kCheckPer = 8;
+
+__device__ __forceinline__ void check_entries(const int64_t* __restrict__ ir, int64_t nnz, int64_t nrows, int64_t block,
+                                              int64_t nblocks, long long& bad, long long& desc) {
+  for (int64_t e0 = block * (kCheckNT * kCheckPer); e0 < nnz; e0 += nblocks * (kCheckNT * kCheckPer)) {
+    int64_t r[kCheckPer], next[kCheckPer];
+#pragma unroll
+    for (int u = 0; u < kCheckPer; ++u) {
+      const int64_t e = e0 + u * kCheckNT + threadIdx.x;
+      r[u] = ir[min(e, nnz - 1)];
+      next[u] = ir[min(e + 1, nnz - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < kCheckPer; ++u) {
+      pin(r[u]);
+      pin(next[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kCheckPer; ++u) {
+      const int64_t e = e0 + u * kCheckNT + threadIdx.x;
+      bad += e < nnz && (r[u] < 0 || r[u] >= nrows);
+      desc += e + 1 < nnz && next[u] <= r[u];
+    }
   }
-  block_add_counts<kCheckNT>(bad, desc, &cnt[0], &cnt[1]);
 }
 
-__global__ __launch_bounds__(kCheckNT) void k_check_columns(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc,
-                                const int64_t* __restrict__ ir, int64_t nzc, int64_t nnz, int64_t ncols,
-                                unsigned long long* __restrict__ cnt) {
-  long long bad = 0, desc = 0;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < nzc; q += stride) {
+__device__ __forceinline__ void check_columns(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc,
+                                              const int64_t* __restrict__ ir, int64_t nzc, int64_t nnz, int64_t ncols,
+                                              int32_t* __restrict__ colmap, int64_t block, int64_t nblocks,
+                                              long long& bad, long long& desc) {
+  for (int64_t q = block * kCheckNT + threadIdx.x; q < nzc; q += nblocks * kCheckNT) {
     const int64_t b = cp[q], e = cp[q + 1], j = jc[q];
     bool err = b < 0 || e <= b || e > nnz || j < 0 || j >= ncols;
     if (q + 1 < nzc) err |= jc[q + 1] <= j;
@@ -83,26 +98,41 @@ __global__ __launch_bounds__(kCheckNT) void k_check_columns(const int64_t* __res
     // a column start inside the entries (a malformed cp elsewhere may still
     // put b at 0: then there is nothing before it to compare with)
     if (!err && q > 0 && b > 0) desc += ir[b] <= ir[b - 1];
+    if (colmap && !err) colmap[j] = (int32_t)q;
   }
-  block_add_counts<kCheckNT>(bad, desc, &cnt[0], &cnt[2]);
+}
+
+// The first ncol workgroups check columns (and note each column's place in
+// colmap), the others entries.
+__global__ __launch_bounds__(kCheckNT) void k_check_structure(const int64_t* __restrict__ cp,
+                                                              const int64_t* __restrict__ jc,
+                                                              const int64_t* __restrict__ ir, int64_t nzc, int64_t nnz,
+                                                              int64_t nrows, int64_t ncols, int32_t* colmap, int ncol,
+                                                              unsigned long long* __restrict__ cnt) {
+  long long bad = 0, desc = 0;
+  const bool columns = (int)blockIdx.x < ncol;
+  if (columns) check_columns(cp, jc, ir, nzc, nnz, ncols, colmap, blockIdx.x, ncol, bad, desc);
+  else check_entries(ir, nnz, nrows, blockIdx.x - ncol, gridDim.x - ncol, bad, desc);
+  block_add_counts<kCheckNT>(bad, desc, &cnt[0], columns ? &cnt[2] : &cnt[1]);
 }
 
 __global__ void k_check_zero(unsigned long long* __restrict__ cnt) {
   if (threadIdx.x < 3) cnt[threadIdx.x] = 0ull;
 }
 
-static unsigned check_blocks(int64_t n) {
-  return (unsigned)std::min<int64_t>(std::max<int64_t>((n + kCheckNT - 1) / kCheckNT, 1), kCheckBlocks);
+static unsigned check_blocks(int64_t n, int per) {
+  return (unsigned)std::min<int64_t>(std::max<int64_t>((n + kCheckNT * per - 1) / (kCheckNT * per), 1), kCheckBlocks);
+}
+
+void dcsc_check_structure_launch(const cbx_dcsc* X, unsigned long long* cnt, int32_t* colmap, hipStream_t s) {
+  const unsigned ncol = check_blocks(X->nzc, 1), nent = X->nnz > 0 ? check_blocks(X->nnz, kCheckPer) : 0;
+  k_check_structure<<<ncol + nent, kCheckNT, 0, s>>>(X->cp, X->jc, X->ir, X->nzc, X->nnz, X->m, X->n, colmap,
+                                                     (int)ncol, cnt);
 }
 
 void dcsc_check_launch(const cbx_dcsc* X, unsigned long long* cnt, hipStream_t s) {
-  dcsc_check_columns_launch(X, cnt, s);
-  if (X->nnz > 0) k_check_entries<<<check_blocks(X->nnz), kCheckNT, 0, s>>>(X->ir, X->nnz, X->m, cnt);
-}
-
-void dcsc_check_columns_launch(const cbx_dcsc* X, unsigned long long* cnt, hipStream_t s) {
   k_check_zero<<<1, 64, 0, s>>>(cnt);
-  k_check_columns<<<check_blocks(X->nzc), kCheckNT, 0, s>>>(X->cp, X->jc, X->ir, X->nzc, X->nnz, X->n, cnt);
+  dcsc_check_structure_launch(X, cnt, nullptr, s);
 }
 
 cbx_status dcsc_check_result(const unsigned long long* cnt, hipStream_t s) {

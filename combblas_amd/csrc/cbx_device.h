@@ -57,6 +57,21 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
   return v;
 }
 
+// Holds v in a register at this point, so that a load of v (and of what its
+// address comes from) is issued before it even where v is only used under a
+// condition: the compiler otherwise sinks the load into the branch, and a
+// lane's independent loads then wait for each other.
+template <class T>
+__device__ __forceinline__ void pin(T& v) {
+  if constexpr (sizeof(T) < 4) {
+    uint32_t x = (uint32_t)v;
+    asm volatile("" : "+v"(x));
+    v = (T)x;
+  } else {
+    asm volatile("" : "+v"(v));
+  }
+}
+
 // The wave's index in its workgroup, in a scalar register.
 __device__ __forceinline__ int wave_id_uniform() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 

@@ -92,99 +92,262 @@ struct GAcc<kSelectMax, float> {
 
 namespace {
 
-__global__ void k_sv_colmap(const int64_t* __restrict__ jc, int64_t nzc, int64_t n, int32_t* __restrict__ colmap) {
+// What one product's kernels count: the structure check of A (cbx_spgemm.h),
+// whether x breaks its rules, the long columns set aside, and y's entries.
+struct SpvFlags {
+  unsigned long long chk[3];
+  int bad_x, nhubs, ny;
+  __device__ __host__ bool malformed() const { return chk[0] || chk[1] != chk[2]; }
+};
+
+template <class T>
+__global__ void k_sv_begin(int32_t* __restrict__ colmap, int64_t n, T* __restrict__ acc, int64_t m, T ident,
+                           uint32_t* __restrict__ bits, int64_t nw, SpvFlags* __restrict__ f) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < n) colmap[i] = -1;
-}
-__global__ void k_sv_colmap_scatter(const int64_t* __restrict__ jc, int64_t nzc, int32_t* __restrict__ colmap) {
-  const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (p < nzc) colmap[jc[p]] = (int32_t)p;
-}
-
-template <class T>
-__global__ void k_sv_init(T* __restrict__ acc, int64_t m, T ident, uint32_t* __restrict__ bits, int64_t nw) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < m) acc[i] = ident;
   if (i < nw) bits[i] = 0u;
+  if (i == 0) *f = SpvFlags{{0ull, 0ull, 0ull}, 0, 0, 0};
 }
 
-// x entries must be valid column indices, ascending and unique.
-__global__ void k_sv_check_x(const int32_t* __restrict__ xind, int32_t nx, int64_t n, int* __restrict__ bad) {
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t >= nx) return;
-  const int32_t k = xind[t];
-  if (k < 0 || k >= n || (t + 1 < nx && xind[t + 1] <= k)) atomicOr(bad, 1);
+// A lane's value of the lane STEP before it in its row of sixteen (`none` in the
+// row's first lanes), or after it.
+template <int STEP>
+__device__ __forceinline__ int row_before(int v, int none) {
+  return __builtin_amdgcn_update_dpp(none, v, 0x110 + STEP, 0xf, 0xf, false);
+}
+__device__ __forceinline__ int row_after(int v, int none) {
+  return __builtin_amdgcn_update_dpp(none, v, 0x101, 0xf, 0xf, false);
 }
 
-// y_acc[i] (+)= A(i,k) (x) x_k for k in x; presence bit per row.
-template <int K, class T, bool BOOLA, int NT, int U>
-__global__ __launch_bounds__(NT) void k_sv_expand(const int64_t* __restrict__ cpA, const int64_t* __restrict__ irA,
-                                                  const void* __restrict__ valA_, const int32_t* __restrict__ colmap,
-                                                  const int32_t* __restrict__ xind, const T* __restrict__ xval,
-                                                  int32_t nx, T* __restrict__ acc, uint32_t* __restrict__ bits) {
+template <int STEP>
+__device__ __forceinline__ void row_or(int at, uint32_t& mask) {
+  const int w = row_before<STEP>(at, -1);
+  const uint32_t o = (uint32_t)row_before<STEP>((int)mask, 0);
+  if (w == at) mask |= o;
+}
+
+// One lane's U products into the accumulator, where there are some (ok), with
+// the loads in flight together; e: places in A (valid also without a product),
+// consecutive along each row of sixteen lanes.  Whole rows call it.
+template <int K, class T, bool BOOLA, int U>
+__device__ __forceinline__ void sv_products(const int64_t* __restrict__ ir, const T* __restrict__ val,
+                                            const int64_t (&e)[U], const bool (&ok)[U], T x, T* __restrict__ acc,
+                                            uint32_t* __restrict__ bits) {
   using SR = Sem<K, T>;
-  __shared__ SegStage<T, NT> st;
-  __shared__ long long wsum[NT / kWave];
-  const T* valA = (const T*)valA_;
-  for (int64_t c0 = (int64_t)blockIdx.x * NT; c0 < nx; c0 += (int64_t)gridDim.x * NT) {
-    const int64_t t = c0 + threadIdx.x;
-    int64_t base = 0;
-    int len = 0;
-    T xv{};
-    if (t < nx) {
-      const int32_t p = colmap[xind[t]];
-      if (p >= 0) {
-        base = cpA[p];
-        len = (int)(cpA[p + 1] - base);
-        xv = xval[t];
-      }
-    }
-    int nseg;
-    const int tot = stage_chunk<T, NT>(st, wsum, base, len, xv, nseg);
-    visit_staged<T, NT, U>(st, nseg, tot, [&](const int64_t(&idx)[U], const T(&xs)[U]) {
-      int64_t r[U];
-      T a[U];
+  int64_t r[U];
+  T a[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        r[u] = -1;
-        if (idx[u] >= 0) {
-          r[u] = irA[idx[u]];
-          if constexpr (!BOOLA) a[u] = valA[idx[u]];
-        }
-      }
+  for (int u = 0; u < U; ++u) {
+    r[u] = ir[e[u]];
+    if constexpr (!BOOLA) a[u] = val[e[u]];
+  }
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (r[u] < 0) continue;
-        T v;
-        if constexpr (BOOLA) v = xs[u];
-        else v = (T)SR::out(SR::mul(a[u], xs[u]));
-        GAcc<K, T>::acc(&acc[r[u]], v);
-        atomicOr(&bits[r[u] >> 5], 1u << (r[u] & 31));
-      }
-    });
+  for (int u = 0; u < U; ++u) {
+    pin(r[u]);
+    if constexpr (!BOOLA) pin(a[u]);
+  }
+  // The rows of a step ascend along a row of sixteen lanes, so its lanes with
+  // one word of the bitmap are neighbours: they set their bits with one atomic.
+  // (Hubs lie next to each other in skewed graphs, and thousands of products
+  // meet in one word: 147 K products of R-MAT s18 took 46 us with this, 79 with
+  // an atomic each.  Looking first whether the bit is set, or whether a maximum
+  // grows, took longer: the loads queue at the same words.)
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int at = ok[u] ? (int)(r[u] >> 5) : -1;
+    uint32_t mask = ok[u] ? 1u << (r[u] & 31) : 0u;
+    row_or<1>(at, mask);
+    row_or<2>(at, mask);
+    row_or<4>(at, mask);
+    row_or<8>(at, mask);
+    if (at >= 0 && row_after(at, -1) != at ) atomicOr(&bits[at], mask);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (!ok[u]) continue;
+    T v;
+    if constexpr (BOOLA) v = x;
+    else v = (T)SR::out(SR::mul(a[u], x));
+    GAcc<K, T>::acc(&acc[r[u]], v);
   }
 }
 
-__global__ void k_sv_wordcnt(const uint32_t* __restrict__ bits, int64_t nw, int32_t* __restrict__ cnt) {
-  const int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (w < nw) cnt[w] = __popc(bits[w]);
+// y_acc[i] (+)= A(i,k) (x) x_k for k in x; presence bit per row.  Sixteen lanes
+// take an entry of x, 64 products a step; columns longer than kSvHub go to a
+// list while it has room (x is short and its columns' lengths skewed: one
+// workgroup for 256 entries of x left the chip idle behind the longest column,
+// 102 us for the 5242 columns of R-MAT s18 that 27 + 19 us take now; lists from
+// 128 or 512 entries on measured the same within 2 us).
+// x entries must be valid column indices, ascending and unique.
+constexpr int kSvExpandNT = 256, kSvGroup = 16;
+constexpr int64_t kSvHub = 256, kSvPiece = 512;
+constexpr int kSvMaxHubs = 2048;
+
+template <int K, class T, bool BOOLA>
+__global__ __launch_bounds__(kSvExpandNT) void k_sv_expand(const int64_t* __restrict__ cpA,
+                                                           const int64_t* __restrict__ irA,
+                                                           const void* __restrict__ valA,
+                                                           const int32_t* __restrict__ colmap, int64_t n,
+                                                           const int32_t* __restrict__ xind,
+                                                           const T* __restrict__ xval, int32_t nx,
+                                                           T* __restrict__ acc, uint32_t* __restrict__ bits,
+                                                           int32_t* __restrict__ hubs, int max_hubs, SpvFlags* f) {
+  constexpr int U = 4, GROUPS = kSvExpandNT / kSvGroup;
+  if (f->malformed()) return;
+  const int l = threadIdx.x % kSvGroup;
+  for (int64_t t = (int64_t)blockIdx.x * GROUPS + threadIdx.x / kSvGroup; t < nx; t += (int64_t)gridDim.x * GROUPS) {
+    const int32_t k = xind[t], next = t + 1 < nx ? xind[t + 1] : INT32_MAX;
+    if (k < 0 || k >= n || next <= k) {
+      f->bad_x = 1;
+      continue;
+    }
+    const int32_t p = colmap[k];
+    if (p < 0) continue;
+    const T x = xval[t];
+    const int64_t b = cpA[p];
+    int64_t end = cpA[p + 1];
+    if (end - b > kSvHub) {
+      int slot = 0;
+      if (l == 0) slot = atomicAdd(&f->nhubs, 1);
+      slot = __shfl(slot, 0, kSvGroup);
+      if (slot < max_hubs) {
+        if (l == 0) hubs[slot] = (int32_t)t;
+        continue;
+      }
+    }
+    for (int64_t i = b; i < end; i += U * kSvGroup) {
+      int64_t e[U];
+      bool ok[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        ok[u] = i + u * kSvGroup + l < end;
+        e[u] = min(i + u * kSvGroup + l, end - 1);
+      }
+      sv_products<K, T, BOOLA, U>(irA, (const T*)valA, e, ok, x, acc, bits);
+    }
+  }
+}
+
+// The listed columns, in pieces of kSvPiece products, one per workgroup at a time.
+template <int K, class T, bool BOOLA>
+__global__ __launch_bounds__(kSvExpandNT) void k_sv_expand_hubs(const int64_t* __restrict__ cpA,
+                                                                const int64_t* __restrict__ irA,
+                                                                const void* __restrict__ valA,
+                                                                const int32_t* __restrict__ colmap,
+                                                                const int32_t* __restrict__ xind,
+                                                                const T* __restrict__ xval, T* __restrict__ acc,
+                                                                uint32_t* __restrict__ bits,
+                                                                const int32_t* __restrict__ hubs, int max_hubs,
+                                                                const SpvFlags* __restrict__ f) {
+  constexpr int PT = kSvMaxHubs / kSvExpandNT, U = (int)(kSvPiece / kSvExpandNT);
+  __shared__ int off[kSvMaxHubs + 1];
+  __shared__ int64_t beg[kSvMaxHubs], end[kSvMaxHubs];
+  __shared__ T xs[kSvMaxHubs];
+  __shared__ int wsum[kSvExpandNT / kWave];
+  const int nh = min(f->nhubs, max_hubs);
+  if (nh == 0) return;
+  int np[PT], sum = 0;
+#pragma unroll
+  for (int k = 0; k < PT; ++k) {
+    const int h = threadIdx.x * PT + k;
+    np[k] = 0;
+    if (h < nh) {
+      const int32_t t = hubs[h], p = colmap[xind[t]];
+      beg[h] = cpA[p];
+      end[h] = cpA[p + 1];
+      xs[h] = xval[t];
+      np[k] = (int)((end[h] - beg[h] + kSvPiece - 1) / kSvPiece);
+    }
+    sum += np[k];
+  }
+  int total;
+  int ex = block_excl_scan<kSvExpandNT>(sum, wsum, total);
+#pragma unroll
+  for (int k = 0; k < PT; ++k) {
+    off[threadIdx.x * PT + k] = ex;
+    ex += np[k];
+  }
+  if (threadIdx.x == 0) off[kSvMaxHubs] = total;
+  __syncthreads();
+  for (int piece = blockIdx.x; piece < total; piece += gridDim.x) {
+    int lo = 0, hi = nh;  // the last h with off[h] <= piece
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (off[mid] <= piece) lo = mid;
+      else hi = mid;
+    }
+    const int64_t i = beg[lo] + (piece - off[lo]) * kSvPiece;
+    int64_t e[U];
+    bool ok[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      ok[u] = i + u * kSvExpandNT + (int)threadIdx.x < end[lo];
+      e[u] = min(i + u * kSvExpandNT + (int)threadIdx.x, end[lo] - 1);
+    }
+    sv_products<K, T, BOOLA, U>(irA, (const T*)valA, e, ok, xs[lo], acc, bits);
+  }
+}
+
+// y's entries in each block of wpb bitmap words; then, with the blocks before
+// it summed by every block (at most kSvMaxSums), the entries themselves: a lane
+// per row.
+constexpr int kSvEmitNT = 256;
+constexpr int64_t kSvMaxSums = 4096;
+
+__global__ __launch_bounds__(kSvEmitNT) void k_sv_count(const uint32_t* __restrict__ bits, int64_t nw, int64_t wpb,
+                                                        int32_t* __restrict__ sums) {
+  __shared__ long long wsum[kSvEmitNT / kWave];
+  const int64_t w0 = blockIdx.x * wpb, w1 = min(nw, w0 + wpb);
+  long long c = 0;
+  for (int64_t w = w0 + threadIdx.x; w < w1; w += kSvEmitNT) c += __popc(bits[w]);
+  c = block_sum_ll<kSvEmitNT>(c, wsum);
+  if (threadIdx.x == 0) sums[blockIdx.x] = (int32_t)c;
 }
 
 template <class T>
-__global__ void k_sv_emit(const uint32_t* __restrict__ bits, const int32_t* __restrict__ off, int64_t nw,
-                          const T* __restrict__ acc, int32_t* __restrict__ yind, T* __restrict__ yval) {
-  const int64_t w = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (w >= nw) return;
-  uint32_t b = bits[w];
-  int32_t q = off[w];
-  while (b) {
-    const int j = __ffs(b) - 1;
-    b &= b - 1;
-    const int32_t i = (int32_t)(w * 32 + j);
-    yind[q] = i;
-    yval[q] = acc[i];
-    ++q;
+__global__ __launch_bounds__(kSvEmitNT) void k_sv_emit(const uint32_t* __restrict__ bits, int64_t nw, int64_t wpb,
+                                                       const int32_t* __restrict__ sums, const T* __restrict__ acc,
+                                                       int32_t* __restrict__ yind, T* __restrict__ yval, SpvFlags* f) {
+  constexpr int NW = kSvEmitNT / kWave, R = kWave / 2 / NW;  // rounds of 64 rows per wave and 64 words
+  __shared__ long long wsum[NW];
+  if (f->malformed() || f->bad_x) return;  // y is left as it was
+  long long before = 0;
+  for (int b = threadIdx.x; b < (int)blockIdx.x; b += kSvEmitNT) before += sums[b];
+  before = block_sum_ll<kSvEmitNT>(before, wsum);
+  int64_t at = before;
+  const int64_t w0 = blockIdx.x * wpb, w1 = min(nw, w0 + wpb);
+  const int lane = lane_id(), wave = wave_id_uniform();
+  for (int64_t w = w0; w < w1; w += kWave) {
+    const uint32_t word = w + lane < w1 ? bits[w + lane] : 0u;
+    const int incl = wave_incl_scan(__popc(word));
+    const int excl = incl - __popc(word);
+    T v[R];
+    bool in[R];
+    unsigned lo[R], hi[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const int j = 2 * (wave * R + k);
+      lo[k] = (unsigned)__builtin_amdgcn_readlane((int)word, j);
+      hi[k] = (unsigned)__builtin_amdgcn_readlane((int)word, j + 1);
+      in[k] = ((lane < 32 ? lo[k] : hi[k]) >> (lane & 31)) & 1u;
+      v[k] = acc[in[k] ? (w + j) * 32 + lane : 0];
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k) pin(v[k]);
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const int j = 2 * (wave * R + k);
+      const int64_t q = at + __builtin_amdgcn_readlane(excl, j) +
+                        (int)__builtin_amdgcn_mbcnt_hi(hi[k], __builtin_amdgcn_mbcnt_lo(lo[k], 0u));
+      if (in[k]) {
+        yind[q] = (int32_t)((w + j) * 32 + lane);
+        yval[q] = v[k];
+      }
+    }
+    at += __builtin_amdgcn_readlane(incl, kWave - 1);
   }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) f->ny = (int)at;
 }
 
 inline unsigned nb(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -202,63 +365,54 @@ T ident_of() {
   return std::numeric_limits<T>::lowest();
 }
 
-__global__ void k_sv_zero(int32_t* __restrict__ a, int32_t* __restrict__ b) {
-  if (threadIdx.x == 0) {
-    *a = 0;
-    *b = 0;
-  }
-}
-
 // Scratch of one SpMSpV: the column map of A (n), the dense accumulator (m
-// values) and presence bitmap (nw words), per-word counts and their scan
-// (nw + 1 each), a flag and the scan's temporary storage.
+// values) and presence bitmap (nw words), the flags, and 2 * (nw + 1) words for
+// the blocks' sums and the list of long columns.
 struct SvWork {
-  int32_t *colmap = nullptr, *cnt = nullptr, *off = nullptr;
+  int32_t *colmap = nullptr, *lists = nullptr;
   void* acc = nullptr;
   uint32_t* bits = nullptr;
-  int* bad = nullptr;
-  void* tmp = nullptr;
-  size_t tb = 0;
+  SpvFlags* flags = nullptr;
 };
 
 inline int64_t sv_words(int64_t m) { return m / 32 + 1; }
 
-template <class T>
-size_t sv_scan_bytes(int64_t m) {
-  size_t tb = 0;
-  const int64_t nw = sv_words(m);
-  (void)hipcub::DeviceScan::ExclusiveSum(nullptr, tb, (int32_t*)nullptr, (int32_t*)nullptr, (int)(nw + 1));
-  return std::max<size_t>(tb, 16);
-}
-
 // The product with its scratch in `w` (every array is initialised here, so
-// the scratch may hold anything on entry).
+// the scratch may hold anything on entry); A has columns and x entries.  The
+// structure check of A runs first; what follows it stops at its verdict.
 template <int K, class T>
 cbx_status spmspv_run(const cbx_dcsc* A, bool boolA, const int32_t* xind, const T* xval, int32_t nx, int32_t* yind,
                       T* yval, int32_t* ny, const SvWork& w, hipStream_t s) {
   const int64_t m = A->m, n = A->n, nw = sv_words(m);
   T* acc = (T*)w.acc;
-  int hbad = 0;
-  k_sv_zero<<<1, 64, 0, s>>>(w.bad, w.cnt + nw);
-  k_sv_check_x<<<nb(nx, 256), 256, 0, s>>>(xind, nx, n, w.bad);
-  CBX_HIP(hipMemcpyAsync(&hbad, w.bad, sizeof(int), hipMemcpyDeviceToHost, s));
-  CBX_HIP(hipStreamSynchronize(s));
-  if (hbad) return set_error(CBX_ERR_INVALID, "cbx_spmspv: x indices must be ascending, unique and below ncols");
-  k_sv_colmap<<<nb(n, 256), 256, 0, s>>>(A->jc, A->nzc, n, w.colmap);
-  k_sv_colmap_scatter<<<nb(A->nzc, 256), 256, 0, s>>>(A->jc, A->nzc, w.colmap);
-  k_sv_init<T><<<nb(std::max(m, nw), 256), 256, 0, s>>>(acc, m, ident_of<K, T>(), w.bits, nw);
-  const unsigned g = std::min<unsigned>(nb(nx, 256), 2048u);
-  if (boolA)
-    k_sv_expand<K, T, true, 256, 4><<<g, 256, 0, s>>>(A->cp, A->ir, A->val, w.colmap, xind, xval, nx, acc, w.bits);
-  else
-    k_sv_expand<K, T, false, 256, 4><<<g, 256, 0, s>>>(A->cp, A->ir, A->val, w.colmap, xind, xval, nx, acc, w.bits);
-  k_sv_wordcnt<<<nb(nw, 256), 256, 0, s>>>(w.bits, nw, w.cnt);
-  size_t tb = w.tb;
-  CBX_HIP(hipcub::DeviceScan::ExclusiveSum(w.tmp, tb, w.cnt, w.off, (int)(nw + 1), s));
-  k_sv_emit<T><<<nb(nw, 256), 256, 0, s>>>(w.bits, w.off, nw, acc, yind, yval);
-  CBX_HIP(hipMemcpyAsync(ny, w.off + nw, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  const int64_t wpb = kWave * ((nw + kWave * kSvMaxSums - 1) / (kWave * kSvMaxSums));
+  const int64_t nblk = (nw + wpb - 1) / wpb;
+  int32_t *sums = w.lists, *hubs = w.lists + nblk;
+  const int max_hubs = (int)std::min<int64_t>(kSvMaxHubs, 2 * (nw + 1) - nblk);
+  k_sv_begin<T><<<nb(std::max(std::max(m, n), nw), 256), 256, 0, s>>>(w.colmap, n, acc, m, ident_of<K, T>(), w.bits,
+                                                                     nw, w.flags);
+  dcsc_check_structure_launch(A, w.flags->chk, w.colmap, s);
+  const unsigned g = std::min(nb(nx, kSvExpandNT / kSvGroup), 16384u), gh = 512;
+  if (boolA) {
+    k_sv_expand<K, T, true><<<g, kSvExpandNT, 0, s>>>(A->cp, A->ir, A->val, w.colmap, n, xind, xval, nx, acc, w.bits,
+                                                     hubs, max_hubs, w.flags);
+    k_sv_expand_hubs<K, T, true><<<gh, kSvExpandNT, 0, s>>>(A->cp, A->ir, A->val, w.colmap, xind, xval, acc, w.bits,
+                                                           hubs, max_hubs, w.flags);
+  } else {
+    k_sv_expand<K, T, false><<<g, kSvExpandNT, 0, s>>>(A->cp, A->ir, A->val, w.colmap, n, xind, xval, nx, acc, w.bits,
+                                                      hubs, max_hubs, w.flags);
+    k_sv_expand_hubs<K, T, false><<<gh, kSvExpandNT, 0, s>>>(A->cp, A->ir, A->val, w.colmap, xind, xval, acc, w.bits,
+                                                            hubs, max_hubs, w.flags);
+  }
+  k_sv_count<<<(unsigned)nblk, kSvEmitNT, 0, s>>>(w.bits, nw, wpb, sums);
+  k_sv_emit<T><<<(unsigned)nblk, kSvEmitNT, 0, s>>>(w.bits, nw, wpb, sums, acc, yind, yval, w.flags);
+  SpvFlags h{};
   CBX_HIP(hipGetLastError());
+  CBX_HIP(hipMemcpyAsync(&h, w.flags, sizeof(h), hipMemcpyDeviceToHost, s));
   CBX_HIP(hipStreamSynchronize(s));
+  if (h.malformed()) return set_error(CBX_ERR_INVALID, "cbx_dcsc_check: malformed DCSC");
+  if (h.bad_x) return set_error(CBX_ERR_INVALID, "cbx_spmspv: x indices must be ascending, unique and below ncols");
+  *ny = h.ny;
   return CBX_OK;
 }
 
@@ -266,35 +420,21 @@ template <int K, class T>
 cbx_status spmspv_typed(const cbx_dcsc* A, bool boolA, const int32_t* xind, const T* xval, int32_t nx, int32_t* yind,
                         T* yval, int32_t* ny, hipStream_t s) {
   const int64_t m = A->m, n = A->n, nw = sv_words(m);
-  *ny = 0;
-  if (nx == 0 || A->nnz == 0) return CBX_OK;
+  ScratchSet ws(s);
   SvWork w;
-  w.tb = sv_scan_bytes<T>(m);
-  auto cleanup = [&]() {
-    for (void* p : {(void*)w.colmap, (void*)w.cnt, (void*)w.off, w.acc, (void*)w.bits, (void*)w.bad, w.tmp})
-      if (p) (void)hipFreeAsync(p, s);
-  };
-  if (hipMallocAsync(&w.colmap, sizeof(int32_t) * std::max<int64_t>(n, 1), s) != hipSuccess ||
-      hipMallocAsync(&w.cnt, sizeof(int32_t) * (nw + 1), s) != hipSuccess ||
-      hipMallocAsync(&w.off, sizeof(int32_t) * (nw + 1), s) != hipSuccess ||
-      hipMallocAsync(&w.acc, sizeof(T) * std::max<int64_t>(m, 1), s) != hipSuccess ||
-      hipMallocAsync(&w.bits, sizeof(uint32_t) * nw, s) != hipSuccess ||
-      hipMallocAsync(&w.bad, sizeof(int), s) != hipSuccess || hipMallocAsync(&w.tmp, w.tb, s) != hipSuccess) {
-    cleanup();
-    (void)hipGetLastError();
+  T* acc = nullptr;
+  if (!ws.take(&w.colmap, std::max<int64_t>(n, 1)) || !ws.take(&w.lists, 2 * (nw + 1)) ||
+      !ws.take(&acc, std::max<int64_t>(m, 1)) || !ws.take(&w.bits, nw) || !ws.take(&w.flags, 1))
     return set_error(CBX_ERR_NOMEM, "cbx_spmspv: workspace allocation failed");
-  }
-  const cbx_status st = spmspv_run<K, T>(A, boolA, xind, xval, nx, yind, yval, ny, w, s);
-  cleanup();
-  CBX_HIP(hipStreamSynchronize(s));
-  return st;
+  w.acc = acc;
+  return spmspv_run<K, T>(A, boolA, xind, xval, nx, yind, yval, ny, w, s);
 }
 
-// Carves the scratch of one SpMSpV (the arrays of SvWork plus the structure
-// check's three counters) out of one caller-given region; with base == null
-// it only adds up the bytes.  Every piece starts on a 256-byte boundary.
+// Carves the scratch of one SpMSpV out of one caller-given region; with base
+// == null it only adds up the bytes.  Every piece starts on a 256-byte
+// boundary.
 template <class T>
-size_t sv_carve(int64_t m, int64_t n, char* base, SvWork* w, unsigned long long** check_cnt) {
+size_t sv_carve(int64_t m, int64_t n, char* base, SvWork* w) {
   const int64_t nw = sv_words(m);
   size_t used = 0;
   auto take = [&](size_t bytes) -> void* {
@@ -303,41 +443,33 @@ size_t sv_carve(int64_t m, int64_t n, char* base, SvWork* w, unsigned long long*
     return p;
   };
   SvWork t;
-  t.tb = sv_scan_bytes<T>(m);
   t.colmap = (int32_t*)take(sizeof(int32_t) * std::max<int64_t>(n, 1));
-  t.cnt = (int32_t*)take(sizeof(int32_t) * (nw + 1));
-  t.off = (int32_t*)take(sizeof(int32_t) * (nw + 1));
+  t.lists = (int32_t*)take(sizeof(int32_t) * 2 * (nw + 1));
   t.acc = take(sizeof(T) * std::max<int64_t>(m, 1));
   t.bits = (uint32_t*)take(sizeof(uint32_t) * nw);
-  t.bad = (int*)take(sizeof(int));
-  t.tmp = take(t.tb);
-  unsigned long long* cnt = (unsigned long long*)take(3 * sizeof(unsigned long long));
+  t.flags = (SpvFlags*)take(sizeof(SpvFlags));
   if (w) *w = t;
-  if (check_cnt) *check_cnt = cnt;
   return used;
 }
 
-// cbx_spmspv with its scratch in `region` (bytes of device memory): the
-// structure check and the product, no allocation.
+// cbx_spmspv with its scratch in `region` (bytes of device memory): no
+// allocation.
 template <int K, class T>
 cbx_status spmspv_in_region(const cbx_dcsc* A, bool boolA, const int32_t* xind, const T* xval, int32_t nx,
                             int32_t* yind, T* yval, int32_t* ny, char* region, size_t bytes, hipStream_t s) {
   *ny = 0;
-  const size_t need = sv_carve<T>(A->m, A->n, nullptr, nullptr, nullptr);
+  const size_t need = sv_carve<T>(A->m, A->n, nullptr, nullptr);
   CBX_RETURN_IF(need > bytes, CBX_ERR_LIMIT,
                 "cbx_spmspv_noalloc: a %lld x %lld matrix needs %zu bytes of scratch, more than the %zu available",
                 (long long)A->m, (long long)A->n, need, bytes);
   SvWork w;
-  unsigned long long* cnt = nullptr;
-  sv_carve<T>(A->m, A->n, region, &w, &cnt);
-  if (A->nzc == 0) {
-    CBX_RETURN_IF(A->nnz != 0, CBX_ERR_INVALID, "cbx_dcsc_check: nnz without columns");
-  } else {
-    dcsc_check_launch(A, cnt, s);  // the kernels index by A's rows and columns
-    const cbx_status st = dcsc_check_result(cnt, s);
-    if (st != CBX_OK) return st;
+  sv_carve<T>(A->m, A->n, region, &w);
+  CBX_RETURN_IF(A->nzc == 0 && A->nnz != 0, CBX_ERR_INVALID, "cbx_dcsc_check: nnz without columns");
+  if (A->nzc == 0) return CBX_OK;
+  if (nx == 0) {  // the structure check all the same
+    dcsc_check_launch(A, w.flags->chk, s);
+    return dcsc_check_result(w.flags->chk, s);
   }
-  if (nx == 0 || A->nnz == 0) return CBX_OK;
   return spmspv_run<K, T>(A, boolA, xind, xval, nx, yind, yval, ny, w, s);
 }
 
@@ -1529,12 +1661,18 @@ extern "C" cbx_status cbx_spmspv(const cbx_dcsc* A, const int32_t* xind, const v
   const bool boolA = A->dtype == CBX_BOOL;
   CBX_RETURN_IF(!boolA && A->dtype != xdtype, CBX_ERR_UNSUPPORTED,
                 "cbx_spmspv: A must be boolean or share the vector's dtype");
-  cbx_status st = cbx_dcsc_check(A);  // the kernels index by A's rows and columns
-  if (st != CBX_OK) return st;
+  *ny = 0;
+  if (A->nzc == 0 || nx == 0) {
+    const cbx_status st = cbx_dcsc_check(A);  // otherwise with the product
+    if (st != CBX_OK) return st;
+  }
+  const cbx_status init = init_device_once();
+  if (init != CBX_OK) return init;
   hipStream_t s = (hipStream_t)stream;
   switch (semiring * 8 + xdtype) {
 #define CBX_SV(SRK, SRE, T, DT)                                                                                     \
   case SRE * 8 + DT:                                                                                                \
+    if (A->nzc == 0 || nx == 0) return CBX_OK;                                                                      \
     return spmspv_typed<SRK, T>(A, boolA, xind, (const T*)xval, nx, yind, (T*)yval, ny, s);
     CBX_SV(kPlusTimes, CBX_SR_PLUS_TIMES, int64_t, CBX_I64)
     CBX_SV(kPlusTimes, CBX_SR_PLUS_TIMES, double, CBX_F64)
