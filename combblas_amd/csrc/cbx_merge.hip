@@ -18,7 +18,8 @@
 // floating-point rounding.
 //
 // cbx_dcsc_from_coo (the Graph500 edge-list constructor, further below) keys
-// the entries, radix-sorts them and assembles with reduce-by-key.
+// the entries, radix-sorts them and combines equal neighbours in one pass that
+// writes the DCSC.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -47,85 +48,16 @@ struct SemAdd {
   }
 };
 
-struct KeyCol {
-  __host__ __device__ __forceinline__ int64_t operator()(const uint64_t& k) const { return (int64_t)(k >> 32); }
-};
-
-__global__ void k_merge_rows(const uint64_t* __restrict__ keys, int64_t n, int64_t* __restrict__ ir) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) ir[i] = (int64_t)(keys[i] & 0xffffffffull);
+// A value of another lane.
+template <class T>
+__device__ __forceinline__ T shfl_down(T v, int d) {
+  if constexpr (sizeof(T) == 1) return (T)__shfl_down((int)v, d, kWave);
+  else return __shfl_down(v, d, kWave);
 }
-
-__global__ void k_merge_close(int64_t* __restrict__ cp, int64_t nzc, int64_t nnz) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) cp[nzc] = nnz;  // after the exclusive scan of the column counts
-}
-
-using ColIt = hipcub::TransformInputIterator<int64_t, KeyCol, const uint64_t*>;
-
-// Temporary bytes of reduce_assemble for up to N sorted entries.
-template <int K, class T>
-hipError_t assemble_tmp_bytes(int N, hipStream_t s, size_t& bytes) {
-  size_t t2 = 0, t3 = 0, t4 = 0;
-  uint64_t* k = nullptr;
-  T* v = nullptr;
-  int64_t* c = nullptr;
-  hipError_t e = hipcub::DeviceReduce::ReduceByKey(nullptr, t2, k, k, v, v, c, SemAdd<K, T>(), N, s);
-  if (e == hipSuccess) e = hipcub::DeviceRunLengthEncode::Encode(nullptr, t3, ColIt(k, KeyCol()), c, c, c, N, s);
-  if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(nullptr, t4, c, c, N, s);
-  bytes = std::max(t2, std::max(t3, t4));
-  return e;
-}
-
-// From N (col, row)-sorted keys and values to a new device DCSC in *out:
-// equal keys combined with the semiring's add (into ukeys/uvals, N entries
-// each), columns from the run lengths of the keys' column halves (counts: N
-// entries; nruns: 2).  out's shape and dtype are set by the caller.
-template <int K, class T>
-cbx_status reduce_assemble(const uint64_t* keys, const T* vals, int N, uint64_t* ukeys, T* uvals, int64_t* nruns,
-                           int64_t* counts, void* tmp, size_t tb, cbx_dcsc* out, hipStream_t s, const char* who) {
-  hipError_t e = hipSuccess;
-  int64_t nnz = 0;  // no entries (every one a dropped loop): an empty matrix
-  if (N > 0) {
-    e = hipcub::DeviceReduce::ReduceByKey(tmp, tb, keys, ukeys, vals, uvals, nruns, SemAdd<K, T>(), N, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(&nnz, nruns, sizeof(int64_t), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-  }
-  if (e != hipSuccess) return set_error(CBX_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
-  cbx_status st = CBX_OK;
-  if ((st = dev_alloc((void**)&out->jc, sizeof(int64_t) * std::max<int64_t>(nnz, 1))) != CBX_OK ||
-      (st = dev_alloc((void**)&out->ir, sizeof(int64_t) * std::max<int64_t>(nnz, 1))) != CBX_OK ||
-      (st = dev_alloc(&out->val, sizeof(T) * std::max<int64_t>(nnz, 1))) != CBX_OK) {
-    cbx_dcsc_free(out);
-    return st;
-  }
-  int64_t nzc = 0;
-  if (nnz > 0) {
-    e = hipcub::DeviceRunLengthEncode::Encode(tmp, tb, ColIt(ukeys, KeyCol()), out->jc, counts, nruns + 1, (int)nnz,
-                                              s);
-    if (e == hipSuccess) e = hipMemcpyAsync(&nzc, nruns + 1, sizeof(int64_t), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-  }
-  if (e == hipSuccess && (st = dev_alloc((void**)&out->cp, sizeof(int64_t) * (nzc + 1))) != CBX_OK) {
-    cbx_dcsc_free(out);
-    return st;
-  }
-  if (e == hipSuccess && nzc > 0) e = hipcub::DeviceScan::ExclusiveSum(tmp, tb, counts, out->cp, (int)nzc, s);
-  if (e == hipSuccess) {
-    k_merge_close<<<1, 64, 0, s>>>(out->cp, nzc, nnz);
-    if (nnz > 0) {
-      k_merge_rows<<<(unsigned)((nnz + kMergeNT - 1) / kMergeNT), kMergeNT, 0, s>>>(ukeys, nnz, out->ir);
-      e = hipMemcpyAsync(out->val, uvals, sizeof(T) * nnz, hipMemcpyDeviceToDevice, s);
-    }
-  }
-  if (e == hipSuccess) e = hipGetLastError();
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  if (e != hipSuccess) {
-    cbx_dcsc_free(out);
-    return set_error(CBX_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
-  }
-  out->nnz = nnz;
-  out->nzc = nzc;
-  return CBX_OK;
+template <class T>
+__device__ __forceinline__ T shfl_from(T v, int lane) {
+  if constexpr (sizeof(T) == 1) return (T)__shfl((int)v, lane, kWave);
+  else return __shfl(v, lane, kWave);
 }
 
 // The parts as column blocks of one matrix: cp shifted by the entries before
@@ -260,27 +192,298 @@ cbx_status merge_typed(int32_t count, const cbx_dcsc* parts, cbx_dcsc* out, hipS
   return st;
 }
 
-// Edge-list input: keys of COO entries.  bad[0] counts entries out of range,
-// bad[1] the self loops dropped (their key is the sentinel (n << 32), past
-// every valid key, so they sort to the end).  vals may be null (value 1).
-template <class T>
+// ------------------------------------------------------- edge list to DCSC
+// Keys of COO entries: column above row in as many bits as the shape needs, as
+// every eight bits are a pass of the sort over keys and values (2^20 x 2^20: 40
+// bits and five passes of 160 us for 16.8 M entries; 53 and seven with the row
+// in a half of its own and a bit for the dropped loops).  A dropped self
+// loop's key is the last one, `drop`, that no entry has (coo_typed).  bad[0]
+// counts entries out of range, bad[1] the loops dropped.
 __global__ __launch_bounds__(kMergeNT) void k_coo_keys(const int64_t* __restrict__ rows,
-                                                       const int64_t* __restrict__ cols,
-                                                       const T* __restrict__ vals, int64_t nnz, int64_t m, int64_t n,
-                                                       int drop_loops, uint64_t* __restrict__ keys,
-                                                       T* __restrict__ out, unsigned long long* __restrict__ bad) {
+                                                       const int64_t* __restrict__ cols, int64_t nnz, int64_t m,
+                                                       int64_t n, int drop_loops, int row_bits, uint64_t drop,
+                                                       uint64_t* __restrict__ keys,
+                                                       unsigned long long* __restrict__ bad) {
+  constexpr int U = 4;
   long long oob = 0, loops = 0;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nnz; i += stride) {
-    const int64_t r = rows[i], c = cols[i];
-    const bool ok = r >= 0 && r < m && c >= 0 && c < n;
-    const bool loop = drop_loops && r == c;
-    oob += !ok;
-    loops += ok && loop;
-    keys[i] = ok && !loop ? ((uint64_t)c << 32) | (uint64_t)r : ((uint64_t)n << 32);
-    out[i] = vals ? vals[i] : (T)1;
+  for (int64_t i0 = blockIdx.x * (int64_t)(kMergeNT * U); i0 < nnz; i0 += (int64_t)gridDim.x * (kMergeNT * U)) {
+    int64_t r[U], c[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t i = min(i0 + u * kMergeNT + threadIdx.x, nnz - 1);
+      r[u] = rows[i];
+      c[u] = cols[i];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      pin(r[u]);
+      pin(c[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t i = i0 + u * kMergeNT + threadIdx.x;
+      if (i >= nnz) continue;
+      const bool ok = r[u] >= 0 && r[u] < m && c[u] >= 0 && c[u] < n;
+      const bool loop = drop_loops && r[u] == c[u];
+      oob += !ok;
+      loops += ok && loop;
+      keys[i] = ok && !loop ? ((uint64_t)c[u] << row_bits) | (uint64_t)r[u] : drop;
+    }
   }
   block_add_counts<kMergeNT>(oob, loops, &bad[0], &bad[1]);
+}
+
+__global__ void k_coo_begin(unsigned long long* __restrict__ bad) {
+  if (threadIdx.x < 2) bad[threadIdx.x] = 0ull;
+}
+
+// The sorted keys are taken in strips of kStrip entries, one per wave, kStrips
+// to a workgroup; a strip's entries are loaded together, 64 at a time to a lane
+// each.  A head is an entry whose key differs from the one before.
+constexpr int kChunks = 8, kStrip = kChunks * kWave, kStrips = kMergeNT / kWave;
+constexpr int kCooTile = kStrip * kStrips;
+
+struct Strip {
+  uint64_t key[kChunks];
+  unsigned long long heads[kChunks], columns[kChunks], live[kChunks];  // lanes (uniform)
+};
+
+__device__ __forceinline__ Strip load_strip(const uint64_t* __restrict__ keys, int64_t e0, int64_t count,
+                                            int row_bits) {
+  Strip st;
+  uint64_t prev[kChunks];
+  const int lane = lane_id();
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    const int64_t i = max(min(e0 + c * kWave + lane, count - 1), (int64_t)0);
+    st.key[c] = keys[i];
+    prev[c] = keys[max(i - 1, (int64_t)0)];
+  }
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    pin(st.key[c]);
+    pin(prev[c]);
+  }
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    const int64_t i = e0 + c * kWave + lane;
+    const bool live = i < count;
+    st.live[c] = __ballot(live);
+    st.heads[c] = __ballot(live && (i == 0 || st.key[c] != prev[c]));
+    st.columns[c] = __ballot(live && (i == 0 || (st.key[c] >> row_bits) != (prev[c] >> row_bits)));
+  }
+  return st;
+}
+
+// Heads (x) and column heads (y) of each tile.  count = nnz less the loops.
+__global__ __launch_bounds__(kMergeNT) void k_coo_count(const uint64_t* __restrict__ keys, int64_t nnz,
+                                                        const unsigned long long* __restrict__ bad, int row_bits,
+                                                        int2* __restrict__ tiles) {
+  __shared__ int sx[kStrips], sy[kStrips];
+  const int64_t count = nnz - (int64_t)bad[1];
+  const int w = wave_id_uniform();
+  const Strip st = load_strip(keys, blockIdx.x * (int64_t)kCooTile + w * kStrip, count, row_bits);
+  int x = 0, y = 0;
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    x += __popcll(st.heads[c]);
+    y += __popcll(st.columns[c]);
+  }
+  if (lane_id() == 0) {
+    sx[w] = x;
+    sy[w] = y;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    x = y = 0;
+    for (int k = 0; k < kStrips; ++k) {
+      x += sx[k];
+      y += sy[k];
+    }
+    tiles[blockIdx.x] = make_int2(x, y);
+  }
+}
+
+// Exclusive prefix sums of the tiles' counts in place, and what the host needs.
+struct CooReport {
+  unsigned long long bad[2];
+  long long nnz, nzc;
+};
+constexpr int kCooScanNT = 1024, kCooScanPer = 8;
+__global__ __launch_bounds__(kCooScanNT) void k_coo_scan(int2* __restrict__ tiles, int64_t ntiles,
+                                                         const unsigned long long* __restrict__ bad,
+                                                         CooReport* __restrict__ rep) {
+  __shared__ long long wsum[kCooScanNT / kWave];
+  long long bx = 0, by = 0;
+  for (int64_t t0 = 0; t0 < ntiles; t0 += kCooScanNT * kCooScanPer) {
+    const int64_t t = t0 + (int64_t)threadIdx.x * kCooScanPer;
+    int2 v[kCooScanPer];
+    long long x = 0, y = 0;
+#pragma unroll
+    for (int k = 0; k < kCooScanPer; ++k) v[k] = tiles[min(t + k, ntiles - 1)];
+#pragma unroll
+    for (int k = 0; k < kCooScanPer; ++k) {
+      pin(v[k].x);
+      pin(v[k].y);
+      if (t + k >= ntiles) v[k] = make_int2(0, 0);
+      x += v[k].x;
+      y += v[k].y;
+    }
+    long long tx, ty;
+    long long ex = bx + block_excl_scan_ll<kCooScanNT>(x, wsum, tx);
+    long long ey = by + block_excl_scan_ll<kCooScanNT>(y, wsum, ty);
+#pragma unroll
+    for (int k = 0; k < kCooScanPer; ++k) {
+      if (t + k < ntiles) tiles[t + k] = make_int2((int)ex, (int)ey);
+      ex += v[k].x;
+      ey += v[k].y;
+    }
+    bx += tx;
+    by += ty;
+  }
+  if (threadIdx.x == 0) *rep = CooReport{{bad[0], bad[1]}, bx, by};
+}
+
+// A value that may be absent (a semiring's add has no identity that every
+// stored value leaves alone: infinity against min-plus's largest number).
+template <class T>
+struct Maybe {
+  T v;
+  bool some;
+};
+
+// What strip s adds to the run that reaches it from the left, and whether that
+// run takes all of it.
+template <class T>
+struct StripLead {
+  T v;
+  int some, whole;
+};
+
+// The DCSC from the sorted entries: each run of equal keys is combined (vals:
+// null for ones) and written at its rank, columns at theirs.  A run is combined
+// within 64 entries by steps that double, as many as its longest run needs;
+// chunks of a strip pass what they add to the run on their left; strips leave
+// it in `lead` for k_coo_join.  Bound by the bytes read and written once: 16.8 M
+// entries (R-MAT s20, int64) take 96 us, and 31 in k_coo_count; the library's
+// reduce-by-key and run lengths, the extraction of rows and a copy of the
+// values, with two waits between, took some 600.
+template <int K, class T>
+__global__ __launch_bounds__(kMergeNT) void k_coo_assemble(const uint64_t* __restrict__ keys,
+                                                           const T* __restrict__ vals, int64_t count, int row_bits,
+                                                           const int2* __restrict__ tiles, int64_t nnz, int64_t nzc,
+                                                           int64_t* __restrict__ cp, int64_t* __restrict__ jc,
+                                                           int64_t* __restrict__ ir, T* __restrict__ val,
+                                                           StripLead<T>* __restrict__ lead) {
+  __shared__ int sx[kStrips], sy[kStrips];
+  const SemAdd<K, T> add;
+  const int w = wave_id_uniform(), lane = lane_id();
+  const int64_t strip = blockIdx.x * (int64_t)kStrips + w, e0 = strip * kStrip;
+  T v[kChunks];
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    v[c] = (T)1;
+    if (vals) v[c] = vals[min(e0 + c * kWave + lane, count - 1)];
+  }
+  const Strip st = load_strip(keys, e0, count, row_bits);
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) pin(v[c]);
+  int x = 0, y = 0;
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) {
+    x += __popcll(st.heads[c]);
+    y += __popcll(st.columns[c]);
+  }
+  if (lane == 0) {
+    sx[w] = x;
+    sy[w] = y;
+  }
+  __syncthreads();
+  int64_t rank = tiles[blockIdx.x].x, crank = tiles[blockIdx.x].y;  // after this strip
+  for (int k = 0; k <= w; ++k) {
+    rank += sx[k];
+    crank += sy[k];
+  }
+  Maybe<T> carry{T{}, false};  // from the chunk on the right
+  bool whole = true;
+#pragma unroll
+  for (int c = kChunks - 1; c >= 0; --c) {
+    const unsigned long long heads = st.heads[c], live = st.live[c];
+    rank -= __popcll(heads);
+    crank -= __popcll(st.columns[c]);
+    // the first lane after this one's run
+    const unsigned long long ends = lane == kWave - 1 ? 0ull : (heads | ~live) >> (lane + 1);
+    const int end = ends ? lane + __ffsll(ends) : kWave;
+    for (int d = 1; __ballot(lane + d < end); d *= 2) {
+      const T o = shfl_down(v[c], d);
+      if (lane + d < end) v[c] = add(v[c], o);
+    }
+    if (end == kWave && carry.some) v[c] = add(v[c], carry.v);
+    const bool head = (heads >> lane) & 1ull;
+    if (head) {
+      const int64_t q = rank + __popcll(heads & ((1ull << lane) - 1ull));
+      ir[q] = (int64_t)(st.key[c] & ((1ull << row_bits) - 1ull));
+      val[q] = v[c];
+      if ((st.columns[c] >> lane) & 1ull) {
+        const int64_t k = crank + __popcll(st.columns[c] & ((1ull << lane) - 1ull));
+        jc[k] = (int64_t)(st.key[c] >> row_bits);
+        cp[k] = q;
+      }
+    }
+    carry.some = (live & 1ull) && !(heads & 1ull);
+    carry.v = shfl_from(v[c], 0);
+    whole = whole && !heads && !~live;
+  }
+  if (lane == 0) lead[strip] = StripLead<T>{carry.v, carry.some, whole};
+  if (blockIdx.x == 0 && threadIdx.x == 0) cp[nzc] = nnz;
+}
+
+// Runs over the ends of strips: the strip in which one has its head adds what
+// the following strips left, up to the first that it does not take whole.  One
+// wave per strip; the last run of strip s is the entry before the strip's end
+// rank, `tiles` and the strips' heads giving that as in the kernel above.
+template <int K, class T>
+__global__ __launch_bounds__(kMergeNT) void k_coo_join(const uint64_t* __restrict__ keys, int64_t count, int row_bits,
+                                                       const int2* __restrict__ tiles, int64_t nstrips,
+                                                       const StripLead<T>* __restrict__ lead, T* __restrict__ val) {
+  __shared__ int sx[kStrips];
+  const SemAdd<K, T> add;
+  const int w = wave_id_uniform(), lane = lane_id();
+  const int64_t strip = blockIdx.x * (int64_t)kStrips + w;
+  const bool open = strip + 1 < nstrips && lead[strip + 1].some && !lead[strip].whole;
+  __shared__ int any;
+  if (threadIdx.x == 0) any = 0;
+  __syncthreads();
+  if (open && lane == 0) any = 1;
+  __syncthreads();
+  if (!any) return;
+  const Strip st = load_strip(keys, strip * kStrip, count, row_bits);
+  int x = 0;
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) x += __popcll(st.heads[c]);
+  if (lane == 0) sx[w] = x;
+  __syncthreads();
+  if (!open) return;
+  int64_t q = (int64_t)tiles[blockIdx.x].x - 1;
+  for (int k = 0; k <= w; ++k) q += sx[k];
+  T sum = val[q];
+  for (int64_t s0 = strip + 1; s0 < nstrips; s0 += kWave) {
+    const bool in = s0 + lane < nstrips;
+    const StripLead<T> l = lead[min(s0 + lane, nstrips - 1)];
+    // lanes up to the first that is not whole
+    const unsigned long long stop = __ballot(!in || !l.whole);
+    const int n = stop ? __ffsll(stop) : kWave;
+    const unsigned long long some = __ballot(in && lane < n && l.some);
+    const int terms = some ? kWave - __clzll(some) : 0;  // (all lanes before the last one have a value)
+    T v = l.v;
+    for (int d = 1; d < terms; d *= 2) {
+      const T o = shfl_down(v, d);
+      if (lane + d < terms) v = add(v, o);
+    }
+    if (terms) sum = add(sum, shfl_from(v, 0));
+    if (stop) break;
+  }
+  if (lane == 0) val[q] = sum;
 }
 
 int bits_for(int64_t v) {  // bits to hold 0..v
@@ -292,51 +495,75 @@ int bits_for(int64_t v) {  // bits to hold 0..v
 template <int K, class T>
 cbx_status coo_typed(int64_t m, int64_t n, const int64_t* rows, const int64_t* cols, const T* vals, int64_t nnz,
                      int drop_loops, cbx_dcsc* out, hipStream_t s) {
+  const char* who = "cbx_dcsc_from_coo";
   const int N = (int)nnz;
-  uint64_t *k0 = nullptr, *k1 = nullptr, *ukeys = nullptr;
-  T *v0 = nullptr, *v1 = nullptr;
-  int64_t *nruns = nullptr, *counts = nullptr;
+  const int row_bits = bits_for(std::max<int64_t>(m - 1, 0));
+  int end_bit = row_bits + bits_for(std::max<int64_t>(n - 1, 0));
+  // dropped loops sort to the end: the last key of so many bits is the entry
+  // (2^row_bits - 1, 2^col_bits - 1), which is out of range or, in a square
+  // matrix, a loop itself; otherwise one bit more
+  if (drop_loops && m != n && m == (int64_t)1 << row_bits && n == (int64_t)1 << (end_bit - row_bits)) ++end_bit;
+  const uint64_t drop = (1ull << end_bit) - 1;
+  const int64_t ntiles = (nnz + kCooTile - 1) / kCooTile, nstrips = ntiles * kStrips;
+  uint64_t *k0 = nullptr, *k1 = nullptr;
+  T* v1 = nullptr;
+  int2* tiles = nullptr;
+  StripLead<T>* lead = nullptr;
   unsigned long long* bad = nullptr;
+  CooReport* rep = nullptr;
   void* tmp = nullptr;
-  size_t tb = 0, t1 = 0, t2 = 0;
-  const int end_bit = 32 + bits_for(n);  // the loop sentinel (col = n) included
-  CBX_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, t1, k0, k1, v0, v1, N, 0, end_bit, s));
-  CBX_HIP((assemble_tmp_bytes<K, T>(N, s, t2)));
-  tb = std::max(t1, t2);
+  size_t tb = 0;
+  if (vals) CBX_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, k0, k1, vals, v1, N, 0, end_bit, s));
+  else CBX_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, tb, k0, k1, N, 0, end_bit, s));
   ScratchSet ws(s);
-  auto cleanup = [&]() { ws.release(); };
-  if (!ws.take(&k0, N) || !ws.take(&k1, N) || !ws.take(&ukeys, N) || !ws.take(&v0, N) || !ws.take(&v1, N) ||
-      !ws.take(&nruns, 2) || !ws.take(&counts, N) || !ws.take(&bad, 2) ||
+  if (!ws.take(&k0, N) || !ws.take(&k1, N) || (vals && !ws.take(&v1, N)) || !ws.take(&tiles, ntiles) ||
+      !ws.take(&lead, nstrips) || !ws.take(&bad, 2) || !ws.take(&rep, 1) ||
       !ws.take_bytes(&tmp, std::max<size_t>(tb, 16))) {
     (void)hipGetLastError();
-    cleanup();
     return set_error(CBX_ERR_NOMEM, "cbx_dcsc_from_coo: workspace allocation failed");
   }
-  unsigned long long hbad[2] = {0, 0};
-  hipError_t e = hipMemsetAsync(bad, 0, 2 * sizeof(unsigned long long), s);
-  if (e == hipSuccess) {
-    const unsigned g = (unsigned)std::min<int64_t>((nnz + kMergeNT - 1) / kMergeNT, 4096);
-    k_coo_keys<T><<<g, kMergeNT, 0, s>>>(rows, cols, vals, nnz, m, n, drop_loops, k0, v0, bad);
+  k_coo_begin<<<1, 64, 0, s>>>(bad);
+  const unsigned g = (unsigned)std::min<int64_t>((nnz + kMergeNT * 4 - 1) / (kMergeNT * 4), 2048);
+  k_coo_keys<<<g, kMergeNT, 0, s>>>(rows, cols, nnz, m, n, drop_loops, row_bits, drop, k0, bad);
+  CBX_HIP(hipGetLastError());
+  if (vals) CBX_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, vals, v1, N, 0, end_bit, s));
+  else CBX_HIP(hipcub::DeviceRadixSort::SortKeys(tmp, tb, k0, k1, N, 0, end_bit, s));
+  k_coo_count<<<(unsigned)ntiles, kMergeNT, 0, s>>>(k1, nnz, bad, row_bits, tiles);
+  k_coo_scan<<<1, kCooScanNT, 0, s>>>(tiles, ntiles, bad, rep);
+  CooReport h{};
+  CBX_HIP(hipGetLastError());
+  CBX_HIP(hipMemcpyAsync(&h, rep, sizeof(h), hipMemcpyDeviceToHost, s));
+  CBX_HIP(hipStreamSynchronize(s));
+  if (h.bad[0])
+    return set_error(CBX_ERR_INVALID, "cbx_dcsc_from_coo: %llu entries outside the %lld x %lld shape", h.bad[0],
+                     (long long)m, (long long)n);
+  const int64_t count = nnz - (int64_t)h.bad[1];
+  cbx_status st = CBX_OK;
+  const int64_t held = std::max<int64_t>(h.nnz, 1);
+  if ((st = dev_alloc((void**)&out->cp, sizeof(int64_t) * (h.nzc + 1))) != CBX_OK ||
+      (st = dev_alloc((void**)&out->jc, sizeof(int64_t) * std::max<int64_t>(h.nzc, 1))) != CBX_OK ||
+      (st = dev_alloc((void**)&out->ir, sizeof(int64_t) * held)) != CBX_OK ||
+      (st = dev_alloc(&out->val, sizeof(T) * held)) != CBX_OK) {
+    cbx_dcsc_free(out);
+    return st;
+  }
+  hipError_t e = hipSuccess;
+  if (count > 0) {
+    k_coo_assemble<K, T><<<(unsigned)ntiles, kMergeNT, 0, s>>>(k1, vals ? v1 : nullptr, count, row_bits, tiles, h.nnz,
+                                                              h.nzc, out->cp, out->jc, out->ir, (T*)out->val, lead);
+    k_coo_join<K, T><<<(unsigned)ntiles, kMergeNT, 0, s>>>(k1, count, row_bits, tiles, nstrips, lead, (T*)out->val);
     e = hipGetLastError();
+  } else {  // every entry a dropped loop
+    e = hipMemsetAsync(out->cp, 0, sizeof(int64_t), s);
   }
-  if (e == hipSuccess) e = hipMemcpyAsync(hbad, bad, sizeof(hbad), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  if (e != hipSuccess || hbad[0]) {
-    cleanup();
-    return e != hipSuccess ? set_error(CBX_ERR_HIP, "cbx_dcsc_from_coo: %s", hipGetErrorString(e))
-                           : set_error(CBX_ERR_INVALID, "cbx_dcsc_from_coo: %llu entries outside the %lld x %lld shape",
-                                       hbad[0], (long long)m, (long long)n);
-  }
-  e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, v0, v1, N, 0, end_bit, s);
   if (e != hipSuccess) {
-    cleanup();
-    return set_error(CBX_ERR_HIP, "cbx_dcsc_from_coo: %s", hipGetErrorString(e));
+    cbx_dcsc_free(out);
+    return set_error(CBX_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
   }
-  // the dropped loops sit at the end of the sorted keys
-  const cbx_status st = reduce_assemble<K, T>(k1, v1, N - (int)hbad[1], ukeys, v0, nruns, counts, tmp, tb, out, s,
-                                              "cbx_dcsc_from_coo");
-  cleanup();
-  return st;
+  out->nnz = h.nnz;
+  out->nzc = h.nzc;
+  return CBX_OK;
 }
 
 }  // namespace
