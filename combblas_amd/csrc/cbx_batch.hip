@@ -11,7 +11,7 @@
 // exactly what a separate call would return.
 //
 // Transpose (SpDCCols::Transpose, include/CombBLAS/SpDCCols.cpp:871-1011)
-// sorts (row, column) keys with a device radix sort and rebuilds DCSC.
+// sorts the entries by row with a (stable) device radix sort and rebuilds DCSC.
 //
 // Galerkin (ReleaseTests/GalerkinNew.cpp:94-112): T = R^T is given, S = T
 // transposed, AT = A*T, SAT = S*AT, all with PlusTimes<double>.
@@ -38,17 +38,6 @@ constexpr int kMaxBatch = 4096;
 
 inline unsigned nblocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// One product's arrays inside a packed batch.
-struct Seg {
-  const int64_t* cp;
-  const int64_t* jc;
-  const int64_t* ir;
-  const void* val;
-  int64_t row_off, col_off;  // added to rows / column ids
-  int64_t nz_off, c_off;     // first entry / first stored column in the packed matrix
-  int64_t m, n, nnz, nzc;    // the member's own shape and sizes (for its bounds)
-};
-
 struct OutSeg {
   int64_t* cp;
   int64_t* jc;
@@ -58,61 +47,129 @@ struct OutSeg {
   int64_t nz_off, c_off, nnz, nzc;
 };
 
-// Index of the segment holding position x: the last s with off[s] <= x.
-__device__ __forceinline__ int find_seg(const int64_t* off, int count, int64_t x) {
+// The last segment s with off(s) <= x among all, and this workgroup's: the
+// number of segments that start at or before x (uniform; a barrier each 256).
+template <class F>
+__device__ __forceinline__ int find_seg(int count, int64_t x, F&& off) {
   int lo = 0, hi = count - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (off[mid] <= x) lo = mid;
+    if (off(mid) <= x) lo = mid;
     else hi = mid - 1;
   }
   return lo;
 }
-
-template <class V>
-__global__ __launch_bounds__(256) void k_pack_entries(const Seg* __restrict__ segs, int count, int64_t total,
-                                                      int64_t* __restrict__ ir, V* __restrict__ val) {
-  __shared__ int64_t off[kMaxBatch];
-  for (int s = threadIdx.x; s < count; s += blockDim.x) off[s] = segs[s].nz_off;
-  __syncthreads();
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
-    const int s = find_seg(off, count, e);
-    const int64_t i = e - off[s];
-    ir[e] = segs[s].ir[i] + segs[s].row_off;
-    val[e] = ((const V*)segs[s].val)[i];
+template <class F>
+__device__ __forceinline__ int block_find_seg(int count, int64_t x, F&& off) {
+  int n = 0;
+  for (int s0 = 0; s0 < count; s0 += 256) {
+    const int s = s0 + (int)threadIdx.x;
+    const int here = __syncthreads_count(s < count && off(s) <= x);
+    n += here;
+    if (here < 256) break;
   }
+  return __builtin_amdgcn_readfirstlane(n - 1);
 }
 
-// Packs the column arrays and checks each member against its own bounds,
-// which the packed matrix's validation cannot see (a row or column id that
-// strays into the next member's block is in range there): column ids in
-// [0, n_i), cp starting at 0 and closing at the member's nnz, and every
-// non-empty column's first and last rows in [0, m_i) — all its rows, since
-// the product's validation of the packed matrix checks that rows ascend
-// within columns.  bad[0] counts violations.
-__global__ __launch_bounds__(256) void k_pack_cols(const Seg* __restrict__ segs, int count, int64_t total,
-                                                   int64_t total_nnz, int64_t* __restrict__ cp,
-                                                   int64_t* __restrict__ jc, unsigned long long* __restrict__ bad) {
-  __shared__ int64_t off[kMaxBatch];
-  for (int s = threadIdx.x; s < count; s += blockDim.x) off[s] = segs[s].c_off;
-  __syncthreads();
-  long long nbad = 0;
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
-    const int s = find_seg(off, count, q);
-    const int64_t i = q - off[s];
-    const Seg& g = segs[s];
-    const int64_t b = g.cp[i], e = g.cp[i + 1], j = g.jc[i];
-    bool err = j < 0 || j >= g.n || (i == 0 && b != 0) || (i + 1 == g.nzc && e != g.nnz);
-    if (!err && 0 <= b && b < e && e <= g.nnz) {  // a non-empty column inside the member's entries
-      const int64_t r0 = g.ir[b], r1 = g.ir[e - 1];
-      err = r0 < 0 || r0 >= g.m || r1 < 0 || r1 >= g.m;
+// Entries and columns are taken in tiles of one workgroup; nearly every tile
+// lies in one member, whose pointers are then the same for all lanes and a
+// thread's entries are in flight together.  (A search per entry, with one entry
+// in flight, moved 1.3 TB/s.)
+constexpr int kPackNT = 256, kPackPer = 8, kPackTile = kPackNT * kPackPer;
+
+// chk: as in the product's validation, [0] violations, [1] descents of rows,
+// [2] those at column starts.
+template <class V>
+__global__ __launch_bounds__(kPackNT) void k_pack_entries(const PackSeg* __restrict__ segs, int count, int64_t total,
+                                                          int64_t* __restrict__ ir, int32_t* __restrict__ rows32,
+                                                          V* __restrict__ val, unsigned long long* __restrict__ chk) {
+  auto off = [&](int s) { return segs[s].nz_off; };
+  long long bad = 0, desc = 0;
+  for (int64_t e0 = blockIdx.x * (int64_t)kPackTile; e0 < total; e0 += gridDim.x * (int64_t)kPackTile) {
+    const int s0 = block_find_seg(count, e0, off);
+    const bool one = s0 + 1 == count || segs[s0 + 1].nz_off >= min(e0 + kPackTile, total);
+    int64_t r[kPackPer], next[kPackPer];
+    V v[kPackPer];
+    if (one) {
+      const PackSeg g = segs[s0];
+      const int64_t i0 = e0 - g.nz_off, left = g.nnz - 1;
+#pragma unroll
+      for (int u = 0; u < kPackPer; ++u) {
+        const int64_t i = i0 + u * kPackNT + threadIdx.x;
+        r[u] = g.ir[min(i, left)];
+        next[u] = g.ir[min(i + 1, left)];
+        v[u] = ((const V*)g.val)[min(i, left)];
+      }
+#pragma unroll
+      for (int u = 0; u < kPackPer; ++u) {
+        pin(r[u]);
+        pin(next[u]);
+        pin(v[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kPackPer; ++u) {
+        const int64_t i = i0 + u * kPackNT + threadIdx.x;
+        if (i > left) continue;
+        bad += r[u] < 0 || r[u] >= g.m;
+        desc += i < left && next[u] <= r[u];
+        r[u] += g.row_off;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kPackPer; ++u) {
+        const int64_t e = e0 + u * kPackNT + threadIdx.x;
+        if (e >= total) continue;
+        const PackSeg& g = segs[find_seg(count, e, off)];
+        const int64_t i = e - g.nz_off;
+        r[u] = g.ir[i];
+        v[u] = ((const V*)g.val)[i];
+        bad += r[u] < 0 || r[u] >= g.m;
+        desc += i + 1 < g.nnz && g.ir[i + 1] <= r[u];
+        r[u] += g.row_off;
+      }
     }
-    nbad += err;
-    cp[q] = b + g.nz_off;
-    jc[q] = j + g.col_off;
+#pragma unroll
+    for (int u = 0; u < kPackPer; ++u) {
+      const int64_t e = e0 + u * kPackNT + threadIdx.x;
+      if (e >= total) continue;
+      if (ir) ir[e] = r[u];
+      if (rows32) rows32[e] = (int32_t)r[u];
+      val[e] = v[u];
+    }
+  }
+  block_add_counts<kPackNT>(bad, desc, &chk[0], &chk[1]);
+}
+
+// The column arrays, and the check's rules for columns, of each member.
+__global__ __launch_bounds__(kPackNT) void k_pack_cols(const PackSeg* __restrict__ segs, int count, int64_t total,
+                                                       int64_t total_nnz, int64_t* __restrict__ cp,
+                                                       int64_t* __restrict__ jc,
+                                                       unsigned long long* __restrict__ chk) {
+  constexpr int PER = 2;
+  auto off = [&](int s) { return segs[s].c_off; };
+  long long bad = 0, desc = 0;
+  for (int64_t q0 = blockIdx.x * (int64_t)(kPackNT * PER); q0 < total; q0 += gridDim.x * (int64_t)(kPackNT * PER)) {
+    const int s0 = block_find_seg(count, q0, off);
+    const bool one = s0 + 1 == count || segs[s0 + 1].c_off >= min(q0 + kPackNT * PER, total);
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int64_t q = q0 + u * kPackNT + threadIdx.x;
+      if (q >= total) continue;
+      const PackSeg& g = segs[one ? s0 : find_seg(count, q, off)];
+      const int64_t i = q - g.c_off;
+      const int64_t b = g.cp[i], e = g.cp[i + 1], j = g.jc[i];
+      bool err = b < 0 || e < b || e > g.nnz || j < 0 || j >= g.n || (i == 0 && b != 0) ||
+                 (i + 1 == g.nzc && e != g.nnz);
+      if (i + 1 < g.nzc) err |= g.jc[i + 1] <= j;
+      bad += err;
+      // a column start with another column's entry before it
+      if (!err && i > 0 && b > 0 && b < g.nnz && g.cp[i - 1] < b) desc += g.ir[b] <= g.ir[b - 1];
+      cp[q] = b + g.nz_off;
+      jc[q] = j + g.col_off;
+    }
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) cp[total] = total_nnz;
-  block_add_counts<256>(nbad, 0, &bad[0], &bad[1]);
+  block_add_counts<kPackNT>(bad, desc, &chk[0], &chk[2]);
 }
 
 // qb[s] = first stored column of the packed matrix with column id >= bound[s].
@@ -133,27 +190,42 @@ __global__ void k_seg_bounds(const int64_t* __restrict__ jc, int64_t nzc, const 
 }
 
 template <class V>
-__global__ __launch_bounds__(256) void k_unpack_entries(const OutSeg* __restrict__ segs, int count, int64_t total,
-                                                        const int64_t* __restrict__ ir, const V* __restrict__ val) {
-  __shared__ int64_t off[kMaxBatch];
-  for (int s = threadIdx.x; s < count; s += blockDim.x) off[s] = segs[s].nz_off;
-  __syncthreads();
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
-    const int s = find_seg(off, count, e);
-    const int64_t i = e - off[s];
-    segs[s].ir[i] = ir[e] - segs[s].row_off;
-    ((V*)segs[s].val)[i] = val[e];
+__global__ __launch_bounds__(kPackNT) void k_unpack_entries(const OutSeg* __restrict__ segs, int count, int64_t total,
+                                                            const int64_t* __restrict__ ir,
+                                                            const V* __restrict__ val) {
+  const int64_t e0 = blockIdx.x * (int64_t)kPackTile;
+  auto off = [&](int s) { return segs[s].nz_off; };
+  const int s0 = block_find_seg(count, e0, off);
+  const bool one = s0 + 1 == count || segs[s0 + 1].nz_off >= min(e0 + kPackTile, total);
+  int64_t r[kPackPer];
+  V v[kPackPer];
+#pragma unroll
+  for (int u = 0; u < kPackPer; ++u) {
+    const int64_t e = min(e0 + u * kPackNT + threadIdx.x, total - 1);
+    r[u] = ir[e];
+    v[u] = val[e];
+  }
+#pragma unroll
+  for (int u = 0; u < kPackPer; ++u) {
+    pin(r[u]);
+    pin(v[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < kPackPer; ++u) {
+    const int64_t e = e0 + u * kPackNT + threadIdx.x;
+    if (e >= total) continue;
+    const OutSeg& g = segs[one ? s0 : find_seg(count, e, off)];
+    g.ir[e - g.nz_off] = r[u] - g.row_off;
+    ((V*)g.val)[e - g.nz_off] = v[u];
   }
 }
 
 __global__ __launch_bounds__(256) void k_unpack_cols(const OutSeg* __restrict__ segs, int count, int64_t total,
                                                      const int64_t* __restrict__ cp, const int64_t* __restrict__ jc) {
-  __shared__ int64_t off[kMaxBatch];
-  for (int s = threadIdx.x; s < count; s += blockDim.x) off[s] = segs[s].c_off;
-  __syncthreads();
+  auto off = [&](int s) { return segs[s].c_off; };
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
-    const int s = find_seg(off, count, q);
-    const int64_t i = q - off[s];
+    const int s = find_seg(count, q, off);
+    const int64_t i = q - segs[s].c_off;
     segs[s].cp[i] = cp[q] - segs[s].nz_off;
     segs[s].jc[i] = jc[q] - segs[s].col_off;
   }
@@ -162,42 +234,51 @@ __global__ __launch_bounds__(256) void k_unpack_cols(const OutSeg* __restrict__ 
     segs[s].cp[segs[s].nzc] = segs[s].nnz;
 }
 
-// Transpose helpers: key = row << 32 | column, payload = entry index.
+// Transpose helpers.  The entries come ordered by column, so a stable sort by
+// row alone puts them in the transpose's order: 32-bit keys of the row's bits
+// (three passes up to 2^24 rows; seven over (row, column) keys of 64 bits took
+// 0.43 ms for 4.7 M entries, these 0.20).  The payload is the entry's place
+// and column.  G lanes take a column (a wave per column of 8 entries waited for
+// its cp: 0.11 ms, now 0.02).
+template <int G>
 __global__ void k_entry_keys(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc,
-                             const int64_t* __restrict__ ir, int64_t nzc, uint64_t* __restrict__ key,
-                             int32_t* __restrict__ idx) {
-  const int64_t q = global_wave();
+                             const int64_t* __restrict__ ir, int64_t nzc, uint32_t* __restrict__ key,
+                             uint64_t* __restrict__ from) {
+  const int64_t q = (global_wave() * kWave + lane_id()) / G;
   if (q >= nzc) return;
   const uint64_t c = (uint64_t)jc[q];
-  for (int64_t e = cp[q] + lane_id(); e < cp[q + 1]; e += kWave) {
-    key[e] = ((uint64_t)ir[e] << 32) | c;
-    idx[e] = (int32_t)e;
+  const int64_t end = cp[q + 1];
+  for (int64_t e = cp[q] + lane_id() % G; e < end; e += G) {
+    key[e] = (uint32_t)ir[e];
+    from[e] = ((uint64_t)e << 32) | c;
   }
 }
 
-__global__ void k_col_heads(const uint64_t* __restrict__ key, int64_t nnz, int32_t* __restrict__ head) {
+__global__ void k_col_heads(const uint32_t* __restrict__ key, int64_t nnz, int32_t* __restrict__ head) {
   const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (e < nnz) head[e] = (e == 0 || (key[e] >> 32) != (key[e - 1] >> 32)) ? 1 : 0;
+  if (e < nnz) head[e] = (e == 0 || key[e] != key[e - 1]) ? 1 : 0;
   if (e == nnz) head[e] = 0;
 }
 
 template <class V>
-__global__ void k_transpose_write(const uint64_t* __restrict__ key, const int32_t* __restrict__ idx,
-                                  const int32_t* __restrict__ head, const int32_t* __restrict__ hpos, int64_t nnz,
-                                  const V* __restrict__ val, int64_t* __restrict__ ocp, int64_t* __restrict__ ojc,
-                                  int64_t* __restrict__ oir, V* __restrict__ oval) {
+__global__ void k_transpose_write(const uint32_t* __restrict__ key, const uint64_t* __restrict__ from,
+                                  const int32_t* __restrict__ hpos, int64_t nnz, const V* __restrict__ val,
+                                  int64_t* __restrict__ ocp, int64_t* __restrict__ ojc, int64_t* __restrict__ oir,
+                                  V* __restrict__ oval) {
   const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (e >= nnz) return;
-  const uint64_t k = key[e];
-  oir[e] = (int64_t)(k & 0xffffffffull);
-  oval[e] = val[idx[e]];
-  if (head[e]) {
-    ojc[hpos[e]] = (int64_t)(k >> 32);
+  const uint64_t f = from[e];
+  oir[e] = (int64_t)(f & 0xffffffffull);
+  oval[e] = val[f >> 32];
+  if (hpos[e + 1] != hpos[e]) {
+    ojc[hpos[e]] = (int64_t)key[e];
     ocp[hpos[e]] = e;
   }
+  if (e == nnz - 1) ocp[hpos[nnz]] = nnz;
 }
 
-cbx_status alloc_dev_dcsc(cbx_dcsc* X, int64_t m, int64_t n, int64_t nnz, int64_t nzc, cbx_dtype dt) {
+cbx_status alloc_dev_dcsc(cbx_dcsc* X, int64_t m, int64_t n, int64_t nnz, int64_t nzc, cbx_dtype dt,
+                          bool rows = true) {
   std::memset(X, 0, sizeof(*X));
   X->m = m;
   X->n = n;
@@ -208,7 +289,7 @@ cbx_status alloc_dev_dcsc(cbx_dcsc* X, int64_t m, int64_t n, int64_t nnz, int64_
   cbx_status st;
   if ((st = dev_alloc((void**)&X->cp, sizeof(int64_t) * (size_t)(nzc + 1))) ||
       (st = dev_alloc((void**)&X->jc, sizeof(int64_t) * (size_t)std::max<int64_t>(nzc, 1))) ||
-      (st = dev_alloc((void**)&X->ir, sizeof(int64_t) * (size_t)std::max<int64_t>(nnz, 1))) ||
+      (rows && (st = dev_alloc((void**)&X->ir, sizeof(int64_t) * (size_t)std::max<int64_t>(nnz, 1)))) ||
       (st = dev_alloc(&X->val, dtype_size(dt) * (size_t)std::max<int64_t>(nnz, 1)))) {
     cbx_dcsc_free(X);
     return st;
@@ -234,59 +315,73 @@ struct DevMem {
 
 unsigned grid_for(int64_t n) { return (unsigned)std::min<int64_t>(std::max<int64_t>(nblocks(n, 256), 1), 65536); }
 
+unsigned pack_tiles(int64_t total) { return nblocks(total, kPackTile); }
+constexpr unsigned kPackGrid = 2048;  // checking workgroups (each adds to the counters once)
+
 template <class V>
-cbx_status launch_pack_entries(const Seg* segs, int count, int64_t total, int64_t* ir, void* val, hipStream_t s) {
-  if (total) k_pack_entries<V><<<grid_for(total), 256, 0, s>>>(segs, count, total, ir, (V*)val);
-  CBX_HIP(hipGetLastError());
-  return CBX_OK;
+void launch_pack_entries(const PackSeg* segs, int count, const cbx_dcsc& out, int32_t* rows32,
+                         unsigned long long* chk, hipStream_t s) {
+  if (out.nnz)
+    k_pack_entries<V><<<std::min(pack_tiles(out.nnz), kPackGrid), kPackNT, 0, s>>>(segs, count, out.nnz, out.ir, rows32, (V*)out.val, chk);
 }
 
 template <class V>
 cbx_status launch_unpack_entries(const OutSeg* segs, int count, int64_t total, const int64_t* ir, const void* val,
                                  hipStream_t s) {
-  if (total) k_unpack_entries<V><<<grid_for(total), 256, 0, s>>>(segs, count, total, ir, (const V*)val);
+  if (total) k_unpack_entries<V><<<pack_tiles(total), kPackNT, 0, s>>>(segs, count, total, ir, (const V*)val);
   CBX_HIP(hipGetLastError());
   return CBX_OK;
 }
 
+__global__ void k_pack_begin(unsigned long long* __restrict__ chk) {
+  if (threadIdx.x < 3) chk[threadIdx.x] = 0ull;
+}
+
 }  // namespace
 
+cbx_status pack_members(const PackSeg* segs, int64_t count, const cbx_dcsc& out, int32_t* rows32, hipStream_t s) {
+  for (int64_t i = 0; i < count; ++i)
+    CBX_RETURN_IF(segs[i].nzc == 0 && segs[i].nnz != 0, CBX_ERR_INVALID, "cbx_dcsc_check: nnz without columns");
+  DevMem dsegs, dchk;
+  PackSeg* d;
+  unsigned long long* chk;
+  CBX_TRY(dsegs.get(&d, count));
+  CBX_TRY(dchk.get(&chk, 3));
+  CBX_HIP(hipMemcpyAsync(d, segs, sizeof(PackSeg) * count, hipMemcpyHostToDevice, s));
+  k_pack_begin<<<1, 64, 0, s>>>(chk);
+  k_pack_cols<<<std::min(std::max(nblocks(out.nzc, kPackNT * 2), 1u), kPackGrid), kPackNT, 0, s>>>(d, (int)count, out.nzc, out.nnz, out.cp,
+                                                                            out.jc, chk);
+  switch (dtype_size(out.dtype)) {
+    case 8: launch_pack_entries<uint64_t>(d, (int)count, out, rows32, chk, s); break;
+    case 4: launch_pack_entries<uint32_t>(d, (int)count, out, rows32, chk, s); break;
+    default: launch_pack_entries<uint8_t>(d, (int)count, out, rows32, chk, s); break;
+  }
+  CBX_HIP(hipGetLastError());
+  unsigned long long h[3] = {0, 0, 0};
+  CBX_HIP(hipMemcpyAsync(h, chk, sizeof(h), hipMemcpyDeviceToHost, s));
+  CBX_HIP(hipStreamSynchronize(s));  // the segment table and counters are released at return
+  // (a member's descents at column starts are among its descents: the sums
+  // agree only if every member's do)
+  return h[0] || h[1] != h[2] ? set_error(CBX_ERR_INVALID, "cbx_dcsc_check: a member is malformed") : CBX_OK;
+}
+
 // Packs X[0..count) into one block-diagonal DCSC (rows and columns offset by
-// the running sums of m and n), checking each member against its own bounds
-// (k_pack_cols); the product validates the packed matrix as any operand.
-static cbx_status pack(const cbx_dcsc* X, int64_t count, cbx_dcsc* out, hipStream_t s) {
-  std::vector<Seg> segs(count);
+// the running sums of m and n); with rows32 its rows are written there, as 32
+// bits, and it has no ir.
+static cbx_status pack(const cbx_dcsc* X, int64_t count, cbx_dcsc* out, DevMem* rows32, int32_t** rows,
+                       hipStream_t s) {
+  std::vector<PackSeg> segs(count);
   int64_t m = 0, n = 0, nnz = 0, nzc = 0;
   for (int64_t i = 0; i < count; ++i) {
-    segs[i] = Seg{X[i].cp, X[i].jc, X[i].ir, X[i].val, m, n, nnz, nzc, X[i].m, X[i].n, X[i].nnz, X[i].nzc};
+    segs[i] = PackSeg{X[i].cp, X[i].jc, X[i].ir, X[i].val, m, n, nnz, nzc, X[i].m, X[i].n, X[i].nnz, X[i].nzc};
     m += X[i].m;
     n += X[i].n;
     nnz += X[i].nnz;
     nzc += X[i].nzc;
   }
-  CBX_TRY(alloc_dev_dcsc(out, m, n, nnz, nzc, X[0].dtype));
-  DevMem dsegs, dbad;
-  Seg* d;
-  unsigned long long* bad;
-  CBX_TRY(dsegs.get(&d, count));
-  CBX_TRY(dbad.get(&bad, 2));
-  CBX_HIP(hipMemcpyAsync(d, segs.data(), sizeof(Seg) * count, hipMemcpyHostToDevice, s));
-  CBX_HIP(hipMemsetAsync(bad, 0, 2 * sizeof(unsigned long long), s));
-  k_pack_cols<<<grid_for(nzc), 256, 0, s>>>(d, (int)count, nzc, nnz, out->cp, out->jc, bad);
-  CBX_HIP(hipGetLastError());
-  switch (dtype_size(X[0].dtype)) {
-    case 8: CBX_TRY(launch_pack_entries<uint64_t>(d, (int)count, nnz, out->ir, out->val, s)); break;
-    case 4: CBX_TRY(launch_pack_entries<uint32_t>(d, (int)count, nnz, out->ir, out->val, s)); break;
-    default: CBX_TRY(launch_pack_entries<uint8_t>(d, (int)count, nnz, out->ir, out->val, s)); break;
-  }
-  unsigned long long hbad = 0;
-  CBX_HIP(hipMemcpyAsync(&hbad, bad, sizeof(hbad), hipMemcpyDeviceToHost, s));
-  CBX_HIP(hipStreamSynchronize(s));  // the segment table and counter are released at return
-  if (hbad) {
-    cbx_dcsc_free(out);
-    return set_error(CBX_ERR_INVALID, "cbx_dcsc_check: a batch member is malformed (index outside its own shape)");
-  }
-  return CBX_OK;
+  CBX_TRY(alloc_dev_dcsc(out, m, n, nnz, nzc, X[0].dtype, rows32 == nullptr));
+  if (rows32) CBX_TRY(rows32->get(rows, nnz));
+  return pack_members(segs.data(), count, *out, rows32 ? *rows : nullptr, s);
 }
 
 // Splits a packed product into count matrices: product i owns the columns
@@ -334,40 +429,46 @@ static cbx_status unpack(const cbx_dcsc* P, int64_t count, const std::vector<int
 
 template <class V>
 static cbx_status transpose_typed(const cbx_dcsc* X, cbx_dcsc* out, hipStream_t s) {
-  const int64_t nnz = X->nnz;
-  DevMem dk0, dk1, di0, di1, dh, dhp, dtmp;
-  uint64_t *k0, *k1;
-  int32_t *i0, *i1, *head, *hpos;
+  const int64_t nnz = X->nnz, nzc = X->nzc;
+  DevMem dk0, dk1, df0, df1, dh, dhp, dtmp;
+  uint32_t *k0, *k1;
+  uint64_t *f0, *f1;
+  int32_t *head, *hpos;
   CBX_TRY(dk0.get(&k0, nnz));
   CBX_TRY(dk1.get(&k1, nnz));
-  CBX_TRY(di0.get(&i0, nnz));
-  CBX_TRY(di1.get(&i1, nnz));
+  CBX_TRY(df0.get(&f0, nnz));
+  CBX_TRY(df1.get(&f1, nnz));
   CBX_TRY(dh.get(&head, nnz + 1));
   CBX_TRY(dhp.get(&hpos, nnz + 1));
-  if (X->nzc) k_entry_keys<<<wave_grid(X->nzc), 256, 0, s>>>(X->cp, X->jc, X->ir, X->nzc, k0, i0);
+  if (nzc && nnz / nzc < 8) k_entry_keys<4><<<wave_grid((nzc + 15) / 16), 256, 0, s>>>(X->cp, X->jc, X->ir, nzc, k0, f0);
+  else if (nzc && nnz / nzc < 32)
+    k_entry_keys<16><<<wave_grid((nzc + 3) / 4), 256, 0, s>>>(X->cp, X->jc, X->ir, nzc, k0, f0);
+  else if (nzc)
+    k_entry_keys<kWave><<<wave_grid(nzc), 256, 0, s>>>(X->cp, X->jc, X->ir, nzc, k0, f0);
   CBX_HIP(hipGetLastError());
   int rbits = 1;
   while (rbits < 31 && ((int64_t)1 << rbits) < X->m) ++rbits;
   size_t tb = 0, tb2 = 0;
-  hipcub::DoubleBuffer<uint64_t> keys(k0, k1);
-  hipcub::DoubleBuffer<int32_t> vals(i0, i1);
-  CBX_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, keys, vals, (int)nnz, 0, 32 + rbits, s));
+  hipcub::DoubleBuffer<uint32_t> keys(k0, k1);
+  hipcub::DoubleBuffer<uint64_t> from(f0, f1);
+  CBX_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, keys, from, (int)nnz, 0, rbits, s));
   CBX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb2, head, hpos, (int)(nnz + 1), s));
   uint8_t* tmp;
   CBX_TRY(dtmp.get(&tmp, std::max(tb, tb2)));
   tb = std::max(tb, tb2);
-  CBX_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, keys, vals, (int)nnz, 0, 32 + rbits, s));
+  CBX_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tb, keys, from, (int)nnz, 0, rbits, s));
   k_col_heads<<<nblocks(nnz + 1, 256), 256, 0, s>>>(keys.Current(), nnz, head);
   CBX_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tb, head, hpos, (int)(nnz + 1), s));
-  int32_t nzc = 0;
-  CBX_HIP(hipMemcpyAsync(&nzc, hpos + nnz, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  int32_t ncols = 0;
+  CBX_HIP(hipMemcpyAsync(&ncols, hpos + nnz, sizeof(int32_t), hipMemcpyDeviceToHost, s));
   CBX_HIP(hipStreamSynchronize(s));
-  CBX_TRY(alloc_dev_dcsc(out, X->n, X->m, nnz, nzc, X->dtype));
+  CBX_TRY(alloc_dev_dcsc(out, X->n, X->m, nnz, ncols, X->dtype));
   if (nnz)
-    k_transpose_write<V><<<nblocks(nnz, 256), 256, 0, s>>>(keys.Current(), vals.Current(), head, hpos, nnz,
+    k_transpose_write<V><<<nblocks(nnz, 256), 256, 0, s>>>(keys.Current(), from.Current(), hpos, nnz,
                                                          (const V*)X->val, out->cp, out->jc, out->ir, (V*)out->val);
+  else
+    CBX_HIP(hipMemsetAsync(out->cp, 0, sizeof(int64_t), s));
   CBX_HIP(hipGetLastError());
-  CBX_HIP(hipMemcpyAsync(out->cp + nzc, &nnz, sizeof(int64_t), hipMemcpyHostToDevice, s));
   CBX_HIP(hipStreamSynchronize(s));
   return CBX_OK;
 }
@@ -417,10 +518,15 @@ static cbx_status spgemm_batched(int64_t count, const cbx_dcsc* A, const cbx_dcs
                                  cbx_spgemm_mode mode, const SpgemmConfig& cfg, cbx_dcsc* C,
                                  cbx_spgemm_stats* st, hipStream_t s) {
   Owned PA, PB, PC;
-  CBX_TRY(pack(A, count, &PA.x, s));
-  CBX_TRY(pack(B, count, &PB.x, s));
+  DevMem rows;
+  int32_t* rows_a = nullptr;
+  CBX_TRY(pack(A, count, &PA.x, &rows, &rows_a, s));
+  CBX_TRY(pack(B, count, &PB.x, nullptr, nullptr, s));
+  SpgemmConfig packed = cfg;
+  packed.trusted_a = packed.trusted_b = true;
+  packed.rows_a = rows_a;
   cbx_spgemm_stats one;
-  CBX_TRY(spgemm_dispatch(&PA.x, &PB.x, sr, mode, cfg, &PC.x, &one, s));
+  CBX_TRY(spgemm_dispatch(&PA.x, &PB.x, sr, mode, packed, &PC.x, &one, s));
   add_stats(st, one);
   std::vector<int64_t> bound(count + 1, 0), roff(count, 0), ms(count), ns(count);
   for (int64_t i = 0; i < count; ++i) {
@@ -435,14 +541,19 @@ static cbx_status spgemm_batched(int64_t count, const cbx_dcsc* A, const cbx_dcs
 static cbx_status galerkin_batched(int64_t count, const cbx_dcsc* A, const cbx_dcsc* T, const SpgemmConfig& cfg,
                                    cbx_dcsc* SAT, cbx_spgemm_stats* st, hipStream_t s) {
   Owned PA, PT, PS, PAT, PSAT;
-  CBX_TRY(pack(A, count, &PA.x, s));
-  CBX_TRY(pack(T, count, &PT.x, s));
+  DevMem rows;
+  int32_t* rows_a = nullptr;
+  CBX_TRY(pack(A, count, &PA.x, &rows, &rows_a, s));
+  CBX_TRY(pack(T, count, &PT.x, nullptr, nullptr, s));
   CBX_TRY(transpose(&PT.x, &PS.x, s));
   cbx_spgemm_stats one;
-  CBX_TRY(spgemm_dispatch(&PA.x, &PT.x, CBX_SR_PLUS_TIMES, CBX_SPGEMM_TWO_PHASE, cfg, &PAT.x, &one, s));
-  add_stats(st, one);
-  SpgemmConfig cfg2 = cfg;  // S (a transpose) and A*T (a product) come from this library
+  // the packed operands are checked; S (a transpose) and A*T (a product) come from this library
+  SpgemmConfig cfg2 = cfg;
   cfg2.trusted_a = cfg2.trusted_b = true;
+  SpgemmConfig packed = cfg2;
+  packed.rows_a = rows_a;
+  CBX_TRY(spgemm_dispatch(&PA.x, &PT.x, CBX_SR_PLUS_TIMES, CBX_SPGEMM_TWO_PHASE, packed, &PAT.x, &one, s));
+  add_stats(st, one);
   CBX_TRY(spgemm_dispatch(&PS.x, &PAT.x, CBX_SR_PLUS_TIMES, CBX_SPGEMM_TWO_PHASE, cfg2, &PSAT.x, &one, s));
   add_stats(st, one);
   std::vector<int64_t> bound(count + 1, 0), roff(count, 0), ms(count), ns(count);

@@ -60,28 +60,6 @@ __device__ __forceinline__ T shfl_from(T v, int lane) {
   else return __shfl(v, lane, kWave);
 }
 
-// The parts as column blocks of one matrix: cp shifted by the entries before
-// the part, jc by the part's first column (its index times n).  Checks what
-// the concatenation's own validation cannot see: column ids in [0, n) (one
-// beyond would fall into the next part's block and merge into the wrong
-// output column) and cp starting at 0 and closing at the part's nnz; *bad
-// counts violations.
-__global__ void k_cat_columns(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc, int64_t nzc,
-                              int64_t nnz, int64_t n, int64_t entry_base, int64_t col_base,
-                              int64_t* __restrict__ cpA, int64_t* __restrict__ jcA, unsigned long long* __restrict__ bad) {
-  const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (q < nzc) {
-    const int64_t b = cp[q], j = jc[q];
-    if (j < 0 || j >= n || (q == 0 && b != 0) || (q + 1 == nzc && cp[q + 1] != nnz)) atomicAdd(bad, 1ull);
-    cpA[q] = b + entry_base;
-    jcA[q] = j + col_base;
-  }
-}
-
-__global__ void k_cat_close(int64_t* __restrict__ cpA, int64_t nzc, int64_t nnz) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) cpA[nzc] = nnz;
-}
-
 // B (c n x n): column j holds c entries, at rows s n + j, each the one.
 template <class T>
 __global__ void k_stacked_identity(int64_t n, int c, T one, int64_t* __restrict__ cpB, int64_t* __restrict__ jcB,
@@ -146,48 +124,39 @@ cbx_status merge_typed(int32_t count, const cbx_dcsc* parts, cbx_dcsc* out, hipS
   B.nnz = (int64_t)count * n;
   B.nzc = n;
   ScratchSet ws(s);
-  int64_t *cpA, *jcA, *irA, *cpB, *jcB, *irB;
+  int64_t *cpA, *jcA, *cpB, *jcB, *irB;
+  int32_t* rowsA;
   T *valA, *valB;
-  unsigned long long* bad;
-  if (!ws.take(&cpA, nzc + 1) || !ws.take(&jcA, nzc) || !ws.take(&irA, nnz) || !ws.take(&valA, nnz) ||
-      !ws.take(&cpB, n + 1) || !ws.take(&jcB, n) || !ws.take(&irB, B.nnz) || !ws.take(&valB, B.nnz) ||
-      !ws.take(&bad, 1))
+  if (!ws.take(&cpA, nzc + 1) || !ws.take(&jcA, nzc) || !ws.take(&rowsA, nnz) || !ws.take(&valA, nnz) ||
+      !ws.take(&cpB, n + 1) || !ws.take(&jcB, n) || !ws.take(&irB, B.nnz) || !ws.take(&valB, B.nnz))
     return set_error(CBX_ERR_NOMEM, "cbx_dcsc_merge: workspace allocation failed");
-  CBX_HIP(hipMemsetAsync(bad, 0, sizeof(unsigned long long), s));
   A.cp = cpA;
   A.jc = jcA;
-  A.ir = irA;
   A.val = valA;
   B.cp = cpB;
   B.jc = jcB;
   B.ir = irB;
   B.val = valB;
+  // the parts as column blocks of one matrix, each checked against its own
+  // bounds (a column id beyond n would fall into the next part's block)
+  std::vector<PackSeg> segs((size_t)count);
   int64_t eb = 0, qb = 0;
   for (int32_t i = 0; i < count; ++i) {
     const cbx_dcsc& P = parts[i];
-    if (P.nzc) {
-      k_cat_columns<<<(unsigned)((P.nzc + kMergeNT - 1) / kMergeNT), kMergeNT, 0, s>>>(
-          P.cp, P.jc, P.nzc, P.nnz, n, eb, (int64_t)i * n, cpA + qb, jcA + qb, bad);
-      CBX_HIP(hipMemcpyAsync(irA + eb, P.ir, sizeof(int64_t) * P.nnz, hipMemcpyDeviceToDevice, s));
-      CBX_HIP(hipMemcpyAsync(valA + eb, P.val, sizeof(T) * P.nnz, hipMemcpyDeviceToDevice, s));
-    }
+    segs[i] = PackSeg{P.cp, P.jc, P.ir, P.val, 0, (int64_t)i * n, eb, qb, m, n, P.nnz, P.nzc};
     eb += P.nnz;
     qb += P.nzc;
   }
-  k_cat_close<<<1, 64, 0, s>>>(cpA, nzc, nnz);
+  cbx_status st = pack_members(segs.data(), count, A, rowsA, s);
+  if (st != CBX_OK) return st;
   k_stacked_identity<T><<<(unsigned)((n + 1 + kMergeNT - 1) / kMergeNT), kMergeNT, 0, s>>>(
       n, count, semiring_one<K, T>(), cpB, jcB, irB, valB);
   CBX_HIP(hipGetLastError());
-  unsigned long long hbad = 0;
-  CBX_HIP(hipMemcpyAsync(&hbad, bad, sizeof(hbad), hipMemcpyDeviceToHost, s));
-  CBX_HIP(hipStreamSynchronize(s));
-  if (hbad) return set_error(CBX_ERR_INVALID, "cbx_dcsc_check: a part is malformed (column outside [0, n) or cp)");
-  // the rest of the parts' structure is validated as A's (rows in range and
-  // ascending per column, columns ascending, cp consistent); B is built here
   SpgemmConfig cfg = current_config();
-  cfg.trusted_b = true;
+  cfg.trusted_a = cfg.trusted_b = true;
+  cfg.rows_a = rowsA;
   const cbx_semiring sr = K == kPlusTimes ? CBX_SR_PLUS_TIMES : K == kMinPlus ? CBX_SR_MIN_PLUS : CBX_SR_SELECT_MAX;
-  const cbx_status st = spgemm_dispatch(&A, &B, sr, CBX_SPGEMM_TWO_PHASE, cfg, out, nullptr, s);
+  st = spgemm_dispatch(&A, &B, sr, CBX_SPGEMM_TWO_PHASE, cfg, out, nullptr, s);
   if (st != CBX_OK) cbx_dcsc_free(out);
   return st;
 }

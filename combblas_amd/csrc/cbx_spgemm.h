@@ -39,6 +39,9 @@ struct SpgemmConfig {
   // Operands the library produced itself (a transpose, an earlier product)
   // are valid by construction and skip the device validation pass.
   bool trusted_a = false, trusted_b = false;
+  // A's rows as 32-bit, where the caller has them (and has checked A): A.ir is
+  // not read then.
+  const int32_t* rows_a = nullptr;
   float capacity_margin = 0.15f;
   // Two-phase mode: share of the free memory the large units' row maps may take (0: none).
   float row_map_share = 0.25f;
@@ -182,6 +185,21 @@ cbx_status dcsc_check_result(const unsigned long long* cnt, hipStream_t s);
 // those at column starts); colmap, if given, receives the place of each column
 // that breaks no rule.
 void dcsc_check_structure_launch(const cbx_dcsc* X, unsigned long long* cnt, int32_t* colmap, hipStream_t s);
+
+// One member of a concatenation, and where its entries, columns, rows and
+// column ids start in it.
+struct PackSeg {
+  const int64_t *cp, *jc, *ir;
+  const void* val;
+  int64_t row_off, col_off, nz_off, c_off;
+  int64_t m, n, nnz, nzc;  // the member's own shape and sizes (for its bounds)
+};
+
+// Writes the members' concatenation to out.cp / jc / val and their rows to
+// out.ir and rows32, where these are not null (out.nnz, nzc, dtype set), and
+// checks every member against its own bounds by the product's rules: the
+// concatenation needs no other check.  CBX_ERR_INVALID if one is malformed.
+cbx_status pack_members(const PackSeg* segs, int64_t count, const cbx_dcsc& out, int32_t* rows32, hipStream_t s);
 
 cbx_status spgemm_dispatch(const cbx_dcsc* A, const cbx_dcsc* B, cbx_semiring sr, cbx_spgemm_mode mode,
                            const SpgemmConfig& cfg, cbx_dcsc* C, cbx_spgemm_stats* stats, hipStream_t s);

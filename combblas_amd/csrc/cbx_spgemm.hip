@@ -303,7 +303,7 @@ __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
 // agree.  cnt[0] violations, cnt[1] descents, cnt[2] descents at starts.
 // With rows32 the pass also writes the rows as 32-bit (garbage where a row is
 // out of range; nothing uses it then): one reading of ir instead of two.
-constexpr int kValNT = 256, kValBlocks = 1024;
+constexpr int kValNT = 256, kValBlocks = 2048, kValPer = 4;  // kValPer entries of a thread in flight together
 
 __global__ __launch_bounds__(kValNT) void k_validate(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc,
                                                      const int64_t* __restrict__ ir, int64_t nzc, int64_t nnz,
@@ -312,13 +312,27 @@ __global__ __launch_bounds__(kValNT) void k_validate(const int64_t* __restrict__
                                                      unsigned long long* __restrict__ cnt) {
   long long bad = 0, desc = 0;
   if ((int)blockIdx.x < eblocks) {  // entries
-    const int64_t stride = (int64_t)eblocks * kValNT;
-    for (int64_t e = blockIdx.x * (int64_t)kValNT + threadIdx.x; e < nnz; e += stride) {
-      const int64_t r = ir[e];
-      const int64_t next = ir[min(e + 1, nnz - 1)];
-      bad += r < 0 || r >= nrows;
-      desc += e + 1 < nnz && next <= r;
-      if (rows32) rows32[e] = (int32_t)r;
+    const int64_t stride = (int64_t)eblocks * (kValNT * kValPer);
+    for (int64_t e0 = blockIdx.x * (int64_t)(kValNT * kValPer); e0 < nnz; e0 += stride) {
+      int64_t r[kValPer], next[kValPer];
+#pragma unroll
+      for (int u = 0; u < kValPer; ++u) {
+        const int64_t e = e0 + u * kValNT + threadIdx.x;
+        r[u] = ir[min(e, nnz - 1)];
+        next[u] = ir[min(e + 1, nnz - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < kValPer; ++u) {
+        pin(r[u]);
+        pin(next[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kValPer; ++u) {
+        const int64_t e = e0 + u * kValNT + threadIdx.x;
+        bad += e < nnz && (r[u] < 0 || r[u] >= nrows);
+        desc += e + 1 < nnz && next[u] <= r[u];
+        if (rows32 && e < nnz) rows32[e] = (int32_t)r[u];
+      }
     }
     block_add_counts<kValNT>(bad, desc, &cnt[0], &cnt[1]);
   } else {  // columns
@@ -346,11 +360,11 @@ __global__ void k_validate_flag(const unsigned long long* __restrict__ cnt, int 
 
 // Launches the validation of X on s; cnt: 3 device counters, cleared before.
 static cbx_status launch_validate(const cbx_dcsc* X, int32_t* rows32, unsigned long long* cnt, hipStream_t s) {
-  auto blocks = [](int64_t n) {
-    return (unsigned)std::min<int64_t>(std::max<int64_t>((n + kValNT - 1) / kValNT, 1), kValBlocks);
+  auto blocks = [](int64_t n, int per) {
+    return (unsigned)std::min<int64_t>(std::max<int64_t>((n + kValNT * per - 1) / (kValNT * per), 1), kValBlocks);
   };
-  const unsigned eb = blocks(X->nnz);
-  k_validate<<<eb + blocks(X->nzc), kValNT, 0, s>>>(X->cp, X->jc, X->ir, X->nzc, X->nnz, X->m, X->n, (int)eb, rows32,
+  const unsigned eb = blocks(X->nnz, kValPer);
+  k_validate<<<eb + blocks(X->nzc, 1), kValNT, 0, s>>>(X->cp, X->jc, X->ir, X->nzc, X->nnz, X->m, X->n, (int)eb, rows32,
                                                     cnt);
   CBX_HIP(hipGetLastError());
   return CBX_OK;
@@ -1098,23 +1112,56 @@ __global__ __launch_bounds__(256) void k_tiny(const int32_t* __restrict__ order,
   }
 }
 
-// Staged tiny columns into place: one wave per column copies its nnzcol[col]
-// entries from its staging slot to cpC[col].
+// Staged tiny columns into place: a wave copies the nnzcol[col] entries of 16
+// columns from their staging slots to cpC[col], four columns' first 64 entries
+// in flight together (one column per wave waited for its place, then for its
+// entries: 0.60 ms for the two products of 16 Galerkin triples, now 0.40).
+constexpr int kPlaceCols = 16;
 template <class T>
-__global__ void k_tiny_place(const int32_t* __restrict__ order, int64_t first, int64_t ncols,
-                             const int64_t* __restrict__ stage_off, const int64_t* __restrict__ nnzcol,
-                             const int64_t* __restrict__ cpC, const int64_t* __restrict__ sir,
-                             const T* __restrict__ sval, int64_t* __restrict__ irC, T* __restrict__ valC,
-                             Filter<T> flt = {}, int* __restrict__ err = nullptr) {
-  const int64_t i = global_wave();
-  if (i >= ncols) return;
-  const int col = order[first + i];
-  const int64_t src = stage_off[i], dst = cpC[col], cnt = nnzcol[col];
-  for (int64_t e = lane_id(); e < cnt; e += kWave) {
-    irC[dst + e] = sir[src + e];
-    valC[dst + e] = sval[src + e];
+__global__ __launch_bounds__(256) void k_tiny_place(
+    const int32_t* __restrict__ order, int64_t first, int64_t ncols, const int64_t* __restrict__ stage_off,
+    const int64_t* __restrict__ nnzcol, const int64_t* __restrict__ cpC, const int64_t* __restrict__ sir,
+    const T* __restrict__ sval, int64_t* __restrict__ irC, T* __restrict__ valC, Filter<T> flt = {},
+    int* __restrict__ err = nullptr) {
+  constexpr int U = 4;
+  const int64_t i0 = global_wave() * kPlaceCols;
+  if (i0 >= ncols) return;
+  const int lane = lane_id(), n = (int)min<int64_t>(ncols - i0, kPlaceCols);
+  const int64_t mine = i0 + min(lane, n - 1);
+  const int col = order[first + mine];
+  const int64_t src = stage_off[mine], dst = cpC[col];
+  const int cnt = lane < n ? (int)nnzcol[col] : 0;
+  if (flt.on && lane < n) filter_add_run(flt, dst, cnt, col, err);  // staged entries are the kept ones
+  for (int c = 0; c < n; c += U) {
+    int64_t s[U], d[U], r[U];
+    T v[U];
+    int k[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      s[u] = readlane_ll(src, c + u);
+      d[u] = readlane_ll(dst, c + u);
+      k[u] = __builtin_amdgcn_readlane(cnt, c + u);
+      const int64_t e = lane < k[u] ? s[u] + lane : 0;
+      r[u] = sir[e];
+      v[u] = sval[e];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      pin(r[u]);
+      pin(v[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (lane < k[u]) {
+        irC[d[u] + lane] = r[u];
+        valC[d[u] + lane] = v[u];
+      }
+      for (int e = kWave + lane; e < k[u]; e += kWave) {
+        irC[d[u] + e] = sir[s[u] + e];
+        valC[d[u] + e] = sval[s[u] + e];
+      }
+    }
   }
-  if (flt.on && lane_id() == 0) filter_add_run(flt, dst, (int)cnt, col, err);  // staged entries are the kept ones
 }
 
 // -------------------------------------------------------- symbolic: dense
@@ -3407,7 +3454,7 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   const int S = use_units ? S4 : S16;
   const int G = kSymRBW * 32 / TR;  // tiles per symbolic pass of the streaming tier
 
-  int32_t *colmap = nullptr, *rowsA, *bpos, *order_s, *P = nullptr;
+  int32_t *colmap = nullptr, *rowsA = nullptr, *bpos, *order_s, *P = nullptr;
   Counters* ctr;
   int64_t *stage_off, *stage_ir = nullptr;  // staged tiny tier (see the symbolic pass)
   T* stage_val = nullptr;
@@ -3417,7 +3464,7 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   const int64_t ctiles = (nzcB + kColTile - 1) / kColTile;
   CBX_TRY(dalloc(ws, 1, &ctr));
   if (nzcA != A->n) CBX_TRY(dalloc(ws, A->n, &colmap));
-  CBX_TRY(dalloc(ws, nnzA, &rowsA));
+  if (!cfg.rows_a) CBX_TRY(dalloc(ws, nnzA, &rowsA));
   CBX_TRY(dalloc(ws, nnzB, &bpos));
   CBX_TRY(dalloc(ws, nzcB + 1, &flop));
   CBX_TRY(dalloc(ws, nzcB, &flop_s));
@@ -3444,7 +3491,8 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   // column map, 32-bit rows, B->A positions, products and order of the columns
   k_init<<<(unsigned)std::min<int64_t>(1024, nblk(std::max<int64_t>({colmap ? A->n : 1, nzcB + 1, 1024}), 256)), 256, 0,
            s>>>(ctr, colmap, A->n, flop, nnzcol, nzcB);
-  if (cfg.trusted_a) k_rows32<<<nblk(nnzA, 256), 256, 0, s>>>(A->ir, nnzA, rowsA);
+  if (cfg.rows_a) rowsA = const_cast<int32_t*>(cfg.rows_a);
+  else if (cfg.trusted_a) k_rows32<<<nblk(nnzA, 256), 256, 0, s>>>(A->ir, nnzA, rowsA);
   else CBX_TRY(launch_validate(A, rowsA, ctr->val, s));
   const bool same = A->cp == B->cp && A->jc == B->jc && A->ir == B->ir && nzcA == nzcB && nnzA == nnzB &&
                     A->m == B->m && A->n == B->n;  // A*A: one look will do
@@ -3702,7 +3750,7 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
     k_num_sort<K, T, 256><<<(unsigned)n_h2, 256, 0, s>>>(order_s, hb[1], nnzcol, B->cp, bpos, valB, A->cp, rowsA, valA,
                                                         cpC, C->ir, (T*)C->val, err, flt);
   if (n_h256 && tiny_staged)
-    k_tiny_place<T><<<wave_grid(n_h256), 256, 0, s>>>(order_s, hb[2], n_h256, stage_off, nnzcol, cpC, stage_ir,
+    k_tiny_place<T><<<wave_grid((n_h256 + kPlaceCols - 1) / kPlaceCols), 256, 0, s>>>(order_s, hb[2], n_h256, stage_off, nnzcol, cpC, stage_ir,
                                                        stage_val, C->ir, (T*)C->val, flt, err);
   else if (n_h256)
     launch_tiny<K, T, false>(cfg, order_s, hb[2], n_h256, B->cp, bpos, valB, A->cp, rowsA, valA, nnzcol, cpC, C->ir,
