@@ -84,8 +84,7 @@ template <class T>
 __global__ __launch_bounds__(256) void k_mcl_stats(const int64_t* __restrict__ cp, const T* __restrict__ val,
                                                    int64_t nzc, T thr, int64_t select, int64_t recover, double pct,
                                                    T* __restrict__ cut, int64_t* __restrict__ cnt,
-                                                   int32_t* __restrict__ job, int32_t* __restrict__ jobs,
-                                                   int32_t* __restrict__ npos, unsigned long long* __restrict__ counters) {
+                                                   int32_t* __restrict__ job, int32_t* __restrict__ npos) {
   const int64_t q = global_wave();
   if (q >= nzc) return;  // whole wave
   const int lane = lane_id();
@@ -98,10 +97,9 @@ __global__ __launch_bounds__(256) void k_mcl_stats(const int64_t* __restrict__ c
   for (int64_t p0 = b; p0 < e; p0 += kWave * kUnroll) {
     T v[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int64_t p = p0 + u * kWave + lane;
-      v[u] = p < e ? val[p] : thr;  // thr: counted as kept, not as above the threshold
-    }
+    for (int u = 0; u < kUnroll; ++u) v[u] = val[min(p0 + u * kWave + lane, e - 1)];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) pin(v[u]);
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       if (p0 + u * kWave + lane >= e) continue;
@@ -124,12 +122,33 @@ __global__ __launch_bounds__(256) void k_mcl_stats(const int64_t* __restrict__ c
     npos[q] = (int32_t)nP;
     cut[q] = thr;
     cnt[q] = nK;
-    if (j != kJobNone) {
-      const unsigned long long slot = atomicAdd(&counters[0], 1ull);
-      jobs[slot] = (int32_t)q;
-      atomicAdd(&counters[j], 1ull);
-    }
   }
+}
+
+// The job columns' list (counters[0] long) and how many of either kind: three
+// atomics per 256 columns (two per job column, all on the same words, were most
+// of k_mcl_stats where many columns are selected: 8.0 ms of an expansion of 500 K
+// columns, now ZZ).
+constexpr int kJobsNT = 256;
+__global__ __launch_bounds__(kJobsNT) void k_mcl_jobs(const int32_t* __restrict__ job, int64_t nzc,
+                                                      int32_t* __restrict__ jobs,
+                                                      unsigned long long* __restrict__ counters) {
+  __shared__ int wsum[kJobsNT / kWave];
+  __shared__ unsigned long long s_base;
+  const int64_t q = blockIdx.x * (int64_t)kJobsNT + threadIdx.x;
+  const int j = q < nzc ? job[q] : kJobNone;
+  int total;
+  // jobs in the low half, recoveries above
+  const int at = block_excl_scan<kJobsNT>(j == kJobNone ? 0 : j == kJobRecover ? 0x10001 : 1, wsum, total);
+  const int all = total & 0xffff, rec = total >> 16;
+  if (all == 0) return;
+  if (threadIdx.x == 0) {
+    s_base = atomicAdd(&counters[0], (unsigned long long)all);
+    if (rec) atomicAdd(&counters[kJobRecover], (unsigned long long)rec);
+    if (all > rec) atomicAdd(&counters[kJobSelect], (unsigned long long)(all - rec));
+  }
+  __syncthreads();
+  if (j != kJobNone) jobs[s_base + (at & 0xffff)] = (int32_t)q;
 }
 
 // k-th largest (1-based, k <= N) of v[0..N) by MSB-first radix select over
@@ -218,19 +237,28 @@ __global__ __launch_bounds__(NT) void k_mcl_select(const int64_t* __restrict__ c
     if (threadIdx.x == 0) ncand = 0;
     __syncthreads();
     const int lane = lane_id();
-    for (int64_t p0 = 0; p0 < N; p0 += NT) {
-      const int64_t p = p0 + threadIdx.x;
-      T x = T(0);
-      bool take = false;
-      if (p < N) {
-        x = v[p];
-        take = !(x <= thr);
+    constexpr int U = 8;  // loads of a thread in flight together
+    for (int64_t p0 = 0; p0 < N; p0 += NT * U) {
+      T x[U];
+      unsigned long long m[U];
+      int total = 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = v[min(p0 + u * NT + threadIdx.x, N - 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) pin(x[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        m[u] = __ballot(p0 + u * NT + threadIdx.x < N && !(x[u] <= thr));
+        total += __popcll(m[u]);
       }
-      const unsigned long long m = __ballot(take);
       int base = 0;
-      if (lane == 0 && m) base = atomicAdd(&ncand, __popcll(m));
-      base = __shfl(base, 0, kWave);
-      if (take) cand[base + __popcll(m & ((1ull << lane) - 1ull))] = x;
+      if (lane == 0 && total) base = atomicAdd(&ncand, total);
+      base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if ((m[u] >> lane) & 1ull) cand[base + __popcll(m[u] & ((1ull << lane) - 1ull))] = x[u];
+        base += __popcll(m[u]);
+      }
     }
     __syncthreads();
   }
@@ -304,22 +332,29 @@ __global__ __launch_bounds__(256) void k_mcl_write(const int64_t* __restrict__ c
   const int64_t end_w = w + cnt[q];
   for (int64_t base0 = b; base0 < e && w < end_w; base0 += kWave * kUnroll) {
     T v[kUnroll];
+    int64_t r[kUnroll];
+    unsigned long long m[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int64_t p = base0 + u * kWave + lane;
-      v[u] = p < e ? val[p] : T(0);
-    }
+    for (int u = 0; u < kUnroll; ++u) v[u] = val[min(base0 + u * kWave + lane, e - 1)];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) pin(v[u]);
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       const int64_t p = base0 + u * kWave + lane;
       const bool keep = p < e && !(v[u] < c);
-      const unsigned long long m = __ballot(keep);
-      if (keep) {
-        const int64_t at = w + __popcll(m & ((1ull << lane) - 1ull));
-        oir[at] = ir[p];
+      m[u] = __ballot(keep);
+      r[u] = ir[keep ? p : b];
+    }
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) pin(r[u]);
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      if ((m[u] >> lane) & 1ull) {
+        const int64_t at = w + __popcll(m[u] & ((1ull << lane) - 1ull));
+        oir[at] = r[u];
         oval[at] = v[u];
       }
-      w += __popcll(m);
+      w += __popcll(m[u]);
     }
   }
   if (lane == 0) {
@@ -411,7 +446,8 @@ static cbx_status mcl_prune_typed(const cbx_dcsc* C, double thr_d, int64_t selec
   CBX_HIP(hipMemsetAsync(flag + nzc, 0, sizeof(int32_t), s));
   if (nzc) {
     k_mcl_stats<T><<<wave_grid(nzc), 256, 0, s>>>(C->cp, (const T*)C->val, nzc, thr, select, recover,
-                                                              pct, cut, cnt, job, jobs, npos, counters);
+                                                              pct, cut, cnt, job, npos);
+    k_mcl_jobs<<<nblocks(nzc, kJobsNT), kJobsNT, 0, s>>>(job, nzc, jobs, counters);
     CBX_HIP(hipGetLastError());
   }
   unsigned long long hc[4] = {0, 0, 0, 0};

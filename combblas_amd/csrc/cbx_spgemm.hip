@@ -3320,18 +3320,40 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
 }
 
 // Gather of the fused threshold's runs: run k (in start order) moves its kept
-// entries from its start in the unfiltered layout to dst[k].
+// entries from its start in the unfiltered layout to dst[k], one wave per run.
 template <class T>
 __global__ __launch_bounds__(256) void k_run_copy(const int32_t* __restrict__ idx, const int64_t* __restrict__ src,
                                                   const int32_t* __restrict__ kept, const int64_t* __restrict__ dst,
                                                   const int64_t* __restrict__ ir, const T* __restrict__ val,
-                                                  int64_t* __restrict__ ir2, T* __restrict__ val2) {
-  const int i = idx[blockIdx.x];
-  const int64_t a = src[i], d = dst[blockIdx.x];
+                                                  int nrun, int64_t* __restrict__ ir2, T* __restrict__ val2) {
+  const int k = (int)global_wave();
+  if (k >= nrun) return;
+  const int i = idx[k];
+  const int64_t a = src[i], d = dst[k];
   const int n = kept[i];
-  for (int e = threadIdx.x; e < n; e += 256) {
-    ir2[d + e] = ir[a + e];
-    val2[d + e] = val[a + e];
+  constexpr int U = 8;  // entries of a lane in flight together
+  for (int e0 = lane_id(); e0 < n; e0 += kWave * U) {
+    int64_t r[U];
+    T v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = min(e0 + u * kWave, n - 1);
+      r[u] = ir[a + e];
+      v[u] = val[a + e];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      pin(r[u]);
+      pin(v[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = e0 + u * kWave;
+      if (e < n) {
+        ir2[d + e] = r[u];
+        val2[d + e] = v[u];
+      }
+    }
   }
 }
 
@@ -3395,8 +3417,8 @@ static cbx_status filter_compact(const Filter<T>& flt, int64_t nzcB, int64_t* nn
     dev_free(ir2);
     return set_error(CBX_ERR_NOMEM, "cbx_spgemm: allocation of the thresholded product failed");
   }
-  if (nrun) k_run_copy<T><<<(unsigned)nrun, 256, 0, s>>>(i2, flt.run_src, flt.run_kept, dst, C->ir, (const T*)C->val,
-                                                        ir2, (T*)val2);
+  if (nrun) k_run_copy<T><<<wave_grid(nrun), 256, 0, s>>>(i2, flt.run_src, flt.run_kept, dst, C->ir, (const T*)C->val,
+                                                         (int)nrun, ir2, (T*)val2);
   CBX_HIP(hipGetLastError());
   CBX_HIP(hipStreamSynchronize(s));
   dev_free(C->ir);
