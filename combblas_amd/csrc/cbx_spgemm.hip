@@ -2458,7 +2458,7 @@ __device__ __forceinline__ int cut_units(int col, float pred, float flop, int lo
   float acc = 0.f, accf = 0.f;
   for (int b = lo; b <= hi; ++b) {
     const float e = scale * distinct_rows(flop, w[b]), ef = flop * w[b];
-    if (ef >= direct_flop) {  // more products than a unit holds in registers: a block of its own, one sweep
+    if (ef >= direct_flop) {  // a block of its own, one sweep
       if (b > start) {
         if (out) out[n] = UnitL{col, start, b};
         ++n;
@@ -2934,8 +2934,13 @@ constexpr int kSymBandNT = 256;                     // banded symbolic pass
 constexpr int kLightNT = 512, kLightK = 3264, kLightDR = 4096, kLightRB = 16;
 constexpr int kHeavyNT = 1024, kHeavyK = 13056, kHeavyDR = 16384, kHeavyRB = 16;
 // learned units: the light units' workgroup shape and window, cut to
-// target * 3264 predicted outputs
-constexpr int kLearnNT = 512, kLearnK = kLightK, kLearnRB = kLightRB, kLearnCR = 2;
+// target * 3264 predicted outputs.  One round of products stays in registers
+// between the sweeps: two spill at the 80 registers of three workgroups per CU
+// (R-MAT s17, int64: 4.5 ms in k_num_learned, 3.7 with one).
+constexpr int kLearnNT = 512, kLearnK = kLightK, kLearnRB = kLightRB, kLearnCR = 1;
+// Expected products from which a block forms a unit of its own, accumulated in
+// one sweep (half of it measured 3.9 ms).
+constexpr int kLearnDirect = 8 * kLearnNT;
 constexpr int kLearnFlopCap = 131072;  // expected products per learned unit
 constexpr int64_t kLearnChunk = 1 << 21;  // workgroups per learned launch
 // Tiny tier launch: `waves` columns (one wave each) per workgroup, grid-stride
@@ -3111,9 +3116,7 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   const float target = cfg.learned_target * (float)kLearnK;
   const float heavy_pred = (float)cfg.heavy_nnz;
   const float fcap = (float)kLearnFlopCap;
-  // a block expected to hold more products than a unit keeps in registers
-  // between its sweeps becomes a single-block unit, accumulated in one sweep
-  const float direct_flop = (float)(kLearnCR * 4 * kLearnNT);
+  const float direct_flop = (float)kLearnDirect;
   k_learned_units<<<nblk(nzcB, 256), 256, 0, s>>>(flop, nzcB, cfg.small_flop_max, logpred, blo, bhi, w, target,
                                                   heavy_pred, fcap, kLearnRB, direct_flop, m, nullptr, ucount,
                                                   nullptr, pred_nnz, heavy_flag);
