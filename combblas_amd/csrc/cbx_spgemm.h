@@ -11,21 +11,22 @@ namespace cbx {
 
 // Tunables of the SpGEMM driver.
 struct SpgemmConfig {
-  // Columns with flop_j <= small_flop_max use the LDS hash tier, the rest the
-  // row-tiled dense tier.  At most 4096 (the largest hash table holds 8192
-  // slots and is kept at most half full).
+  // Columns with flop_j <= small_flop_max are formed by one workgroup (sort
+  // tier), the rest by row-range units.  At most 4096 (four products per thread
+  // of the largest workgroup; the counting hash table of 8192 slots is kept at
+  // most half full).
   int64_t small_flop_max = 4096;
-  // Hash tier table sizes: flop_j in (hash_mid_flop, small_flop_max] use the
-  // 8192-slot table, (tiny_flop, hash_mid_flop] the 2048-slot table (each
-  // table kept at most half full); columns with flop_j <= tiny_flop (<= 256)
-  // take one wave each (the tiny tier).
+  // Sort tier sizes: flop_j in (hash_mid_flop, small_flop_max] are counted in
+  // the 8192-slot table and sorted by 512 threads (1024 beyond 2048 products),
+  // (tiny_flop, hash_mid_flop] in the 2048-slot table by 256; columns with
+  // flop_j <= tiny_flop (<= 256) take one wave each (the tiny tier).
   int64_t hash_mid_flop = 1024;
   int64_t tiny_flop = 256;
   // Learned mode: columns predicted to exceed heavy_nnz outputs are computed
   // exactly (symbolic, then two-phase units).
   int64_t heavy_nnz = 65536;
   // Unit tier: columns whose exact output exceeds unit_split_nnz use the
-  // large (16384-output) units.
+  // large units.
   int64_t unit_split_nnz = 131072;
   // Learned mode: device parameters of the nnz predictor (null = not loaded),
   // unit size target as a fraction of the value window, and the headroom of

@@ -10,18 +10,18 @@
 // This file keeps those phases but maps them to the GPU as follows.
 //
 // Column tiers (by flop_j, after sorting columns by flop descending):
-//   hash tier  flop_j <= small_flop_max: one workgroup per column; the rows
+//   tiny tier  flop_j <= tiny_flop: one wave per column (k_tiny).
+//   sort tier  flop_j <= small_flop_max: one workgroup per column; the rows
 //              are counted in an LDS linear-probing hash table, and the
 //              products sorted by row in LDS (k_num_sort).
-//   dense tier the rest: one workgroup per column walks the rows in tiles of
-//              TR rows; each tile accumulates into a dense LDS array with a
-//              presence bitmap and is emitted in row order by a block scan
-//              of the bitmap, so no sort is needed.  The A-entries of a tile
-//              are found through a precomputed tile-pointer table
-//              P[a][s] = #entries of A's a-th stored column with row < s*TR.
-// Within every wave, the A-column segments of up to 64 B entries are
-// flattened with a prefix sum so that all 64 lanes work on products even
-// when most segments are short (R-MAT columns are).
+//   unit tier  the rest: a symbolic pass cuts each column into row ranges
+//              (units) of one workgroup each, which accumulate in LDS.  The
+//              A entries of a row range are found through a precomputed
+//              tile-pointer table.  (Matrices taller than 2^24 rows walk
+//              dense row tiles per column instead.)
+// The A-column segments of a workgroup's B entries are flattened, so that all
+// lanes work on products even when most segments are short (R-MAT columns
+// are).
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -103,7 +103,7 @@ __device__ __forceinline__ int ceil_log2_dev(long long x) {
 constexpr int kBR = 4096;        // rows per block (also the tile-pointer granularity)
 constexpr int kBRW = kBR / 32;   // 32-bit bitmap words per block
 // Row lists (k_sym_units) cover the blocks with at most this many outputs:
-// sixteen denser blocks already fill a 4096-output unit, so a unit holding a
+// sixteen denser blocks already fill a small unit, so a unit holding a
 // denser block spans at most 16 blocks and takes its ranks from a bitmap.
 constexpr int kListBlockMax = 256;
 
@@ -2858,14 +2858,13 @@ __global__ void k_unit_permute(const Unit* __restrict__ src, const int32_t* __re
   if (i < n) dst[i] = src[idx[i]];
 }
 
-// A copy of units[0, n) sorted by blk_lo (stable), kept in `keep`.
 __global__ void k_gather_flop(const int32_t* __restrict__ cols, int64_t n, const int64_t* __restrict__ flop,
                               int64_t* __restrict__ key) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < n) key[i] = flop[cols[i]];
 }
 
-// Reorders cols[0..n) by descending flop (into `keep`, returned in *out), so a
+// Reorders cols[0..n) by descending flop (into *out), so a
 // per-column launch over them starts its longest columns first, as the
 // two-phase path's flop-sorted order does.
 cbx_status sort_cols_by_flop(const int32_t* cols, int64_t n, const int64_t* flop, ScratchSet& ws, int32_t** out) {
@@ -2884,6 +2883,7 @@ cbx_status sort_cols_by_flop(const int32_t* cols, int64_t n, const int64_t* flop
   return CBX_OK;
 }
 
+// A copy of units[0, n) sorted by blk_lo (stable), in *out.
 cbx_status sort_units_by_block(const Unit* units, int n, int S, ScratchSet& ws, Unit** out) {
   hipStream_t s = ws.s;
   int32_t *k1, *k2, *i1, *i2;

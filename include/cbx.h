@@ -180,19 +180,21 @@ enum {
  * workload by combblas_amd/autotune.py; defaults {4096, 1024, 256, 65536,
  * 131072, 0.75, 0.15, 0.25, 4, 1, 0, 0, 1, 1, 0}. */
 typedef struct cbx_spgemm_config {
-  int64_t hash_max_flop;   /* columns with flop_j <= this use the LDS hash tier (<= 4096) */
-  int64_t hash_mid_flop;   /* ... with flop_j > this use the 8192-slot table, else the 2048-slot one (<= 1024) */
-  int64_t tiny_flop;       /* columns with flop_j <= this take one wave each, sorted in registers (<= 256) */
+  int64_t hash_max_flop;   /* columns with flop_j <= this are formed by one workgroup in LDS: counted by a hash
+                              table, their products sorted (<= 4096) */
+  int64_t hash_mid_flop;   /* ... with flop_j > this by 512 or (above 2048) 1024 threads and an 8192-slot table,
+                              else by 256 threads and a 2048-slot one (<= 1024) */
+  int64_t tiny_flop;       /* columns with flop_j <= this take one wave each (<= 256) */
   int64_t heavy_nnz;       /* learned mode: columns predicted to hold more outputs are computed exactly (symbolic
                               pass, then two-phase units) after the single pass (>= 4096) */
-  int64_t unit_split_nnz;  /* unit tier: columns with more (exact) outputs use the 16384-output units, the
-                              others the 4096-output ones (>= 4096) */
-  float learned_target;    /* learned mode: predicted outputs per unit as a fraction of the 4096-output value
+  int64_t unit_split_nnz;  /* unit tier: columns with more (exact) outputs use the large units (13056 outputs
+                              or 16384 rows), the others the small ones (3264 or 4096; >= 4096) */
+  float learned_target;    /* learned mode: predicted outputs per unit as a fraction of the 3264-output value
                               window; above 1 units are cut larger than their window and re-swept in windows
                               (exact, slower) */
   float capacity_margin;   /* learned mode: output capacity headroom over the predicted total */
   float row_map_share;     /* two-phase mode: at most this share of the free device memory holds the symbolic
-                              pass's row maps of the columns that can form 16384-output units, which those
+                              pass's row maps of the columns that can form large units, which those
                               units then read instead of rebuilding them (0 disables; in [0, 1]) */
   int32_t tiny_wg_waves;   /* workgroup shape of the tiny tier: columns (one wave each) per workgroup, 1, 2 or 4 */
   int32_t unit_order;      /* order of the exactly sized row-range units in the numeric pass: 0 as the symbolic
@@ -339,7 +341,7 @@ cbx_status cbx_spmspv(const cbx_dcsc* A, const int32_t* xind, const void* xval, 
  * it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments, results and errors as cbx_spmspv; the structure check of A and
- * every scratch array (column map, dense accumulator, bitmap, scan storage)
+ * every scratch array (column map, dense accumulator, bitmap, lists)
  * live in one static device array of CBX_SPMSPV_NOALLOC_SCRATCH_BYTES per GPU,
  * kept until the process ends.  It needs about 4*n + sizeof(value)*m + m/4
  * bytes plus a few KiB (12.4 MiB for m = n = 2^20 with 8-byte values); a
