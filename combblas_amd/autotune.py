@@ -1,7 +1,7 @@
 """Autotuner for the SpGEMM tunables (cbx_spgemm_set_config).
 
 The reference hard-codes its bin switch and hash-table sizing
-(mtSpGEMM.h:311, :366-367).  Here the flop bound of the LDS hash tier, the
+(mtSpGEMM.h:311, :366-367).  Here the flop bound of the LDS sort tier, the
 flop bounds of its table sizes (the LDS table sizes), the tiny tier's bound
 and workgroup shape, the output size that sends a column to the large units
 (the other unit workgroup shape) and the learned pass's unit target and
@@ -108,20 +108,19 @@ def _mcl_workload(n: int, mode: str):
 
 
 GRID = {
-    "hash_max_flop": [1024, 2048],
+    "hash_max_flop": [1024, 2048, 4096],
     "hash_mid_flop": [1024],
     "tiny_flop": [256],
     "unit_split_nnz": [131072, 262144],
     "unit_order": [1],
-    "tiny_algo": [0, 1],
     "sym_band": [0, 16],
     "unit_lists": [0, 1],
     "unit_xcd_group": [0, 32],
 }
-# the learned single pass adds its own knobs; the hash tiers are swept more
+# the learned single pass adds its own knobs; the lower tiers are swept more
 # coarsely there to keep the product of the grids small
 LEARNED_GRID = {
-    "hash_max_flop": [1024, 2048],
+    "hash_max_flop": [1024, 4096],
     "hash_mid_flop": [1024],
     "tiny_flop": [256],
     "unit_split_nnz": [131072],
@@ -131,16 +130,15 @@ LEARNED_GRID = {
     "unit_lists": [0, 1],
 }
 # Galerkin columns hold 216 (A*T) and 64 (S*(A*T)) products: the tiny tier's
-# bound, form and workgroup shape decide where they run
+# bound and workgroup shape decide where they run
 GALERKIN_GRID = {
     "tiny_flop": [128, 256],
     "hash_mid_flop": [256, 1024],
     "tiny_wg_waves": [1, 2, 4],
-    "tiny_algo": [0, 1],
 }
 MCL_GRID = {
-    "hash_max_flop": [1024, 2048],
-    "unit_split_nnz": [262144],
+    "hash_max_flop": [1024, 2048, 4096],
+    "unit_split_nnz": [131072, 262144],
     "sym_band": [0, 16],
     "mcl_fuse": [0, 1],
     "unit_lists": [0, 1],
@@ -150,7 +148,6 @@ MCL_GRID = {
 MERGE_GRID = {
     "hash_max_flop": [1024, 2048, 4096],
     "hash_mid_flop": [1024],
-    "tiny_algo": [0, 1],
     "unit_lists": [0, 1],
 }
 MCL_LEARNED_GRID = {
