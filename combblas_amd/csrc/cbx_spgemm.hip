@@ -816,8 +816,9 @@ __global__ __launch_bounds__(NT) void k_sym_hash(const int32_t* __restrict__ ord
 // A bitonic network over the 256 elements in registers took some 430
 // cross-lane moves through LDS a column whatever its distinct rows: 4.0 ms for
 // the two products of 16 Galerkin blocks (4.1e5 columns each of 216 and 64
-// products, FP64); this takes 1.45 ms.  Bound by LDS latency at seven waves per
-// SIMD (23 KB for four waves).
+// products, FP64); this takes 1.2 ms (1.7 with the loads of one register waited
+// for before the next's are issued).  Bound by LDS latency at six waves per SIMD
+// (27 KB for four waves).
 constexpr int kTinyMax = 256;
 constexpr int kTinyHash = 2 * kTinyMax;  // slots per wave at most
 constexpr int kTinyWaves = 4;            // waves per workgroup at most (launch bound 256)
@@ -882,27 +883,39 @@ __device__ __forceinline__ int tiny_gather(L& ws, int64_t b0, int64_t b1, const 
     wave_lds_sync();
     const int end = min(filled + total, kTinyMax);
     int before = 0;
+    int32_t r[kE];
+    T a[kE], b[kE];
 #pragma unroll
     for (int u = 0; u < kE; ++u) {
+      r[u] = 0;
+      a[u] = b[u] = T{};
       const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)ws.starts[u]);
       const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(ws.starts[u] >> 32));
       // registers whose 64 elements miss this chunk's range stay as they are
       if ((u + 1) * kWave > filled && u * kWave < end) {
-        const int e = u * kWave + lane;
         const int s = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, (unsigned)before));
         // lanes outside repeat the chunk's first or last product
-        const int32_t idx = min(max(e, filled), end - 1) + ws.delta[s];
-        int32_t r = rowsA[idx];
-        pin(r);
-        const bool mine = e >= filled && e < end;
+        const int32_t idx = min(max(u * kWave + lane, filled), end - 1) + ws.delta[s];
+        r[u] = rowsA[idx];
         if constexpr (!SYM) {
-          T a = valA[idx], b = ws.bval[s];
-          pin(a);
-          if (mine) val[u] = SR::mul(a, b);
+          a[u] = valA[idx];
+          b[u] = ws.bval[s];
         }
-        if (mine) key[u] = r;
       }
       before += __popc(lo) + __popc(hi);
+    }
+#pragma unroll
+    for (int u = 0; u < kE; ++u) {
+      pin(r[u]);
+      if constexpr (!SYM) pin(a[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kE; ++u) {
+      const int e = u * kWave + lane;
+      if (e >= filled && e < end) {
+        key[u] = r[u];
+        if constexpr (!SYM) val[u] = SR::mul(a[u], b[u]);
+      }
     }
     filled += total;
     wave_lds_sync();  // the chunk's segments have been read
