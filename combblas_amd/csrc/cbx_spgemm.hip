@@ -465,25 +465,34 @@ __global__ __launch_bounds__(kFlopNT) void k_flops(const int64_t* __restrict__ c
   if (c && !(counts_valid(c->val) && counts_valid(c->val + 3))) return;
   const int64_t t0 = blockIdx.x * (int64_t)kFlopTile;
   const int n = (int)min((int64_t)kFlopTile, nnzB - t0);
+  // (each step's four loads in flight together)
+  int64_t k[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) k[u] = irB[t0 + min(u * kFlopNT + (int)threadIdx.x, n - 1)];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) pin(k[u]);
   int32_t p[4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int64_t k = irB[t0 + min(u * kFlopNT + (int)threadIdx.x, n - 1)];
-    p[u] = colmap ? colmap[k] : (int32_t)k;
-    pin(p[u]);
-  }
-  int l[4];
+  for (int u = 0; u < 4; ++u) p[u] = colmap ? colmap[k[u]] : (int32_t)k[u];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) pin(p[u]);
+  int64_t b[4], e[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int32_t q = max(p[u], 0);
-    l[u] = (int)(cpA[q + 1] - cpA[q]);
-    pin(l[u]);
+    b[u] = cpA[q];
+    e[u] = cpA[q + 1];
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    pin(b[u]);
+    pin(e[u]);
   }
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int i = u * kFlopNT + threadIdx.x;
     if (i < n) bpos[t0 + i] = p[u];
-    len[i] = i < n && p[u] >= 0 ? l[u] : 0;
+    len[i] = i < n && p[u] >= 0 ? (int)(e[u] - b[u]) : 0;
   }
   __syncthreads();
   const int4 v = reinterpret_cast<const int4*>(len)[threadIdx.x];
