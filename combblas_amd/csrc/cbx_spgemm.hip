@@ -33,6 +33,7 @@
 
 #include "cbx_device.h"
 #include "cbx_flatten.h"
+#include "cbx_index.h"
 #include "cbx_semiring.h"
 #include "cbx_spgemm.h"
 
@@ -2768,8 +2769,7 @@ __global__ __launch_bounds__(256) void k_learned_place(const UnitL* __restrict__
 
 // Tile pointers (Tiles): thread per stored A column and run of kTileRun tiles,
 // so a wave's stores cover 64 consecutive columns of one tile.  Each pointer
-// is searched for from the previous one, doubling the step: one or two probes
-// for the short segments of sparse columns, a logarithm for the long ones.
+// is searched for from the previous one.
 constexpr int kTileRun = 32;
 __global__ __launch_bounds__(256) void k_tiles(const int64_t* __restrict__ cpA, int64_t nzcA,
                                                const int32_t* __restrict__ rowsA, int S, int32_t* __restrict__ at) {
@@ -2779,18 +2779,7 @@ __global__ __launch_bounds__(256) void k_tiles(const int64_t* __restrict__ cpA, 
   int32_t lo = (int32_t)cpA[p];
   const int t0 = (int)blockIdx.y * kTileRun, t1 = min(S + 1, t0 + kTileRun);
   for (int t = t0; t < t1; ++t) {
-    const int64_t key = (int64_t)t * kBR;
-    int32_t step = 1, hi = lo;  // rows before lo are below key
-    while (hi < end && rowsA[hi] < key) {
-      lo = hi + 1;
-      hi = min(end, lo + step);
-      step = min(step * 2, 1 << 29);
-    }
-    while (lo < hi) {  // first entry in [lo, hi] with row >= key
-      const int32_t mid = lo + (hi - lo) / 2;
-      if (rowsA[mid] < key) lo = mid + 1;
-      else hi = mid;
-    }
+    lo = first_from([&](int32_t i) { return rowsA[i]; }, lo, end, (int64_t)t * kBR);
     at[t * nzcA + p] = lo;
   }
 }
