@@ -31,4 +31,12 @@ CBX_HD int32_t first_from(Row&& row, int32_t lo, int32_t end, int64_t key) {
   return lo;
 }
 
+// Entry `off` of those from `first` (below end) on, and whether there is one
+// (ok): past the end the last entry's index.
+CBX_HD int32_t entry_from(int32_t first, int32_t end, int32_t off, bool& ok) {
+  const int32_t left = end - first;
+  ok = off < left;
+  return first + (ok ? off : left - 1);
+}
+
 }  // namespace cbx

@@ -33,6 +33,7 @@
 
 #include "cbx_device.h"
 #include "cbx_flatten.h"
+#include "cbx_index.h"
 #include "cbx_semiring.h"
 #include "cbx_spgemm.h"
 
@@ -730,10 +731,8 @@ __global__ __launch_bounds__(NT) void k_bfs_expand_hubs(const int2* __restrict__
     bool ok[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int e = e0 + u * NT + (int)threadIdx.x;
-      ok[u] = e < rg.y;
       ks[u] = v;
-      r[u] = rows[min(e, rg.y - 1)];
+      r[u] = rows[entry_from(e0, rg.y, u * NT + (int)threadIdx.x, ok[u])];
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) pin(r[u]);

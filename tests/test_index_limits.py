@@ -44,3 +44,25 @@ int main() {
   }
 }
 """)
+
+
+def test_entries_of_a_piece_at_the_last_index(tmp_path):
+    """Pieces of 1024 entries of ranges that end at 2^31 - 1: every index lies in its piece."""
+    _run(tmp_path, r"""
+int main() {
+  const int32_t last = 0x7fffffff;
+  for (int32_t len : {1, 1023, 1024, 1025, 5000}) {
+    for (int32_t end : {last, last - 1, last - 1024, len}) {
+      for (int32_t first = end - len; end - first > 0; first += 1024) {
+        for (int32_t off = 0; off < 1024; ++off) {
+          bool ok;
+          const int32_t e = cbx::entry_from(first, end, off, ok);
+          CHECK(ok == ((int64_t)first + off < end));
+          CHECK(e == (ok ? first + off : end - 1));
+        }
+        if (end - first <= 1024) break;
+      }
+    }
+  }
+}
+""")
