@@ -132,6 +132,8 @@ def lib() -> C.CDLL:
         L.cbx_dcsc_transpose.argtypes = [P(cbx_dcsc), P(cbx_dcsc), C.c_void_p]
         L.cbx_dcsc_merge.argtypes = [C.c_int32, P(cbx_dcsc), C.c_int32, P(cbx_dcsc), C.c_void_p]
         L.cbx_dcsc_merge.restype = C.c_int32
+        L.cbx_dcsc_merge_in_ranges.argtypes = [C.c_int32, P(cbx_dcsc), C.c_int32, C.c_int64, P(cbx_dcsc), C.c_void_p]
+        L.cbx_dcsc_merge_in_ranges.restype = C.c_int32
         L.cbx_dcsc_from_coo.argtypes = [C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int32,
                                         C.c_int32, C.c_int32, P(cbx_dcsc), C.c_void_p]
         L.cbx_dcsc_from_coo.restype = C.c_int32
@@ -497,12 +499,18 @@ def transpose(X: DeviceDcsc, stream: int | None = None) -> DeviceDcsc:
     return DeviceDcsc(out)
 
 
-def merge(parts: list[DeviceDcsc], semiring: str = "plus_times", stream: int | None = None) -> DeviceDcsc:
-    """MultiwayMerge<SR> on the device: the semiring sum of same-shape parts (SUMMA's stage merge)."""
+def merge(parts: list[DeviceDcsc], semiring: str = "plus_times", stream: int | None = None,
+          max_entries: int | None = None) -> DeviceDcsc:
+    """MultiwayMerge<SR> on the device: the semiring sum of same-shape parts (SUMMA's stage merge).
+    max_entries: in column ranges of at most so many entries of the parts (cbx_dcsc_merge_in_ranges)."""
     if not parts:
         raise ValueError("merge needs at least one part")
     out = cbx_dcsc()
-    _check(lib().cbx_dcsc_merge(len(parts), _desc_array(parts), SEMIRINGS[semiring], C.byref(out), stream))
+    if max_entries is None:
+        _check(lib().cbx_dcsc_merge(len(parts), _desc_array(parts), SEMIRINGS[semiring], C.byref(out), stream))
+    else:
+        _check(lib().cbx_dcsc_merge_in_ranges(len(parts), _desc_array(parts), SEMIRINGS[semiring], int(max_entries),
+                                              C.byref(out), stream))
     return DeviceDcsc(out)
 
 

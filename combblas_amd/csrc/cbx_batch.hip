@@ -157,13 +157,13 @@ __global__ __launch_bounds__(kPackNT) void k_pack_cols(const PackSeg* __restrict
       if (q >= total) continue;
       const PackSeg& g = segs[one ? s0 : find_seg(count, q, off)];
       const int64_t i = q - g.c_off;
-      const int64_t b = g.cp[i], e = g.cp[i + 1], j = g.jc[i];
+      const int64_t b = g.cp[i] - g.nz_base, e = g.cp[i + 1] - g.nz_base, j = g.jc[i] - g.col_base;
       bool err = b < 0 || e < b || e > g.nnz || j < 0 || j >= g.n || (i == 0 && b != 0) ||
                  (i + 1 == g.nzc && e != g.nnz);
-      if (i + 1 < g.nzc) err |= g.jc[i + 1] <= j;
+      if (i + 1 < g.nzc) err |= g.jc[i + 1] - g.col_base <= j;
       bad += err;
       // a column start with another column's entry before it
-      if (!err && i > 0 && b > 0 && b < g.nnz && g.cp[i - 1] < b) desc += g.ir[b] <= g.ir[b - 1];
+      if (!err && i > 0 && b > 0 && b < g.nnz && g.cp[i - 1] - g.nz_base < b) desc += g.ir[b] <= g.ir[b - 1];
       cp[q] = b + g.nz_off;
       jc[q] = j + g.col_off;
     }
@@ -373,7 +373,8 @@ static cbx_status pack(const cbx_dcsc* X, int64_t count, cbx_dcsc* out, DevMem* 
   std::vector<PackSeg> segs(count);
   int64_t m = 0, n = 0, nnz = 0, nzc = 0;
   for (int64_t i = 0; i < count; ++i) {
-    segs[i] = PackSeg{X[i].cp, X[i].jc, X[i].ir, X[i].val, m, n, nnz, nzc, X[i].m, X[i].n, X[i].nnz, X[i].nzc};
+    segs[i] = PackSeg{X[i].cp, X[i].jc, X[i].ir, X[i].val, m, n, nnz, nzc, X[i].m, X[i].n, X[i].nnz, X[i].nzc,
+                      0, 0};
     m += X[i].m;
     n += X[i].n;
     nnz += X[i].nnz;

@@ -85,43 +85,67 @@ T semiring_one() {
   }
 }
 
-template <int K, class T>
-cbx_status merge_typed(int32_t count, const cbx_dcsc* parts, cbx_dcsc* out, hipStream_t s) {
-  const int64_t m = parts[0].m, n = parts[0].n;
-  int64_t nnz = 0, nzc = 0;
-  for (int32_t i = 0; i < count; ++i) {
-    nnz += parts[i].nnz;
-    nzc += parts[i].nzc;
-  }
+// The product's kernels hold places in A's entries and A's stored columns as
+// 32-bit numbers: so many of either in one concatenation at most.
+constexpr int64_t kMergeMost = (1ll << 31) - 1;
+
+// A matrix to merge, or a range of its columns (entries from nz_base on, column
+// ids from col_base on).
+struct MergePart {
+  const int64_t *cp, *jc, *ir;
+  const void* val;
+  int64_t nnz, nzc, nz_base, col_base;
+};
+
+struct MergeResult {
+  cbx_dcsc x{};
+  MergeResult() = default;
+  MergeResult(MergeResult&& o) noexcept : x(o.x) { o.x = cbx_dcsc{}; }
+  MergeResult(const MergeResult&) = delete;
+  ~MergeResult() { cbx_dcsc_free(&x); }
+  MergePart part() const { return MergePart{x.cp, x.jc, x.ir, x.val, x.nnz, x.nzc, 0, 0}; }
+};
+
+cbx_status merge_empty(int64_t m, int64_t n, cbx_dtype dtype, cbx_dcsc* out, hipStream_t s) {
   std::memset(out, 0, sizeof(*out));
   out->m = m;
   out->n = n;
-  out->dtype = parts[0].dtype;
+  out->dtype = dtype;
   out->location = CBX_DEVICE;
-  if (nnz == 0) {  // an empty m x n matrix
-    cbx_status st = CBX_OK;
-    if ((st = dev_alloc((void**)&out->cp, sizeof(int64_t))) != CBX_OK ||
-        (st = dev_alloc((void**)&out->jc, sizeof(int64_t))) != CBX_OK ||
-        (st = dev_alloc((void**)&out->ir, sizeof(int64_t))) != CBX_OK ||
-        (st = dev_alloc(&out->val, sizeof(int64_t))) != CBX_OK) {
-      cbx_dcsc_free(out);
-      return st;
-    }
-    CBX_HIP(hipMemsetAsync(out->cp, 0, sizeof(int64_t), s));
-    CBX_HIP(hipStreamSynchronize(s));
-    return CBX_OK;
+  cbx_status st = CBX_OK;
+  if ((st = dev_alloc((void**)&out->cp, sizeof(int64_t))) != CBX_OK ||
+      (st = dev_alloc((void**)&out->jc, sizeof(int64_t))) != CBX_OK ||
+      (st = dev_alloc((void**)&out->ir, sizeof(int64_t))) != CBX_OK ||
+      (st = dev_alloc(&out->val, sizeof(int64_t))) != CBX_OK) {
+    cbx_dcsc_free(out);
+    return st;
+  }
+  CBX_HIP(hipMemsetAsync(out->cp, 0, sizeof(int64_t), s));
+  CBX_HIP(hipStreamSynchronize(s));
+  return CBX_OK;
+}
+
+// The merge of n columns as one product.
+template <int K, class T>
+cbx_status merge_product(const std::vector<MergePart>& parts, int64_t m, int64_t n, cbx_dtype dtype, cbx_dcsc* out,
+                         hipStream_t s) {
+  const int64_t count = (int64_t)parts.size();
+  int64_t nnz = 0, nzc = 0;
+  for (const MergePart& P : parts) {
+    nnz += P.nnz;
+    nzc += P.nzc;
   }
   CBX_RETURN_IF((double)count * (double)n >= 9.0e18, CBX_ERR_LIMIT, "cbx_dcsc_merge: too many columns in the parts");
   cbx_dcsc A{}, B{};
   A.m = m;
-  A.n = (int64_t)count * n;
+  A.n = count * n;
   A.nnz = nnz;
   A.nzc = nzc;
-  A.dtype = B.dtype = parts[0].dtype;
+  A.dtype = B.dtype = dtype;
   A.location = B.location = CBX_DEVICE;
   B.m = A.n;
   B.n = n;
-  B.nnz = (int64_t)count * n;
+  B.nnz = count * n;
   B.nzc = n;
   ScratchSet ws(s);
   int64_t *cpA, *jcA, *cpB, *jcB, *irB;
@@ -141,16 +165,16 @@ cbx_status merge_typed(int32_t count, const cbx_dcsc* parts, cbx_dcsc* out, hipS
   // bounds (a column id beyond n would fall into the next part's block)
   std::vector<PackSeg> segs((size_t)count);
   int64_t eb = 0, qb = 0;
-  for (int32_t i = 0; i < count; ++i) {
-    const cbx_dcsc& P = parts[i];
-    segs[i] = PackSeg{P.cp, P.jc, P.ir, P.val, 0, (int64_t)i * n, eb, qb, m, n, P.nnz, P.nzc};
+  for (int64_t i = 0; i < count; ++i) {
+    const MergePart& P = parts[i];
+    segs[i] = PackSeg{P.cp, P.jc, P.ir, P.val, 0, i * n, eb, qb, m, n, P.nnz, P.nzc, P.nz_base, P.col_base};
     eb += P.nnz;
     qb += P.nzc;
   }
   cbx_status st = pack_members(segs.data(), count, A, rowsA, s);
   if (st != CBX_OK) return st;
   k_stacked_identity<T><<<(unsigned)((n + 1 + kMergeNT - 1) / kMergeNT), kMergeNT, 0, s>>>(
-      n, count, semiring_one<K, T>(), cpB, jcB, irB, valB);
+      n, (int)count, semiring_one<K, T>(), cpB, jcB, irB, valB);
   CBX_HIP(hipGetLastError());
   SpgemmConfig cfg = current_config();
   cfg.trusted_a = cfg.trusted_b = true;
@@ -159,6 +183,174 @@ cbx_status merge_typed(int32_t count, const cbx_dcsc* parts, cbx_dcsc* out, hipS
   st = spgemm_dispatch(&A, &B, sr, CBX_SPGEMM_TWO_PHASE, cfg, out, nullptr, s);
   if (st != CBX_OK) cbx_dcsc_free(out);
   return st;
+}
+
+// Of each part: its first stored column (x) at or after column id `col`, and
+// that column's first entry (y), both counted in the part's range.
+__global__ __launch_bounds__(kMergeNT) void k_merge_below(const MergePart* __restrict__ parts, int64_t count,
+                                                          int64_t col, longlong2* __restrict__ below) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= count) return;
+  const MergePart P = parts[i];
+  int64_t lo = 0, hi = P.nzc;
+  while (lo < hi) {
+    const int64_t mid = lo + (hi - lo) / 2;
+    if (P.jc[mid] - P.col_base < col) lo = mid + 1;
+    else hi = mid;
+  }
+  below[i] = make_longlong2(lo, P.nzc ? P.cp[lo] - P.nz_base : 0);
+}
+
+// A range's columns into the output's arrays at its place (cp: one more, the
+// next range's first or the end).
+__global__ __launch_bounds__(kMergeNT) void k_merge_columns(const int64_t* __restrict__ cp,
+                                                            const int64_t* __restrict__ jc, int64_t nzc,
+                                                            int64_t entries, int64_t first, int64_t* __restrict__ ocp,
+                                                            int64_t* __restrict__ ojc) {
+  const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (q > nzc) return;
+  ocp[q] = cp[q] + entries;
+  if (q < nzc) ojc[q] = jc[q] + first;
+}
+
+// The merge of n columns whose parts hold too much for one product: column
+// ranges that fit, one after the other, and their results one after the other
+// in the output.  A single column that does not fit is merged in two halves of
+// the parts first.  Nothing of the parts is trusted here beyond their sizes:
+// the cuts are checked below, and each range is checked as it is packed.
+template <int K, class T>
+cbx_status merge_columns(const std::vector<MergePart>& parts, int64_t m, int64_t n, cbx_dtype dtype, int64_t most,
+                         cbx_dcsc* out, hipStream_t s) {
+  const size_t count = parts.size();
+  int64_t nnz = 0, nzc = 0;
+  for (const MergePart& P : parts) {
+    nnz += P.nnz;
+    nzc += P.nzc;
+  }
+  if (nzc == 0) return merge_empty(m, n, dtype, out, s);
+  if (nnz <= most && nzc <= most) return merge_product<K, T>(parts, m, n, dtype, out, s);
+  std::memset(out, 0, sizeof(*out));
+  cbx_status st = CBX_OK;
+  if (n == 1) {
+    CBX_RETURN_IF(count < 3, CBX_ERR_LIMIT, "cbx_dcsc_merge: a column of two partial sums holds %lld entries, more than %lld",
+                  (long long)nnz, (long long)most);
+    MergeResult half[2];
+    for (int h = 0; h < 2; ++h) {
+      const std::vector<MergePart> some(parts.begin() + (h ? count / 2 : 0), h ? parts.end() : parts.begin() + count / 2);
+      if ((st = merge_columns<K, T>(some, m, 1, dtype, most, &half[h].x, s)) != CBX_OK) return st;
+    }
+    return merge_columns<K, T>({half[0].part(), half[1].part()}, m, 1, dtype, most, out, s);
+  }
+  ScratchSet ws(s);
+  MergePart* dparts;
+  longlong2* dbelow;
+  if (!ws.take(&dparts, count) || !ws.take(&dbelow, count))
+    return set_error(CBX_ERR_NOMEM, "cbx_dcsc_merge: workspace allocation failed");
+  CBX_HIP(hipMemcpyAsync(dparts, parts.data(), sizeof(MergePart) * count, hipMemcpyHostToDevice, s));
+  std::vector<longlong2> from(count, make_longlong2(0, 0)), to(count);
+  // what the columns [from, col) hold; malformed: they are no range of a part
+  auto upto = [&](int64_t col, int64_t& entries, int64_t& columns) -> cbx_status {
+    if (col == n) {
+      for (size_t i = 0; i < count; ++i) to[i] = make_longlong2(parts[i].nzc, parts[i].nnz);
+    } else {
+      k_merge_below<<<(unsigned)((count + kMergeNT - 1) / kMergeNT), kMergeNT, 0, s>>>(dparts, (int64_t)count, col,
+                                                                                     dbelow);
+      CBX_HIP(hipGetLastError());
+      CBX_HIP(hipMemcpyAsync(to.data(), dbelow, sizeof(longlong2) * count, hipMemcpyDeviceToHost, s));
+      CBX_HIP(hipStreamSynchronize(s));
+    }
+    entries = columns = 0;
+    for (size_t i = 0; i < count; ++i) {
+      CBX_RETURN_IF(to[i].x < from[i].x || to[i].y < from[i].y || to[i].y > parts[i].nnz, CBX_ERR_INVALID,
+                    "cbx_dcsc_check: a part is malformed");
+      entries += to[i].y - from[i].y;
+      columns += to[i].x - from[i].x;
+    }
+    return CBX_OK;
+  };
+  struct Range {
+    int64_t first, columns, entries;  // column id, and stored columns and entries before its own in the output
+    MergeResult merged;
+  };
+  std::vector<Range> ranges;
+  int64_t cols_out = 0, entries_out = 0;
+  for (int64_t c0 = 0; c0 < n;) {
+    int64_t lo = c0 + 1, hi = n, entries = 0, columns = 0;  // the last end of a range that fits, one column at least
+    while (lo < hi) {
+      const int64_t mid = lo + (hi - lo + 1) / 2;
+      if ((st = upto(mid, entries, columns)) != CBX_OK) return st;
+      if (entries <= most && columns <= most) lo = mid;
+      else hi = mid - 1;
+    }
+    if ((st = upto(lo, entries, columns)) != CBX_OK) return st;
+    std::vector<MergePart> some;
+    for (size_t i = 0; i < count; ++i) {
+      const MergePart& P = parts[i];
+      if (to[i].x == from[i].x) {
+        CBX_RETURN_IF(to[i].y != from[i].y, CBX_ERR_INVALID, "cbx_dcsc_check: a part is malformed");
+        continue;
+      }
+      some.push_back(MergePart{P.cp + from[i].x, P.jc + from[i].x, P.ir + from[i].y, (const T*)P.val + from[i].y,
+                               to[i].y - from[i].y, to[i].x - from[i].x, P.nz_base + from[i].y, P.col_base + c0});
+    }
+    if (!some.empty()) {
+      ranges.push_back(Range{c0, cols_out, entries_out, {}});
+      cbx_dcsc& x = ranges.back().merged.x;
+      if ((st = merge_columns<K, T>(some, m, lo - c0, dtype, most, &x, s)) != CBX_OK) return st;
+      cols_out += x.nzc;
+      entries_out += x.nnz;
+    }
+    c0 = lo;
+    from = to;
+  }
+  ws.release();
+  out->m = m;
+  out->n = n;
+  out->dtype = dtype;
+  out->location = CBX_DEVICE;
+  // array by array, each range's given back before the next is allocated
+  auto fail = [&](cbx_status why) {
+    (void)hipStreamSynchronize(s);
+    cbx_dcsc_free(out);
+    return why;
+  };
+  if ((st = dev_alloc((void**)&out->cp, sizeof(int64_t) * (size_t)(cols_out + 1))) != CBX_OK ||
+      (st = dev_alloc((void**)&out->jc, sizeof(int64_t) * (size_t)std::max<int64_t>(cols_out, 1))) != CBX_OK)
+    return fail(st);
+  for (const Range& r : ranges)
+    k_merge_columns<<<(unsigned)((r.merged.x.nzc + kMergeNT) / kMergeNT), kMergeNT, 0, s>>>(
+        r.merged.x.cp, r.merged.x.jc, r.merged.x.nzc, r.entries, r.first, out->cp + r.columns, out->jc + r.columns);
+  hipError_t e = hipGetLastError();
+  auto gather = [&](auto member, void** to_all, size_t size) -> cbx_status {
+    const cbx_status ast = dev_alloc(to_all, size * (size_t)std::max<int64_t>(entries_out, 1));
+    if (ast != CBX_OK) return ast;
+    for (Range& r : ranges)
+      if (e == hipSuccess && r.merged.x.nnz)
+        e = hipMemcpyAsync((char*)*to_all + size * (size_t)r.entries, *member(r.merged.x), size * (size_t)r.merged.x.nnz,
+                           hipMemcpyDeviceToDevice, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    for (Range& r : ranges) {
+      dev_free(*member(r.merged.x));
+      *member(r.merged.x) = nullptr;
+    }
+    return CBX_OK;
+  };
+  if ((st = gather([](cbx_dcsc& x) { return (void**)&x.ir; }, (void**)&out->ir, sizeof(int64_t))) != CBX_OK ||
+      (st = gather([](cbx_dcsc& x) { return &x.val; }, &out->val, sizeof(T))) != CBX_OK)
+    return fail(st);
+  if (e != hipSuccess) return fail(set_error(CBX_ERR_HIP, "cbx_dcsc_merge: %s", hipGetErrorString(e)));
+  out->nnz = entries_out;
+  out->nzc = cols_out;
+  return CBX_OK;
+}
+
+template <int K, class T>
+cbx_status merge_typed(int32_t count, const cbx_dcsc* parts, int64_t most, cbx_dcsc* out, hipStream_t s) {
+  std::memset(out, 0, sizeof(*out));
+  std::vector<MergePart> all((size_t)count);
+  for (int32_t i = 0; i < count; ++i)
+    all[i] = MergePart{parts[i].cp, parts[i].jc, parts[i].ir, parts[i].val, parts[i].nnz, parts[i].nzc, 0, 0};
+  return merge_columns<K, T>(all, parts[0].m, parts[0].n, parts[0].dtype, most, out, s);
 }
 
 // ------------------------------------------------------- edge list to DCSC
@@ -542,6 +734,13 @@ using namespace cbx;
 
 extern "C" cbx_status cbx_dcsc_merge(int32_t count, const cbx_dcsc* parts, cbx_semiring semiring, cbx_dcsc* out,
                                      void* stream) {
+  return cbx_dcsc_merge_in_ranges(count, parts, semiring, kMergeMost, out, stream);
+}
+
+extern "C" cbx_status cbx_dcsc_merge_in_ranges(int32_t count, const cbx_dcsc* parts, cbx_semiring semiring,
+                                               int64_t max_entries, cbx_dcsc* out, void* stream) {
+  CBX_RETURN_IF(max_entries < 1 || max_entries > kMergeMost, CBX_ERR_INVALID,
+                "cbx_dcsc_merge_in_ranges: max_entries must be in [1, 2^31)");
   CBX_RETURN_IF(!parts || !out || count < 1, CBX_ERR_INVALID, "cbx_dcsc_merge: need at least one part and an output");
   cbx_status st = init_device_once();
   if (st != CBX_OK) return st;
@@ -555,7 +754,7 @@ extern "C" cbx_status cbx_dcsc_merge(int32_t count, const cbx_dcsc* parts, cbx_s
   switch (semiring * 8 + dt) {
 #define CBX_MG(SRK, SRE, T, DT) \
   case SRE * 8 + DT:            \
-    return merge_typed<SRK, T>(count, parts, out, s);
+    return merge_typed<SRK, T>(count, parts, max_entries, out, s);
     CBX_MG(kPlusTimes, CBX_SR_PLUS_TIMES, int64_t, CBX_I64)
     CBX_MG(kPlusTimes, CBX_SR_PLUS_TIMES, double, CBX_F64)
     CBX_MG(kPlusTimes, CBX_SR_PLUS_TIMES, float, CBX_F32)

@@ -193,7 +193,8 @@ struct PackSeg {
   const int64_t *cp, *jc, *ir;
   const void* val;
   int64_t row_off, col_off, nz_off, c_off;
-  int64_t m, n, nnz, nzc;  // the member's own shape and sizes (for its bounds)
+  int64_t m, n, nnz, nzc;    // the member's own shape and sizes (for its bounds)
+  int64_t nz_base, col_base; // of a column range of a matrix: its first entry (cp counts from there) and column id
 };
 
 // Writes the members' concatenation to out.cp / jc / val and their rows to

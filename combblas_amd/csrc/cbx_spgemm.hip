@@ -3469,6 +3469,10 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
     return CBX_OK;
   }
 
+  // places in A's entries and stored columns are 32-bit numbers in the kernels (tile pointers, segment bases, bpos)
+  CBX_RETURN_IF(nnzA >= (1ll << 31) || nzcA >= (1ll << 31), CBX_ERR_LIMIT,
+                "cbx_spgemm: the left operand must hold fewer than 2^31 nonzeros");
+
   // Three waits for the device per product: after the setup (the tiers' sizes),
   // after the symbolic pass (the output's), at the end.  Kernels report into
   // the slot's pinned page; counters are cleared together, and all scratch is

@@ -469,6 +469,17 @@ cbx_status cbx_dcsc_transpose(const cbx_dcsc* X, cbx_dcsc* out, void* stream);
  * m x n (CBX_ERR_INVALID). */
 cbx_status cbx_dcsc_merge(int32_t count, const cbx_dcsc* parts, cbx_semiring semiring, cbx_dcsc* out, void* stream);
 
+/* The same in column ranges whose parts hold at most max_entries entries, in
+ * [1, 2^31), one after the other: the same result, with workspace (4 bytes and
+ * a value per entry of the concatenation, and the product's own) for one range
+ * at a time, and up to one more copy of the result's values.
+ * cbx_dcsc_merge does this by itself with 2^31 - 1, the product's limit; parts
+ * of up to that many entries in all are merged at once.  A single column that
+ * holds more is merged part by part; CBX_ERR_LIMIT if two of its partial sums
+ * hold more. */
+cbx_status cbx_dcsc_merge_in_ranges(int32_t count, const cbx_dcsc* parts, cbx_semiring semiring, int64_t max_entries,
+                                    cbx_dcsc* out, void* stream);
+
 /* Edge list to matrix on the device: the Graph500 constructor SpTuples(maxnnz,
  * m, n, edges, removeloops) (SpTuples.cpp:70-110: values 1, duplicates summed,
  * self loops dropped) and SpTuples::RemoveDuplicates(BinOp) (SpTuples.cpp:271)
