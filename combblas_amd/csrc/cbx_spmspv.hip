@@ -1771,6 +1771,7 @@ extern "C" cbx_status cbx_spmv_dense(const cbx_dcsc* A, const void* x, void* y, 
                 "cbx_spmv_dense: A must be boolean or share the vectors' dtype");
   // (the structure check, the rules of cbx_dcsc_check, runs with the product)
   CBX_RETURN_IF(A->nzc == 0 && A->nnz != 0, CBX_ERR_INVALID, "cbx_dcsc_check: nnz without columns");
+  CBX_RETURN_IF(A->m <= 0 && A->nnz != 0, CBX_ERR_INVALID, "cbx_dcsc_check: nnz without rows");
   const cbx_status init = init_device_once();
   if (init != CBX_OK) return init;
   hipStream_t s = (hipStream_t)stream;
