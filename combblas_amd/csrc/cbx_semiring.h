@@ -16,8 +16,10 @@
 // (ds_add_f32 takes 193 cycles a wave instruction at random addresses,
 // ds_add_f64 21, ds_add_u64 11).  Identities:
 //   PlusTimes integers 0; floating point -0.0 (so a lone -0.0 stays -0.0);
-//   MinPlus   max();
-//   SelectMax lowest() (the reference's id() of -1 is not an identity of max
+//   MinPlus   max(); floating point NaN, which loses against every number:
+//             with max() or infinity a column's infinite products would come
+//             back as max(), or its NaN products as infinity;
+//   SelectMax lowest(), NaN likewise (the reference's id() of -1 is not an identity of max
 //             for products below -1, so it is not used here);
 //   bool      0 in a 32-bit word accumulated with OR.
 // Whether an entry exists is tracked separately (bitmap or hash key), so
@@ -57,16 +59,16 @@ __device__ __forceinline__ void lds_max(A* p, A v) {
   __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Floating min/max through a compare-and-swap loop on the bit pattern, with
-// std::min / std::max semantics: the stored value is replaced only when the
-// new value is strictly smaller (larger).
+// Floating min/max through a compare-and-swap loop on the bit pattern: the
+// stored value is replaced when the new one is strictly smaller (larger) or it
+// is NaN, as ds_min_f64 / ds_max_f64 do.
 template <class F, class U>
 __device__ __forceinline__ void lds_cas_minmax(F* p, F v, bool is_min) {
   U* up = reinterpret_cast<U*>(p);
   U old = __hip_atomic_load(up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   while (true) {
     F cur = __builtin_bit_cast(F, old);
-    bool better = is_min ? (v < cur) : (cur < v);
+    bool better = (is_min ? (v < cur) : (cur < v)) || cur != cur;
     if (!better) return;
     U want = __builtin_bit_cast(U, v);
     if (__hip_atomic_compare_exchange_strong(up, &old, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
@@ -147,7 +149,7 @@ template <>
 struct Sem<kMinPlus, double> : LdsAsAcc<Sem<kMinPlus, double>, double, double> {
   using S = double;
   using Acc = double;
-  static __device__ __forceinline__ Acc ident() { return std::numeric_limits<double>::max(); }
+  static __device__ __forceinline__ Acc ident() { return std::numeric_limits<double>::quiet_NaN(); }
   static __device__ __forceinline__ Acc mul(S a, S b) { return inf_plus(a, b); }
   static __device__ __forceinline__ void acc(Acc* p, Acc v) { lds_min(p, v); }
   static __device__ __forceinline__ Acc add(Acc a, Acc b) { return b < a ? b : a; }
@@ -157,7 +159,7 @@ template <>
 struct Sem<kMinPlus, float> : LdsAsAcc<Sem<kMinPlus, float>, float, float> {
   using S = float;
   using Acc = float;
-  static __device__ __forceinline__ Acc ident() { return std::numeric_limits<float>::max(); }
+  static __device__ __forceinline__ Acc ident() { return std::numeric_limits<float>::quiet_NaN(); }
   static __device__ __forceinline__ Acc mul(S a, S b) { return inf_plus(a, b); }
   static __device__ __forceinline__ void acc(Acc* p, Acc v) { lds_cas_minmax<float, unsigned int>(p, v, true); }
   static __device__ __forceinline__ Acc add(Acc a, Acc b) { return b < a ? b : a; }
@@ -179,7 +181,7 @@ template <>
 struct Sem<kSelectMax, double> : LdsAsAcc<Sem<kSelectMax, double>, double, double> {
   using S = double;
   using Acc = double;
-  static __device__ __forceinline__ Acc ident() { return -std::numeric_limits<double>::infinity(); }
+  static __device__ __forceinline__ Acc ident() { return std::numeric_limits<double>::quiet_NaN(); }
   static __device__ __forceinline__ Acc mul(S a, S b) { return a * b; }
   static __device__ __forceinline__ void acc(Acc* p, Acc v) { lds_max(p, v); }
   static __device__ __forceinline__ Acc add(Acc a, Acc b) { return a < b ? b : a; }
@@ -189,7 +191,7 @@ template <>
 struct Sem<kSelectMax, float> : LdsAsAcc<Sem<kSelectMax, float>, float, float> {
   using S = float;
   using Acc = float;
-  static __device__ __forceinline__ Acc ident() { return -std::numeric_limits<float>::infinity(); }
+  static __device__ __forceinline__ Acc ident() { return std::numeric_limits<float>::quiet_NaN(); }
   static __device__ __forceinline__ Acc mul(S a, S b) { return a * b; }
   static __device__ __forceinline__ void acc(Acc* p, Acc v) { lds_cas_minmax<float, unsigned int>(p, v, false); }
   static __device__ __forceinline__ Acc add(Acc a, Acc b) { return a < b ? b : a; }

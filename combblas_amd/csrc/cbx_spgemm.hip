@@ -1087,6 +1087,27 @@ __global__ __launch_bounds__(256) void k_tiny(const int32_t* __restrict__ order,
 #pragma unroll
       for (int u = 0; u < kE; ++u)
         if (u * kWave + lane < filled) SR::acc(&ws.vals[ws.keys[slot[u]]], val[u]);
+      if constexpr (K != kPlusTimes && std::is_floating_point<T>::value) {
+        // the semiring's add keeps a NaN that comes first (b < a ? b : a), the
+        // accumulator one that is alone: rare, so product by product
+        wave_lds_sync();
+#pragma unroll
+        for (int u = 0; u < kE; ++u) {
+          unsigned long long nan = __ballot(u * kWave + lane < filled && val[u] != val[u]);
+          while (nan) {
+            const int l = __ffsll(nan) - 1;
+            nan &= nan - 1;
+            const int at = __builtin_amdgcn_readlane(slot[u], l);
+            unsigned long long before = 0ull;  // products of the row before this one
+#pragma unroll
+            for (int w2 = 0; w2 <= u; ++w2) {
+              const unsigned long long same = __ballot(w2 * kWave + lane < filled && slot[w2] == at);
+              before |= w2 < u ? same : same & ((1ull << l) - 1ull);
+            }
+            if (!before && lane == 0) ws.vals[ws.keys[at]] = SR::lident();
+          }
+        }
+      }
       // the column's allocation from the symbolic pass; or, staged (no symbolic
       // pass), its slot of flop_j entries in the staging buffer, and the count
       // is recorded for the copy into place
