@@ -62,13 +62,15 @@ template <>
 struct GAcc<kSelectMax, int64_t> {
   static __device__ void acc(int64_t* p, int64_t v) { atomicMax((long long*)p, (long long)v); }
 };
+// SR::add on a value in memory, which keeps a NaN there; with `empty_nan` a NaN
+// is an accumulator without products yet.
 template <class F, class U>
-__device__ void gcas_minmax(F* p, F v, bool is_min) {
+__device__ void gcas_minmax(F* p, F v, bool is_min, bool empty_nan = false) {
   U* up = reinterpret_cast<U*>(p);
   U old = __hip_atomic_load(up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   while (true) {
     const F cur = __builtin_bit_cast(F, old);
-    if (!(is_min ? (v < cur) : (cur < v))) return;
+    if (!((is_min ? (v < cur) : (cur < v)) || (empty_nan && cur != cur))) return;
     if (__hip_atomic_compare_exchange_strong(up, &old, __builtin_bit_cast(U, v), __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT))
       return;
@@ -90,6 +92,17 @@ template <>
 struct GAcc<kSelectMax, float> {
   static __device__ void acc(float* p, float v) { gcas_minmax<float, unsigned int>(p, v, false); }
 };
+
+// Into an accumulator that started at ident_of().
+template <int K, class T>
+__device__ __forceinline__ void acc_new(T* p, T v) {
+  if constexpr (K == kPlusTimes || !std::is_floating_point<T>::value) {
+    GAcc<K, T>::acc(p, v);
+  } else {
+    using Bits = typename std::conditional<sizeof(T) == 8, unsigned long long, unsigned int>::type;
+    gcas_minmax<T, Bits>(p, v, K == kMinPlus, true);
+  }
+}
 
 namespace {
 
@@ -170,7 +183,7 @@ __device__ __forceinline__ void sv_products(const int64_t* __restrict__ ir, cons
     T v;
     if constexpr (BOOLA) v = x;
     else v = (T)SR::out(SR::mul(a[u], x));
-    GAcc<K, T>::acc(&acc[r[u]], v);
+    acc_new<K, T>(&acc[r[u]], v);
   }
 }
 
@@ -362,6 +375,7 @@ inline unsigned nb(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 template <int K, class T>
 T ident_of() {
   if (K == kPlusTimes) return std::is_floating_point<T>::value ? (T)-0.0 : (T)0;
+  if (std::is_floating_point<T>::value) return std::numeric_limits<T>::quiet_NaN();  // (as in cbx_semiring.h)
   if (K == kMinPlus) return std::numeric_limits<T>::max();
   return std::numeric_limits<T>::lowest();
 }

@@ -2,7 +2,8 @@
 product has that product; infinities take part like numbers.  Of several
 products, the semiring's add keeps a NaN that comes first and passes over
 later ones (the columns of few products, merges and the dense SpMV do so);
-columns of many products have NaN only where every product is."""
+columns of many products and the product with a sparse vector have NaN only
+where every product is."""
 from __future__ import annotations
 
 import numpy as np
@@ -103,3 +104,19 @@ def test_dense_spmv(nnz, semiring, dtype):
     x, y = rng.integers(1, 4, n).astype(dtype), _special(rng, m, dtype)
     got = cb.spmv_dense(A.to_device(), x, y, semiring)
     assert np.array_equal(got, oracle.spmv_dense(A, x, y, semiring), equal_nan=True)
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("semiring,dtype", KINDS)
+def test_sparse_vector(noalloc, semiring, dtype):
+    rng = np.random.default_rng(8)
+    lengths = np.append(rng.integers(1, 40, 60), [300, 700])  # and two columns that are set aside
+    rows = np.concatenate([np.sort(rng.choice(2000, d, replace=False)) for d in lengths])
+    A = cb.Dcsc.from_coo(2000, lengths.size, rows, np.repeat(np.arange(lengths.size), lengths),
+                         _special(rng, rows.size, dtype), dtype)
+    x = np.arange(lengths.size, dtype=np.int32)
+    xv = rng.integers(1, 4, x.size).astype(dtype)
+    per = np.repeat(xv, lengths)
+    at, want = _by_row(A.ir, A.val + per if semiring == "min_plus" else A.val * per, semiring, _many)
+    gi, gv = cb.spmspv(A.to_device(), x, xv, semiring, noalloc=noalloc)
+    assert np.array_equal(gi, at) and np.array_equal(gv, want, equal_nan=True)
