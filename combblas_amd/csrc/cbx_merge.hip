@@ -39,12 +39,21 @@ namespace {
 constexpr int kMergeNT = 256;
 
 // The semiring's add on stored values (SR::add of the reference's semirings).
+// Min and max keep a NaN on the left and pass over one on the right, which is
+// not associative: in a tree, (5 + NaN) + (NaN + 3) would lose the 3.  `join`
+// passes over NaN on either side; a run's fold from left to right is then its
+// first value if that is NaN, and otherwise the join of all in any shape.
 template <int K, class T>
 struct SemAdd {
+  static constexpr bool kKeepsNan = K != kPlusTimes && std::is_floating_point<T>::value;
   __device__ __forceinline__ T operator()(const T& a, const T& b) const {
     using SR = Sem<K, T>;
     using Acc = typename SR::Acc;
     return (T)SR::out(SR::add((Acc)a, (Acc)b));
+  }
+  __device__ __forceinline__ T join(const T& a, const T& b) const {
+    if (kKeepsNan && a != a) return b;
+    return (*this)(a, b);
   }
 };
 
@@ -575,16 +584,17 @@ __global__ __launch_bounds__(kMergeNT) void k_coo_assemble(const uint64_t* __res
     // the first lane after this one's run
     const unsigned long long ends = lane == kWave - 1 ? 0ull : (heads | ~live) >> (lane + 1);
     const int end = ends ? lane + __ffsll(ends) : kWave;
+    const T own = v[c];
     for (int d = 1; __ballot(lane + d < end); d *= 2) {
       const T o = shfl_down(v[c], d);
-      if (lane + d < end) v[c] = add(v[c], o);
+      if (lane + d < end) v[c] = add.join(v[c], o);
     }
-    if (end == kWave && carry.some) v[c] = add(v[c], carry.v);
+    if (end == kWave && carry.some) v[c] = add.join(v[c], carry.v);
     const bool head = (heads >> lane) & 1ull;
     if (head) {
       const int64_t q = rank + __popcll(heads & ((1ull << lane) - 1ull));
       ir[q] = (int64_t)(st.key[c] & ((1ull << row_bits) - 1ull));
-      val[q] = v[c];
+      val[q] = add.kKeepsNan && own != own ? own : v[c];
       if ((st.columns[c] >> lane) & 1ull) {
         const int64_t k = crank + __popcll(st.columns[c] & ((1ull << lane) - 1ull));
         jc[k] = (int64_t)(st.key[c] >> row_bits);
@@ -639,9 +649,9 @@ __global__ __launch_bounds__(kMergeNT) void k_coo_join(const uint64_t* __restric
     T v = l.v;
     for (int d = 1; d < terms; d *= 2) {
       const T o = shfl_down(v, d);
-      if (lane + d < terms) v = add(v, o);
+      if (lane + d < terms) v = add.join(v, o);
     }
-    if (terms) sum = add(sum, shfl_from(v, 0));
+    if (terms) sum = add(sum, shfl_from(v, 0));  // (a NaN so far is the run's first)
     if (stop) break;
   }
   if (lane == 0) val[q] = sum;

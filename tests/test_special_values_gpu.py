@@ -120,3 +120,16 @@ def test_sparse_vector(noalloc, semiring, dtype):
     at, want = _by_row(A.ir, A.val + per if semiring == "min_plus" else A.val * per, semiring, _many)
     gi, gv = cb.spmspv(A.to_device(), x, xv, semiring, noalloc=noalloc)
     assert np.array_equal(gi, at) and np.array_equal(gv, want, equal_nan=True)
+
+
+@pytest.mark.parametrize("count,spread", [(3, 1), (64, 1), (700, 5), (20_000, 1), (20_000, 300), (200_000, 2)])
+@pytest.mark.parametrize("semiring,dtype", KINDS)
+def test_edge_list(count, spread, semiring, dtype):
+    """Equal entries are folded in input order, in runs within a wave and over many strips."""
+    rng = np.random.default_rng(count + spread)
+    rows, cols = rng.integers(0, spread, count), rng.integers(0, 2, count)
+    vals = _special(rng, count, dtype)
+    at, want = _by_row(cols * spread + rows, vals, semiring, _fold)
+    dr, dc, dv = (cb.DeviceArray.from_host(a) for a in (rows, cols, vals))
+    got = cb.from_coo_device(spread, 2, dr, dc, dv, dtype=dtype, semiring=semiring).to_host()
+    assert np.array_equal(got.col_ids() * spread + got.ir, at) and np.array_equal(got.val, want, equal_nan=True)
