@@ -11,6 +11,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "cbx_blocks.h"
 #include "cbx_device.h"
 #include "cbx_spgemm.h"
 
@@ -66,11 +67,8 @@ cbx_status check_dcsc(const cbx_dcsc* X, const char* name, cbx_location loc) {
 // a small caching allocator: cbx_dcsc_free returns blocks to a per-process
 // free list and the next allocation of a similar size reuses them, so
 // repeated products of the same shape do not pay hipMalloc/hipFree (which
-// costs seconds for outputs of hundreds of GB).  New blocks are rounded up to
-// an eighth of their leading power of two, so that products whose sizes differ
-// by a few percent (the column phases of an MCL expansion) find each other's:
-// unrounded, every new matrix added its own set of blocks until the card was
-// full, and giving them all back took 1.3 s.
+// costs seconds for outputs of hundreds of GB).  New blocks are rounded up
+// (block_bytes).
 namespace {
 struct Cache {
   std::mutex mu;
@@ -84,7 +82,7 @@ Cache& cache() {
 }
 }  // namespace
 
-cbx_status dev_alloc(void** p, size_t bytes) {
+cbx_status dev_alloc(void** p, size_t bytes, bool exact) {
   bytes = std::max<size_t>(bytes, 256);
   Cache& c = cache();
   {
@@ -98,9 +96,7 @@ cbx_status dev_alloc(void** p, size_t bytes) {
       return CBX_OK;
     }
   }
-  size_t step = 256;
-  while (step * 16 <= bytes) step *= 2;  // an eighth of the leading power of two
-  size_t want = (bytes + step - 1) / step * step;
+  size_t want = exact ? bytes : block_bytes(bytes);
   hipError_t e = hipMalloc(p, want);
   if (e != hipSuccess) {
     (void)hipGetLastError();
@@ -130,6 +126,20 @@ void dev_free(void* p) {
   c.idle.emplace(it->second, p);
   c.idle_bytes += it->second;
   c.live.erase(it);
+}
+
+cbx_status dev_alloc_entries(int64_t** ir, void** val, int64_t nnz, size_t value_size) {
+  const size_t n = (size_t)std::max<int64_t>(nnz, 1);
+  for (const bool exact : {false, true}) {
+    cbx_status st = dev_alloc((void**)ir, sizeof(int64_t) * n, exact);
+    if (st == CBX_OK) st = dev_alloc(val, value_size * n, exact);
+    if (st == CBX_OK) return st;
+    dev_free(*ir);
+    *ir = nullptr;
+    release_cache();
+    if (exact) return st;
+  }
+  return CBX_ERR_NOMEM;
 }
 
 size_t cache_idle_bytes() {

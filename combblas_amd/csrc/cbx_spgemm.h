@@ -87,7 +87,10 @@ void mlp_infer_launch(const float* params, const float* X, int64_t n, float* out
 const float* predictor_params();
 
 // Cached device allocations for arrays handed to callers (see cbx_runtime.hip).
-cbx_status dev_alloc(void** p, size_t bytes);
+cbx_status dev_alloc(void** p, size_t bytes, bool exact = false);  // exact: a new block is not rounded up
+// A matrix's ir and val; where one does not fit beside the other's surplus, both
+// at their own sizes.  Both null on failure.
+cbx_status dev_alloc_entries(int64_t** ir, void** val, int64_t nnz, size_t value_size);
 void dev_free(void* p);
 void release_cache();
 size_t cache_idle_bytes();  // bytes held by the cache and free for reuse

@@ -3276,11 +3276,7 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
     if (herr & ~512) return set_error(CBX_ERR_HIP, "cbx_spgemm: learned pass inconsistency (flag %d)", herr);
     return CBX_OK;
   }
-  auto alloc_out = [&]() -> cbx_status {
-    if (!C->ir) CBX_TRY(dev_alloc((void**)&C->ir, sizeof(int64_t) * std::max<int64_t>(info.nnzC, 1)));
-    if (!C->val) CBX_TRY(dev_alloc(&C->val, sizeof(T) * std::max<int64_t>(info.nnzC, 1)));
-    return CBX_OK;
-  };
+  auto alloc_out = [&]() { return dev_alloc_entries(&C->ir, &C->val, info.nnzC, sizeof(T)); };
   cbx_status ast = alloc_out();
   if (ast != CBX_OK && rm.p) {  // give the row maps back; the large units then count in a sweep
     dev_free(rm.p);             // (the stream is idle)
@@ -3447,11 +3443,8 @@ static cbx_status filter_compact(const Filter<T>& flt, int64_t nzcB, int64_t* nn
   }
   int64_t* ir2 = nullptr;
   void* val2 = nullptr;
-  CBX_TRY(dev_alloc((void**)&ir2, sizeof(int64_t) * std::max<int64_t>(total, 1)));
-  if (dev_alloc(&val2, sizeof(T) * std::max<int64_t>(total, 1)) != CBX_OK) {
-    dev_free(ir2);
+  if (dev_alloc_entries(&ir2, &val2, total, sizeof(T)) != CBX_OK)
     return set_error(CBX_ERR_NOMEM, "cbx_spgemm: allocation of the thresholded product failed");
-  }
   if (nrun) k_run_copy<T><<<wave_grid(nrun), 256, 0, s>>>(i2, flt.run_src, flt.run_kept, dst, C->ir, (const T*)C->val,
                                                          (int)nrun, ir2, (T*)val2);
   CBX_HIP(hipGetLastError());
@@ -3746,11 +3739,7 @@ static cbx_status spgemm_typed_once(const cbx_dcsc* A, const cbx_dcsc* B, cbx_sp
   }
 
   // --- output allocation (cached: repeated products reuse the arrays)
-  auto alloc_out = [&]() -> cbx_status {
-    if (!C->ir) CBX_TRY(dev_alloc((void**)&C->ir, sizeof(int64_t) * std::max<int64_t>(nnzC, 1)));
-    if (!C->val) CBX_TRY(dev_alloc(&C->val, sizeof(T) * std::max<int64_t>(nnzC, 1)));
-    return CBX_OK;
-  };
+  auto alloc_out = [&]() { return dev_alloc_entries(&C->ir, &C->val, nnzC, sizeof(T)); };
   cbx_status ast = alloc_out();
   if (ast != CBX_OK && rmap) {  // give the row maps back and use the two-sweep numeric pass
     CBX_HIP(hipStreamSynchronize(s));

@@ -1,0 +1,82 @@
+"""The caching allocator's block sizes: near their request, and a product's
+output given its exact size where the surplus does not fit."""
+from __future__ import annotations
+
+import ctypes as C
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+import combblas_amd as cb
+
+CSRC = Path(__file__).resolve().parents[1] / "combblas_amd" / "csrc"
+GB = 1 << 30
+
+
+def test_block_sizes(tmp_path):
+    src, exe = tmp_path / "t.cpp", tmp_path / "t"
+    src.write_text(r"""
+#include <cstdio>
+#include "cbx_blocks.h"
+int main() {
+  size_t last = 0;
+  for (int e = 8; e < 39; ++e)
+    for (size_t k = 0; k < 64; ++k) {
+      const size_t bytes = ((size_t)1 << e) + (k << e) / 64 + k % 3, got = cbx::block_bytes(bytes);
+      const bool ok = got >= bytes && (got - bytes) * 8 <= bytes + 8 * 256 && got - bytes < (size_t)1 << 30 &&
+                      got >= last && got % 256 == 0;
+      if (!ok) return std::printf("%zu -> %zu\n", bytes, got), 1;
+      last = got;
+    }
+  // sizes a few percent apart share a block
+  return cbx::block_bytes((size_t)20 << 20) == cbx::block_bytes(((size_t)20 << 20) - (1 << 19)) ? 0 : 2;
+}
+""")
+    subprocess.run(["g++", "-O1", "-std=c++17", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+
+
+def _free():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert cb.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def leave(free):
+    """Blocks that leave about `free` bytes of device memory (of sizes that the allocator does not round)."""
+    held = []
+    for size in (64 * GB, GB, GB // 16):
+        while _free() - size >= free:
+            held.append(cb.DeviceArray(size, np.uint8))
+    return held
+
+
+@pytest.mark.gpu
+def test_output_that_fits_without_its_surplus():
+    m, n = 40_000, 27_200  # 1.09 G outputs: ir and val of 8.1 GiB, 9 each when rounded up
+    A = cb.Dcsc.from_coo(m, 1, np.arange(m), np.zeros(m, np.int64), np.arange(m) % 9 + 1).to_device()
+    B = cb.Dcsc.from_coo(1, n, np.zeros(n, np.int64), np.arange(n), np.arange(n) % 5 + 1).to_device()
+    base = cb.get_config()
+    held = []
+    try:
+        cb.set_config(unit_lists=0)
+        cb.release_cached_memory()
+        before = _free()
+        C_, _ = cb.spgemm(A, B)
+        sums = C_.column_checksums(1)
+        C_.release()
+        used = before - _free()  # the output and the scratch, in the cache now
+        assert used > 18 * GB
+        cb.release_cached_memory()
+        held = leave(used - GB)  # one surplus less is not enough, two are
+        C_, _ = cb.spgemm(A, B)
+        assert C_.nnz == m * n and np.array_equal(C_.column_checksums(1), sums)
+        C_.release()
+    finally:
+        cb.set_config(**base)
+        for h in held:
+            h.release()
+        cb.release_cached_memory()
