@@ -1,8 +1,10 @@
-// Sizes of the blocks that the caching allocator asks the driver for, free of
-// HIP so that the host can test them.
+// The caching allocator's block sizes and lists, free of HIP so that the host
+// can test them.
 #pragma once
 
 #include <cstddef>
+#include <map>
+#include <unordered_map>
 
 namespace cbx {
 
@@ -20,5 +22,52 @@ inline size_t block_bytes(size_t bytes) {
   while (step < kBlockStep && step * 16 <= bytes) step *= 2;
   return (bytes + step - 1) / step * step;
 }
+
+// Blocks in use and idle ones, by device (not thread-safe).
+class BlockLists {
+  struct Block {
+    int device;
+    size_t bytes;
+  };
+  std::unordered_map<void*, Block> live_;
+  std::map<int, std::multimap<size_t, void*>> idle_;
+  std::map<int, size_t> idle_bytes_;
+
+ public:
+  // An idle block of the device for `bytes`, not much larger; null if there is none.
+  void* take(int device, size_t bytes) {
+    auto& blocks = idle_[device];
+    const auto it = blocks.lower_bound(bytes);
+    if (it == blocks.end() || it->first > bytes + bytes / 4 + (1u << 20)) return nullptr;
+    void* p = it->second;
+    live_[p] = Block{device, it->first};
+    idle_bytes_[device] -= it->first;
+    blocks.erase(it);
+    return p;
+  }
+  // A block newly allocated on the device.
+  void add(void* p, int device, size_t bytes) { live_[p] = Block{device, bytes}; }
+  // A block in use becomes idle; false if p is none.
+  bool give_back(void* p) {
+    const auto it = live_.find(p);
+    if (it == live_.end()) return false;
+    idle_[it->second.device].emplace(it->second.bytes, p);
+    idle_bytes_[it->second.device] += it->second.bytes;
+    live_.erase(it);
+    return true;
+  }
+  size_t idle_bytes(int device) const {
+    const auto it = idle_bytes_.find(device);
+    return it == idle_bytes_.end() ? 0 : it->second;
+  }
+  // Every idle block to f, and off the lists.
+  template <class F>
+  void release(F&& f) {
+    for (auto& d : idle_)
+      for (auto& b : d.second) f(b.second);
+    idle_.clear();
+    idle_bytes_.clear();
+  }
+};
 
 }  // namespace cbx

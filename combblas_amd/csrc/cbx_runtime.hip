@@ -6,9 +6,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <map>
 #include <mutex>
-#include <unordered_map>
 #include <vector>
 
 #include "cbx_blocks.h"
@@ -68,33 +66,30 @@ cbx_status check_dcsc(const cbx_dcsc* X, const char* name, cbx_location loc) {
 // free list and the next allocation of a similar size reuses them, so
 // repeated products of the same shape do not pay hipMalloc/hipFree (which
 // costs seconds for outputs of hundreds of GB).  New blocks are rounded up
-// (block_bytes).
+// (block_bytes).  Each device has idle blocks of its own.
 namespace {
 struct Cache {
   std::mutex mu;
-  std::unordered_map<void*, size_t> live;
-  std::multimap<size_t, void*> idle;
-  size_t idle_bytes = 0;
+  BlockLists blocks;
 };
 Cache& cache() {
   static Cache* c = new Cache();  // never destroyed: outlives static teardown order
   return *c;
+}
+int current_device() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) (void)hipGetLastError();
+  return dev;
 }
 }  // namespace
 
 cbx_status dev_alloc(void** p, size_t bytes, bool exact) {
   bytes = std::max<size_t>(bytes, 256);
   Cache& c = cache();
+  const int dev = current_device();
   {
     std::lock_guard<std::mutex> g(c.mu);
-    auto it = c.idle.lower_bound(bytes);
-    if (it != c.idle.end() && it->first <= bytes + bytes / 4 + (1u << 20)) {
-      *p = it->second;
-      c.live[*p] = it->first;
-      c.idle_bytes -= it->first;
-      c.idle.erase(it);
-      return CBX_OK;
-    }
+    if ((*p = c.blocks.take(dev, bytes))) return CBX_OK;
   }
   size_t want = exact ? bytes : block_bytes(bytes);
   hipError_t e = hipMalloc(p, want);
@@ -110,7 +105,7 @@ cbx_status dev_alloc(void** p, size_t bytes, bool exact) {
     return set_error(CBX_ERR_NOMEM, "device allocation of %zu bytes failed: %s", bytes, hipGetErrorString(e));
   }
   std::lock_guard<std::mutex> g(c.mu);
-  c.live[*p] = want;
+  c.blocks.add(*p, dev, want);
   return CBX_OK;
 }
 
@@ -118,14 +113,7 @@ void dev_free(void* p) {
   if (!p) return;
   Cache& c = cache();
   std::lock_guard<std::mutex> g(c.mu);
-  auto it = c.live.find(p);
-  if (it == c.live.end()) {
-    (void)hipFree(p);
-    return;
-  }
-  c.idle.emplace(it->second, p);
-  c.idle_bytes += it->second;
-  c.live.erase(it);
+  if (!c.blocks.give_back(p)) (void)hipFree(p);
 }
 
 cbx_status dev_alloc_entries(int64_t** ir, void** val, int64_t nnz, size_t value_size) {
@@ -145,7 +133,7 @@ cbx_status dev_alloc_entries(int64_t** ir, void** val, int64_t nnz, size_t value
 size_t cache_idle_bytes() {
   Cache& c = cache();
   std::lock_guard<std::mutex> g(c.mu);
-  return c.idle_bytes;
+  return c.blocks.idle_bytes(current_device());
 }
 
 namespace {
@@ -208,9 +196,7 @@ void release_cache() {
   Cache& c = cache();
   {
     std::lock_guard<std::mutex> g(c.mu);
-    for (auto& kv : c.idle) (void)hipFree(kv.second);
-    c.idle.clear();
-    c.idle_bytes = 0;
+    c.blocks.release([](void* p) { (void)hipFree(p); });
   }
   // and the stream pool's reserve (scratch freed by finished calls), so that
   // a large hipMalloc can use it

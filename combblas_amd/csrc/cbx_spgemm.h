@@ -93,7 +93,7 @@ cbx_status dev_alloc(void** p, size_t bytes, bool exact = false);  // exact: a n
 cbx_status dev_alloc_entries(int64_t** ir, void** val, int64_t nnz, size_t value_size);
 void dev_free(void* p);
 void release_cache();
-size_t cache_idle_bytes();  // bytes held by the cache and free for reuse
+size_t cache_idle_bytes();  // bytes of the current device held by the cache and free for reuse
 
 // The scratch blocks of one call, from the caching allocator above, released
 // together once the stream's kernels are done (at the latest when the set goes

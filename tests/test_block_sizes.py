@@ -39,6 +39,39 @@ int main() {
     assert r.returncode == 0, r.stdout
 
 
+def test_idle_blocks_stay_on_their_device(tmp_path):
+    src, exe = tmp_path / "t.cpp", tmp_path / "t"
+    src.write_text(r"""
+#include <cstdio>
+#include "cbx_blocks.h"
+#define CHECK(x) do { if (!(x)) return std::printf("line %d: %s\n", __LINE__, #x), 1; } while (0)
+int main() {
+  char mem[4];
+  cbx::BlockLists b;
+  b.add(mem, 0, 1000);
+  b.add(mem + 1, 1, 5 << 20);
+  b.add(mem + 2, 0, 5 << 20);
+  CHECK(!b.take(0, 1000));  // in use
+  CHECK(b.give_back(mem) && b.give_back(mem + 1) && b.give_back(mem + 2));
+  CHECK(!b.give_back(mem) && !b.give_back(mem + 3));
+  CHECK(b.idle_bytes(0) == 1000 + (5 << 20) && b.idle_bytes(1) == 5 << 20 && b.idle_bytes(2) == 0);
+  CHECK(!b.take(1, 6 << 20) && !b.take(2, 1000));
+  CHECK(b.take(1, 4 << 20) == mem + 1 && !b.take(1, 4 << 20));  // device 0 has another
+  CHECK(!b.take(0, 3 << 20) || !"more than a quarter and 1 MB larger");
+  CHECK(b.take(0, 1000) == mem && b.take(0, 5 << 20) == mem + 2 && b.idle_bytes(0) == 0);
+  b.give_back(mem);
+  b.give_back(mem + 1);
+  int n = 0;
+  b.release([&](void* p) { n += p == mem || p == mem + 1; });
+  CHECK(n == 2 && !b.take(0, 1000) && b.idle_bytes(1) == 0 && b.give_back(mem + 2));
+  return 0;
+}
+""")
+    subprocess.run(["g++", "-O1", "-std=c++17", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+
+
 def _free():
     free, total = C.c_size_t(), C.c_size_t()
     assert cb.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
