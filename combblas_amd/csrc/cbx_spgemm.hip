@@ -3855,14 +3855,16 @@ static cbx_status spgemm_typed(const cbx_dcsc* A, const cbx_dcsc* B, cbx_spgemm_
                                cbx_dcsc* C, cbx_spgemm_stats* stats, hipStream_t s,
                                int64_t* symbolic_out = nullptr) {
   bool lists_used = false;
-  const cbx_status st = spgemm_typed_once<K, T>(A, B, mode, cfg, C, stats, s, symbolic_out, &lists_used);
+  cbx_status st = spgemm_typed_once<K, T>(A, B, mode, cfg, C, stats, s, symbolic_out, &lists_used);
   if (st != CBX_OK) cbx_dcsc_free(C);
   if (st != CBX_ERR_NOMEM || !lists_used) return st;
   (void)hipStreamSynchronize(s);
   release_cache();
   SpgemmConfig plain = cfg;
   plain.unit_lists = 0;
-  return spgemm_typed_once<K, T>(A, B, mode, plain, C, stats, s, symbolic_out, nullptr);
+  st = spgemm_typed_once<K, T>(A, B, mode, plain, C, stats, s, symbolic_out, nullptr);
+  if (st != CBX_OK) cbx_dcsc_free(C);
+  return st;
 }
 
 // The operands as the features and the sampling estimator read them: validated

@@ -1,5 +1,5 @@
-"""The caching allocator's block sizes: near their request, and a product's
-output given its exact size where the surplus does not fit."""
+"""The caching allocator's block sizes and lists, and products at the limit of
+the card's memory."""
 from __future__ import annotations
 
 import ctypes as C
@@ -87,11 +87,16 @@ def leave(free):
     return held
 
 
+def _outer():
+    """Operands of a full 40,000 x 27,200 product: ir and val of 8.1 GiB, 9 each when rounded up."""
+    m, n = 40_000, 27_200
+    A = cb.Dcsc.from_coo(m, 1, np.arange(m), np.zeros(m, np.int64), np.arange(m) % 9 + 1).to_device()
+    return A, cb.Dcsc.from_coo(1, n, np.zeros(n, np.int64), np.arange(n), np.arange(n) % 5 + 1).to_device()
+
+
 @pytest.mark.gpu
 def test_output_that_fits_without_its_surplus():
-    m, n = 40_000, 27_200  # 1.09 G outputs: ir and val of 8.1 GiB, 9 each when rounded up
-    A = cb.Dcsc.from_coo(m, 1, np.arange(m), np.zeros(m, np.int64), np.arange(m) % 9 + 1).to_device()
-    B = cb.Dcsc.from_coo(1, n, np.zeros(n, np.int64), np.arange(n), np.arange(n) % 5 + 1).to_device()
+    A, B = _outer()
     base = cb.get_config()
     held = []
     try:
@@ -106,10 +111,31 @@ def test_output_that_fits_without_its_surplus():
         cb.release_cached_memory()
         held = leave(used - GB)  # one surplus less is not enough, two are
         C_, _ = cb.spgemm(A, B)
-        assert C_.nnz == m * n and np.array_equal(C_.column_checksums(1), sums)
+        assert C_.nnz == A.m * B.n and np.array_equal(C_.column_checksums(1), sums)
         C_.release()
     finally:
         cb.set_config(**base)
         for h in held:
             h.release()
         cb.release_cached_memory()
+
+
+@pytest.mark.gpu
+def test_product_that_does_not_fit_leaves_nothing():
+    A, B = _outer()
+    C_, _ = cb.spgemm(A, B)  # (what the runtime itself takes for the kernels)
+    C_.release()
+    held = []
+    try:
+        cb.release_cached_memory()
+        before = _free()
+        held = leave(15 * GB)  # room for the row lists, but in no attempt for the output
+        out = cb.cbx_dcsc()
+        st = cb.lib().cbx_spgemm(C.byref(A.s), C.byref(B.s), 0, 0, C.byref(out), None, None)
+        assert st == cb.ERR_NOMEM
+        assert not (out.cp or out.jc or out.ir or out.val)
+    finally:
+        for h in held:
+            h.release()
+        cb.release_cached_memory()
+    assert _free() >= before - GB // 64
