@@ -3238,10 +3238,21 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
     k_learned_units<<<nblk(nzcB, 256), 256, 0, s>>>(flop, nzcB, cfg.small_flop_max, logpred, blo, bhi, w, target,
                                                     heavy_pred, fcap, kLearnRB, direct_flop, m, ubase, nullptr,
                                                     units, nullptr, nullptr);
-  // staging capacity from the predictions; where it does not fit, the exact
-  // two-phase path computes the product
+  // staging capacity from the predictions; where it does not fit beside the
+  // output (the exactly sized columns and the predictions), the exact two-phase
+  // path computes the product, before anything is done twice
   LearnedStage<T> stage;
   stage.cap = (int64_t)(pred_sum * (1.0 + cfg.capacity_margin)) + (1 << 20);
+  const double staged = (double)stage.cap * (double)(sizeof(int32_t) + sizeof(T));
+  const double output = ((double)hash_total + pred_sum) * (double)(sizeof(int64_t) + sizeof(T));
+  if (rm.p && !fits(staged + output, 1.0)) {  // without the row maps the large units count in a sweep
+    dev_free(rm.p);                           // (the stream is idle)
+    rm.p = nullptr;
+  }
+  if (!fits(staged + output, 1.0)) {
+    info.over_capacity = true;
+    return CBX_OK;
+  }
   int64_t* upto;
   if (dalloc(ws, nunits + 1, &stage.cnt) != CBX_OK || dalloc(ws, nunits + 1, &stage.at) != CBX_OK ||
       dalloc(ws, nunits + 1, &upto) != CBX_OK || dalloc(ws, 1, &stage.taken) != CBX_OK ||

@@ -169,7 +169,9 @@ enum {
    * exact size comes from its own presence bitmap, its outputs go to a staging
    * area and from there into place once all sizes are known; units larger than
    * predicted are re-run exactly, and an exceeded staging capacity falls back
-   * to the two-phase path.
+   * to the two-phase path.  The staging area takes 4 bytes and a value per
+   * predicted output (and capacity_margin of them) beside the output; where
+   * both do not fit the free memory the two-phase path is taken at once.
    * Output identical to CBX_SPGEMM_TWO_PHASE. */
   CBX_SPGEMM_LEARNED = 2
 };
@@ -234,8 +236,8 @@ typedef struct cbx_spgemm_stats {
   int64_t predicted_nnz;  /* learned mode: sum of the predicted sizes of the columns the single pass
                              sized by prediction */
   int64_t actual_nnz_predicted; /* learned mode: their exact sizes (the product's outputs in those columns) */
-  int64_t learned_fallback; /* learned mode: 1 if the predicted output capacity was exceeded and the
-                               product was recomputed by the exact two-phase path */
+  int64_t learned_fallback; /* learned mode: 1 if the exact two-phase path computed the product, because the
+                               predicted output capacity was exceeded or the staging area did not fit */
   int64_t units_light;    /* row-range units of the numeric pass (small/large) */
   int64_t units_heavy;
   int64_t nnz_main;       /* outputs written by the row-range-unit kernels */

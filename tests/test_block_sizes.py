@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import combblas_amd as cb
+from combblas_amd import predictor
 
 CSRC = Path(__file__).resolve().parents[1] / "combblas_amd" / "csrc"
 GB = 1 << 30
@@ -139,3 +140,37 @@ def test_product_that_does_not_fit_leaves_nothing():
             h.release()
         cb.release_cached_memory()
     assert _free() >= before - GB // 64
+
+
+@pytest.mark.gpu
+def test_learned_pass_is_not_begun_where_its_staging_area_does_not_fit():
+    """Beside the output, that is: the pass would be done and then done again."""
+    A = cb.gen_rmat(18, 16).to_device()
+    base = cb.get_config()
+    held = []
+    cb.set_predictor(predictor.load())
+    try:
+        cb.set_config(learned_target=2.0)  # a pass then has units to re-run, and counts them
+        C_, st = cb.spgemm(A, A, mode="learned")
+        assert st["overflow_cols"] > 0 and st["learned_fallback"] == 0
+        staging = 12 * st["predicted_nnz"]
+        assert staging > 10 * GB
+        sums = C_.column_checksums(1)
+        C_.release()
+        cb.release_cached_memory()
+        before = _free()
+        C_, _ = cb.spgemm(A, A)
+        C_.release()
+        used = before - _free()  # by the two-phase product
+        cb.release_cached_memory()
+        held = leave(used + 2 * GB)
+        C_, st = cb.spgemm(A, A, mode="learned")
+        assert st["learned_fallback"] == 1 and st["overflow_cols"] == 0
+        assert np.array_equal(C_.column_checksums(1), sums)
+        C_.release()
+    finally:
+        cb.set_predictor(None)
+        cb.set_config(**base)
+        for h in held:
+            h.release()
+        cb.release_cached_memory()
