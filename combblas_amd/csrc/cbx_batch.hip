@@ -239,18 +239,50 @@ __global__ __launch_bounds__(256) void k_unpack_cols(const OutSeg* __restrict__ 
 // (three passes up to 2^24 rows; seven over (row, column) keys of 64 bits took
 // 0.43 ms for 4.7 M entries, these 0.20).  The payload is the entry's place
 // and column.  G lanes take a column (a wave per column of 8 entries waited for
-// its cp: 0.11 ms, now 0.02).
+// its cp: 0.11 ms, now 0.02), up to 64 entries of it; the wave takes the rest of
+// its longer columns together, four loads of a lane in flight.  (With sixteen
+// lanes on the longest of R-MAT s18's columns, 15,803 entries where the mean is
+// 26, the transpose took 0.65 ms; with a wave per column, one load in flight,
+// 0.61; so 0.39.)
 template <int G>
-__global__ void k_entry_keys(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc,
-                             const int64_t* __restrict__ ir, int64_t nzc, uint32_t* __restrict__ key,
-                             uint64_t* __restrict__ from) {
-  const int64_t q = (global_wave() * kWave + lane_id()) / G;
-  if (q >= nzc) return;
-  const uint64_t c = (uint64_t)jc[q];
-  const int64_t end = cp[q + 1];
-  for (int64_t e = cp[q] + lane_id() % G; e < end; e += G) {
+__global__ __launch_bounds__(256) void k_entry_keys(const int64_t* __restrict__ cp, const int64_t* __restrict__ jc,
+                                                    const int64_t* __restrict__ ir, int64_t nzc,
+                                                    uint32_t* __restrict__ key, uint64_t* __restrict__ from) {
+  const int lane = lane_id();
+  const int64_t q = (global_wave() * kWave + lane) / G;
+  int64_t b = 0, end = 0;
+  uint32_t c = 0;
+  if (q < nzc) {
+    b = cp[q];
+    end = cp[q + 1];
+    c = (uint32_t)jc[q];
+  }
+  const int64_t own = min(end, b + kWave);
+  for (int64_t e = b + lane % G; e < own; e += G) {
     key[e] = (uint32_t)ir[e];
     from[e] = ((uint64_t)e << 32) | c;
+  }
+  unsigned long long more = __ballot(lane % G == 0 && own < end);
+  while (more) {
+    const int l = __ffsll(more) - 1;
+    more &= more - 1;
+    const int64_t e1 = readlane_ll(end, l);
+    const uint64_t col = (uint32_t)__builtin_amdgcn_readlane((int)c, l);
+    constexpr int U = 4;
+    for (int64_t e0 = readlane_ll(own, l); e0 < e1; e0 += U * kWave) {
+      int64_t r[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) r[u] = ir[min(e0 + u * kWave + lane, e1 - 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) pin(r[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t e = e0 + u * kWave + lane;
+        if (e >= e1) continue;
+        key[e] = (uint32_t)r[u];
+        from[e] = ((uint64_t)e << 32) | col;
+      }
+    }
   }
 }
 
