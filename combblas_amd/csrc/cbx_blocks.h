@@ -5,6 +5,7 @@
 #include <cstddef>
 #include <map>
 #include <unordered_map>
+#include <vector>
 
 namespace cbx {
 
@@ -29,44 +30,49 @@ class BlockLists {
     int device;
     size_t bytes;
   };
+  struct Idle {
+    std::multimap<size_t, void*> blocks;
+    size_t bytes = 0;
+  };
   std::unordered_map<void*, Block> live_;
-  std::map<int, std::multimap<size_t, void*>> idle_;
-  std::map<int, size_t> idle_bytes_;
+  std::vector<Idle> idle_;  // by device
 
  public:
   // An idle block of the device for `bytes`, not much larger; null if there is none.
   void* take(int device, size_t bytes) {
-    auto& blocks = idle_[device];
-    const auto it = blocks.lower_bound(bytes);
-    if (it == blocks.end() || it->first > bytes + bytes / 4 + (1u << 20)) return nullptr;
+    if ((size_t)device >= idle_.size()) return nullptr;
+    Idle& d = idle_[(size_t)device];
+    const auto it = d.blocks.lower_bound(bytes);
+    if (it == d.blocks.end() || it->first > bytes + bytes / 4 + (1u << 20)) return nullptr;
     void* p = it->second;
     live_[p] = Block{device, it->first};
-    idle_bytes_[device] -= it->first;
-    blocks.erase(it);
+    d.bytes -= it->first;
+    d.blocks.erase(it);
     return p;
   }
   // A block newly allocated on the device.
-  void add(void* p, int device, size_t bytes) { live_[p] = Block{device, bytes}; }
+  void add(void* p, int device, size_t bytes) {
+    if ((size_t)device >= idle_.size()) idle_.resize((size_t)device + 1);
+    live_[p] = Block{device, bytes};
+  }
   // A block in use becomes idle; false if p is none.
   bool give_back(void* p) {
     const auto it = live_.find(p);
     if (it == live_.end()) return false;
-    idle_[it->second.device].emplace(it->second.bytes, p);
-    idle_bytes_[it->second.device] += it->second.bytes;
+    Idle& d = idle_[(size_t)it->second.device];
+    d.blocks.emplace(it->second.bytes, p);
+    d.bytes += it->second.bytes;
     live_.erase(it);
     return true;
   }
-  size_t idle_bytes(int device) const {
-    const auto it = idle_bytes_.find(device);
-    return it == idle_bytes_.end() ? 0 : it->second;
-  }
+  size_t idle_bytes(int device) const { return (size_t)device < idle_.size() ? idle_[(size_t)device].bytes : 0; }
   // Every idle block to f, and off the lists.
   template <class F>
   void release(F&& f) {
-    for (auto& d : idle_)
-      for (auto& b : d.second) f(b.second);
-    idle_.clear();
-    idle_bytes_.clear();
+    for (Idle& d : idle_) {
+      for (auto& b : d.blocks) f(b.second);
+      d = Idle{};
+    }
   }
 };
 
