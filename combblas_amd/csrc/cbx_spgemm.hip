@@ -999,8 +999,15 @@ __device__ __forceinline__ void tiny_sort(L& ws, int D) {
   }
 }
 
+// Six waves per SIMD, as its LDS allows, where the compiler would stop at 81
+// VGPRs and five (FP64 min-plus, whose NaN rule is live to the end).
 template <int K, class T, bool SYM>
-__global__ __launch_bounds__(256) void k_tiny(const int32_t* __restrict__ order, int64_t first, int64_t ncols,
+struct TinyWavesPerSimd {
+  static constexpr int value = K == kMinPlus && std::is_same<T, double>::value && !SYM ? 6 : 1;
+};
+
+template <int K, class T, bool SYM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TinyWavesPerSimd<K, T, SYM>::value))) void k_tiny(const int32_t* __restrict__ order, int64_t first, int64_t ncols,
                                               const int64_t* __restrict__ cpB, const int32_t* __restrict__ bpos,
                                               const T* __restrict__ valB, const int64_t* __restrict__ cpA,
                                               const int32_t* __restrict__ rowsA, const T* __restrict__ valA,
