@@ -1573,10 +1573,11 @@ __global__ __launch_bounds__(NT) void k_num_dense(const int32_t* __restrict__ or
 // takes ranks from the list instead of a bitmap.
 //
 // Eight waves per SIMD: the pass is latency-bound on its gathers, so the
-// kernel asks for 64 VGPRs (six of its values spill to scratch) and keeps
-// its LDS under 40 KB (the unit staging lives in the bitmap, idle while a
-// pass is cut), four workgroups per CU.  At the compiler's own choice (80
-// VGPRs, 47 KB: six waves) the pass took 64 ms at R-MAT s20, here 55.7 ms.
+// kernel asks for 64 VGPRs at most (it takes 55, and 60 with seven waves if
+// left alone) and keeps its LDS under 40 KB (the unit staging lives in the
+// bitmap, idle while a pass is cut), four workgroups per CU.  At R-MAT s20 it
+// takes 30.9 ms; before the products were flattened by bitmaps, 55.7, and 64
+// with the 80 VGPRs, 47 KB and six waves of then.
 template <int NT, int U, int IBLK>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_sym_units(
     const int32_t* __restrict__ order, int64_t first,
@@ -1715,8 +1716,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void
     __syncthreads();
     const int pass_total = bpre[nblk - 1];
     if (threadIdx.x == 0) {
-      // greedy cut into units (a single block never exceeds kBR <= kmax);
-      // a small-unit pass with its list written is cut by count alone
+      // greedy cut into units of at most kmax outputs (a unit of one block may
+      // have more, up to kBR: it is direct, its rows fit the value window); a
+      // small-unit pass with its list written is cut by count alone
       const bool heavy = pass_total > heavy_thr;
       const bool by_list = !heavy && listok;
       const int kmax = heavy ? kmax_h : kmax_l, rblk = heavy ? rblk_h : rblk_l;
@@ -2001,8 +2003,8 @@ __device__ __forceinline__ void unit_emit(bool direct, int nw32, int cnt, const 
 // registers between the sweeps, so sweep 2 re-reads nothing for them.
 // Waves per SIMD the small-unit kernel asks for, as many as its LDS allows:
 // eight for a value window of at most 16 KB (4-byte accumulators; 64 VGPRs),
-// else six (three 512-thread workgroups of 51 KB; 80 VGPRs).  Left alone, the
-// compiler keeps 81, and a third workgroup stays out.
+// else six (three 512-thread workgroups of 53 KB; 80 VGPRs).  Left alone, the
+// compiler takes 84 to 86 for 8-byte values, and a third workgroup stays out.
 template <class Lds, int NT, int DR>
 struct UnitWaves {
   static constexpr int value = NT != 512 ? 1 : sizeof(Lds) * DR <= 16384 ? 8 : 6;
@@ -2964,7 +2966,7 @@ constexpr int kDenseTR = 32 * kDenseNT;       // rows per numeric tile (16384)
 constexpr int kSymNT = 512;
 constexpr int kSymRBW = 32768;                // bitmap words per symbolic pass (2^20 rows)
 // unit tier
-constexpr int kSymUnitNT = 512, kSymUnitIBLK = 64;  // 32 KB bitmap: three workgroups per CU
+constexpr int kSymUnitNT = 512, kSymUnitIBLK = 64;  // 32 KB bitmap (38 KB in all): four workgroups per CU
 constexpr int kSymBandNT = 256;                     // banded symbolic pass
 // Light units: at most 16 blocks (64K rows) and 3264 outputs, whose 8-byte
 // accumulators and 16-bit rows share the 32 KB of a direct unit's 4096 rows:
@@ -2972,6 +2974,7 @@ constexpr int kSymBandNT = 256;                     // banded symbolic pass
 // Heavy units: 13056 outputs or 16384 direct rows, 128 KB.
 constexpr int kLightNT = 512, kLightK = 3264, kLightDR = 4096, kLightRB = 16;
 constexpr int kHeavyNT = 1024, kHeavyK = 13056, kHeavyDR = 16384, kHeavyRB = 16;
+static_assert(kLightDR >= kBR && kHeavyDR >= kBR, "a unit of one block is direct, whatever its outputs");
 // learned units: the light units' workgroup shape and window, cut to
 // target * 3264 predicted outputs.  One round of products stays in registers
 // between the sweeps: two spill at the 80 registers of three workgroups per CU
@@ -3089,7 +3092,7 @@ struct LearnedInfo {
 };
 
 // Learned single pass for the unit-tier columns (see the learned tier above).
-// On entry nnzcol holds the exact sizes of the hash-tier columns (0 for the
+// On entry nnzcol holds the exact sizes of the sort- and tiny-tier columns (0 for the
 // rest).  On success C->ir / C->val are allocated and the unit-tier outputs
 // written, nnzcol holds every column's size and cpC its exclusive scan.
 template <int K, class T>
@@ -3164,7 +3167,7 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
   // columns predicted heavy: exact sizes from the symbolic unit pass (their
   // units then go through the two-phase unit kernels), so the single pass
   // covers the many light columns and its outputs are placed around the heavy columns'
-  // sizes up front, like the hash tier's
+  // sizes up front, like the sort tier's
   int64_t hash_only = 0;
   {
     size_t need = 0, need2 = 0;
@@ -3180,7 +3183,7 @@ static cbx_status learned_numeric(const cbx_dcsc* A, const cbx_dcsc* B, const Sp
     CBX_HIP(hipMemcpyAsync(&hash_only, nh_dev, sizeof(int64_t), hipMemcpyDeviceToHost, s));
     CBX_HIP(hipcub::DeviceSelect::Flagged(t2, tb2, hipcub::CountingInputIterator<int32_t>(0), heavy_flag, hcols,
                                           nh_dev, (int)nzcB, s));
-    CBX_HIP(hipStreamSynchronize(s));  // b_tmp2 is released at scope exit
+    CBX_HIP(hipStreamSynchronize(s));  // hash_only
   }
   int64_t nheavy = 0;
   CBX_HIP(hipMemcpyAsync(&nheavy, nh_dev, sizeof(int64_t), hipMemcpyDeviceToHost, s));

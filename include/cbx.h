@@ -45,7 +45,13 @@ enum {
  *               multiply = inf_plus, saturating at numeric_limits<T>::max()
  *               (Semirings.h:40-47).
  *   SELECT_MAX  SelectMaxSRing<T,T>   (Semirings.h:165-190): add = max,
- *               multiply = a*b. */
+ *               multiply = a*b.
+ * Floating-point min and max take infinities as numbers.  An entry with one
+ * product has that product, NaN too; an entry all of whose products are NaN is
+ * NaN.  Among several, NaN is passed over, except that the add keeps one that
+ * comes first (min(a, b) = b < a ? b : a) where products are few: in columns of
+ * at most tiny_flop products, most merges among them, in cbx_dcsc_from_coo and
+ * for cbx_spmv_dense's y. */
 typedef int32_t cbx_semiring;
 enum { CBX_SR_PLUS_TIMES = 0, CBX_SR_MIN_PLUS = 1, CBX_SR_SELECT_MAX = 2 };
 
